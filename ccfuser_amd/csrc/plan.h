@@ -81,9 +81,11 @@ __host__ __device__ inline int skinny_m_tiles(int r, int limit) {
 constexpr int kSkinnyMaxWgs = 4;                     // per XCD
 constexpr int kSkinnyHead = 8;                       // header integers in front of the entries
 __host__ __device__ inline size_t skinny_ints(int max_rows, int E, int n_tiles_n) {
-  const int by_rows = (max_rows + kSkinnyRows - 1) / kSkinnyRows;
-  const int most = 2 * E < by_rows ? 2 * E : by_rows;  // at most two skinny M tiles per expert
-  return kSkinnyHead + 4 * static_cast<size_t>(most > 0 ? most : 0) * n_tiles_n;
+  // An expert with any row may have a skinny M tile, and a second one from kSkinnyRows + 1 rows on: a few rows per
+  // expert make as many M tiles as there are experts, however few rows that is in all.
+  const int ones = E < max_rows ? E : max_rows, twos = max_rows / (kSkinnyRows + 1);
+  const int most = ones + (twos < E ? twos : E);
+  return kSkinnyHead + 4 * static_cast<size_t>(most < 2 * E ? most : 2 * E) * n_tiles_n;
 }
 
 // n / d for 0 <= n < 2^24, d > 0 and a quotient below 2^22 (every count a plan divides is far below: at

@@ -547,6 +547,36 @@ def test_fused_layer_random_shapes(T, d, f, E, k, cap, seed):
     assert torch.equal(fused, _staged_forward(ops, args, E, k, cap))
 
 
+@pytest.mark.parametrize("T,d,f,E,k", [(1, 256, 1024, 8, 2), (2, 512, 512, 8, 2), (48, 256, 1024, 16, 2),
+                                       (97, 1024, 256, 32, 2), (130, 256, 512, 4, 2), (64, 320, 832, 32, 1)])
+def test_fused_layer_with_a_few_rows_per_expert(T, d, f, E, k):
+    """Fewer rows than 64 per expert: every expert is a skinny M tile of its own, more of them than
+    64-row blocks fit the rows (the list of skinny tiles is sized by experts, not by rows).  Against
+    the oracle, the staged path bit for bit, and a second call bit for bit."""
+    from ccfuser_amd import ops
+    _say(f"few rows per expert T={T} d={d} f={f} E={E} k={k}")
+    g = torch.Generator().manual_seed(100 * T + d)
+
+    def r(*s, std=1.0):
+        return (torch.randn(*s, generator=g) * std).half()
+
+    t = {"x": r(T, d), "wg": r(E, d, std=0.05), "bg": r(E, std=0.02), "w1": r(E, f, d, std=0.02), "b1": r(E, f, std=0.02),
+         "w2": r(E, d, f, std=0.02), "b2": r(E, d, std=0.02)}
+    args = [v.cuda() for v in t.values()]
+    out, routing = ops.moe_forward(*args, k, return_routing=True)
+    torch.cuda.synchronize()
+    ref = O.moe_layer_forward(*t.values(), k, capacity=-1)
+    assert torch.equal(routing["counts"].cpu(), ref["counts"])
+    assert O.max_abs_err(out.cpu(), ref["out"]) <= MAX_ABS and O.mean_rel_err(out.cpu(), ref["out"]) <= MEAN_REL
+    assert torch.equal(out, ops.moe_forward(*args, k))
+    x, wg, bg, w1, b1, w2, b2 = args
+    idx, score = ops.gate_topk_softmax(x, wg, bg, k)
+    m = ops.route(idx.view(-1), E, k)
+    h = ops.ffn1(x, m["src_row"], m["offsets"], T * k, w1, b1)
+    y = ops.ffn2(h, m["dst_row"], m["offsets"], T * k, w2, b2, torch.empty(T * k, d, dtype=torch.float16, device="cuda"))
+    assert torch.equal(out, ops.combine(y, score.view(-1), k, m["inv_pos"]))
+
+
 def _forced_plan_cases(count, seed):
     g = torch.Generator().manual_seed(seed)
     ri = lambda lo, hi: int(torch.randint(lo, hi + 1, (1,), generator=g))
