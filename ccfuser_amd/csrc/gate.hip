@@ -598,56 +598,186 @@ gate_stream_kernel(const half_t *__restrict__ x, const half_t *__restrict__ wg, 
   }
 }
 
-// fp32 gate on the vector unit, one wavefront per token: a lane takes one (expert, part)
-// pair at a time and walks the part in ascending K, multiply and add rounded separately;
-// lanes then add each expert's part sums in order.  The logits of the token wait in LDS
-// for the selection.
-__global__ void __launch_bounds__(64)
+// fp32 gate on the vector unit.  Each product is rounded before it is added, which no MFMA does, so the floor is
+// two vector instructions per product: 8192 tokens x 64 experts x 2048 are 33.6 M wavefront instructions, 33 K per
+// SIMD, ~40 us at the issue rate of a few wavefronts per SIMD.  What the kernel has to do is feed them:
+//
+// * A wavefront computes a tile of 8 TT tokens x 8 EE experts over one part of K (lane l: tokens l / 8 + 8 i,
+//   experts l % 8 + 8 j), so four K elements of TT + EE rows read from LDS feed 8 TT EE instructions (12 reads for
+//   256 at the full tile).  The wavefronts of a workgroup take different parts of the same tile.
+// * Operands come in stages of 16 K elements: four lanes per row fetch its 64 bytes a stage ahead into registers,
+//   which go into the other half of the wavefront's own LDS behind the stage's arithmetic: no barrier in the loop.
+// * Rows are 80 bytes apart: the eight rows that a read touches start 20 banks apart, none in conflict.
+// * Behind a round of parts their sums meet in LDS and are added in ascending order onto the running sums.
+//
+// TT shrinks with the tokens, so that there is a workgroup per CU from 2048 tokens on, EE with the experts.
+// 8192 tokens x 2048, 64 experts, top-2: 66 us, 988 us as one wavefront per token whose lanes each walked
+// rows of their own (and left the selection to one lane).
+constexpr int kF32StageK = 16;                     // K elements of a stage
+constexpr int kF32Row = kF32StageK + 4;            // row stride in LDS, floats
+
+template <int TT, int EE>
+struct GateF32Tile {
+  static constexpr int WT = 8 * TT, WE = 8 * EE;   // tokens and experts of a tile
+  static constexpr int ROWS = WT + WE;
+  static constexpr int LOADS = (ROWS + 15) / 16;   // 16 rows per load instruction of a wavefront
+  static constexpr int BUF = LOADS * 16 * kF32Row; // one stage, floats
+  static constexpr int LD = WE + 1;                // row stride of the part sums and of the logits
+  static constexpr int REGION = 2 * BUF > WT * LD ? 2 * BUF : WT * LD;   // a wavefront's LDS, floats
+};
+
+template <int KS>
+__device__ inline void gate_f32_select(const float *row, int e0, int ne, int k, Best<KS> &best) {
+  for (int e = 0; e < ne; ++e) best.offer(row[e], e0 + e, k);
+}
+
+template <int TT, int EE, int KS>
+__global__ void __launch_bounds__(kMaxWaves * 64)
 gate_f32_kernel(const float *__restrict__ x, const float *__restrict__ wg, const float *__restrict__ bg,
-                int tokens, int d, int E, int k, int group, int64_t *__restrict__ idx_out,
+                int tokens, int d, int E, int k, int64_t *__restrict__ idx_out,
                 float *__restrict__ score_out, float *__restrict__ logits_out) {
 #pragma clang fp contract(off)
+  using C = GateF32Tile<TT, EE>;
   extern __shared__ float s_mem[];
-  const int lane = threadIdx.x;
+  const int waves = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  float *region = s_mem + static_cast<size_t>(wave) * C::REGION;
+  float *s_logit = s_mem + static_cast<size_t>(waves) * C::REGION;       // [WT][LD] running sums, then logits
+  const int t0 = blockIdx.x * C::WT;
   const int nparts = (d + kPart - 1) / kPart;
-  float *s_logit = s_mem;                          // [E]
-  float *s_part = s_mem + E;                       // [group][nparts]: `group` experts at a time
-  const int t = blockIdx.x;
-  const float *xrow = x + static_cast<size_t>(t) * d;
-  for (int e0 = 0; e0 < E; e0 += group) {
-    const int ne = (E - e0) < group ? (E - e0) : group;
-    for (int q = lane; q < ne * nparts; q += kWave) {   // part fastest: neighbours read neighbouring K
-      const int e = e0 + q / nparts, p = q % nparts;
-      const float *wrow = wg + static_cast<size_t>(e) * d;
-      const int k_end = (p + 1) * kPart < d ? (p + 1) * kPart : d;
-      float acc = 0.0f;
-      for (int kk = p * kPart; kk < k_end; kk += 4) {
-        const float4v xv = *reinterpret_cast<const float4v *>(xrow + kk);
-        const float4v wv = *reinterpret_cast<const float4v *>(wrow + kk);
+  const int l_row = lane >> 2, l_piece = lane & 3;                       // as a loader
+  const int my_t = lane >> 3, my_e = lane & 7;                           // as a reader
+  Best<KS> best;
+  best.clear();
+  for (int e0 = 0; e0 < E; e0 += C::WE) {
+    // rows of this lane's loads: the tile's tokens, then its experts (past the end: a repeated row, never used)
+    const float *src[C::LOADS];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float prod = xv[j] * wv[j];
-          acc = acc + prod;
+    for (int i = 0; i < C::LOADS; ++i) {
+      const int r = 16 * i + l_row;
+      const int t = t0 + r < tokens ? t0 + r : tokens - 1;
+      int e = e0 + r - C::WT;
+      e = e < 0 ? 0 : (e < E ? e : E - 1);
+      src[i] = (r < C::WT ? x + static_cast<size_t>(t) * d : wg + static_cast<size_t>(e) * d) + l_piece * 4;
+    }
+    for (int p0 = 0; p0 < nparts; p0 += waves) {
+      const int part = p0 + wave;
+      float acc[TT][EE];
+#pragma unroll
+      for (int i = 0; i < TT; ++i)
+#pragma unroll
+        for (int j = 0; j < EE; ++j) acc[i][j] = 0.0f;
+      if (part < nparts) {                                               // uniform per wavefront
+        const int k_lo = part * kPart;
+        const int k_hi = k_lo + kPart < d ? k_lo + kPart : d;
+        float4v reg[C::LOADS];
+        // K past the part's end reads as zero, which adds nothing (a running sum is never -0)
+        auto fetch = [&](int kk) {
+          const bool in = kk + l_piece * 4 < k_hi;                       // d is a multiple of 8
+#pragma unroll
+          for (int i = 0; i < C::LOADS; ++i) {
+            const float4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            reg[i] = in ? *reinterpret_cast<const float4v *>(src[i] + kk) : zero;
+          }
+        };
+        auto park = [&](float *buf) {
+#pragma unroll
+          for (int i = 0; i < C::LOADS; ++i)
+            *reinterpret_cast<float4v *>(buf + (16 * i + l_row) * kF32Row + l_piece * 4) = reg[i];
+        };
+        fetch(k_lo);
+        park(region);
+        int half = 0;
+        for (int kk = k_lo; kk < k_hi; kk += kF32StageK) {
+          const bool more = kk + kF32StageK < k_hi;
+          if (more) fetch(kk + kF32StageK);
+          const float *buf = region + half * C::BUF;
+          // four K elements at a time, the next four read from LDS ahead of their use; the empty asm keeps
+          // it at that: left alone, the compiler reads the whole stage up front and spills
+          float4v xv[2][TT], wv[2][EE];
+          auto take = [&](int c, float4v (&xr)[TT], float4v (&wr)[EE]) {
+#pragma unroll
+            for (int i = 0; i < TT; ++i) xr[i] = *reinterpret_cast<const float4v *>(buf + (my_t + 8 * i) * kF32Row + c);
+#pragma unroll
+            for (int j = 0; j < EE; ++j)
+              wr[j] = *reinterpret_cast<const float4v *>(buf + (C::WT + my_e + 8 * j) * kF32Row + c);
+          };
+          take(0, xv[0], wv[0]);
+#pragma unroll
+          for (int c = 0; c < kF32StageK / 4; ++c) {
+            asm volatile("" ::: "memory");
+            if (c + 1 < kF32StageK / 4) take(4 * (c + 1), xv[(c + 1) & 1], wv[(c + 1) & 1]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+              for (int i = 0; i < TT; ++i)
+#pragma unroll
+                for (int j = 0; j < EE; ++j) {
+                  const float prod = xv[c & 1][i][q] * wv[c & 1][j][q];
+                  acc[i][j] = acc[i][j] + prod;
+                }
+#pragma unroll
+            for (int i = 0; i < TT; ++i)
+#pragma unroll
+              for (int j = 0; j < EE; ++j) asm volatile("" : "+v"(acc[i][j]));
+          }
+          half ^= 1;
+          if (more) park(region + half * C::BUF);
         }
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+#pragma unroll
+          for (int j = 0; j < EE; ++j) region[(my_t + 8 * i) * C::LD + my_e + 8 * j] = acc[i][j];
       }
-      s_part[q] = acc;
+      __syncthreads();
+      const int np = nparts - p0 < waves ? nparts - p0 : waves;
+      const bool last = p0 + waves >= nparts;
+      for (int o = threadIdx.x; o < C::WT * C::WE; o += blockDim.x) {
+        const int t = o / C::WE, e = o % C::WE;
+        const int at = t * C::LD + e;
+        float s = p0 == 0 ? s_mem[at] : s_logit[at] + s_mem[at];
+        for (int w = 1; w < np; ++w) s = s + s_mem[static_cast<size_t>(w) * C::REGION + at];
+        if (last && e0 + e < E) {
+          if (bg) s = s + bg[e0 + e];
+          if (logits_out && t0 + t < tokens) logits_out[static_cast<size_t>(t0 + t) * E + e0 + e] = s;
+        }
+        s_logit[at] = s;
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    for (int g = lane; g < ne; g += kWave) {
-      float s = s_part[g * nparts];
-      for (int p = 1; p < nparts; ++p) s = s + s_part[g * nparts + p];
-      if (bg) s = s + bg[e0 + g];
-      s_logit[e0 + g] = s;
-      if (logits_out) logits_out[static_cast<size_t>(t) * E + e0 + g] = s;
-    }
-    __syncthreads();
+    if (threadIdx.x < C::WT)
+      gate_f32_select<KS>(s_logit + threadIdx.x * C::LD, e0, (E - e0) < C::WE ? (E - e0) : C::WE, k, best);
+    // the next tile's logits are written behind the barrier that follows its first round's part sums
   }
-  if (lane == 0) {
-    Best<kMaxTopK> best;
-    best.clear();
-    for (int e = 0; e < E; ++e) best.offer(s_logit[e], e, k);
-    best.write<float>(t, k, idx_out, score_out);
+  if (threadIdx.x < C::WT && t0 + threadIdx.x < tokens) best.template write<float>(t0 + threadIdx.x, k, idx_out, score_out);
+}
+
+template <int TT, int EE>
+int launch_gate_f32(const float *x, const float *wg, const float *bg, int tokens, int d, int E, int k, int64_t *idx_out,
+                    float *score_out, float *logits_out, hipStream_t stream) {
+  using C = GateF32Tile<TT, EE>;
+  const int nparts = (d + kPart - 1) / kPart;
+  const int waves = nparts < kMaxWaves ? nparts : kMaxWaves;
+  const size_t lds = sizeof(float) * (static_cast<size_t>(waves) * C::REGION + C::WT * C::LD);
+  static_assert(sizeof(float) * (kMaxWaves * C::REGION + C::WT * C::LD) <= 160 * 1024, "LDS of a CU");
+  auto kern = k <= 2 ? gate_f32_kernel<TT, EE, 2> : gate_f32_kernel<TT, EE, kMaxTopK>;
+  if (lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       static_cast<int>(lds));
+    if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate: LDS attribute: %s", hipGetErrorString(e));
   }
+  hipLaunchKernelGGL(kern, dim3((tokens + C::WT - 1) / C::WT), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
+                     idx_out, score_out, logits_out);
+  return check_launch("gate_f32_kernel");
+}
+
+template <int TT>
+int launch_gate_f32_experts(const float *x, const float *wg, const float *bg, int tokens, int d, int E, int k,
+                            int64_t *idx_out, float *score_out, float *logits_out, hipStream_t stream) {
+  auto launch = E <= 8 ? launch_gate_f32<TT, 1> : (E <= 16 ? launch_gate_f32<TT, 2>
+                                                           : (E <= 32 ? launch_gate_f32<TT, 4> : launch_gate_f32<TT, 8>));
+  return launch(x, wg, bg, tokens, d, E, k, idx_out, score_out, logits_out, stream);
 }
 
 }  // namespace
@@ -672,16 +802,11 @@ int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int 
   if (tokens == 0) return CCF_OK;
   const int nparts = (d_model + kPart - 1) / kPart;
   if (dtype == CCF_F32) {
-    // part sums of as many experts at a time as 32 KB hold
-    int group = 8192 / nparts;
-    group = group < 1 ? 1 : (group > tot_expert ? tot_expert : group);
-    const size_t lds = sizeof(float) * (static_cast<size_t>(tot_expert) + static_cast<size_t>(group) * nparts);
-    CCF_REQUIRE(lds <= 64 * 1024, CCF_ERR_SHAPE, "gate: fp32 d_model=%d needs %zu bytes of LDS", d_model, lds);
-    hipLaunchKernelGGL(gate_f32_kernel, dim3(tokens), dim3(64), lds, as_stream(stream),
-                       static_cast<const float *>(x), static_cast<const float *>(wg),
-                       static_cast<const float *>(bg), tokens, d_model, tot_expert, top_k, group, idx_out,
-                       static_cast<float *>(score_out), static_cast<float *>(logits_out));
-    return check_launch("gate_f32_kernel");
+    auto launch = tokens > 4096 ? launch_gate_f32_experts<4>
+                                : (tokens > 2048 ? launch_gate_f32_experts<2> : launch_gate_f32_experts<1>);
+    return launch(static_cast<const float *>(x), static_cast<const float *>(wg), static_cast<const float *>(bg), tokens,
+                  d_model, tot_expert, top_k, idx_out, static_cast<float *>(score_out), static_cast<float *>(logits_out),
+                  as_stream(stream));
   }
   // Tile and slots.  With S slots a wavefront covers 64 / S tokens, so S grows while there
   // are fewer than four workgroups per CU and K has parts for the slots.

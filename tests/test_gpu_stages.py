@@ -53,6 +53,24 @@ def test_gate_bit_exact(T, d, E, k, dtype, seed):
     assert torch.allclose(score.float().sum(-1).cpu(), torch.ones(T), atol=2e-3)
 
 
+@pytest.mark.parametrize("T,d,E,k", [(1, 8, 8, 2), (9, 136, 9, 1), (2049, 128, 16, 2), (2055, 1160, 33, 3), (4097, 256, 8, 1),
+                                     (4127, 520, 64, 2), (4100, 2048, 65, 8), (100, 128, 130, 2)])
+def test_gate_fp32_tiles(T, d, E, k):
+    """Every tile of the fp32 gate (8, 16 or 32 tokens by 8 to 64 experts), ragged in tokens and experts, with
+    fewer parts of K than wavefronts, more, and a short last part: the oracle's bits."""
+    from ccfuser_amd import ops
+    _say(f"fp32 gate T={T} d={d} E={E} k={k}")
+    g = torch.Generator().manual_seed(T + d + E)
+    x, wg, bg = torch.randn(T, d, generator=g), torch.randn(E, d, generator=g) * 0.05, torch.randn(E, generator=g) * 0.05
+    idx_ref, score_ref, logits_ref = O.naive_gate(x, wg, bg, k)
+    idx, score, logits = ops.gate_topk_softmax(dev(x), dev(wg), dev(bg), k, return_logits=True)
+    assert torch.equal(logits.cpu(), logits_ref), "logits differ bitwise"
+    assert torch.equal(idx.cpu(), idx_ref), "expert choice differs"
+    assert torch.allclose(score.cpu(), score_ref, rtol=1e-5, atol=1e-7)
+    idx2, _ = ops.gate_topk_softmax(dev(x), dev(wg), None, k)
+    assert torch.equal(idx2.cpu(), O.naive_gate(x, wg, None, k)[0])
+
+
 _GATE_CASES = {}
 
 
