@@ -595,10 +595,13 @@ __device__ __forceinline__ void skinny_tail_role(const GroupedArgs &p, int w, in
     skinny_mainloop<kKN>(p, list[t], k0, k1 - k0, acc, a_off, b_off, tid, lds, lds_base);
     float4v *out = reinterpret_cast<float4v *>(p.sk_partial) +
                    static_cast<size_t>(w * kSkTailSegs + seg) * (C::TM * C::TN * 256) + tid;
+    const int rows = __builtin_amdgcn_readfirstlane(list[t][2]);
 #pragma unroll
-    for (int tm = 0; tm < C::TM; ++tm)
+    for (int tm = 0; tm < C::TM; ++tm) {
+      if (tm * 16 >= rows) break;                    // row blocks without real rows are not read back
 #pragma unroll
       for (int tn = 0; tn < C::TN; ++tn) out[(tm * C::TN + tn) * 256] = acc[tm][tn];
+    }
   }
   wait_vmcnt<0>();
   block_barrier();                                   // every wavefront is done with LDS before a caller's next tile loads
@@ -935,6 +938,7 @@ grouped_gemm_persistent_kernel(GroupedArgs p, int slots_per_xcd) {
       const int tid = fresh_tid();
       static_for<0, TM>([&](auto T) {
         constexpr int tm = T.value;
+        if (tm >= live_m) return;                     // uniform; row blocks without real rows are not read back
         const int tr = acc16_row<Cfg>(tm, tid);
         static_for<0, TN>([&](auto J) {
           constexpr int tn = J.value;
@@ -1049,6 +1053,7 @@ __device__ __forceinline__ void reduce_split_tile(const GroupedArgs &p, int t, i
   const int4v ent = reinterpret_cast<const int4v *>(p.tail + 64)[first_wg];
   const int e = ent[0], row0 = ent[1], rows = ent[2], n0 = (ent[3] & 0xffff) * Cfg::BN;
   if (e < 0) return;
+  if (!R::row_is_real(blockIdx.y * 16, rows)) return;  // a row block's first row is real if any of them is
   const int c4 = threadIdx.x & 63;                     // which group of four columns
   const int col = n0 + 4 * c4;
   if (col >= p.N) return;
@@ -1270,10 +1275,14 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   g.grid = persistent ? cus : 0;
   // the last, partly filled round is cut along K and spread over all workgroups (forward forms;
   // worth its two small launches only where a tile is long: K of 4096 and more)
-  g.split = opt.split_tail && (b_kn ? epi == kEpiPlain : epi <= kEpiGeluKeep) && g.grid >= 8 && g.grid <= g.wgs &&
+  // A launch with a split round or skinny tiles has all CUs' workgroups, also where the plan has fewer entries: few
+  // tiles are where cutting them along K pays most.  One token, top-2 of 8 experts, 4096 / 14336: FFN2's 32 tiles
+  // 235 us on 32 workgroups, 52 us cut over 256.
+  g.split = opt.split_tail && (b_kn ? epi == kEpiPlain : epi <= kEpiGeluKeep) && g.grid >= 8 &&
             g.grid <= kTailMaxParts && v.bm == Cfg5::BM && v.bn == Cfg5::BN && K / 64 >= opt.split_tail_min_kt;
   // remainder rows as skinny tiles: forward epilogues of the persistent 256 x 256 kernel (either weight layout)
-  g.skinny = opt.skinny_pct != 0 && (b_kn ? epi == kEpiPlain && N % 256 == 0 : epi <= kEpiGeluKeep) && g.grid >= 64 && g.grid <= g.wgs &&
+  g.skinny = opt.skinny_pct != 0 && (b_kn ? epi == kEpiPlain && N % 256 == 0 : epi <= kEpiGeluKeep) && g.grid >= 64 &&
+             (g.grid <= g.wgs || K / 64 >= opt.split_tail_min_kt) &&   // few short tiles: not worth the reduction launch
              v.bm == Cfg5::BM && v.bn == Cfg5::BN && v.persistent_plain && (!wide || g.split);
   // skinny tiles may be cut along K (partial tiles in the split scratch, summed by the reduction launch) at any K,
   // also where the last round of 256-row tiles is not split
@@ -1348,7 +1357,8 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
   p.zero_row = nullptr;
   p.skinny = gs.skinny ? gs.skinny_list : nullptr;
   if (grid >= 8) {
-    const long long g = grid < wgs ? grid : wgs;                // wgs is a multiple of 8
+    // one workgroup per CU; without parts or skinny tiles to share out, none without a plan entry (wgs is a multiple of 8)
+    const long long g = (split || gs.skinny || grid < wgs) ? grid : wgs;
     // the parts of a split last round: run by the persistent workgroups themselves behind their tiles (the
     // four-wavefront kernels; part i is workgroup i's), else by a launch of their own
     const bool parts_inside = split && g_split_inside && gs.v != &kVariants[kFwd8Variant];

@@ -577,6 +577,39 @@ def test_fused_layer_with_a_few_rows_per_expert(T, d, f, E, k):
     assert torch.equal(out, ops.combine(y, score.view(-1), k, m["inv_pos"]))
 
 
+@pytest.mark.parametrize("counts", [[1], [5, 0, 70], [300, 17, 129, 64], [0, 513, 0, 256]])
+def test_few_tiles_of_a_long_contraction(counts):
+    """Fewer plan entries than compute units, each a contraction over 4160: cut along K over all of them, as
+    skinny tiles or as the split last round.  Both products, the pre-activation form and the input gradient on
+    the stored [K][N] weight, against fp32 (fp16 results of sums of 4160 products of order 1e-2: half an fp16
+    step of the result, 2^-11, plus 4160 * 2^-24 relative for the order of the sums)."""
+    from ccfuser_amd import ops
+    _say(f"few tiles, counts={counts}")
+    E, n, K, N = len(counts), sum(counts), 4160, 256
+    g = torch.Generator().manual_seed(n)
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    a = torch.randn(n, K, generator=g).half().cuda()
+    w = (torch.randn(E, N, K, generator=g) * 0.02).half().cuda()
+    b = torch.randn(E, N, generator=g).half().cuda()
+    e_of = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ref = torch.cat([a[e_of.cuda() == e].float() @ w[e].float().t() + b[e].float() for e in range(E)])
+
+    def close(got, want):
+        assert float((got.float() - want).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(want.abs().max()) + 1e-4
+
+    y = ops.ffn2(a, None, off, n, w, b, torch.empty(n, N, dtype=torch.float16, device="cuda"))
+    close(y, ref)
+    assert torch.equal(y, ops.ffn2(a, None, off, n, w, b, torch.empty_like(y)))
+    close(ops.ffn1(a, None, off, n, w, b), torch.nn.functional.gelu(ref))
+    act, pre = ops.ffn1_keep(a, None, off, n, w, b)
+    close(pre, ref)
+    close(act, torch.nn.functional.gelu(ref))
+    w1 = (torch.randn(E, K, N, generator=g) * 0.02).half().cuda()          # [out = 4160, in = 256]
+    x = torch.randn(n, N, generator=g).half().cuda()
+    gx, _, _ = ops.ffn1_backward(a, x, None, None, off, n, w1, n)
+    close(gx, torch.cat([a[e_of.cuda() == e].float() @ w1[e].float() for e in range(E)]))
+
+
 def _forced_plan_cases(count, seed):
     g = torch.Generator().manual_seed(seed)
     ri = lambda lo, hi: int(torch.randint(lo, hi + 1, (1,), generator=g))
