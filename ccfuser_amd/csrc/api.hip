@@ -103,6 +103,28 @@ SegWs carve_seg(void *ws, int total_rows, int d, int f, int E) {
   return w;
 }
 
+struct BlocksWs {
+  int32_t *counts, *offsets, *token_rows, *flat_rows;
+  char *ffn_ws;
+  size_t ffn_bytes;
+  half_t *h;
+  size_t total;
+};
+
+BlocksWs carve_blocks(void *ws, int rows, int d, int f, int E) {
+  Carver c(ws);
+  BlocksWs w;
+  w.counts = c.take<int32_t>(E);
+  w.offsets = c.take<int32_t>(E + 1);
+  w.token_rows = c.take<int32_t>(rows);
+  w.flat_rows = c.take<int32_t>(rows);
+  w.ffn_bytes = ccf_ffn_workspace_bytes(rows, E, d, f);
+  w.ffn_ws = c.take<char>(w.ffn_bytes);
+  w.h = c.take<half_t>(static_cast<size_t>(rows) * f);
+  w.total = c.used;
+  return w;
+}
+
 // Optional per-stage timing: events recorded on the layer's stream before the
 // gate and after each of the five stages of the next ccf_moe_forward calls
 // (ccf_moe_ffn_segments records the same six; its gate and combine stages are empty).
@@ -263,4 +285,45 @@ extern "C" int ccf_moe_ffn_segments(const void *x, const int32_t *seg_start, con
   mark_stage(4, st);
   mark_stage(5, st);                                  // no combine either
   return rc;
+}
+
+extern "C" size_t ccf_blocks_workspace_bytes(int n_blocks, int block_size, int num_expert, int d_model, int d_ffn) {
+  if (n_blocks < 0 || block_size <= 0 || num_expert <= 0 || d_model <= 0 || d_ffn <= 0) return 0;
+  if (static_cast<long long>(n_blocks) * block_size >= (1ll << 31)) return 0;
+  return ccf::carve_blocks(nullptr, n_blocks * block_size, d_model, d_ffn, num_expert).total;
+}
+
+// _MixMOE::forward (mix_moe/csrc/mix_moe.h:507-598) from the block arrays of its planner: the rows go from the
+// tokens to the flat outputs through row indices, no padded buffer in between.
+extern "C" int ccf_moe_ffn_blocks(const void *x, int n_tokens, const int64_t *pos, int n_pos, int top_k,
+                                  const int32_t *expert_ids, const int32_t *lens, const int32_t *start_addrs,
+                                  int n_blocks, int block_size, int d_model, int d_ffn, int num_expert,
+                                  const void *w1, int w1_kn, const void *b1, const void *w2, int w2_kn, const void *b2,
+                                  void *y, void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
+  using namespace ccf;
+  if (n_blocks == 0) return CCF_OK;
+  CCF_REQUIRE(x && pos && expert_ids && lens && start_addrs && w1 && b1 && w2 && b2 && y, CCF_ERR_ARG,
+              "moe_ffn_blocks: null pointer");
+  CCF_REQUIRE(n_blocks >= 0 && block_size > 0 && num_expert > 0 && num_expert <= 1024 && top_k >= 1 && d_model > 0 && d_ffn > 0,
+              CCF_ERR_ARG, "moe_ffn_blocks: bad size");
+  CCF_REQUIRE(static_cast<long long>(n_blocks) * block_size < (1ll << 31), CCF_ERR_SHAPE, "moe_ffn_blocks: too many rows");
+  CCF_REQUIRE(n_tokens > 0 && n_pos > 0, CCF_ERR_ARG, "moe_ffn_blocks: blocks of no tokens");
+  const size_t need = ccf_blocks_workspace_bytes(n_blocks, block_size, num_expert, d_model, d_ffn);
+  CCF_REQUIRE(workspace && workspace_bytes >= need, CCF_ERR_WORKSPACE,
+              "moe_ffn_blocks: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+  const int rows = n_blocks * block_size;
+  BlocksWs w = carve_blocks(workspace, rows, d_model, d_ffn, num_expert);
+  hipStream_t st = as_stream(stream);
+  PlanReq plans[2];
+  const GemmOptions opt = forward_options();
+  const bool planned = forward_plan_request(1, rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[0], w1_kn != 0) &&
+                       forward_plan_request(2, rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[1], w2_kn != 0);
+  if (int rc = blocks_with_plans(pos, n_pos, top_k, n_tokens, expert_ids, lens, start_addrs, n_blocks, block_size,
+                                 num_expert, w.counts, w.offsets, w.token_rows, w.flat_rows, st, plans, planned ? 2 : 0))
+    return rc;
+  if (int rc = ffn1_forward(x, w.token_rows, nullptr, w.offsets, rows, num_expert, d_model, d_ffn, w1, b1, 1, w.h,
+                            w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr, w1_kn != 0))
+    return rc;
+  return ffn2_forward(w.h, nullptr, w.flat_rows, w.offsets, rows, num_expert, d_model, d_ffn, w2, b2, nullptr, y,
+                      w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr, w2_kn != 0);
 }

@@ -96,6 +96,9 @@ __device__ __forceinline__ int tile_row_to_local(int r, int rows) {
 // `ent`: K element 0 of the (clamped) A row and B row, at this lane's K chunk.
 // Padded A rows re-read the tile's last real row, B rows past N the last row.
 // tid: threadIdx.x, or fresh_tid() where what is derived from it must not be kept from an earlier call.
+// First column (of eight) that a load of a [K][N] operand fetches: past the matrix, the last eight again.
+__device__ __forceinline__ int kn_column(int c, int N) { return c < N - 8 ? c : N - 8; }
+
 template <class Cfg, bool kSeg = false, bool kKN = false>
 __device__ __forceinline__ void tile_sources(const GroupedArgs &p, const int4v ent,
                                              const half_t *(&a_src)[Cfg::A_DMA],
@@ -125,12 +128,12 @@ __device__ __forceinline__ void tile_sources(const GroupedArgs &p, const int4v e
     }
   }
   if constexpr (kKN) {
-    // B is [E, K, N]: K row r of the tile, the columns LDS unit u of that row holds (N % BN == 0)
+    // B is [E, K, N]: K row r of the tile, the columns LDS unit u of that row holds (units past N: the last one again)
     using R = RingFor<Cfg, true>;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {                          // loads 0 and 1; load i >= 2 is 16 rows below load i - 2
       const int r = R::kn_dma_row(i, tid);
-      b_src[i] = Be + static_cast<size_t>(r) * p.N + n0 + R::kn_col(r, R::kn_dma_unit(tid));
+      b_src[i] = Be + static_cast<size_t>(r) * p.N + kn_column(n0 + R::kn_col(r, R::kn_dma_unit(tid)), p.N);
     }
   } else {
 #pragma unroll
@@ -434,10 +437,10 @@ __device__ __forceinline__ void skinny_mainloop(const GroupedArgs &p, const int4
 #pragma unroll
   for (int j = 0; j < C::B_DMA; ++j) {
     if constexpr (kKN) {
-      // a load is two K rows of 256 columns (N % 256 == 0); which columns a 16-byte unit holds: the main loop's layout
+      // a load is two K rows of 256 columns; which columns a 16-byte unit holds: the main loop's layout
       using KN = SkinnyKN;
       const int r = KN::kn_dma_row(j, tid);
-      b_src[j] = Be + static_cast<size_t>(r) * p.N + n0 + KN::kn_col(r, KN::kn_dma_unit(tid));
+      b_src[j] = Be + static_cast<size_t>(r) * p.N + kn_column(n0 + KN::kn_col(r, KN::kn_dma_unit(tid)), p.N);
     } else {
       const int r = (j * 4 + wave) * 8 + (lane >> 3);
       const int n = (n0 + r) < p.N ? (n0 + r) : p.N - 1;
@@ -909,7 +912,7 @@ grouped_gemm_persistent_kernel(GroupedArgs p, int slots_per_xcd) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const int r = R::kn_dma_row(i, tid1);
-          b_src[i] = Be + (static_cast<size_t>(r) + n_k0) * p.N + n0 + R::kn_col(r, R::kn_dma_unit(tid1));
+          b_src[i] = Be + (static_cast<size_t>(r) + n_k0) * p.N + kn_column(n0 + R::kn_col(r, R::kn_dma_unit(tid1)), p.N);
         }
       } else {
 #pragma unroll
@@ -1188,8 +1191,13 @@ const Launch kVariants[] = {// forward: "plain" = bias and row scale, "gelu" = b
                              grouped_gemm_persistent_kernel<Cfg5, kEpiCombine>, nullptr},
                             // forward, eight wavefronts (persistent only)
                             {Cfg8::BM, Cfg8::BN, Cfg8::THREADS, nullptr, nullptr, grouped_gemm_persistent_kernel<Cfg8, kEpiPlain>,
-                             grouped_gemm_persistent_kernel<Cfg8, kEpiGelu>}};
-constexpr int kFwdVariant = 0, kKnVariant = 1, kTrainVariant = 2, kCombineVariant = 3, kFwd8Variant = 4;
+                             grouped_gemm_persistent_kernel<Cfg8, kEpiGelu>},
+                            // forward on weights stored [E, K, N]
+                            {Cfg5::BM, Cfg5::BN, Cfg5::THREADS, grouped_gemm_kernel<Cfg5, kEpiPlain, false, true>,
+                             grouped_gemm_kernel<Cfg5, kEpiGelu, false, true>,
+                             grouped_gemm_persistent_kernel<Cfg5, kEpiPlain, false, true>,
+                             grouped_gemm_persistent_kernel<Cfg5, kEpiGelu, false, true>}};
+constexpr int kFwdVariant = 0, kKnVariant = 1, kTrainVariant = 2, kCombineVariant = 3, kFwd8Variant = 4, kFwdKnVariant = 5;
 
 // Compute units of the current device, rounded down to whole XCD rounds of 8.
 int persistent_grid() {
@@ -1264,11 +1272,11 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   const bool persistent = opt.variant != 1 && kt_all >= kPersistentMinKT && cus >= 8;
   // eight wavefronts: the two plain forward epilogues, short K (or forced)
   const bool wide = persistent && !b_kn && epi <= kEpiGelu && (opt.variant == 3 || (opt.variant == 0 && kt_all <= kWideMaxKT));
-  g.v = &kVariants[b_kn ? kKnVariant : (epi == kEpiCombine ? kCombineVariant : (epi >= kEpiGeluKeep ? kTrainVariant :
+  g.v = &kVariants[b_kn ? (epi == kEpiGelu ? kFwdKnVariant : kKnVariant) : (epi == kEpiCombine ? kCombineVariant : (epi >= kEpiGeluKeep ? kTrainVariant :
                                                                                    (wide ? kFwd8Variant : kFwdVariant)))];
   const Launch &v = *g.v;
   // which of the entry's two kernels: the K-N and training entries hold the GELU-gradient form in the second slot
-  g.second = b_kn ? epi == kEpiGeluGrad : (epi == kEpiCombine ? false : (epi >= kEpiGeluKeep ? epi == kEpiGeluGrad : gelu));
+  g.second = b_kn ? epi != kEpiPlain : (epi == kEpiCombine ? false : (epi >= kEpiGeluKeep ? epi == kEpiGeluGrad : gelu));
   const int max_tiles = max_tiles_for(max_rows, E, v.bm);
   const int n_tiles_n = (N + v.bn - 1) / v.bn;
   g.wgs = launched_wgs(max_tiles, n_tiles_n);                   // worst-case tile count
@@ -1278,10 +1286,10 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   // A launch with a split round or skinny tiles has all CUs' workgroups, also where the plan has fewer entries: few
   // tiles are where cutting them along K pays most.  One token, top-2 of 8 experts, 4096 / 14336: FFN2's 32 tiles
   // 235 us on 32 workgroups, 52 us cut over 256.
-  g.split = opt.split_tail && (b_kn ? epi == kEpiPlain : epi <= kEpiGeluKeep) && g.grid >= 8 &&
+  g.split = opt.split_tail && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 8 &&
             g.grid <= kTailMaxParts && v.bm == Cfg5::BM && v.bn == Cfg5::BN && K / 64 >= opt.split_tail_min_kt;
   // remainder rows as skinny tiles: forward epilogues of the persistent 256 x 256 kernel (either weight layout)
-  g.skinny = opt.skinny_pct != 0 && (b_kn ? epi == kEpiPlain && N % 256 == 0 : epi <= kEpiGeluKeep) && g.grid >= 64 &&
+  g.skinny = opt.skinny_pct != 0 && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 64 &&
              (g.grid <= g.wgs || K / 64 >= opt.split_tail_min_kt) &&   // few short tiles: not worth the reduction launch
              v.bm == Cfg5::BM && v.bn == Cfg5::BN && v.persistent_plain && (!wide || g.split);
   // skinny tiles may be cut along K (partial tiles in the split scratch, summed by the reduction launch) at any K,
@@ -1309,10 +1317,12 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
               "%s: epilogue %d needs the pre-activation buffer", what, epi);
   CCF_REQUIRE(epi != kEpiCombine || (c_rows && row_scale && scale_rows && !b_kn && N % 8 == 0), CCF_ERR_ARG,
               "%s: the combine epilogue needs token rows, scores and their index", what);
-  // b_kn: B is [E, K, N] (the stored weight of the layer whose input gradient this is); Cfg5 kernels only
-  CCF_REQUIRE(!b_kn || (N % Cfg5::BN == 0 && (epi == kEpiPlain || epi == kEpiGeluGrad) &&
-                        static_cast<long long>(K) * N < (1ll << 31)), CCF_ERR_SHAPE,
-              "%s: the [K][N] weight form needs N=%d to be a multiple of %d", what, N, Cfg5::BN);
+  // b_kn: B is [E, K, N] (the stored weight of the layer whose input gradient this is, or a transposed one);
+  // Cfg5 kernels only
+  CCF_REQUIRE(!b_kn || epi == kEpiPlain || epi == kEpiGelu || epi == kEpiGeluGrad, CCF_ERR_ARG,
+              "%s: no [K][N] weight form of epilogue %d", what, epi);
+  CCF_REQUIRE(!b_kn || static_cast<long long>(K) * N < (1ll << 31), CCF_ERR_SHAPE,
+              "%s: a [K][N] weight of %d x %d is too large", what, K, N);
   CCF_REQUIRE(max_rows >= 0 && E > 0 && N > 0 && K > 0, CCF_ERR_ARG, "%s: bad size", what);
   CCF_REQUIRE(E <= 1024, CCF_ERR_SHAPE, "%s: num_expert=%d exceeds 1024", what, E);
   CCF_REQUIRE(K % 64 == 0, CCF_ERR_SHAPE, "%s: K=%d is not a multiple of 64", what, K);
@@ -1594,7 +1604,7 @@ int linear_backward(half_t *grad_out, const int32_t *g_rows, const half_t *in,
   // gelu'(pre) and writes them back, so that everything below sees the gradient of the pre-activation.
   CCF_REQUIRE(!pre_inplace || !g_rows, CCF_ERR_ARG, "%s: the in-place GELU gradient needs rows in expert order", what);
   // input gradient: on the stored weight read as [K][N] where the shape allows, else on a transposed copy
-  const bool kn = !g_dgrad_transpose && n_in % Cfg5::BN == 0 && static_cast<long long>(n_out) * n_in < (1ll << 31);
+  const bool kn = !g_dgrad_transpose && static_cast<long long>(n_out) * n_in < (1ll << 31);
   const int dgrad_epi = gelu_pre ? kEpiGeluGrad : kEpiPlain;
   // the launch that lays out the K ranges also builds the tile plans of both GEMMs
   const PlanReq rows_plan = setup_gemm(max_rows, E, n_in, n_out, dgrad_epi, kn, ws.plan_rows, 0, current_options()).req;
@@ -1725,11 +1735,11 @@ namespace ccf {
 GemmOptions forward_options() { return current_options(); }
 
 bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *workspace, const GemmOptions &opt,
-                          PlanReq *out) {
+                          PlanReq *out, bool w_kn) {
   if (!workspace || max_rows <= 0 || E <= 0 || E > 1024 || d <= 0 || f <= 0 || d % 64 || f % 64) return false;
   const int N = which == 1 ? f : d, K = which == 1 ? d : f;
   const GemmSetup gs = setup_gemm(max_rows, E, N, K, which == 1 ? kEpiGelu : (which == 3 ? kEpiCombine : kEpiPlain),
-                                  false, workspace, which == 1 ? 0 : 1, opt);
+                                  w_kn, workspace, which == 1 ? 0 : 1, opt);
   if (gs.wgs >= (1ll << 24)) return false;
   *out = gs.req;
   return true;
@@ -1738,7 +1748,7 @@ bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *wo
 int ffn1_forward(const void *x, const int32_t *src_row, const int32_t *dst_row, const int32_t *offsets,
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w1, const void *b1,
                  int apply_gelu, void *h, void *workspace, size_t workspace_bytes, hipStream_t stream,
-                 const GemmOptions *planned) {
+                 const GemmOptions *planned, bool w_kn) {
   const bool plan_ready = planned != nullptr;
   const size_t need = ccf_ffn_workspace_bytes(max_rows, num_expert, d_model, d_ffn);
   CCF_REQUIRE(workspace && workspace_bytes >= need, CCF_ERR_WORKSPACE,
@@ -1746,13 +1756,13 @@ int ffn1_forward(const void *x, const int32_t *src_row, const int32_t *dst_row, 
   return grouped_gemm(static_cast<const half_t *>(x), src_row, offsets, max_rows, num_expert, d_ffn,
                       d_model, static_cast<const half_t *>(w1), static_cast<const half_t *>(b1),
                       apply_gelu != 0 ? kEpiGelu : kEpiPlain, static_cast<half_t *>(h), dst_row, nullptr,
-                      workspace, stream, "ffn1", false, nullptr, 0, plan_ready && apply_gelu != 0, planned);
+                      workspace, stream, "ffn1", w_kn, nullptr, 0, plan_ready && apply_gelu != 0, planned);
 }
 
 int ffn2_forward(const void *h, const int32_t *src_row, const int32_t *dst_row, const int32_t *offsets,
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w2, const void *b2,
                  const void *row_scale, void *y, void *workspace, size_t workspace_bytes,
-                 hipStream_t stream, const GemmOptions *planned) {
+                 hipStream_t stream, const GemmOptions *planned, bool w_kn) {
   const bool plan_ready = planned != nullptr;
   const size_t need = ccf_ffn_workspace_bytes(max_rows, num_expert, d_model, d_ffn);
   CCF_REQUIRE(workspace && workspace_bytes >= need, CCF_ERR_WORKSPACE,
@@ -1760,7 +1770,7 @@ int ffn2_forward(const void *h, const int32_t *src_row, const int32_t *dst_row, 
   return grouped_gemm(static_cast<const half_t *>(h), src_row, offsets, max_rows, num_expert, d_model,
                       d_ffn, static_cast<const half_t *>(w2), static_cast<const half_t *>(b2), kEpiPlain,
                       static_cast<half_t *>(y), dst_row, static_cast<const half_t *>(row_scale),
-                      workspace, stream, "ffn2", false, nullptr, 1, plan_ready, planned);
+                      workspace, stream, "ffn2", w_kn, nullptr, 1, plan_ready, planned);
 }
 
 // FFN2 with the combine in its epilogue: out[token_row[j]] += (h[j] * w2[e]^T + b2[e]) * score[flat_row[j]].
@@ -1795,6 +1805,24 @@ extern "C" int ccf_ffn2_forward(const void *h, const int32_t *src_row, const int
                                 ccf_stream_t stream) {
   return ccf::ffn2_forward(h, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w2, b2,
                            row_scale, y, workspace, workspace_bytes, ccf::as_stream(stream), nullptr);
+}
+
+// The same on weights stored [E, K, N], as the reference hands them to its extension (linear.py:74, 129).
+extern "C" int ccf_ffn1_forward_kn(const void *x, const int32_t *src_row, const int32_t *dst_row,
+                                   const int32_t *offsets, int max_rows, int num_expert, int d_model,
+                                   int d_ffn, const void *w1, const void *b1, int apply_gelu, void *h,
+                                   void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
+  return ccf::ffn1_forward(x, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w1, b1,
+                           apply_gelu, h, workspace, workspace_bytes, ccf::as_stream(stream), nullptr, true);
+}
+
+extern "C" int ccf_ffn2_forward_kn(const void *h, const int32_t *src_row, const int32_t *dst_row,
+                                   const int32_t *offsets, int max_rows, int num_expert, int d_model,
+                                   int d_ffn, const void *w2, const void *b2, const void *row_scale,
+                                   void *y, void *workspace, size_t workspace_bytes,
+                                   ccf_stream_t stream) {
+  return ccf::ffn2_forward(h, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w2, b2,
+                           row_scale, y, workspace, workspace_bytes, ccf::as_stream(stream), nullptr, true);
 }
 
 extern "C" int ccf_ffn_plan_info(const void *workspace, int max_rows, int num_expert, int d_model, int d_ffn,

@@ -499,15 +499,16 @@ struct GemmOptions {
 };
 GemmOptions forward_options();
 bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *workspace, const GemmOptions &opt,
-                          PlanReq *out);
+                          PlanReq *out, bool w_kn = false);   // w_kn: the weight is stored [E, K, N]
 int ffn1_forward(const void *x, const int32_t *src_row, const int32_t *dst_row, const int32_t *offsets,
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w1, const void *b1,
                  int apply_gelu, void *h, void *workspace, size_t workspace_bytes, hipStream_t stream,
-                 const GemmOptions *planned);   // planned: the options the plan in the workspace was built under, or NULL
+                 const GemmOptions *planned,    // planned: the options the plan in the workspace was built under, or NULL
+                 bool w_kn = false);
 int ffn2_forward(const void *h, const int32_t *src_row, const int32_t *dst_row, const int32_t *offsets,
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w2, const void *b2,
                  const void *row_scale, void *y, void *workspace, size_t workspace_bytes,
-                 hipStream_t stream, const GemmOptions *planned);
+                 hipStream_t stream, const GemmOptions *planned, bool w_kn = false);
 int ffn2_forward_combine(const void *h, const int32_t *token_row, const int32_t *flat_row, const int32_t *offsets,
                          int max_rows, int num_expert, int d_model, int d_ffn, const void *w2, const void *b2,
                          const void *score, void *out, void *workspace, size_t workspace_bytes, hipStream_t stream,
@@ -529,6 +530,11 @@ int route_with_plans(const int64_t *gate_idx, int n_flat, int num_expert, int to
 int segments_with_plans(const int32_t *seg_start, const int32_t *seg_len, const int32_t *seg_expert, int n_seg,
                         int num_expert, int total_rows, int32_t *counts, int32_t *offsets, int32_t *rows,
                         hipStream_t stream, const PlanReq *plans, int n_plans);
+// route.hip: the same from the reference's block arrays (pos, expert_ids, lens, start_addrs)
+int blocks_with_plans(const int64_t *pos, int n_pos, int top_k, int n_tokens, const int32_t *expert_ids,
+                      const int32_t *lens, const int32_t *starts, int n_blocks, int block_size, int num_expert,
+                      int32_t *counts, int32_t *offsets, int32_t *token_rows, int32_t *flat_rows, hipStream_t stream,
+                      const PlanReq *plans, int n_plans);
 // most entries of a table of per-run expert counts that the routing stage takes from the gate kernel
 long long route_rows_max_ints();
 

@@ -287,11 +287,26 @@ pos_kernel(const int64_t *__restrict__ idx, int n, int E, int nbits, int top_k, 
 
 // (start, len, expert) triples -> counts, offsets, row list grouped by expert.
 // Inside an expert the rows keep the order of the triple list, then row order.
-__global__ void __launch_bounds__(1024)
+// The first `row_wgs` workgroups write the rows, a wavefront per triple (each repeats the counts: a few hundred
+// integers), the others build the plans.  The launch on 64 triples of 16384 rows: 15 us, 22 with all rows in one
+// workgroup; what is left is the plans.
+//
+// With `pos` the triples are the reference's block arrays (mix_moe/csrc/mix_moe.h:507-598): block s holds the padded
+// rows [s block_size, s block_size + len), padded row p is sorted entry starts[p / block_size] + p % block_size of
+// pos, and what is written per row is its token (rows) and its flat index (flat_rows).
+constexpr int kSegThreads = 256;
+struct SegBlocks {
+  const int64_t *pos;        // NULL: plain triples
+  const int32_t *starts;     // [n_seg]
+  int n_pos, block_size, top_k, n_tokens;
+  int32_t *flat_rows;
+};
+
+__global__ void __launch_bounds__(kSegThreads)
 segments_kernel(const int32_t *__restrict__ seg_start, const int32_t *__restrict__ seg_len,
                 const int32_t *__restrict__ seg_expert, int n_seg, int E, int total_rows,
                 int32_t *__restrict__ counts, int32_t *__restrict__ offsets,
-                int32_t *__restrict__ rows, int plan_wgs, PlanReq plan0, PlanReq plan1) {
+                int32_t *__restrict__ rows, SegBlocks blk, int row_wgs, int plan_wgs, PlanReq plan0, PlanReq plan1) {
   __shared__ int s_cnt[kMaxExpert];
   __shared__ int s_off[kMaxExpert + 1];
   // every workgroup: rows per expert (a thread per triple, integer adds in LDS), then the experts' starts
@@ -319,31 +334,45 @@ segments_kernel(const int32_t *__restrict__ seg_start, const int32_t *__restrict
     if (lane == 0) s_off[E] = carry;
   }
   __syncthreads();
-  // workgroups past the first build the tile plans of the GEMMs that follow (the offsets are final)
-  if (blockIdx.x > 0) {
-    const int r = static_cast<int>(blockIdx.x) - 1;
+  // workgroups past the rows build the tile plans of the GEMMs that follow (the offsets are final)
+  if (static_cast<int>(blockIdx.x) >= row_wgs) {
+    const int r = static_cast<int>(blockIdx.x) - row_wgs;
     build_plan(r < plan_wgs ? plan0 : plan1, s_off, E, r % plan_wgs, plan_wgs);
     return;
   }
-  for (int e = threadIdx.x; e <= E; e += blockDim.x) {
-    offsets[e] = s_off[e];
-    if (e < E) counts[e] = s_cnt[e];
-  }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nwave = blockDim.x >> 6;
+  if (blockIdx.x == 0)
+    for (int e = threadIdx.x; e <= E; e += blockDim.x) {
+      offsets[e] = s_off[e];
+      if (e < E) counts[e] = s_cnt[e];
+    }
+  const int lane = threadIdx.x & 63, nwave = row_wgs * (kSegThreads / 64);
+  const int wave = static_cast<int>(blockIdx.x) * (kSegThreads / 64) + (threadIdx.x >> 6);
   for (int s = wave; s < n_seg; s += nwave) {
     const int e = seg_expert[s];
-    const int len = seg_len[s], st = seg_start[s];
+    const int len = seg_len[s], st = blk.pos ? s * blk.block_size : seg_start[s];
     if (e < 0 || e >= E || len <= 0) continue;     // uniform per wavefront
     int before = 0;                                // rows of earlier triples of this expert
-    for (int q = lane; q < s; q += 64)
-      if (seg_expert[q] == e && seg_len[q] > 0) before += seg_len[q];
+#pragma unroll 4
+    for (int q = lane; q < s; q += 64) {
+      const int qe = seg_expert[q], ql = seg_len[q];
+      before += (qe == e && ql > 0) ? ql : 0;
+    }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off, 64);
     const int dst = s_off[e] + before;
-    for (int r = lane; r < len; r += 64) {
+    for (int r = lane; r < len && dst + r < total_rows; r += 64) {
       int row = st + r;                            // keep malformed triples inside the buffer
       row = row < 0 ? 0 : (row >= total_rows ? total_rows - 1 : row);
-      if (dst + r < total_rows) rows[dst + r] = row;
+      if (blk.pos) {
+        int i = blk.starts[row / blk.block_size] + row % blk.block_size;
+        i = i < 0 ? 0 : (i >= blk.n_pos ? blk.n_pos - 1 : i);
+        const int64_t at = blk.pos[i];             // and malformed positions inside the tensors
+        const int flat = at < 0 ? 0 : (at >= blk.n_pos ? blk.n_pos - 1 : static_cast<int>(at));
+        const int token = flat / blk.top_k;
+        blk.flat_rows[dst + r] = flat;
+        row = token < blk.n_tokens ? token : blk.n_tokens - 1;
+      }
+      rows[dst + r] = row;
     }
   }
 }
@@ -610,6 +639,21 @@ extern "C" int ccf_route_static(const int64_t *gate_idx, int n_flat, int num_exp
 }
 
 namespace ccf {
+namespace {
+int launch_segments(const int32_t *seg_start, const int32_t *seg_len, const int32_t *seg_expert, int n_seg, int E,
+                    int total_rows, int32_t *counts, int32_t *offsets, int32_t *rows, const SegBlocks &blk,
+                    hipStream_t stream, const PlanReq *plans, int n_plans) {
+  const PlanReq none{0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  const int plan_wgs = 8;
+  int row_wgs = (n_seg + kSegThreads / 64 - 1) / (kSegThreads / 64);
+  row_wgs = row_wgs < 1 ? 1 : (row_wgs > 512 ? 512 : row_wgs);
+  hipLaunchKernelGGL(segments_kernel, dim3(row_wgs + n_plans * plan_wgs), dim3(kSegThreads), 0, stream, seg_start, seg_len,
+                     seg_expert, n_seg, E, total_rows, counts, offsets, rows, blk, row_wgs, plan_wgs,
+                     n_plans > 0 ? plans[0] : none, n_plans > 1 ? plans[1] : none);
+  return check_launch("segments_kernel");
+}
+}  // namespace
+
 // ccf_segments_to_rows(), whose launch also builds n_plans (0..2) tile plans from the offsets.
 int segments_with_plans(const int32_t *seg_start, const int32_t *seg_len, const int32_t *seg_expert, int n_seg,
                         int num_expert, int total_rows, int32_t *counts, int32_t *offsets, int32_t *rows,
@@ -621,12 +665,18 @@ int segments_with_plans(const int32_t *seg_start, const int32_t *seg_len, const 
   CCF_REQUIRE(num_expert <= kMaxExpert, CCF_ERR_SHAPE, "segments_to_rows: num_expert=%d exceeds %d",
               num_expert, kMaxExpert);
   CCF_REQUIRE(n_plans >= 0 && n_plans <= 2 && (n_plans == 0 || plans), CCF_ERR_ARG, "segments_to_rows: bad plan requests");
-  const PlanReq none{0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
-  const int plan_wgs = 4;                            // of 1024 threads: 64 wavefronts per plan
-  hipLaunchKernelGGL(segments_kernel, dim3(1 + n_plans * plan_wgs), dim3(1024), 0, stream, seg_start, seg_len,
-                     seg_expert, n_seg, num_expert, total_rows, counts, offsets, rows, plan_wgs,
-                     n_plans > 0 ? plans[0] : none, n_plans > 1 ? plans[1] : none);
-  return check_launch("segments_kernel");
+  return launch_segments(seg_start, seg_len, seg_expert, n_seg, num_expert, total_rows, counts, offsets, rows,
+                         SegBlocks{}, stream, plans, n_plans);
+}
+
+// The same from the reference's block arrays: tokens and flat indices of the routed rows in expert order.
+int blocks_with_plans(const int64_t *pos, int n_pos, int top_k, int n_tokens, const int32_t *expert_ids,
+                      const int32_t *lens, const int32_t *starts, int n_blocks, int block_size, int num_expert,
+                      int32_t *counts, int32_t *offsets, int32_t *token_rows, int32_t *flat_rows, hipStream_t stream,
+                      const PlanReq *plans, int n_plans) {
+  return launch_segments(nullptr, lens, expert_ids, n_blocks, num_expert, n_blocks * block_size, counts, offsets,
+                         token_rows, SegBlocks{pos, starts, n_pos, block_size, top_k, n_tokens, flat_rows}, stream, plans,
+                         n_plans);
 }
 }  // namespace ccf
 

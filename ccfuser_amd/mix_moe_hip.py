@@ -55,16 +55,20 @@ def cpy_data2tensor(data: List[int], tensor: torch.Tensor) -> None:
         tensor.view(-1)[:n].copy_(torch.tensor(data, dtype=torch.int32))
 
 
-def _stored_layout(weight: torch.Tensor, n_out: int, k_in: int) -> torch.Tensor:
-    """The reference passes ``weight.transpose(-2, -1).contiguous()``, i.e. [E, K, N]
-    (mix_moe/mix_moe/linear.py:74); the kernels here read [E, N, K].  A tensor
-    already in [E, N, K] is used as is; a [E, K, N] one is transposed back."""
+def _weight_form(weight: torch.Tensor, n_out: int, k_in: int):
+    """(weight, is_kn): the reference passes ``weight.transpose(-2, -1).contiguous()``, i.e. [E, K, N]
+    (mix_moe/mix_moe/linear.py:74), which the GEMM reads as it is; a tensor already in [E, N, K] is used as
+    well.  Transposing the weights back first took 549 of 1069 us of a layer of 16 experts, 1024 / 4096, and
+    8192 tokens."""
     if weight.dim() != 3:
         raise ValueError("expert weight must be 3-D")
     if tuple(weight.shape[1:]) == (n_out, k_in) and n_out != k_in:
-        return weight.contiguous()
+        return weight.contiguous(), False
     if tuple(weight.shape[1:]) == (k_in, n_out):
-        return weight.transpose(-2, -1).contiguous()
+        if k_in * n_out >= 1 << 31:                  # the [K, N] loads index an expert's weight with 31 bits
+            return weight.transpose(-2, -1).contiguous(), False
+        weight = weight.contiguous()
+        return (weight if weight.data_ptr() % 16 == 0 else weight.clone()), True
     raise ValueError(f"expert weight {tuple(weight.shape)} matches neither [E,{k_in},{n_out}] nor [E,{n_out},{k_in}]")
 
 
@@ -113,32 +117,32 @@ class MixMOE:
         return flat_of_padded, valid, offsets, rows
 
     def first_gemm_forward(self, inp, pos, expert_ids, ranks, expert_lens, start_addrs,
-                           total_block_num, remote_block_num, weight, bias, _gelu=False):
+                           total_block_num, remote_block_num, weight, bias):
         if inp.dtype != torch.float16:
             raise TypeError("moe input data type must be float 16")
         E = weight.shape[0]
-        w = _stored_layout(weight, self._ffn_hidden_size, self._hidden_size)
+        w, kn = _weight_form(weight, self._ffn_hidden_size, self._hidden_size)
         flat_of_padded, valid, offsets, rows = self._plan(pos, expert_ids, expert_lens, start_addrs,
                                                           total_block_num, E)
         src_of_padded = torch.div(flat_of_padded, self._top_k, rounding_mode="floor")
         a_rows = src_of_padded[rows.long()].to(torch.int32)
         M = int(total_block_num) * self._block_size
         ffn1_out = torch.zeros(M, self._ffn_hidden_size, dtype=inp.dtype, device=inp.device)
-        ops.ffn1(inp.contiguous(), a_rows, offsets, M, w, bias.contiguous(), gelu=_gelu,
-                 out=ffn1_out, dst_row=rows)
+        ops.ffn1(inp.contiguous(), a_rows, offsets, M, w, bias.contiguous(), gelu=False,
+                 out=ffn1_out, dst_row=rows, w_kn=kn)
         merged_input = inp[src_of_padded] * valid[:, None].to(inp.dtype)
         return [merged_input, ffn1_out]
 
     def second_gemm_forward(self, ffn1_out, pos, expert_ids, ranks, expert_lens, start_addrs,
                             total_block_num, remote_block_num, weight, bias):
         E = weight.shape[0]
-        w = _stored_layout(weight, self._hidden_size, self._ffn_hidden_size)
+        w, kn = _weight_form(weight, self._hidden_size, self._ffn_hidden_size)
         flat_of_padded, valid, offsets, rows = self._plan(pos, expert_ids, expert_lens, start_addrs,
                                                           total_block_num, E)
         c_rows = flat_of_padded[rows.long()].to(torch.int32)
         M = int(total_block_num) * self._block_size
         output = torch.zeros(pos.numel(), self._hidden_size, dtype=ffn1_out.dtype, device=ffn1_out.device)
-        ops.ffn2(ffn1_out.contiguous(), c_rows, offsets, M, w, bias.contiguous(), output, src_row=rows)
+        ops.ffn2(ffn1_out.contiguous(), c_rows, offsets, M, w, bias.contiguous(), output, src_row=rows, w_kn=kn)
         return [ffn1_out, output]
 
     def forward(self, inp, pos, expert_ids, ranks, expert_lens, start_addrs, total_block_num,
@@ -148,10 +152,14 @@ class MixMOE:
         (mix_moe/csrc/mix_moe.h:507-598)."""
         if self._w1 is None:
             raise RuntimeError("MixMOE.forward needs the expert weights passed to the constructor")
-        _, h = self.first_gemm_forward(inp, pos, expert_ids, ranks, expert_lens, start_addrs,
-                                       total_block_num, remote_block_num, self._w1, self._b1, _gelu=True)
-        return self.second_gemm_forward(h, pos, expert_ids, ranks, expert_lens, start_addrs,
-                                        total_block_num, remote_block_num, self._w2, self._b2)[1]
+        if inp.dtype != torch.float16:
+            raise TypeError("moe input data type must be float 16")
+        w1, kn1 = _weight_form(self._w1, self._ffn_hidden_size, self._hidden_size)
+        w2, kn2 = _weight_form(self._w2, self._hidden_size, self._ffn_hidden_size)
+        nb = int(total_block_num)
+        arrays = [t[:nb].to(torch.int32).contiguous() for t in (expert_ids, expert_lens, start_addrs)]
+        return ops.moe_ffn_blocks(inp.contiguous(), pos.to(torch.int64).contiguous(), *arrays, self._block_size,
+                                  self._top_k, w1, self._b1.contiguous(), w2, self._b2.contiguous(), kn1, kn2)
 
     @staticmethod
     def _stored(weight: torch.Tensor, n_out: int, k_in: int) -> torch.Tensor:

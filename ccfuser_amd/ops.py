@@ -270,24 +270,25 @@ def ffn_plan_info(workspace: torch.Tensor, max_rows: int, E: int, d: int, f: int
     return dict(zip(names, list(info)))
 
 
-def _check_expert(w: torch.Tensor, b: torch.Tensor, name: str) -> None:
+def _check_expert(w: torch.Tensor, b: torch.Tensor, name: str, kn: bool = False) -> None:
     _check(w, f"{name} weight", dtype=torch.float16, ndim=3)
     _check(b, f"{name} bias", dtype=torch.float16, ndim=2)
-    if b.shape[0] != w.shape[0] or b.shape[1] != w.shape[1]:
+    if b.shape[0] != w.shape[0] or b.shape[1] != w.shape[2 if kn else 1]:
         raise ValueError(f"{name}: bias {tuple(b.shape)} does not match weight {tuple(w.shape)}")
 
 
 def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor, max_rows: int,
          w1: torch.Tensor, b1: torch.Tensor, gelu: bool = True,
          out: Optional[torch.Tensor] = None, dst_row: Optional[torch.Tensor] = None,
-         workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """h [max_rows, f] (or ``out``); rows nothing maps to are left as they were."""
+         workspace: Optional[torch.Tensor] = None, w_kn: bool = False) -> torch.Tensor:
+    """h [max_rows, f] (or ``out``); rows nothing maps to are left as they were.  ``w_kn``: the weight is
+    stored [E, d, f] (input width first)."""
     if x.dtype != torch.float16:
         raise TypeError("moe input data type must be float 16")
     _check(x, "x", dtype=torch.float16, ndim=2)
-    _check_expert(w1, b1, "ffn1")
+    _check_expert(w1, b1, "ffn1", w_kn)
     _check(offsets, "offsets", dtype=torch.int32, ndim=1)
-    E, f, d = w1.shape
+    E, f, d = (w1.shape[0], w1.shape[2], w1.shape[1]) if w_kn else w1.shape
     if x.shape[1] != d or offsets.numel() != E + 1:
         raise ValueError("ffn1: x/offsets do not match the weight shape")
     if src_row is not None:
@@ -306,7 +307,7 @@ def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor
         raise ValueError("ffn1: output buffer too small")
     with torch.cuda.device(x.device):
         ws = workspace if workspace is not None else ffn_workspace(max_rows, E, d, f, x)
-        _lib.call("ccf_ffn1_forward", _ptr(x), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
+        _lib.call("ccf_ffn1_forward_kn" if w_kn else "ccf_ffn1_forward", _ptr(x), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
                   _ptr(w1), _ptr(b1), int(bool(gelu)), _ptr(h), _ptr(ws), ws.numel(), _stream(x))
     return h
 
@@ -339,13 +340,15 @@ def ffn1_keep(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.T
 def ffn2(h: torch.Tensor, dst_row: Optional[torch.Tensor], offsets: torch.Tensor, max_rows: int,
          w2: torch.Tensor, b2: torch.Tensor, y: torch.Tensor,
          row_scale: Optional[torch.Tensor] = None,
-         src_row: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Writes ``y[dst_row[j]]`` for the routed rows and returns ``y``."""
+         src_row: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None,
+         w_kn: bool = False) -> torch.Tensor:
+    """Writes ``y[dst_row[j]]`` for the routed rows and returns ``y``.  ``w_kn``: the weight is stored
+    [E, f, d] (input width first)."""
     _check(h, "h", dtype=torch.float16, ndim=2)
-    _check_expert(w2, b2, "ffn2")
+    _check_expert(w2, b2, "ffn2", w_kn)
     _check(offsets, "offsets", dtype=torch.int32, ndim=1)
     _check(y, "y", dtype=torch.float16, ndim=2)
-    E, d, f = w2.shape
+    E, d, f = (w2.shape[0], w2.shape[2], w2.shape[1]) if w_kn else w2.shape
     if h.shape[1] != f or offsets.numel() != E + 1 or y.shape[1] != d:
         raise ValueError("ffn2: h/offsets/y do not match the weight shape")
     if src_row is not None:
@@ -364,7 +367,7 @@ def ffn2(h: torch.Tensor, dst_row: Optional[torch.Tensor], offsets: torch.Tensor
         _check(row_scale, "row_scale", dtype=torch.float16, ndim=1)
     with torch.cuda.device(h.device):
         ws = workspace if workspace is not None else ffn_workspace(max_rows, E, d, f, h)
-        _lib.call("ccf_ffn2_forward", _ptr(h), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
+        _lib.call("ccf_ffn2_forward_kn" if w_kn else "ccf_ffn2_forward", _ptr(h), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
                   _ptr(w2), _ptr(b2), _ptr(row_scale), _ptr(y), _ptr(ws), ws.numel(), _stream(h))
     return y
 
@@ -553,4 +556,34 @@ def moe_ffn_segments(x, seg_start, seg_len, seg_expert, w1, b1, w2, b2,
         _lib.call("ccf_moe_ffn_segments", _ptr(x), _ptr(seg_start), _ptr(seg_len), _ptr(seg_expert),
                   seg_start.numel(), R, d, f, E, _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(y),
                   _ptr(ws), ws.numel(), _stream(x))
+    return y
+
+
+def moe_ffn_blocks(x, pos, expert_ids, lens, start_addrs, block_size: int, top_k: int, w1, b1, w2, b2,
+                   w1_kn: bool = False, w2_kn: bool = False) -> torch.Tensor:
+    """Expert FFN over the reference's block arrays: y [pos.numel(), d] in flat token order, zero at rows no
+    block covers.  ``w1_kn`` / ``w2_kn``: that weight is stored [E, K, N]."""
+    if x.dtype != torch.float16:
+        raise TypeError("moe input data type must be float 16")
+    _check(x, "x", dtype=torch.float16, ndim=2)
+    _check(pos, "pos", dtype=torch.int64, ndim=1)
+    for t, nm in ((expert_ids, "expert_ids"), (lens, "expert_lens"), (start_addrs, "start_addrs")):
+        _check(t, nm, dtype=torch.int32, ndim=1)
+    _check_expert(w1, b1, "ffn1", w1_kn)
+    _check_expert(w2, b2, "ffn2", w2_kn)
+    E, f = b1.shape
+    T, d = x.shape
+    nb = expert_ids.numel()
+    if w1.numel() != E * f * d or w2.numel() != E * f * d or tuple(b2.shape) != (E, d):
+        raise ValueError("moe_ffn_blocks: x and the weights do not match")
+    if lens.numel() != nb or start_addrs.numel() != nb:
+        raise ValueError("moe_ffn_blocks: the block arrays differ in length")
+    if nb and (not T or not pos.numel()):
+        raise ValueError("moe_ffn_blocks: blocks of no tokens")
+    y = torch.zeros(pos.numel(), d, dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        ws = _workspace(_lib.lib().ccf_blocks_workspace_bytes(nb, int(block_size), E, d, f), x)
+        _lib.call("ccf_moe_ffn_blocks", _ptr(x), T, _ptr(pos), pos.numel(), int(top_k), _ptr(expert_ids), _ptr(lens),
+                  _ptr(start_addrs), nb, int(block_size), d, f, E, _ptr(w1), int(w1_kn), _ptr(b1), _ptr(w2),
+                  int(w2_kn), _ptr(b2), _ptr(y), _ptr(ws), ws.numel(), _stream(x))
     return y

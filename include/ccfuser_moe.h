@@ -375,6 +375,43 @@ int ccf_moe_ffn_segments(const void *x, const int32_t *seg_start,
                          void *workspace, size_t workspace_bytes,
                          ccf_stream_t stream);
 
+/*
+ * The reference's MixMOE.forward (mix_moe/csrc/mix_moe.h:507-598) on the block
+ * arrays of its planner (transformer.py:242-250).  Block b holds lens[b] rows of
+ * expert expert_ids[b]: entries start_addrs[b] .. of pos, each a flat index
+ * token * top_k + slot below n_pos.  y [n_pos, d_model] is written at the rows
+ * the blocks cover; the caller clears it when they may not cover all.
+ * w1_kn / w2_kn != 0: the weight is stored [E, K, N] (linear.py:74, 129), 0:
+ * [E, N, K].  An [E, K, N] weight has K * N < 2^31.
+ */
+size_t ccf_blocks_workspace_bytes(int n_blocks, int block_size, int num_expert,
+                                  int d_model, int d_ffn);
+int ccf_moe_ffn_blocks(const void *x, int n_tokens, const int64_t *pos,
+                       int n_pos, int top_k, const int32_t *expert_ids,
+                       const int32_t *lens, const int32_t *start_addrs,
+                       int n_blocks, int block_size, int d_model, int d_ffn,
+                       int num_expert, const void *w1, int w1_kn,
+                       const void *b1, const void *w2, int w2_kn,
+                       const void *b2, void *y, void *workspace,
+                       size_t workspace_bytes, ccf_stream_t stream);
+
+/*
+ * ccf_ffn1_forward / ccf_ffn2_forward on weights stored [E, K, N], as the
+ * reference passes them to its extension (mix_moe/mix_moe/linear.py:74, 129).
+ */
+int ccf_ffn1_forward_kn(const void *x, const int32_t *src_row,
+                        const int32_t *dst_row, const int32_t *offsets,
+                        int max_rows, int num_expert, int d_model, int d_ffn,
+                        const void *w1, const void *b1, int apply_gelu, void *h,
+                        void *workspace, size_t workspace_bytes,
+                        ccf_stream_t stream);
+int ccf_ffn2_forward_kn(const void *h, const int32_t *src_row,
+                        const int32_t *dst_row, const int32_t *offsets,
+                        int max_rows, int num_expert, int d_model, int d_ffn,
+                        const void *w2, const void *b2, const void *row_scale,
+                        void *y, void *workspace, size_t workspace_bytes,
+                        ccf_stream_t stream);
+
 /* ------------------------------------------------------------ backward */
 
 /*

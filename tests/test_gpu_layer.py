@@ -610,6 +610,44 @@ def test_few_tiles_of_a_long_contraction(counts):
     close(gx, torch.cat([a[e_of.cuda() == e].float() @ w1[e].float() for e in range(E)]))
 
 
+@pytest.mark.parametrize("T,d,f,E,k,bs,stored", [(1, 64, 192, 4, 2, 64, False), (333, 320, 832, 5, 2, 64, False),
+                                                  (700, 256, 256, 3, 1, 32, False), (900, 512, 1024, 8, 2, 64, True),
+                                                  (60, 4160, 512, 2, 2, 64, False)])
+def test_block_arrays_on_kn_weights(T, d, f, E, k, bs, stored):
+    """``MixMOE.forward`` from block arrays (blocks of 64 and 32 rows, short ones, an expert without rows) on
+    [E, K, N] weights of widths that are no multiple of the column tile, square ones and [E, N, K] ones, against
+    the staged calls on the [E, N, K] form: the same products in the same order, so the same bits wherever no
+    tile is cut along K, and the tolerance everywhere.  A weight at an odd 2-byte offset is taken too."""
+    from ccfuser_amd import mix_moe_hip, ops
+    _say(f"block arrays T={T} d={d} f={f} E={E} k={k} bs={bs}")
+    g = torch.Generator().manual_seed(T + d)
+    r = lambda *s, sc=1.0: (torch.randn(*s, generator=g) * sc).half().cuda()
+    x, w1, b1, w2, b2 = r(T, d), r(E, f, d, sc=0.05), r(E, f), r(E, d, f, sc=0.05), r(E, d)
+    idx = torch.randint(0, E - 1, (T * k,), generator=g).cuda()            # the last expert has no rows
+    m = ops.route(idx, E, k)
+    plan = ops.plan_blocks(m["counts"], T * k, bs)
+    total, remote = plan["block_nums"].tolist()
+    blocks = (plan["expert_ids"], plan["ranks"], plan["lens"], plan["start_addrs"], total, remote)
+    h = ops.ffn1(x, m["src_row"], m["offsets"], T * k, w1, b1)
+    want = ops.ffn2(h, m["dst_row"], m["offsets"], T * k, w2, b2, torch.empty(T * k, d, dtype=torch.float16, device="cuda"))
+    kn = [w if stored else w.transpose(-2, -1).contiguous() for w in (w1, w2)]
+    odd = torch.empty(kn[0].numel() + 1, dtype=torch.float16, device="cuda")[1:].view(kn[0].shape)
+    odd.copy_(kn[0])
+    for first in ([kn[0]] if stored else [kn[0], odd]):
+        got = mix_moe_hip.MixMOE(1, T, E, k, d, f, bs, first, kn[1], b1, b2).forward(x, m["pos"], *blocks)
+        err = float((got.float() - want.float()).abs().max())
+        assert err <= 2.0 ** -9 * float(want.float().abs().max())          # two fp16 steps of the largest result
+        if max(d, f) < 4096:
+            assert torch.equal(got, want)
+    m3 = mix_moe_hip.MixMOE(1, T, E, k, d, f, bs)
+    _, pre = m3.first_gemm_forward(x, m["pos"], *blocks, kn[0], b1)
+    y = m3.second_gemm_forward(torch.nn.functional.gelu(pre.float()).half(), m["pos"], *blocks, kn[1], b2)[1]
+    assert float((y.float() - want.float()).abs().max()) <= 2.0 ** -8 * float(want.float().abs().max())
+    # a block count below the arrays' length, and none: rows that no block covers are zero
+    part = mix_moe_hip.MixMOE(1, T, E, k, d, f, bs, *kn, b1, b2).forward(x, m["pos"], *blocks[:4], 0, 0)
+    assert part.shape == want.shape and not part.any()
+
+
 def _forced_plan_cases(count, seed):
     g = torch.Generator().manual_seed(seed)
     ri = lambda lo, hi: int(torch.randint(lo, hi + 1, (1,), generator=g))
