@@ -204,25 +204,26 @@ extern "C" int ccf_moe_forward(const void *x, const void *wg, const void *bg, co
   const bool direct = top_k == 1 && capacity < 0;
   // top-2 with the option on: FFN2's epilogue adds score * y into the zero-filled output
   const bool fuse = opt.fused_combine && top_k == 2 && d_model % 8 == 0;
-  const bool planned = forward_plan_request(1, n, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[0]) &&
-                       forward_plan_request(fuse ? 3 : 2, n, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[1]);
+  // (a GEMM of few rows per expert needs none)
+  const bool planned1 = forward_plan_request(1, n, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[0]);
+  const bool planned2 = forward_plan_request(fuse ? 3 : 2, n, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[planned1 ? 1 : 0]);
   if ((rc = route_with_plans(w.idx, n, num_expert, top_k, capacity, w.counts, w.offsets, w.pos, w.src_row,
                              w.dst_row, w.inv_pos, w.idx_kept, w.route_ws, w.route_bytes, st, plans,
-                             planned ? 2 : 0, gate_tokens * top_k)))
+                             planned1 + planned2, gate_tokens * top_k)))
     return rc;
   mark_stage(2, st);
   if ((rc = ffn1_forward(x, w.src_row, nullptr, w.offsets, n, num_expert, d_model, d_ffn, w1, b1, 1, w.h,
-                         w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr)))
+                         w.ffn_ws, w.ffn_bytes, st, planned1 ? &opt : nullptr)))
     return rc;
   mark_stage(3, st);
   if (fuse) {
     if ((rc = launch_zero(static_cast<half_t *>(out), static_cast<size_t>(tokens) * d_model, st))) return rc;
     if ((rc = ffn2_forward_combine(w.h, w.src_row, w.dst_row, w.offsets, n, num_expert, d_model, d_ffn, w2, b2,
-                                   w.score, out, w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr)))
+                                   w.score, out, w.ffn_ws, w.ffn_bytes, st, planned2 ? &opt : nullptr)))
       return rc;
     mark_stage(4, st);
   } else if ((rc = ffn2_forward(w.h, nullptr, w.dst_row, w.offsets, n, num_expert, d_model, d_ffn, w2, b2,
-                         nullptr, direct ? out : w.y_flat, w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr)))
+                         nullptr, direct ? out : w.y_flat, w.ffn_ws, w.ffn_bytes, st, planned2 ? &opt : nullptr)))
     return rc;
   if (!fuse) mark_stage(4, st);
   if (!direct && !fuse) {
@@ -270,18 +271,18 @@ extern "C" int ccf_moe_ffn_segments(const void *x, const int32_t *seg_start, con
   // the tile plans of both GEMMs are built by more workgroups of the regrouping launch, as in ccf_moe_forward
   PlanReq plans[2];
   const GemmOptions opt = forward_options();
-  const bool planned = forward_plan_request(1, total_rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[0]) &&
-                       forward_plan_request(2, total_rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[1]);
+  const bool planned1 = forward_plan_request(1, total_rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[0]);
+  const bool planned2 = forward_plan_request(2, total_rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[planned1 ? 1 : 0]);
   if ((rc = segments_with_plans(seg_start, seg_len, seg_expert, n_seg, num_expert, total_rows, w.counts, w.offsets,
-                                w.rows, st, plans, planned ? 2 : 0)))
+                                w.rows, st, plans, planned1 + planned2)))
     return rc;
   mark_stage(2, st);
   if ((rc = ffn1_forward(x, w.rows, nullptr, w.offsets, total_rows, num_expert, d_model, d_ffn, w1, b1, 1,
-                         w.h, w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr)))
+                         w.h, w.ffn_ws, w.ffn_bytes, st, planned1 ? &opt : nullptr)))
     return rc;
   mark_stage(3, st);
   rc = ffn2_forward(w.h, nullptr, w.rows, w.offsets, total_rows, num_expert, d_model, d_ffn, w2, b2,
-                    nullptr, y, w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr);
+                    nullptr, y, w.ffn_ws, w.ffn_bytes, st, planned2 ? &opt : nullptr);
   mark_stage(4, st);
   mark_stage(5, st);                                  // no combine either
   return rc;
@@ -316,14 +317,14 @@ extern "C" int ccf_moe_ffn_blocks(const void *x, int n_tokens, const int64_t *po
   hipStream_t st = as_stream(stream);
   PlanReq plans[2];
   const GemmOptions opt = forward_options();
-  const bool planned = forward_plan_request(1, rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[0], w1_kn != 0) &&
-                       forward_plan_request(2, rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[1], w2_kn != 0);
+  const bool planned1 = forward_plan_request(1, rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[0], w1_kn != 0);
+  const bool planned2 = forward_plan_request(2, rows, num_expert, d_model, d_ffn, w.ffn_ws, opt, &plans[planned1 ? 1 : 0], w2_kn != 0);
   if (int rc = blocks_with_plans(pos, n_pos, top_k, n_tokens, expert_ids, lens, start_addrs, n_blocks, block_size,
-                                 num_expert, w.counts, w.offsets, w.token_rows, w.flat_rows, st, plans, planned ? 2 : 0))
+                                 num_expert, w.counts, w.offsets, w.token_rows, w.flat_rows, st, plans, planned1 + planned2))
     return rc;
   if (int rc = ffn1_forward(x, w.token_rows, nullptr, w.offsets, rows, num_expert, d_model, d_ffn, w1, b1, 1, w.h,
-                            w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr, w1_kn != 0))
+                            w.ffn_ws, w.ffn_bytes, st, planned1 ? &opt : nullptr, w1_kn != 0))
     return rc;
   return ffn2_forward(w.h, nullptr, w.flat_rows, w.offsets, rows, num_expert, d_model, d_ffn, w2, b2, nullptr, y,
-                      w.ffn_ws, w.ffn_bytes, st, planned ? &opt : nullptr, w2_kn != 0);
+                      w.ffn_ws, w.ffn_bytes, st, planned2 ? &opt : nullptr, w2_kn != 0);
 }

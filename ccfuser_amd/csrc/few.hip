@@ -1,0 +1,442 @@
+// Grouped GEMM of few rows per expert for gfx950: decoding batches, short prompts, small layers.
+//
+// The 256-row tiles of ffn.hip leave most of the chip idle there: 32 rows per expert fill an eighth of a
+// tile, and a layer of a few hundred rows makes a few dozen tiles for 256 CUs.  This kernel has tiles of 32,
+// 64 or 128 rows by 64, 128 or 256 columns, picks among them on the device from the experts' row counts, and
+// runs all of K in one workgroup: no plan launch in front, no partial tiles, no reduction behind.
+//
+//   * every workgroup derives its own tiles from the offsets (a scan over the experts and one binary search
+//     per tile), so the launch stands alone;
+//   * tiles of one column range lie side by side on an XCD, so an expert's second M tile reads the weights
+//     from that XCD's L2;
+//   * operands go to LDS with direct loads, 64 K elements per stage, as many stages as fit; the pipeline
+//     runs on across a workgroup's tiles (the stages of the next tile are loaded under the last steps of
+//     this one).  One workgroup of eight wavefronts per CU: two workgroups of four with half of the LDS each
+//     measured the same at many tiles and up to a quarter slower at one tile per CU, whose weights then stream
+//     through a pipeline of half the depth;
+//   * accumulation runs over K in 32-wide steps in ascending order, as in the 256-row tiles: same bits.
+//
+// Bound by streaming the weights from HBM at 5.3 - 5.7 TB/s where they are large, by the latency of a few dependent
+// steps where they are small.  FFN1 / FFN2 including their plan and reduction launches, 256-row tiles -> here:
+// 8 experts of 4096 / 14336, 32 rows each: 205 -> 165 and 176 -> 172 us, 83 rows each: 213 -> 191 and 201 -> 177;
+// 4 experts of 256 / 1024, 128 rows each: 20 -> 10 and 28 -> 10; 8 experts of 768 / 3072, 500 rows each: 44 -> 43 and
+// 70 -> 38; 16 experts of 1024 / 4096, 64 rows each: 37 -> 28 and 53 -> 31.
+#include "ccf_common.h"
+#include "gelu.h"
+#include "gemm_tile.h"
+#include "plan.h"
+
+#include <cmath>
+
+namespace ccf {
+namespace {
+
+constexpr int kFewThreads = 512;
+constexpr int kFewLds = 163840;
+constexpr int kFewMaxRounds = 64;      // most tiles of a workgroup: one per lane of the tile table
+constexpr int kBK = 64;
+// A K step of 64 by tile shape [rows 64, 128][columns 64, 128, 256] in microseconds, operands in L2 (measured)
+constexpr double kFewStepUs[2][3] = {{0.36, 0.45, 0.80}, {0.42, 0.62, 1.20}};
+
+// Tile of 16 TM rows x 32 DB columns, 64 K elements per stage.  Eight wavefronts, 2 along the rows (wavefront half m
+// holds the 16-row blocks m, m + 2, ...) x 4 along the columns (16 NB columns each): two wavefronts per SIMD, so one's
+// LDS reads run under the other's MFMAs.
+template <int TM_, int DB_>
+struct FewCfg {
+  static constexpr int TM = TM_, DB = DB_, TMW = TM / 2, NB = DB / 2, BN = 32 * DB;
+  static constexpr int A_DMA = TM / 4, B_DMA = DB / 2, LOADS = A_DMA + B_DMA;             // 1 KB loads per wavefront and stage
+  static constexpr int A_BYTES = 16 * TM * kBK * 2, STAGE = A_BYTES + BN * kBK * 2;
+  static constexpr int FIT = kFewLds / STAGE, STAGES = FIT > 8 ? 8 : FIT;
+  static_assert(TM % 4 == 0 && DB % 2 == 0 && STAGES >= 3 && (STAGES - 2) * LOADS < 63, "tile shape");
+};
+
+// One substep's fragments, waited for in the block that reads them: row blocks 32 rows (4096 bytes) apart, column
+// blocks 16 rows (2048 bytes) apart.
+template <int TMW, int NB>
+__device__ __forceinline__ void few_frags(half8 (&a)[TMW], half8 (&b)[NB], uint32_t ra, uint32_t rb);
+#define CCF_RD(o, base, off) "ds_read_b128 %" #o ", %" #base " offset:" #off "\n"
+#define CCF_LGKM "s_waitcnt lgkmcnt(0)"
+#define CCF_A2 "=&v"(a[0]), "=&v"(a[1])
+#define CCF_A4 CCF_A2, "=&v"(a[2]), "=&v"(a[3])
+#define CCF_B1 "=&v"(b[0])
+#define CCF_B2 CCF_B1, "=&v"(b[1])
+#define CCF_B4 CCF_B2, "=&v"(b[2]), "=&v"(b[3])
+#define CCF_FRAGS(TMW, NB, READS, ...)                                                                             \
+  template <>                                                                                                      \
+  __device__ __forceinline__ void few_frags<TMW, NB>(half8 (&a)[TMW], half8 (&b)[NB], uint32_t ra, uint32_t rb) { \
+    asm volatile(READS CCF_LGKM : __VA_ARGS__ : "v"(ra), "v"(rb) : "memory");                                      \
+  }
+CCF_FRAGS(2, 1, CCF_RD(0, 4, 0) CCF_RD(1, 3, 0) CCF_RD(2, 3, 4096), CCF_B1, CCF_A2)
+CCF_FRAGS(2, 2, CCF_RD(0, 5, 0) CCF_RD(1, 5, 2048) CCF_RD(2, 4, 0) CCF_RD(3, 4, 4096), CCF_B2, CCF_A2)
+CCF_FRAGS(2, 4, CCF_RD(0, 7, 0) CCF_RD(1, 7, 2048) CCF_RD(2, 7, 4096) CCF_RD(3, 7, 6144) CCF_RD(4, 6, 0) CCF_RD(5, 6, 4096),
+          CCF_B4, CCF_A2)
+CCF_FRAGS(4, 1, CCF_RD(0, 6, 0) CCF_RD(1, 5, 0) CCF_RD(2, 5, 4096) CCF_RD(3, 5, 8192) CCF_RD(4, 5, 12288), CCF_B1, CCF_A4)
+CCF_FRAGS(4, 2, CCF_RD(0, 7, 0) CCF_RD(1, 7, 2048) CCF_RD(2, 6, 0) CCF_RD(3, 6, 4096) CCF_RD(4, 6, 8192) CCF_RD(5, 6, 12288),
+          CCF_B2, CCF_A4)
+CCF_FRAGS(4, 4, CCF_RD(0, 9, 0) CCF_RD(1, 9, 2048) CCF_RD(2, 9, 4096) CCF_RD(3, 9, 6144) CCF_RD(4, 8, 0) CCF_RD(5, 8, 4096)
+                    CCF_RD(6, 8, 8192) CCF_RD(7, 8, 12288),
+          CCF_B4, CCF_A4)
+
+// The same for weights stored [K][N]: a column block's fragment is two transposing reads, K rows 0..3 and 4..7 of the
+// lane's eight (PITCH = 8 BN bytes apart), at the lane's address XOR 32 J.
+template <int TMW, int NB, int PITCH4>
+__device__ __forceinline__ void few_frags_kn(half8 (&a)[TMW], half8 (&b)[NB], uint32_t ra, uint32_t rb) {
+  static_assert((TMW == 2 || TMW == 4) && (NB == 2 || NB == 4), "written out below");
+  half4 lo[NB], hi[NB];
+#define CCF_TR(o, base) "ds_read_b64_tr_b16 %" #o ", %" #base "\n"
+#define CCF_TRH(o, base, off) "ds_read_b64_tr_b16 %" #o ", %" #base " offset:%" #off "\n"
+  if constexpr (NB == 2) {
+    if constexpr (TMW == 2)
+      asm volatile(CCF_TR(0, 7) CCF_TRH(1, 7, 9) CCF_TR(2, 8) CCF_TRH(3, 8, 9) CCF_RD(4, 6, 0) CCF_RD(5, 6, 4096) CCF_LGKM
+                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), CCF_A2
+                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "n"(PITCH4)
+                   : "memory");
+    else
+      asm volatile(CCF_TR(0, 9) CCF_TRH(1, 9, 11) CCF_TR(2, 10) CCF_TRH(3, 10, 11) CCF_RD(4, 8, 0) CCF_RD(5, 8, 4096)
+                   CCF_RD(6, 8, 8192) CCF_RD(7, 8, 12288) CCF_LGKM
+                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), CCF_A4
+                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "n"(PITCH4)
+                   : "memory");
+  } else {
+    if constexpr (TMW == 2)
+      asm volatile(CCF_TR(0, 11) CCF_TRH(1, 11, 15) CCF_TR(2, 12) CCF_TRH(3, 12, 15) CCF_TR(4, 13) CCF_TRH(5, 13, 15) CCF_TR(6, 14)
+                   CCF_TRH(7, 14, 15) CCF_RD(8, 10, 0) CCF_RD(9, 10, 4096) CCF_LGKM
+                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3]),
+                     CCF_A2
+                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "v"(rb ^ 64), "v"(rb ^ 96), "n"(PITCH4)
+                   : "memory");
+    else
+      asm volatile(CCF_TR(0, 13) CCF_TRH(1, 13, 17) CCF_TR(2, 14) CCF_TRH(3, 14, 17) CCF_TR(4, 15) CCF_TRH(5, 15, 17) CCF_TR(6, 16)
+                   CCF_TRH(7, 16, 17) CCF_RD(8, 12, 0) CCF_RD(9, 12, 4096) CCF_RD(10, 12, 8192) CCF_RD(11, 12, 12288) CCF_LGKM
+                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3]),
+                     CCF_A4
+                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "v"(rb ^ 64), "v"(rb ^ 96), "n"(PITCH4)
+                   : "memory");
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) b[i] = __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// A [K][N] weight tile in LDS: 64 K rows of BN columns, the 32-byte chunks of each span of 128 columns XOR-swizzled by
+// the row (the layout of the 256-row tiles' main loop, gemm_tile.h).
+__device__ __forceinline__ int few_kn_swz(int row) { return (row & 3) | (((row >> 3) & 1) << 2); }
+
+// One lane's tile table entry.
+struct FewTile {
+  int e, row0, rows, n0;
+};
+
+__device__ __forceinline__ FewTile tile_at(const FewTile &mine, int r) {
+  return FewTile{__builtin_amdgcn_readlane(mine.e, r), __builtin_amdgcn_readlane(mine.row0, r),
+                 __builtin_amdgcn_readlane(mine.rows, r), __builtin_amdgcn_readlane(mine.n0, r)};
+}
+
+// The workgroup's `nr` (>= 1) tiles, one after the other.  mine: lane r holds tile r.
+template <class C, int kEpi, bool kKN>
+__device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, int nr, lds_char *lds) {
+  constexpr int TMW = C::TMW, NB = C::NB, S = C::STAGES;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 2, wn = wave & 3;
+  const int KT = p.K / kBK;
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+
+  // this lane's fragment chunk of its first blocks, per K half: row lane % 16, K chunk lane / 16
+  uint32_t a_off[2], b_off[2];
+  {
+    const int ra = wm * 16 + (lane & 15), rb = wn * (16 * NB) + (lane & 15);
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      const int c = sub * 4 + (lane >> 4);
+      a_off[sub] = lds_base + (ra * 8 + (c ^ swz<8>(ra))) * 16;
+      if constexpr (kKN) {
+        // source lane i of its group of 16 points at K row 8 * group + i / 4, columns 4 (i % 4) ..
+        const int i = lane & 15, row = sub * 32 + 8 * (lane >> 4) + (i >> 2), blk = wn * NB;
+        b_off[sub] = lds_base + C::A_BYTES + row * (2 * C::BN) + (blk >> 3) * 256 + ((few_kn_swz(row) ^ (blk & 7)) << 5) + ((i & 3) << 3);
+      } else {
+        b_off[sub] = lds_base + C::A_BYTES + (rb * 8 + (c ^ swz<8>(rb))) * 16;
+      }
+    }
+  }
+
+  // The load side runs STAGES - 1 stages ahead: tile `it`, K tile `ik` of it.  Load j of a wavefront is 1 KB at
+  // 1024 (8 j + wave) of the operand's part of the stage: eight 128-byte rows, or 1024 / (2 BN) K rows of a [K][N] tile.
+  const half_t *a_src[C::A_DMA], *b_src[C::B_DMA];
+  int it = 0, ik = 0;
+  const size_t b_step = kKN ? static_cast<size_t>(kBK) * p.N : kBK;
+  auto sources = [&](const FewTile &t) {
+    const half_t *Be = p.B + static_cast<size_t>(t.e) * p.N * p.K;
+#pragma unroll
+    for (int j = 0; j < C::A_DMA; ++j) {
+      const int r = (j * 8 + wave) * 8 + (lane >> 3);
+      int g = t.row0 + (r < t.rows ? r : t.rows - 1);              // padded tile rows re-read the last real row
+      if (p.a_rows) g = p.a_rows[g];
+      a_src[j] = p.A + static_cast<size_t>(g) * p.K + ((lane & 7) ^ swz<8>(r)) * 8;
+    }
+#pragma unroll
+    for (int j = 0; j < C::B_DMA; ++j) {
+      if constexpr (kKN) {
+        constexpr int UNITS = C::BN / 8;                           // 16-byte units of a K row
+        const int r = (j * 8 + wave) * (64 / UNITS) + lane / UNITS, u = lane % UNITS, chunk = u >> 1;
+        const int c = t.n0 + (chunk >> 3) * 128 + (((chunk & 7) ^ few_kn_swz(r)) << 4) + ((u & 1) << 3);
+        b_src[j] = Be + static_cast<size_t>(r) * p.N + (c < p.N - 8 ? c : p.N - 8);
+      } else {
+        const int r = (j * 8 + wave) * 8 + (lane >> 3);
+        const int n = (t.n0 + r) < p.N ? (t.n0 + r) : p.N - 1;
+        b_src[j] = Be + static_cast<size_t>(n) * p.K + ((lane & 7) ^ swz<8>(r)) * 8;
+      }
+    }
+  };
+  auto issue = [&](int stage) {
+    lds_char *base = lds + stage * C::STAGE;
+#pragma unroll
+    for (int j = 0; j < C::A_DMA; ++j) lds_dma16(a_src[j], base + (j * 8 + wave) * 1024);
+#pragma unroll
+    for (int j = 0; j < C::B_DMA; ++j) lds_dma16(b_src[j], base + C::A_BYTES + (j * 8 + wave) * 1024);
+    if (ik + 1 < KT) {
+      ++ik;
+#pragma unroll
+      for (int j = 0; j < C::A_DMA; ++j) a_src[j] += kBK;
+#pragma unroll
+      for (int j = 0; j < C::B_DMA; ++j) b_src[j] += b_step;
+    } else if (it + 1 < nr) {
+      ++it;
+      ik = 0;
+      sources(tile_at(mine, it));
+    }                                                              // past the end: the last K tile again, read by nobody
+  };
+  sources(tile_at(mine, 0));
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s) issue(s);
+
+  int stage = 0;
+  for (int r = 0; r < nr; ++r) {
+    const FewTile t = tile_at(mine, r);
+    const int live = (t.rows + 15) / 16;                           // 16-row blocks with real rows
+    float4v acc[TMW][NB];
+#pragma unroll
+    for (int tm = 0; tm < TMW; ++tm)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[tm][nb] = float4v{0, 0, 0, 0};
+    for (int kt = 0; kt < KT; ++kt) {
+      // this step's stage has landed for this wavefront (the later ones may be in flight), then for all; behind
+      // the barrier everyone is also done with the stage of the step before, which takes the next load
+      wait_vmcnt<(S - 2) * C::LOADS>();
+      block_barrier();
+      issue(stage == 0 ? S - 1 : stage - 1);
+      const uint32_t so = stage * C::STAGE;
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub) {
+        half8 a[TMW], b[NB];
+        if constexpr (kKN) few_frags_kn<TMW, NB, 8 * C::BN>(a, b, so + a_off[sub], so + b_off[sub]);
+        else few_frags<TMW, NB>(a, b, so + a_off[sub], so + b_off[sub]);
+        static_for<0, TMW>([&](auto I) {
+          constexpr int tm = I.value;
+          if (2 * tm + wm < live) {                                // uniform
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[tm][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[nb], a[tm], acc[tm][nb], 0, 0, 0);
+          }
+        });
+      }
+      stage = stage == S - 1 ? 0 : stage + 1;
+    }
+    // a lane holds one row and four consecutive columns of every block
+    const half_t *bias_e = p.bias + static_cast<size_t>(t.e) * p.N;
+    const int colb = t.n0 + wn * (16 * NB) + 4 * (lane >> 4);
+#pragma unroll
+    for (int tm = 0; tm < TMW; ++tm) {
+      const int lr = (2 * tm + wm) * 16 + (lane & 15);
+      if (2 * tm + wm >= live) break;                              // uniform
+      const bool real = lr < t.rows;
+      const int j = t.row0 + (real ? lr : t.rows - 1);
+      const size_t crow = p.c_rows ? static_cast<size_t>(p.c_rows[j]) : static_cast<size_t>(j);
+      const float sc = p.row_scale ? static_cast<float>(p.row_scale[j]) : 1.0f;
+      half_t *dst = p.C + crow * p.N;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const int col = colb + 16 * nb;
+        if (!real || col >= p.N) continue;
+        half4 bv = {0, 0, 0, 0};
+        if (p.bias) bv = *reinterpret_cast<const half4 *>(bias_e + col);
+        half4 o, pre;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          float x = acc[tm][nb][c] + static_cast<float>(bv[c]);
+          if (kEpi == kFewPlain) {
+            x *= sc;
+          } else {
+            pre[c] = static_cast<half_t>(x);
+            x = gelu_erf(x);
+          }
+          o[c] = static_cast<half_t>(x);
+        }
+        *reinterpret_cast<half4 *>(dst + col) = o;
+        if (kEpi == kFewGeluKeep) *reinterpret_cast<half4 *>(p.C2 + static_cast<size_t>(j) * p.N + col) = pre;
+      }
+    }
+  }
+  wait_vmcnt<0>();                                                 // no load into LDS outlives the workgroup
+}
+
+// Candidate tile shapes: index = 3 * (rows: 0 = 64, 1 = 128) + (columns: 0 = 64, 1 = 128, 2 = 256).
+constexpr int kFewShapes = 6;
+
+template <int kEpi, bool kKN>
+__global__ void __launch_bounds__(kFewThreads)
+few_rows_kernel(FewArgs p) {
+  __shared__ __attribute__((aligned(1024))) char buf[kFewLds];
+  int *s_off = reinterpret_cast<int *>(buf), *s_mt = s_off + 1056;  // tables of the tile search, before the pipeline starts
+  static_assert(2 * 1056 * sizeof(int) <= kFewLds, "tables of 1024 experts");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int E = p.E;
+  for (int e = tid; e <= E; e += kFewThreads) {
+    const int v = p.offsets[e];
+    s_off[e] = v < p.max_rows ? v : p.max_rows;                     // never past the caller's bound
+  }
+  __syncthreads();
+  // M tiles of each height over all experts (every wavefront for itself)
+  int m64 = 0, m128 = 0;
+  for (int e = lane; e < E; e += 64) {
+    int cnt = s_off[e + 1] - s_off[e];
+    cnt = cnt > 0 ? cnt : 0;
+    m64 += (cnt + 63) >> 6;
+    m128 += (cnt + 127) >> 7;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    m64 += __shfl_xor(m64, off, 64);
+    m128 += __shfl_xor(m128, off, 64);
+  }
+  // price the shapes, one per lane: rounds of tiles times the rows of both operands that a K step loads (of the
+  // measured shapes the best, or within 4 % of it, in every case above)
+  const int slots = gridDim.x >> 3;                                 // workgroups per XCD
+  const int ci = lane < kFewShapes ? lane : 0;
+  const int rsel = ci / 3, csel = ci - 3 * rsel;
+  const int mt_l = rsel == 0 ? m64 : m128;
+  const int per_x_l = (mt_l * ((p.N + (64 << csel) - 1) >> (6 + csel)) + 7) >> 3;
+  const int rounds_l = (per_x_l + slots - 1) / slots;
+  int key = INT_MAX;
+  if (lane < kFewShapes && rounds_l <= kFewMaxRounds && (!kKN || csel > 0)) {      // no [K][N] layout of 64 columns
+    key = (rounds_l * ((64 << rsel) + (64 << csel))) << 4 | lane;
+  }
+  if (lane == p.force && key != INT_MAX) key = lane;                // below every price
+#pragma unroll
+  for (int off = 4; off >= 1; off >>= 1) {
+    const int other = __shfl_xor(key, off, 64);
+    key = other < key ? other : key;
+  }
+  key = __builtin_amdgcn_readfirstlane(key);
+  const int shape = key & 15;
+  const int rs = shape / 3, cs = shape - 3 * rs;
+  const int MT = __builtin_amdgcn_readfirstlane(rs == 0 ? m64 : m128);
+  if (MT == 0) return;
+  const int n_col = (p.N + (64 << cs) - 1) >> (6 + cs);
+  const int T = MT * n_col, per_x = (T + 7) >> 3;
+  // exclusive scan of the chosen M tiles
+  if (tid < 64) {
+    int carry = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      int cnt = e0 + lane < E ? s_off[e0 + lane + 1] - s_off[e0 + lane] : 0;
+      cnt = cnt > 0 ? cnt : 0;
+      const int v = (cnt + (64 << rs) - 1) >> (6 + rs);
+      int inc = v;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += o;
+      }
+      if (e0 + lane < E) s_mt[e0 + lane] = carry + inc - v;
+      carry += __shfl(inc, 63, 64);
+    }
+    if (lane == 0) s_mt[E] = carry;
+  }
+  __syncthreads();
+  // workgroup j of XCD x has tiles x * per_x + j, + slots, ...; lane r finds tile r.  Tile order: expert, column
+  // range, M tile.
+  const int x = blockIdx.x & 7, first = blockIdx.x >> 3;
+  int left = T - x * per_x;
+  left = left < per_x ? left : per_x;                               // tiles of this XCD
+  const int nr = first < left ? (left - first + slots - 1) / slots : 0;
+  if (nr <= 0) return;
+  FewTile mine;
+  {
+    const int i = first + (lane < nr ? lane : 0) * slots;
+    const int t = x * per_x + i;
+    int lo = 0, hi = E - 1;                                         // last expert whose tiles start at or before t
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (s_mt[mid] * n_col <= t) lo = mid;
+      else hi = mid - 1;
+    }
+    const int mts = s_mt[lo + 1] - s_mt[lo], local = t - s_mt[lo] * n_col;
+    const int ct = local / mts, m = local - ct * mts;
+    const int cnt = s_off[lo + 1] - s_off[lo], r0 = m << (6 + rs), bm = 64 << rs;
+    mine.e = lo;
+    mine.row0 = s_off[lo] + r0;
+    mine.rows = cnt - r0 < bm ? cnt - r0 : bm;
+    mine.n0 = ct << (6 + cs);
+  }
+  __syncthreads();                                                  // the tables have been read
+  lds_char *lds = (lds_char *)buf;
+  auto go = [&](auto CI) {
+    constexpr int i = CI.value;
+    if constexpr (!kKN || i % 3 > 0)
+      if (shape == i) few_run<FewCfg<4 << (i / 3), 2 << (i % 3)>, kEpi, kKN>(p, mine, nr, lds);
+  };
+  static_for<0, kFewShapes>(go);
+}
+
+}  // namespace
+
+int g_few_rows = 1;          // 0: never, 1: by the rule below, 2: always, 16 + i: always and with tile shape i
+
+bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cus) {
+  if (!g_few_rows || epi > kFewGeluKeep || (b_kn && epi == kFewGeluKeep) || cus < 8 || K % kBK || E > 1024) return false;
+  // the tile table holds kFewMaxRounds tiles per workgroup of the largest shape
+  const long long worst = (static_cast<long long>(max_rows) / 128 + E) * ((N + 255) / 256);
+  if (worst >= static_cast<long long>(kFewMaxRounds - 1) * cus) return false;
+  if (g_few_rows >= 2) return true;
+  // The 256-row tiles do 1.48 PFLOP/s inside a K step, the largest tile here 0.9: they win where they fill the chip
+  // (150 rows per expert of 4096 / 14336: 225 and 225 us there, 306 and 278 here; 1024 rows of 768 / 3072, FFN1: 67 and
+  // 80), and lose where a few of them cannot (figures at the top).  Both priced in microseconds for evenly popular experts.  M tiles of an expert: the ceiling, which a load
+  // within two standard deviations of a whole number of tiles may miss by one either way.
+  const int used = E < max_rows ? E : max_rows;
+  const double avg = static_cast<double>(max_rows) / used, sd = std::sqrt(avg), kt = K / kBK;
+  auto near = [&](double gap) { return gap < 2 * sd ? 0.5 - 0.25 * gap / sd : 0.0; };
+  auto m_tiles = [&](int bm) {
+    const double base = std::ceil(avg / bm);
+    return used * (base + near(base * bm - avg) - (base > 1 ? near(avg - (base - 1) * bm) : 0.0));
+  };
+  const double epi_us = epi == kFewPlain ? 3 : 6;
+  double mine = 1e30;
+  for (int rs = 0; rs < 2; ++rs)
+    for (int cs = b_kn ? 1 : 0; cs < 3; ++cs) {
+      const int bm = 64 << rs, bn = 64 << cs;
+      const double rounds = std::ceil(m_tiles(bm) * ((N + bn - 1) / bn) / cus);
+      const double t = rounds * (kt * kFewStepUs[rs][cs] + epi_us * bm * bn / 32768);
+      mine = t < mine ? t : mine;
+    }
+  const double weights = 2.0 * used * N * K / 5.5e6;                // every weight once, from HBM
+  mine = (mine > weights ? mine : weights) + 6;
+  // 256 x 256 tiles: 1.45 us a K step and the epilogue; a last round of at most half the CUs is cut along K
+  const double tile = kt * 1.45 + (epi == kFewPlain ? 7 : 13);
+  const double rounds = m_tiles(256) * ((N + 255) / 256) / cus, full = std::floor(rounds), part = rounds - full;
+  double last = part > 0 ? tile : 0.0;
+  if (part > 0 && kt >= 64 && part <= 0.5) {
+    const double cut = kt / std::fmin(std::floor(1 / part), 8.0) * 1.45 + 35;
+    last = cut < tile ? cut : tile;
+  }
+  double big = full * tile + last;
+  big = (big > weights ? big : weights) + 6;
+  return mine < 0.95 * big;
+}
+
+int few_rows_gemm(FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {
+  p.force = g_few_rows >= 16 ? g_few_rows & 15 : -1;
+  void (*kernel)(FewArgs) = b_kn ? (epi == kFewPlain ? few_rows_kernel<kFewPlain, true> : few_rows_kernel<kFewGelu, true>)
+                                 : (epi == kFewPlain ? few_rows_kernel<kFewPlain, false>
+                                                     : (epi == kFewGelu ? few_rows_kernel<kFewGelu, false> : few_rows_kernel<kFewGeluKeep, false>));
+  hipLaunchKernelGGL(kernel, dim3(cus), dim3(kFewThreads), 0, stream, p);
+  return check_launch(what);
+}
+
+}  // namespace ccf

@@ -1146,7 +1146,8 @@ constexpr int kSplitTailMinKT = 64;
 int g_split_tail_min_kt = kSplitTailMinKT;
 int g_split_max_parts = 8;
 int g_fused_combine = 0;     // 1: top-2 layers add the gate-weighted expert outputs in the second GEMM's epilogue
-int g_skinny_pct = 70;       // a K step of a skinny tile in percent of a 256-row tile's (plan model); 0: no skinny tiles
+constexpr int kSkinnyPct = 70;
+int g_skinny_pct = kSkinnyPct;       // a K step of a skinny tile in percent of a 256-row tile's (plan model); 0: no skinny tiles
 int g_skinny_positions = 0;  // skinny ranges inside the persistent launch: 0 = a point per round of tiles, 2 = in front of / behind all tiles
 int g_split_inside = 1;      // 1: the parts of a split last round run inside the persistent launch, 0: as a launch of their own
 int g_skinny_tail = 0;       // 0: skinny tiles never run as a launch of their own
@@ -1156,7 +1157,7 @@ int g_skinny_tail = 0;       // 0: skinny tiles never run as a launch of their o
 // between the routing stage (which builds the plans of the layer's forward call) and the GEMMs.
 GemmOptions current_options() {
   return GemmOptions{g_variant, g_split_tail, g_split_tail_min_kt, g_split_max_parts, g_skinny_pct, g_fused_combine,
-                     g_skinny_tail};
+                     g_skinny_tail, g_few_rows};
 }
 
 // The kernels of one family of epilogues: `first` and `second` are two epilogue forms, each as
@@ -1303,6 +1304,12 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   return g;
 }
 
+// Few rows per expert: the kernel of few.hip, unless a knob asks for a form of the 256-row tiles.
+bool use_few_rows(int max_rows, int E, int N, int K, int epi, bool b_kn, const GemmOptions &opt) {
+  return opt.few_rows && opt.variant == kDefaultVariant && opt.skinny_pct == kSkinnyPct && opt.split_tail == 1 &&
+         opt.split_tail_min_kt == kSplitTailMinKT && few_rows_fits(max_rows, E, N, K, epi, b_kn, persistent_grid());
+}
+
 // plan_ready: the plan (and the split list) of this very call was already built in `region`
 // by forward_plan_request()'s request.
 int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets, int max_rows, int E,
@@ -1331,6 +1338,9 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
               "%s: operands must be 16-byte aligned", what);
   CCF_REQUIRE(!(gelu && row_scale), CCF_ERR_ARG, "%s: the GELU epilogue takes no row scale", what);
   if (max_rows == 0) return CCF_OK;
+  if (use_few_rows(max_rows, E, N, K, epi, b_kn, opt ? *opt : current_options()))
+    return few_rows_gemm(FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1}, epi,
+                         b_kn, persistent_grid(), stream, what);
   const GemmSetup gs = setup_gemm(max_rows, E, N, K, epi, b_kn, workspace, region, opt ? *opt : current_options());
   const Launch &v = *gs.v;
   const bool second = gs.second, split = gs.split;
@@ -1607,11 +1617,13 @@ int linear_backward(half_t *grad_out, const int32_t *g_rows, const half_t *in,
   const bool kn = !g_dgrad_transpose && static_cast<long long>(n_out) * n_in < (1ll << 31);
   const int dgrad_epi = gelu_pre ? kEpiGeluGrad : kEpiPlain;
   // the launch that lays out the K ranges also builds the tile plans of both GEMMs
-  const PlanReq rows_plan = setup_gemm(max_rows, E, n_in, n_out, dgrad_epi, kn, ws.plan_rows, 0, current_options()).req;
+  const GemmOptions opt = current_options();
+  const bool few = use_few_rows(max_rows, E, n_in, n_out, dgrad_epi, kn, opt);       // needs no plan
+  const PlanReq rows_plan = setup_gemm(max_rows, E, n_in, n_out, dgrad_epi, kn, ws.plan_rows, 0, opt).req;
   const PlanReq w_plan = wgrad_plan_request(E, n_out, n_in, ws.plan_w);
   const bool plans = max_rows > 0 && static_cast<long long>(E) * n_out < (1ll << 31);
   if (int rc = launch_kseg(offsets, E, max_rows, n_out, ws.n_blk, ws.k_seg, ws.row_off, ws.blk_row0,
-                           ws.blk_cnt, ws.row_lo, ws.zero_row, plans ? &rows_plan : nullptr, plans ? &w_plan : nullptr,
+                           ws.blk_cnt, ws.row_lo, ws.zero_row, plans && !few ? &rows_plan : nullptr, plans ? &w_plan : nullptr,
                            stream))
     return rc;
   // rows form: gathered gradient rows go to a_t as a plain [rows, n_out] matrix; rows already in expert order stay
@@ -1626,7 +1638,7 @@ int linear_backward(half_t *grad_out, const int32_t *g_rows, const half_t *in,
   CCF_REQUIRE(!gelu_pre || !gi_rows, CCF_ERR_ARG, "%s: the GELU gradient needs rows in expert order", what);
   if (int rc = grouped_gemm(grad_out, g_rows, offsets, max_rows, E, n_in, n_out, kn ? w : ws.w_t, nullptr,
                             dgrad_epi, grad_in, gi_rows, nullptr, ws.plan_rows, stream,
-                            what, kn, const_cast<half_t *>(gelu_pre), 0, plans))
+                            what, kn, const_cast<half_t *>(gelu_pre), 0, plans && !few, &opt))
     return rc;
   // weight and bias gradients
   const half_t *in_mat = (rows_form && !in_rows) ? in : ws.b_t;
@@ -1670,7 +1682,7 @@ extern "C" int ccf_set_option(const char *name, int value) {
                                              // launch of their own
     CCF_REQUIRE(value >= -kSkinnyMaxWgs - 2 && value <= 400, CCF_ERR_ARG, "set_option: skinny %d outside %d..400", value,
                 -kSkinnyMaxWgs - 2);
-    g_skinny_pct = value == 1 ? 70 : value;
+    g_skinny_pct = value == 1 ? kSkinnyPct : value;
     return CCF_OK;
   }
   if (!strcmp(name, "skinny_tail")) {
@@ -1691,6 +1703,12 @@ extern "C" int ccf_set_option(const char *name, int value) {
   }
   if (!strcmp(name, "wgrad_transpose")) {
     g_wgrad_transpose = value != 0;
+    return CCF_OK;
+  }
+  if (!strcmp(name, "few_rows")) {
+    CCF_REQUIRE((value >= 0 && value <= 2) || (value >= 16 && value < 22), CCF_ERR_ARG,
+                "set_option: few_rows %d is neither 0..2 nor 16..21", value);
+    g_few_rows = value;
     return CCF_OK;
   }
   if (!strcmp(name, "gate_waves")) {
@@ -1738,6 +1756,7 @@ bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *wo
                           PlanReq *out, bool w_kn) {
   if (!workspace || max_rows <= 0 || E <= 0 || E > 1024 || d <= 0 || f <= 0 || d % 64 || f % 64) return false;
   const int N = which == 1 ? f : d, K = which == 1 ? d : f;
+  if (use_few_rows(max_rows, E, N, K, which == 1 ? kEpiGelu : (which == 3 ? kEpiCombine : kEpiPlain), w_kn, opt)) return false;
   const GemmSetup gs = setup_gemm(max_rows, E, N, K, which == 1 ? kEpiGelu : (which == 3 ? kEpiCombine : kEpiPlain),
                                   w_kn, workspace, which == 1 ? 0 : 1, opt);
   if (gs.wgs >= (1ll << 24)) return false;
@@ -1836,6 +1855,7 @@ extern "C" int ccf_ffn_plan_info(const void *workspace, int max_rows, int num_ex
   const GemmSetup gs = setup_gemm(max_rows, num_expert, N, K, which == 1 ? kEpiGelu : kEpiPlain, false,
                                   const_cast<void *>(workspace), which == 1 ? 0 : 1, current_options());
   for (int i = 0; i < 8; ++i) info[i] = 0;
+  if (use_few_rows(max_rows, num_expert, N, K, which == 1 ? kEpiGelu : kEpiPlain, false, current_options())) return CCF_OK;   // no plan
   hipStream_t st = as_stream(stream);
   hipError_t e = hipSuccess;
   if (gs.split || gs.cut) e = hipMemcpyAsync(info, gs.tail, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, st);

@@ -495,7 +495,7 @@ __device__ inline void build_plan(const PlanReq &rq, const int32_t *__restrict__
 // ffn.hip
 // Snapshot of the tuning knobs (ccf_set_option) that a grouped GEMM's plan and launches depend on.
 struct GemmOptions {
-  int variant, split_tail, split_tail_min_kt, split_max_parts, skinny_pct, fused_combine, skinny_tail;
+  int variant, split_tail, split_tail_min_kt, split_max_parts, skinny_pct, fused_combine, skinny_tail, few_rows;
 };
 GemmOptions forward_options();
 bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *workspace, const GemmOptions &opt,
@@ -535,6 +535,24 @@ int blocks_with_plans(const int64_t *pos, int n_pos, int top_k, int n_tokens, co
                       const int32_t *lens, const int32_t *starts, int n_blocks, int block_size, int num_expert,
                       int32_t *counts, int32_t *offsets, int32_t *token_rows, int32_t *flat_rows, hipStream_t stream,
                       const PlanReq *plans, int n_plans);
+// few.hip: the forward GEMMs of few rows per expert.  C[c_rows[j]] = epilogue(A[a_rows[j]] * B[e]^T + bias[e]) for the
+// rows offsets[e] <= j < offsets[e+1]; the forms are those of the grouped GEMM's epilogues 0, 1 and 2.
+constexpr int kFewPlain = 0, kFewGelu = 1, kFewGeluKeep = 2;
+struct FewArgs {
+  const half_t *A;
+  const int32_t *a_rows;     // or NULL (identity)
+  const half_t *B, *bias;    // [E, N, K], [E, N] or NULL
+  half_t *C, *C2;            // C2: pre-activations in expert order (kFewGeluKeep)
+  const int32_t *c_rows;     // or NULL (identity)
+  const half_t *row_scale;   // or NULL
+  const int32_t *offsets;
+  int max_rows, E, N, K;
+  int force;                 // tile shape, or -1: chosen by the kernel; filled in by few_rows_gemm
+};
+bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cus);
+int few_rows_gemm(FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what);
+extern int g_few_rows;
+
 // most entries of a table of per-run expert counts that the routing stage takes from the gate kernel
 long long route_rows_max_ints();
 

@@ -78,6 +78,10 @@ const char *ccf_last_error(void);
  *   "skinny_positions" 0 (default) or n >= 2: over how many points in time the fourth way spreads the
  *                     workgroups' ranges (0: one in front of every round of tiles and one behind the last;
  *                     2: half of the workgroups in front of all their tiles, half behind)
+ *   "few_rows"        1 (default): a forward or input-gradient GEMM whose 256-row tiles would leave most of the
+ *                     chip idle (few rows per expert, small layers) runs as tiles of 64 or 128 rows in a kernel that
+ *                     needs no plan; 0 = never, 2 = always, 16..21 = always, and with that tile shape.  The knobs
+ *                     above apply to the 256-row tiles: with any of the first six away from its default, they are used
  *   "fused_combine"   0/1 (default 0): ccf_moe_forward with top_k = 2 adds the gate-weighted expert outputs
  *                     into the output in the second GEMM's epilogue (packed fp16 atomic adds onto zeros)
  *                     instead of running the combine pass; measured slower, kept for comparison

@@ -487,6 +487,62 @@ def test_eight_wavefront_kernel_gives_the_four_wavefront_bits(R, d, f, E, skew, 
     assert torch.equal(res[2][1], res[3][1]), "second GEMM"
 
 
+@pytest.mark.parametrize("shape", range(6))
+@pytest.mark.parametrize("counts,N,K", [
+    ([0, 1, 63, 64, 65, 127, 128, 129, 0], 264, 64),          # edges of both tile heights, a ragged last column tile
+    ([300, 0, 17], 72, 320),                                  # several M tiles per expert; columns end inside the first tile
+    ([2] * 70, 520, 192),                                     # more experts than lanes, several tiles per workgroup
+    ([40], 8, 1024),                                          # one expert, the narrowest output
+])
+def test_few_rows_kernel(shape, counts, N, K):
+    """Every tile shape of the kernel for few rows per expert, both weight layouts and all epilogues, through row
+    indices: the bits of the 256-row tiles, which add over K in the same order, and the fp32 product."""
+    from ccfuser_amd import ops
+    g = torch.Generator().manual_seed(shape * 100 + N)
+    E, R = len(counts), sum(counts)
+    pad = 5                                                   # max_rows may exceed the rows
+    _say(f"few rows shape={shape} E={E} R={R} N={N} K={K}")
+    x = dev(torch.randn(R + 9, K, generator=g).half())
+    w = dev((torch.randn(E, N, K, generator=g) * K ** -0.5).half())
+    b = dev(torch.randn(E, N, generator=g).half())
+    off = dev(torch.tensor([0] + counts).cumsum(0).int())
+    src = dev(torch.cat([torch.randperm(R + 9, generator=g)[:R], torch.zeros(pad, dtype=torch.int64)]).int())
+    dst = dev(torch.cat([torch.randperm(R, generator=g), torch.zeros(pad, dtype=torch.int64)]).int())
+    wk = w.transpose(1, 2).contiguous()
+    scale = dev(torch.rand(R + pad, generator=g).half())
+
+    def outputs():
+        res = [ops.ffn1(x, src, off, R + pad, w, b, gelu=True, out=torch.zeros(R, N, dtype=torch.float16, device="cuda"), dst_row=dst),
+               ops.ffn1(x, src, off, R + pad, wk, b, gelu=True, out=torch.zeros(R, N, dtype=torch.float16, device="cuda"),
+                        dst_row=dst, w_kn=True)]
+        for ww, kn in ((w, False), (wk, True)):
+            res.append(ops.ffn2(x, dst, off, R + pad, ww, b, torch.zeros(R, N, dtype=torch.float16, device="cuda"), src_row=src,
+                                row_scale=scale, w_kn=kn))
+        act, pre = ops.ffn1_keep(x, src, off, R + pad, w, b)
+        torch.cuda.synchronize()
+        return res + [act[:R], pre[:R]]
+
+    ops.set_option("few_rows", 16 + shape)
+    try:
+        got = outputs()
+        ops.set_option("few_rows", 0)
+        ops.set_option("split_tail", 0)
+        ops.set_option("skinny", 0)
+        tiles = outputs()
+    finally:
+        ops.set_option("few_rows", 1)
+        ops.set_option("split_tail", 1)
+        ops.set_option("skinny", 1)
+    for i, (a, t) in enumerate(zip(got, tiles)):
+        assert torch.equal(a, t), f"output {i} differs from the 256-row tiles"
+    e_of = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).cuda()
+    pre = torch.cat([x[src[:R].long()][e_of == e].float() @ w[e].float().t() + b[e].float() for e in range(E)])
+    assert O.mean_rel_err(got[5].cpu(), pre.cpu()) <= MEAN_REL
+    plain = torch.zeros_like(pre)
+    plain[dst[:R].long()] = pre * scale[:R, None].float()
+    assert O.mean_rel_err(got[2].cpu(), plain.cpu()) <= MEAN_REL
+
+
 def test_ffn_special_cases():
     """Closed forms: zero weights give the bias path; a single expert is a dense MLP."""
     from ccfuser_amd import ops
