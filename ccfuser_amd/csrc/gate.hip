@@ -950,8 +950,198 @@ gate_bias_reduce_kernel(const float *__restrict__ partial, int n_wg, int E, half
   grad_bias[e] = static_cast<half_t>(acc);
 }
 
+// ---- the whole backward of the gate ------------------------------------------------------
+// A token has k selected experts, so both products with the [T, E] gradient of the logits are sparse:
+//   grad_x[t, :] = sum_j g[t, j] wg[e(t, j), :],   grad_wg[e, :] = sum over the (t, j) with e(t, j) = e of g[t, j] x[t, :],
+// and the dense matrix is never made.  A workgroup takes a run of tokens and 512 columns, two per thread: it reads
+// x once, writes grad_x, and adds the expert rows up in LDS, where a thread alone touches its two columns
+// of every expert, so the order is the tokens' and two runs agree bit for bit.  gate_products_reduce_kernel adds the
+// workgroups' partial rows in order and rounds once.  Bound by the chain of LDS additions of a run and by reading x and
+// writing grad_x.  Against the softmax kernel, its reduction and two library products, GPU time: 1000 tokens of 256, 16
+// experts 33 -> 16 us, 1999 of 768, 8: 22 -> 18, 4096 of 4096, 8: 42 -> 33, 32768 of 768, 8: 150 -> 65; and two launches
+// instead of four, the products' 15 us of host time each (1999 tokens, host included: 58 -> 23).  More than 16 experts
+// keep the products: the sums take so much LDS that a CU has one workgroup (8192 of 1024, 32: 47 against 57).
+//
+// A wavefront holds the values of 64 tokens in its lanes and broadcasts them through scalar registers; the expert
+// rows of wg sit in LDS, and the sums are plain reads and writes there (LDS float atomics run at ~190 cycles an
+// instruction: 91 us instead of 18 for the 1999 tokens).
+constexpr int kGpCols = 512;
+constexpr int kGpMaxExpert = 16;                     // [E][512] floats and [E][512] halves of LDS: 48 KB
+
+template <int KS>                                    // top_k <= KS
+__global__ void __launch_bounds__(256)
+gate_products_kernel(const half_t *__restrict__ score, const half_t *__restrict__ grad_score,
+                     const int64_t *__restrict__ idx, const half_t *__restrict__ x, const half_t *__restrict__ wg,
+                     int tokens, int top_k, int E, int d, int run, half_t *__restrict__ grad_x,
+                     float *__restrict__ partial /* [n_run][E][d], or NULL */,
+                     float *__restrict__ partial_b /* [n_run][E], or NULL */) {
+  extern __shared__ float s_rows[];                  // [E][512] sums, then [E][512] halves of wg
+  half_t *s_wg = reinterpret_cast<half_t *>(s_rows + E * kGpCols);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int c = blockIdx.x * kGpCols + 2 * t;
+  const bool in = c < d;                             // d is even
+  const int cc = in ? c : 0;
+  const int tok0 = blockIdx.y * run, tok1 = tok0 + run < tokens ? tok0 + run : tokens;
+  // a thread reads and writes its own two columns only: no barrier
+  for (int e0 = 0; e0 < E; e0 += 8) {
+    half2v w[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) w[u] = *reinterpret_cast<const half2v *>(wg + static_cast<size_t>(e0 + u < E ? e0 + u : E - 1) * d + cc);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (e0 + u < E) {
+        *reinterpret_cast<float2 *>(s_rows + (e0 + u) * kGpCols + 2 * t) = float2{0.0f, 0.0f};
+        *reinterpret_cast<half2v *>(s_wg + (e0 + u) * kGpCols + 2 * t) = w[u];
+      }
+  }
+  float bias = 0.0f;                                 // first wavefront of the first column range: expert = lane
+  const bool want_b = partial_b && blockIdx.x == 0 && wave == 0;
+  for (int base = tok0; base < tok1; base += 64) {
+    const int n = tok1 - base < 64 ? tok1 - base : 64;
+    float g[KS];
+    int ex[KS];
+    {
+      const size_t at = static_cast<size_t>(base + (lane < n ? lane : n - 1)) * top_k;
+      float dot = 0.0f, s[KS];
+#pragma unroll
+      for (int j = 0; j < KS; ++j) {
+        const bool on = j < top_k;
+        s[j] = on ? static_cast<float>(score[at + (on ? j : 0)]) : 0.0f;
+        g[j] = on ? static_cast<float>(grad_score[at + (on ? j : 0)]) : 0.0f;
+        const int64_t e = on ? idx[at + (on ? j : 0)] : -1;
+        ex[j] = e >= 0 && e < E ? static_cast<int>(e) : -1;
+        if (on) dot = fmaf(s[j], g[j], dot);
+      }
+#pragma unroll
+      for (int j = 0; j < KS; ++j) {
+        g[j] = ex[j] >= 0 ? s[j] * (g[j] - dot) : 0.0f;
+        ex[j] = ex[j] >= 0 ? ex[j] : 0;              // nobody's choice: adds zero
+      }
+    }
+    constexpr int U = 8;                             // tokens whose loads leave together
+    for (int q0 = 0; q0 < n; q0 += U) {
+      half2v xv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u < n ? q0 + u : n - 1;
+        xv[u] = *reinterpret_cast<const half2v *>(x + static_cast<size_t>(base + q) * d + cc);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u;
+        if (q >= n) break;                           // uniform
+        const float x0 = static_cast<float>(xv[u][0]), x1 = static_cast<float>(xv[u][1]);
+        float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+          if (j >= top_k) break;
+          const float gj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g[j]), q));
+          const int e = __builtin_amdgcn_readlane(ex[j], q);
+          const half2v w = *reinterpret_cast<const half2v *>(s_wg + e * kGpCols + 2 * t);
+          a0 = fmaf(gj, static_cast<float>(w[0]), a0);
+          a1 = fmaf(gj, static_cast<float>(w[1]), a1);
+          float *row = s_rows + e * kGpCols + 2 * t;
+          float2 sum = *reinterpret_cast<const float2 *>(row);
+          sum.x = fmaf(gj, x0, sum.x);
+          sum.y = fmaf(gj, x1, sum.y);
+          *reinterpret_cast<float2 *>(row) = sum;
+          if (want_b) bias += lane == e ? gj : 0.0f;
+        }
+        if (grad_x && in)
+          *reinterpret_cast<half2v *>(grad_x + static_cast<size_t>(base + q) * d + c) = half2v{static_cast<half_t>(a0), static_cast<half_t>(a1)};
+      }
+    }
+  }
+  if (partial && in) {
+    float *out = partial + static_cast<size_t>(blockIdx.y) * E * d + c;
+    for (int e = 0; e < E; ++e)
+      *reinterpret_cast<float2 *>(out + static_cast<size_t>(e) * d) = *reinterpret_cast<const float2 *>(s_rows + e * kGpCols + 2 * t);
+  }
+  if (want_b && lane < E) partial_b[static_cast<size_t>(blockIdx.y) * E + lane] = bias;
+}
+
+// grad_wg (two columns per thread) and, in the workgroups behind them, grad_bias from the runs' partial sums, in order
+__global__ void __launch_bounds__(256)
+gate_products_reduce_kernel(const float *__restrict__ partial, const float *__restrict__ partial_b, int n_run, int E, int d,
+                            half_t *__restrict__ grad_w, half_t *__restrict__ grad_bias, int w_wgs) {
+  if (static_cast<int>(blockIdx.x) >= w_wgs) {
+    const int e = threadIdx.x;
+    if (e >= E) return;
+    float acc = 0.0f;
+    for (int r = 0; r < n_run; ++r) acc += partial_b[static_cast<size_t>(r) * E + e];
+    grad_bias[e] = static_cast<half_t>(acc);
+    return;
+  }
+  const size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 2, n = static_cast<size_t>(E) * d;
+  if (i >= n) return;
+  float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll 16
+  for (int r = 0; r < n_run; ++r) {
+    const float2 v = *reinterpret_cast<const float2 *>(partial + static_cast<size_t>(r) * n + i);
+    a0 += v.x;
+    a1 += v.y;
+  }
+  *reinterpret_cast<half2v *>(grad_w + i) = half2v{static_cast<half_t>(a0), static_cast<half_t>(a1)};
+}
+
+// Tokens per run: about two workgroups per CU, and runs of 32 and more, which keeps the sums of the reduction short.
+int products_run(int tokens, int d) {
+  const int chunks = (d + kGpCols - 1) / kGpCols;
+  const int most = 512 / chunks < 16 ? 16 : 512 / chunks;
+  const int run = (tokens + most - 1) / most;
+  return (run + 31) / 32 * 32;
+}
+
 }  // namespace
 }  // namespace ccf
+
+extern "C" size_t ccf_gate_backward_products_workspace_bytes(int tokens, int d_model, int tot_expert) {
+  if (tokens <= 0 || d_model <= 0 || tot_expert <= 0 || tot_expert > ccf::kGpMaxExpert) return 0;
+  const int run = ccf::products_run(tokens, d_model);
+  return sizeof(float) * static_cast<size_t>((tokens + run - 1) / run) * tot_expert * (static_cast<size_t>(d_model) + 1);
+}
+
+extern "C" int ccf_gate_backward_products(const void *score, const void *grad_score, const int64_t *idx, const void *x,
+                                          const void *wg, int tokens, int d_model, int tot_expert, int top_k, void *grad_x,
+                                          void *grad_wg, void *grad_bias, void *workspace, size_t workspace_bytes,
+                                          ccf_stream_t stream) {
+  using namespace ccf;
+  CCF_REQUIRE(score && grad_score && idx && x && wg && (grad_x || grad_wg || grad_bias), CCF_ERR_ARG,
+              "gate_backward_products: null pointer");
+  CCF_REQUIRE(tokens > 0 && d_model > 0 && d_model % 2 == 0 && tot_expert > 0 && tot_expert <= kGpMaxExpert, CCF_ERR_SHAPE,
+              "gate_backward_products: %d tokens of %d and %d experts (tokens, an even width and 1..%d experts)", tokens,
+              d_model, tot_expert, kGpMaxExpert);
+  CCF_REQUIRE(top_k >= 1 && top_k <= kMaxTopK && top_k <= tot_expert, CCF_ERR_SHAPE,
+              "gate_backward_products: top_k=%d outside 1..min(%d, tot_expert=%d)", top_k, kMaxTopK, tot_expert);
+  const auto aligned4 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; };
+  CCF_REQUIRE(aligned4(x) && aligned4(wg) && aligned4(grad_x) && aligned4(grad_wg), CCF_ERR_ARG,
+              "gate_backward_products: operands must be 4-byte aligned");
+  const size_t need = ccf_gate_backward_products_workspace_bytes(tokens, d_model, tot_expert);
+  CCF_REQUIRE(workspace && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0, CCF_ERR_WORKSPACE,
+              "gate_backward_products: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+  const int run = products_run(tokens, d_model), n_run = (tokens + run - 1) / run;
+  float *partial = static_cast<float *>(workspace);
+  float *partial_b = partial + static_cast<size_t>(n_run) * tot_expert * d_model;
+  const size_t lds = (sizeof(float) + sizeof(half_t)) * kGpCols * tot_expert;
+  const auto kernel = top_k <= 2 ? gate_products_kernel<2> : gate_products_kernel<kMaxTopK>;
+  if (lds > 32768) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       static_cast<int>(lds));
+    if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate_backward_products: LDS attribute: %s", hipGetErrorString(e));
+  }
+  hipLaunchKernelGGL(kernel, dim3((d_model + kGpCols - 1) / kGpCols, n_run), dim3(256), lds, as_stream(stream),
+                     static_cast<const half_t *>(score), static_cast<const half_t *>(grad_score), idx,
+                     static_cast<const half_t *>(x), static_cast<const half_t *>(wg), tokens, top_k, tot_expert, d_model, run,
+                     static_cast<half_t *>(grad_x), grad_wg ? partial : nullptr, grad_bias ? partial_b : nullptr);
+  if (int rc = check_launch("gate_products_kernel")) return rc;
+  if (!grad_wg && !grad_bias) return CCF_OK;
+  const size_t pairs = static_cast<size_t>(tot_expert) * d_model / 2;
+  const int w_wgs = grad_wg ? static_cast<int>((pairs + 255) / 256) : 0;
+  hipLaunchKernelGGL(gate_products_reduce_kernel, dim3(w_wgs + (grad_bias ? 1 : 0)), dim3(256), 0, as_stream(stream), partial,
+                     partial_b, n_run, tot_expert, d_model, static_cast<half_t *>(grad_wg), static_cast<half_t *>(grad_bias),
+                     w_wgs);
+  return check_launch("gate_products_reduce_kernel");
+}
 
 extern "C" size_t ccf_gate_backward_workspace_bytes(int tokens, int tot_expert) {
   if (tokens <= 0 || tot_expert <= 0) return 0;

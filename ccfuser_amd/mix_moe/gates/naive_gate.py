@@ -21,9 +21,10 @@ def _zero_on(device):
 class _GateFunction(torch.autograd.Function):
     """The fused gate kernel with the backward autograd derives for the reference's
     linear -> topk -> softmax (naive_gate.py:31-38): softmax over the k selected
-    logits, the selection as a scatter into [T, E], then the linear layer.  For fp16 the
-    first two are one HIP kernel (``ops.gate_backward``); the two products with the [T, E]
-    gradient are small library GEMMs."""
+    logits, the selection as a scatter into [T, E], then the linear layer.  In fp16 with up
+    to 16 experts that is one HIP kernel and a reduction (``ops.gate_backward_products``),
+    which use that a token has k experts only; otherwise the first two are one HIP kernel
+    (``ops.gate_backward``) and the two products with the [T, E] gradient library GEMMs."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, top_k, return_logits):
@@ -45,6 +46,10 @@ class _GateFunction(torch.autograd.Function):
         if grad_score is None:                           # the scores were not used
             return None, None, None, None, None
         want_bias = ctx.has_bias and ctx.needs_input_grad[2]
+        if not torch.is_grad_enabled() and ops.gate_products_fit(x, weight):     # grad mode is on for create_graph
+            grad_x, grad_w, grad_b = ops.gate_backward_products(score, grad_score.contiguous(), idx, x, weight,
+                                                                ctx.needs_input_grad[0], ctx.needs_input_grad[1], want_bias)
+            return grad_x, grad_w, grad_b, None, None
         if x.dtype == torch.float16:
             g16, grad_b = ops.gate_backward(score, grad_score.contiguous(), idx, weight.shape[0], want_bias)
         else:

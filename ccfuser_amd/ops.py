@@ -91,6 +91,35 @@ def gate_backward(score: torch.Tensor, grad_score: torch.Tensor, idx: torch.Tens
     return g_logits, g_bias
 
 
+def gate_backward_products(score: torch.Tensor, grad_score: torch.Tensor, idx: torch.Tensor, x: torch.Tensor,
+                           weight: torch.Tensor, want_x: bool = True, want_weight: bool = True, want_bias: bool = True):
+    """(grad_x [T, d], grad_weight [E, d], grad_bias [E]) of the fp16 gate, each None when not wanted.
+    At most 16 experts (``gate_products_fit``)."""
+    for t, nm in ((score, "score"), (grad_score, "grad_score"), (x, "x"), (weight, "gate weight")):
+        _check(t, nm, dtype=torch.float16, ndim=2)
+    _check(idx, "idx", dtype=torch.int64, ndim=2)
+    T, k = score.shape
+    E, d = weight.shape
+    if grad_score.shape != score.shape or idx.shape != score.shape or tuple(x.shape) != (T, d):
+        raise ValueError("gate_backward_products: shapes do not match")
+    g_x = torch.empty_like(x) if want_x else None
+    g_w = torch.empty_like(weight) if want_weight else None
+    g_b = torch.empty(E, dtype=torch.float16, device=x.device) if want_bias else None
+    if want_x or want_weight or want_bias:
+        with torch.cuda.device(x.device):
+            ws = _workspace(_lib.lib().ccf_gate_backward_products_workspace_bytes(T, d, E), x)
+            _lib.call("ccf_gate_backward_products", _ptr(score), _ptr(grad_score), _ptr(idx), _ptr(x), _ptr(weight), T, d,
+                      E, k, _ptr(g_x), _ptr(g_w), _ptr(g_b), _ptr(ws), ws.numel(), _stream(x))
+    return g_x, g_w, g_b
+
+
+def gate_products_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``gate_backward_products`` takes these operands."""
+    return (x.dtype == torch.float16 and weight.dtype == torch.float16 and x.is_contiguous() and weight.is_contiguous()
+            and x.shape[0] > 0 and x.shape[1] % 2 == 0 and weight.shape[0] <= 16
+            and x.data_ptr() % 4 == 0 and weight.data_ptr() % 4 == 0)
+
+
 # --------------------------------------------------------------- routing
 def expert_count(gate_idx: torch.Tensor, expert_count_out: torch.Tensor) -> None:
     """Accumulate the histogram of ``gate_idx`` into ``expert_count_out`` (int32)."""

@@ -116,6 +116,39 @@ def test_gate_backward_of_softmax_and_selection(T, k, E, seed):
     assert none is None and torch.equal(gl3, gl)
 
 
+@pytest.mark.parametrize("T,d,E,k", [(1, 2, 1, 1), (63, 510, 8, 2), (65, 514, 9, 1), (257, 512, 16, 8), (1999, 768, 8, 2),
+                                     (5000, 130, 16, 2), (1100, 16386, 5, 3)])
+def test_gate_backward_products(T, d, E, k):
+    """The gate's input, weight and bias gradients from the k selected experts only, against the dense products in
+    fp64: each within one rounding of fp16 plus a fp32 sum; two runs give the same bits."""
+    from ccfuser_amd import ops
+    g = torch.Generator().manual_seed(T + d)
+    x, w = torch.randn(T, d, generator=g).half(), (torch.randn(E, d, generator=g) * 0.1).half()
+    idx = torch.rand(T, E, generator=g).topk(k, -1).indices
+    score = torch.softmax(torch.randn(T, k, generator=g), -1).half()
+    gs = torch.randn(T, k, generator=g).half()
+    args = [t.cuda() for t in (score, gs, idx, x, w)]
+    got = ops.gate_backward_products(*args)
+    again = ops.gate_backward_products(*args)
+    only_w = ops.gate_backward_products(*args, want_x=False, want_bias=False)
+    torch.cuda.synchronize()
+    s, q = score.double(), gs.double()
+    val = s * (q - (s * q).sum(-1, keepdim=True))
+    dense = torch.zeros(T, E, dtype=torch.float64).scatter_(1, idx, val)
+    mag = torch.zeros(T, E, dtype=torch.float64).scatter_(1, idx, s * (q.abs() + (s * q).abs().sum(-1, keepdim=True)))
+    # fp16 rounds by half a unit in 2^11 (absolute below 2^-14); a sum of n terms, and the cancellation inside val, by
+    # n units in 2^24 of the sum of magnitudes
+    for out, ref, terms, n in ((got[0], dense @ w.double(), mag @ w.double().abs(), k),
+                               (got[1], dense.t() @ x.double(), mag.t() @ x.double().abs(), T),
+                               (got[2], dense.sum(0), mag.sum(0), T)):
+        err = (out.cpu().double() - ref).abs()
+        bound = ref.abs() * 2.0 ** -11 + 2.0 ** -25 + terms * (min(n, 600) + 8) * 2.0 ** -24
+        assert (err <= bound).all(), (err - bound).max()
+    for a, b in zip(got, again):
+        assert torch.equal(a, b)
+    assert only_w[0] is None and only_w[2] is None and torch.equal(only_w[1], got[1])
+
+
 @pytest.mark.parametrize("mode", [-1, -3, -5, -6, 1])
 def test_input_gradient_with_skinny_tiles(mode):
     """The input-gradient GEMM on the stored [K][N] weight with every expert's remainder rows
