@@ -26,6 +26,7 @@ SIGNATURES = {
     "ccf_set_option": (_i, [C.c_char_p, _i]),
     "ccf_gate_topk_softmax": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p]),
     "ccf_gate_backward_workspace_bytes": (_sz, [_i, _i]),
+    "ccf_zero_ranges": (_i, [_p, _sz, _p, _sz, _p]),
     "ccf_gate_backward_products_workspace_bytes": (_sz, [_i, _i, _i]),
     "ccf_gate_backward_products": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _sz, _p]),
     "ccf_gate_backward": (_i, [_p, _p, _p, _i, _i, _i, _p, _p, _p, _sz, _p]),

@@ -245,6 +245,17 @@ int launch_zero(half_t *dst, size_t halves, hipStream_t stream) {
   return check_launch("zero_kernel");
 }
 
+// Two ranges in one launch: the first `wgs_a` workgroups take the first.
+__global__ void __launch_bounds__(256)
+zero_ranges_kernel(half_t *__restrict__ a, size_t chunks_a, half_t *__restrict__ b, size_t chunks_b, int wgs_a) {
+  const half8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+  const bool first = static_cast<int>(blockIdx.x) < wgs_a;
+  half8 *dst = reinterpret_cast<half8 *>(first ? a : b);
+  const size_t chunks = first ? chunks_a : chunks_b;
+  const size_t wgs = first ? wgs_a : gridDim.x - wgs_a, wg = first ? blockIdx.x : blockIdx.x - wgs_a;
+  for (size_t c = wg * 256 + threadIdx.x; c < chunks; c += wgs * 256) dst[c] = z;
+}
+
 int padded_rows(int max_rows, int E) {
   return static_cast<int>(round_up(static_cast<size_t>(max_rows) + static_cast<size_t>(kPadK) * E, kTile));
 }
@@ -297,6 +308,21 @@ int launch_bias_reduce(const float *partial, const int32_t *k_seg, int E, int C,
 }
 
 }  // namespace ccf
+
+extern "C" int ccf_zero_ranges(void *a, size_t halves_a, void *b, size_t halves_b, ccf_stream_t stream) {
+  using namespace ccf;
+  CCF_REQUIRE((a || !halves_a) && (b || !halves_b), CCF_ERR_ARG, "zero_ranges: null pointer");
+  CCF_REQUIRE(halves_a % 8 == 0 && halves_b % 8 == 0 && aligned16(a) && aligned16(b), CCF_ERR_SHAPE,
+              "zero_ranges: ranges must be whole, aligned groups of 16 bytes");
+  if (!halves_a && !halves_b) return CCF_OK;
+  const auto wgs = [](size_t halves) {
+    const size_t n = (halves / 8 + 255) / 256;
+    return static_cast<int>(n < 4096 ? n : 4096);
+  };
+  hipLaunchKernelGGL(zero_ranges_kernel, dim3(wgs(halves_a) + wgs(halves_b)), dim3(256), 0, as_stream(stream),
+                     static_cast<half_t *>(a), halves_a / 8, static_cast<half_t *>(b), halves_b / 8, wgs(halves_a));
+  return check_launch("zero_ranges_kernel");
+}
 
 extern "C" int ccf_combine_backward(const void *grad_out, const void *y_flat, const void *score,
                                     const int32_t *inv_pos, int tokens, int top_k, int hidden,

@@ -39,8 +39,11 @@ def _param_grads(weight, E):
     grad_w = torch.empty_like(weight)
     grad_b = torch.empty(weight.shape[0], weight.shape[1], dtype=weight.dtype, device=weight.device)
     if weight.shape[0] > E:
-        grad_w[E:].zero_()
-        grad_b[E:].zero_()
+        if weight.dtype == torch.float16 and weight.is_contiguous() and weight.shape[1] % 8 == 0:
+            ops.zero_tails(grad_w, grad_b, E)
+        else:
+            grad_w[E:].zero_()
+            grad_b[E:].zero_()
     return grad_w, grad_b
 
 

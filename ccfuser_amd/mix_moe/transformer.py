@@ -68,6 +68,19 @@ class BlockInfos(dict):
         return dict.__getitem__(self, key)
 
 
+def _any_requires_grad(module):
+    """``any(p.requires_grad for p in module.parameters())`` without the generators over names, which cost more host
+    time than the launches of a small layer."""
+    todo = [module]
+    while todo:
+        m = todo.pop()
+        for p in m._parameters.values():
+            if p is not None and p.requires_grad:
+                return True
+        todo.extend(c for c in m._modules.values() if c is not None)
+    return False
+
+
 class _Expert(nn.Module):
     """Two grouped linear layers with an activation between them
     (reference transformer.py:70-91)."""
@@ -236,15 +249,12 @@ class MixMOETransformerMLP(MixMOE):
             self.async_ = False
             output = super().forward(inp, pos, gate_score, infos)
         elif self.fused and self.experts._gelu_is_fusable() and not (
-                torch.is_grad_enabled() and (inp.requires_grad or
-                                             any(p.requires_grad for p in self.parameters()))):
+                torch.is_grad_enabled() and (inp.requires_grad or _any_requires_grad(self))):
             ex = self.experts
             with torch.no_grad():
-                output = ops.moe_forward(inp, self.gate.gate.weight.detach(),
-                                         None if self.gate.gate.bias is None else self.gate.gate.bias.detach(),
-                                         ex.htoh4.weight.detach()[:E], ex.htoh4.bias.detach()[:E],
-                                         ex.h4toh.weight.detach()[:E], ex.h4toh.bias.detach()[:E],
-                                         self.top_k, self._capacity(inp.shape[0]))
+                lin, up, down = self.gate.gate, ex.htoh4, ex.h4toh
+                output = ops.moe_forward(inp, lin.weight, lin.bias, up.weight[:E], up.bias[:E], down.weight[:E],
+                                         down.bias[:E], self.top_k, self._capacity(inp.shape[0]))
         else:
             self.async_expert_assign.capacity = self._capacity(inp.shape[0])
             pos, gate_score, infos = self.async_expert_assign.process_data(

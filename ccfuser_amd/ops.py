@@ -8,6 +8,7 @@ mix_moe/csrc/mix_moe.h:242-245, or asserts, mix_moe/csrc/cuda/utils.h:4-6).
 """
 from __future__ import annotations
 
+import contextlib
 from typing import Dict, Optional, Tuple
 
 import torch
@@ -22,7 +23,15 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(t: torch.Tensor):
+    """A context in which t's device is current; entering one that already is costs as much as a kernel launch."""
+    return _HERE if t.get_device() == torch._C._cuda_getDevice() else torch.cuda.device(t.device)
 
 
 def _check(t: torch.Tensor, name: str, dtype=None, ndim=None) -> None:
@@ -63,7 +72,7 @@ def gate_topk_softmax(x: torch.Tensor, wg: torch.Tensor, bg: Optional[torch.Tens
     idx = torch.empty(T, top_k, dtype=torch.int64, device=x.device)
     score = torch.empty(T, top_k, dtype=x.dtype, device=x.device)
     logits = torch.empty(T, E, dtype=x.dtype, device=x.device) if return_logits else None
-    with torch.cuda.device(x.device):
+    with _on(x):
         _lib.call("ccf_gate_topk_softmax", _ptr(x), _ptr(wg), _ptr(bg), T, d, E, int(top_k),
                   CCF_F16 if x.dtype == torch.float16 else CCF_F32, _ptr(idx), _ptr(score),
                   _ptr(logits), _stream(x))
@@ -83,7 +92,7 @@ def gate_backward(score: torch.Tensor, grad_score: torch.Tensor, idx: torch.Tens
     E = int(tot_expert)
     g_logits = torch.empty(T, E, dtype=torch.float16, device=score.device)
     g_bias = torch.empty(E, dtype=torch.float16, device=score.device) if want_bias else None
-    with torch.cuda.device(score.device):
+    with _on(score):
         nbytes = _lib.lib().ccf_gate_backward_workspace_bytes(T, E) if want_bias else 0
         ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=score.device) if want_bias else None
         _lib.call("ccf_gate_backward", _ptr(score), _ptr(grad_score), _ptr(idx), T, k, E, _ptr(g_logits),
@@ -106,7 +115,7 @@ def gate_backward_products(score: torch.Tensor, grad_score: torch.Tensor, idx: t
     g_w = torch.empty_like(weight) if want_weight else None
     g_b = torch.empty(E, dtype=torch.float16, device=x.device) if want_bias else None
     if want_x or want_weight or want_bias:
-        with torch.cuda.device(x.device):
+        with _on(x):
             ws = _workspace(_lib.lib().ccf_gate_backward_products_workspace_bytes(T, d, E), x)
             _lib.call("ccf_gate_backward_products", _ptr(score), _ptr(grad_score), _ptr(idx), _ptr(x), _ptr(weight), T, d,
                       E, k, _ptr(g_x), _ptr(g_w), _ptr(g_b), _ptr(ws), ws.numel(), _stream(x))
@@ -125,7 +134,7 @@ def expert_count(gate_idx: torch.Tensor, expert_count_out: torch.Tensor) -> None
     """Accumulate the histogram of ``gate_idx`` into ``expert_count_out`` (int32)."""
     _check(gate_idx, "gate_idx", dtype=torch.int64)
     _check(expert_count_out, "expert_count", dtype=torch.int32, ndim=1)
-    with torch.cuda.device(gate_idx.device):
+    with _on(gate_idx):
         _lib.call("ccf_expert_count", _ptr(gate_idx), gate_idx.numel(), _ptr(expert_count_out),
                   expert_count_out.numel(), _stream(gate_idx))
 
@@ -138,7 +147,7 @@ def assign_pos(cum_count: torch.Tensor, gate: torch.Tensor, pos: torch.Tensor) -
     n, E = gate.numel(), cum_count.numel()
     if pos.numel() > n:
         raise ValueError("pos is longer than the gate index list")
-    with torch.cuda.device(gate.device):
+    with _on(gate):
         nbytes = _lib.lib().ccf_route_workspace_bytes(n, E)
         ws = _workspace(nbytes, gate)
         # pos may be shorter than n (dropped entries); the kernel bounds writes by n, so hand it
@@ -168,7 +177,7 @@ def route(gate_idx: torch.Tensor, num_expert: int, top_k: int, capacity: int = -
         "inv_pos": torch.empty(n, dtype=torch.int32, device=dev),
         "idx_kept": torch.empty(n, dtype=torch.int64, device=dev),
     }
-    with torch.cuda.device(dev):
+    with _on(gate_idx):
         ws = _workspace(_lib.lib().ccf_route_workspace_bytes(n, num_expert), gate_idx)
         _lib.call("ccf_route", _ptr(gate_idx), n, int(num_expert), int(top_k), int(capacity),
                   _ptr(out["counts"]), _ptr(out["offsets"]), _ptr(out["pos"]), _ptr(out["src_row"]),
@@ -196,7 +205,7 @@ def route_static(gate_idx: torch.Tensor, num_expert: int, top_k: int, capacity: 
             "inv_pos": torch.empty(n, dtype=torch.int32, device=dev),
             "idx_kept": torch.empty(n, dtype=torch.int64, device=dev),
         }
-    with torch.cuda.device(dev):
+    with _on(gate_idx):
         _lib.call("ccf_route_static", _ptr(gate_idx), n, int(num_expert), int(top_k), int(capacity),
                   _ptr(out["counts"]), _ptr(out["offsets"]), _ptr(out["pos"]), _ptr(out["src_row"]),
                   _ptr(out["dst_row"]), _ptr(out["inv_pos"]), _ptr(out["idx_kept"]), _stream(gate_idx))
@@ -219,7 +228,7 @@ def plan_blocks(counts: torch.Tensor, max_rows: int, block_size: int = 64, rank:
     out = {k: torch.zeros(cap, dtype=torch.int32, device=dev) for k in names}
     out["expert_block_id_idxs"] = torch.empty(E + 1, dtype=torch.int32, device=dev)
     out["block_nums"] = torch.empty(2, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(counts):
         _lib.call("ccf_plan_blocks", _ptr(counts), E, int(block_size), int(rank), cap,
                   *[_ptr(out[k]) for k in names], _ptr(out["expert_block_id_idxs"]),
                   _ptr(out["block_nums"]), _stream(counts))
@@ -233,7 +242,7 @@ def segments_to_rows(seg_start, seg_len, seg_expert, num_expert: int, total_rows
     counts = torch.empty(num_expert, dtype=torch.int32, device=dev)
     offsets = torch.empty(num_expert + 1, dtype=torch.int32, device=dev)
     rows = torch.zeros(total_rows, dtype=torch.int32, device=dev)   # entries past offsets[-1] stay 0
-    with torch.cuda.device(dev):
+    with _on(seg_start):
         _lib.call("ccf_segments_to_rows", _ptr(seg_start), _ptr(seg_len), _ptr(seg_expert),
                   seg_start.numel(), int(num_expert), int(total_rows), _ptr(counts), _ptr(offsets),
                   _ptr(rows), _stream(seg_start))
@@ -246,7 +255,7 @@ def local_scatter(inp: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
     _check(inp, "inp", dtype=torch.float16, ndim=2)
     _check(pos, "pos", dtype=torch.int32, ndim=1)
     out = torch.empty(pos.numel(), inp.shape[1], dtype=inp.dtype, device=inp.device)
-    with torch.cuda.device(inp.device):
+    with _on(inp):
         _lib.call("ccf_local_scatter", _ptr(inp), _ptr(out), _ptr(pos), pos.numel(), inp.shape[1],
                   _stream(inp))
     return out
@@ -259,7 +268,7 @@ def local_gather(inp: torch.Tensor, pos: torch.Tensor, out_rows: int) -> torch.T
     if pos.numel() != inp.shape[0]:
         raise ValueError("pos and inp disagree on the number of rows")
     out = torch.zeros(out_rows, inp.shape[1], dtype=inp.dtype, device=inp.device)
-    with torch.cuda.device(inp.device):
+    with _on(inp):
         _lib.call("ccf_local_gather", _ptr(inp), _ptr(out), _ptr(pos), pos.numel(), inp.shape[1],
                   _stream(inp))
     return out
@@ -275,7 +284,7 @@ def combine(y_flat: torch.Tensor, score: torch.Tensor, top_k: int,
     if n % top_k or score.numel() != n or (inv_pos is not None and inv_pos.numel() != n):
         raise ValueError("combine: sizes do not match tokens*top_k")
     out = torch.empty(n // top_k, d, dtype=y_flat.dtype, device=y_flat.device)
-    with torch.cuda.device(y_flat.device):
+    with _on(y_flat):
         _lib.call("ccf_combine", _ptr(y_flat), _ptr(score), _ptr(inv_pos), _ptr(out), n // top_k,
                   int(top_k), d, _stream(y_flat))
     return out
@@ -292,7 +301,7 @@ def ffn_plan_info(workspace: torch.Tensor, max_rows: int, E: int, d: int, f: int
     call decided (diagnostic; synchronises)."""
     import ctypes as C
     info = (C.c_int32 * 8)()
-    with torch.cuda.device(workspace.device):
+    with _on(workspace):
         _lib.call("ccf_ffn_plan_info", _ptr(workspace), int(max_rows), E, d, f, int(which), info, _stream(workspace))
     names = ("split_tiles", "split_parts", "skinny_tiles", "skinny_wgs_per_xcd", "skinny_per_xcd", "skinny_tail_steps",
              "persistent_wgs", "worst_case_tiles")
@@ -334,7 +343,7 @@ def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor
     _check(h, "h", dtype=torch.float16, ndim=2)
     if h.shape[1] != f or (dst_row is None and h.shape[0] < max_rows):
         raise ValueError("ffn1: output buffer too small")
-    with torch.cuda.device(x.device):
+    with _on(x):
         ws = workspace if workspace is not None else ffn_workspace(max_rows, E, d, f, x)
         _lib.call("ccf_ffn1_forward_kn" if w_kn else "ccf_ffn1_forward", _ptr(x), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
                   _ptr(w1), _ptr(b1), int(bool(gelu)), _ptr(h), _ptr(ws), ws.numel(), _stream(x))
@@ -359,7 +368,7 @@ def ffn1_keep(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.T
         raise ValueError("ffn1_keep: x has fewer rows than max_rows")
     act = torch.empty(max_rows, f, dtype=x.dtype, device=x.device)
     h_pre = torch.empty_like(act)
-    with torch.cuda.device(x.device):
+    with _on(x):
         ws = _workspace(_lib.lib().ccf_ffn_workspace_bytes(max_rows, E, d, f), x)
         _lib.call("ccf_ffn1_forward_keep", _ptr(x), _ptr(src_row), _ptr(offsets), int(max_rows), E, d, f,
                   _ptr(w1), _ptr(b1), _ptr(h_pre), _ptr(act), _ptr(ws), ws.numel(), _stream(x))
@@ -394,7 +403,7 @@ def ffn2(h: torch.Tensor, dst_row: Optional[torch.Tensor], offsets: torch.Tensor
         raise ValueError("ffn2: y has fewer rows than max_rows")
     if row_scale is not None:
         _check(row_scale, "row_scale", dtype=torch.float16, ndim=1)
-    with torch.cuda.device(h.device):
+    with _on(h):
         ws = workspace if workspace is not None else ffn_workspace(max_rows, E, d, f, h)
         _lib.call("ccf_ffn2_forward_kn" if w_kn else "ccf_ffn2_forward", _ptr(h), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
                   _ptr(w2), _ptr(b2), _ptr(row_scale), _ptr(y), _ptr(ws), ws.numel(), _stream(h))
@@ -417,10 +426,23 @@ def combine_backward(grad_out: torch.Tensor, y_flat: torch.Tensor, score: torch.
         raise ValueError("combine_backward: sizes do not match tokens*top_k")
     g_y = torch.empty_like(y_flat)
     g_s = torch.empty(n, dtype=torch.float16, device=y_flat.device)
-    with torch.cuda.device(y_flat.device):
+    with _on(y_flat):
         _lib.call("ccf_combine_backward", _ptr(grad_out), _ptr(y_flat), _ptr(score), _ptr(inv_pos), T,
                   int(top_k), d, _ptr(g_y), _ptr(g_s), _stream(y_flat))
     return g_y, g_s
+
+
+def zero_tails(a: torch.Tensor, b: torch.Tensor, first: int) -> None:
+    """``a[first:] = 0`` and ``b[first:] = 0`` in one launch (contiguous fp16 tensors of one leading size whose rows
+    are multiples of 8 elements)."""
+    for t in (a, b):
+        _check(t, "tensor", dtype=torch.float16)
+    rows = a.shape[0] - first
+    na, nb = a.numel() // a.shape[0], b.numel() // b.shape[0]
+    if b.shape[0] != a.shape[0] or first < 0 or rows < 0:
+        raise ValueError("zero_tails: sizes do not match")
+    with _on(a):
+        _lib.call("ccf_zero_ranges", a.data_ptr() + 2 * first * na, rows * na, b.data_ptr() + 2 * first * nb, rows * nb, _stream(a))
 
 
 def _backward_ws(max_rows: int, E: int, d: int, f: int, like: torch.Tensor) -> torch.Tensor:
@@ -468,7 +490,7 @@ def ffn2_backward(grad_y_flat: torch.Tensor, act: torch.Tensor, dst_row: Optiona
     dev = act.device
     g_act = (torch.zeros if may_drop else torch.empty)(max_rows, f, dtype=torch.float16, device=dev)
     g_w, g_b = _grad_outputs(w2, grad_w, grad_b)
-    with torch.cuda.device(dev):
+    with _on(act):
         ws = _backward_ws(max_rows, E, d, f, act)
         _lib.call("ccf_ffn2_backward", _ptr(grad_y_flat), _ptr(act), _ptr(h_pre), _ptr(dst_row), _ptr(offsets),
                   int(max_rows), E, d, f, _ptr(w2), _ptr(g_act), _ptr(g_w), _ptr(g_b), _ptr(ws),
@@ -509,7 +531,7 @@ def ffn1_backward(grad_h: torch.Tensor, x: torch.Tensor, src_row: Optional[torch
     dev = x.device
     g_x = (torch.zeros if may_drop else torch.empty)(n_flat, d, dtype=torch.float16, device=dev)
     g_w, g_b = _grad_outputs(w1, grad_w, grad_b)
-    with torch.cuda.device(dev):
+    with _on(x):
         ws = _backward_ws(max_rows, E, d, f, x)
         if h_pre is not None:
             _lib.call("ccf_ffn1_backward_gelu", _ptr(grad_h), _ptr(h_pre), _ptr(x), _ptr(src_row), _ptr(dst_row),
@@ -548,7 +570,7 @@ def moe_forward(x, wg, bg, w1, b1, w2, b2, top_k: int, capacity: int = -1,
                  "pos": torch.empty(n, dtype=torch.int64, device=dev),
                  "counts": torch.empty(E, dtype=torch.int32, device=dev),
                  "offsets": torch.empty(E + 1, dtype=torch.int32, device=dev)}
-    with torch.cuda.device(dev):
+    with _on(x):
         need = _lib.lib().ccf_moe_workspace_bytes(T, d, f, E, int(top_k))
         ws = workspace if workspace is not None else _workspace(need, x)
         _lib.call("ccf_moe_forward", _ptr(x), _ptr(wg), _ptr(bg), _ptr(w1), _ptr(b1), _ptr(w2),
@@ -579,7 +601,7 @@ def moe_ffn_segments(x, seg_start, seg_len, seg_expert, w1, b1, w2, b2,
     E, f, _ = w1.shape
     if y is None:
         y = torch.zeros(R, d, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x):
         need = _lib.lib().ccf_segments_workspace_bytes(R, seg_start.numel(), E, d, f)
         ws = _workspace(need, x)
         _lib.call("ccf_moe_ffn_segments", _ptr(x), _ptr(seg_start), _ptr(seg_len), _ptr(seg_expert),
@@ -610,7 +632,7 @@ def moe_ffn_blocks(x, pos, expert_ids, lens, start_addrs, block_size: int, top_k
     if nb and (not T or not pos.numel()):
         raise ValueError("moe_ffn_blocks: blocks of no tokens")
     y = torch.zeros(pos.numel(), d, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x):
         ws = _workspace(_lib.lib().ccf_blocks_workspace_bytes(nb, int(block_size), E, d, f), x)
         _lib.call("ccf_moe_ffn_blocks", _ptr(x), T, _ptr(pos), pos.numel(), int(top_k), _ptr(expert_ids), _ptr(lens),
                   _ptr(start_addrs), nb, int(block_size), d, f, E, _ptr(w1), int(w1_kn), _ptr(b1), _ptr(w2),

@@ -122,11 +122,17 @@ int ccf_gate_topk_softmax(const void *x, const void *wg, const void *bg,
                           int dtype, int64_t *idx_out, void *score_out,
                           void *logits_out, ccf_stream_t stream);
 
-/* Backward of the whole fp16 gate (top-k softmax, selection and linear layer): grad_x [tokens, d_model],
+/* Bytes of workspace ccf_gate_backward_products needs (no counterpart in the reference). */
+size_t ccf_gate_backward_products_workspace_bytes(int tokens, int d_model, int tot_expert);
+/* a[0 .. halves_a) = 0 and b[0 .. halves_b) = 0 in one launch (no counterpart in the reference); sizes are multiples
+ * of 8, pointers 16-byte aligned. */
+int ccf_zero_ranges(void *a, size_t halves_a, void *b, size_t halves_b, ccf_stream_t stream);
+
+/* Backward of the whole fp16 gate (top-k softmax, selection and linear layer; in the reference autograd derives it
+ * from gates/naive_gate.py:31-38, so it has no counterpart in the reference): grad_x [tokens, d_model],
  * grad_wg [tot_expert, d_model] and grad_bias [tot_expert], each NULL when not wanted (at least one is).  The sums are
  * fp32, in a fixed order.  tokens >= 1, an even d_model, tot_expert <= 16; x, wg and the gradients 4-byte, the
  * workspace 8-byte aligned. */
-size_t ccf_gate_backward_products_workspace_bytes(int tokens, int d_model, int tot_expert);
 int ccf_gate_backward_products(const void *score, const void *grad_score, const int64_t *idx, const void *x, const void *wg,
                                int tokens, int d_model, int tot_expert, int top_k, void *grad_x, void *grad_wg,
                                void *grad_bias, void *workspace, size_t workspace_bytes, ccf_stream_t stream);

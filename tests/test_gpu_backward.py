@@ -415,3 +415,12 @@ def test_ffn_backward_random_shapes(T, d, f, E, k, cap, seed):
     """Widths from 64 to 640 in steps of 64 (one K tile, partial M and N tiles, both weight
     forms), 1 to 600 tokens, 1 to 9 experts, top-1 to top-3, with and without capacity."""
     _ffn_backward_stages(T, d, f, E, k, cap, False, seed)
+
+
+@pytest.mark.parametrize("E,first,shape", [(5, 2, (8,)), (3, 3, (16, 8)), (4, 0, (24, 40)), (11, 8, (768, 64))])
+def test_zero_tails(E, first, shape):
+    from ccfuser_amd import ops
+    a, b = torch.ones(E, *shape, dtype=torch.float16, device="cuda"), torch.ones(E, shape[0], dtype=torch.float16, device="cuda")
+    ops.zero_tails(a, b, first)
+    for t in (a, b):
+        assert (t[:first] == 1).all() and (t[first:] == 0).all()
