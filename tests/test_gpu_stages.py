@@ -487,6 +487,28 @@ def test_eight_wavefront_kernel_gives_the_four_wavefront_bits(R, d, f, E, skew, 
     assert torch.equal(res[2][1], res[3][1]), "second GEMM"
 
 
+@pytest.mark.parametrize("n", [1, 63, 1023, 1024, 1025, 2048, 2049])
+@pytest.mark.parametrize("E", [1, 8, 300, 1024])
+@pytest.mark.parametrize("capacity", [-1, 3])
+def test_route_of_few_indices(n, E, capacity):
+    """One or two chunks of indices, counted by the launch that writes the positions, and the sizes next to them:
+    the results of the three-launch form, also with indices that name no expert."""
+    from ccfuser_amd import ops
+    g = torch.Generator().manual_seed(n + E)
+    idx = torch.randint(0, E, (n,), generator=g)
+    idx[torch.rand(n, generator=g) < 0.1] = -1
+    got = ops.route(dev(idx), E, 1, capacity)
+    ops.set_option("route_rows_max", 0)
+    try:
+        ref = ops.route(dev(idx), E, 1, capacity)
+    finally:
+        ops.set_option("route_rows_max", 16384)
+    kept = int(ref["offsets"][-1])
+    for k, v in ref.items():
+        m = kept if k in ("pos", "src_row", "dst_row") else v.numel()
+        assert torch.equal(got[k][:m], v[:m]), k
+
+
 @pytest.mark.parametrize("shape", range(6))
 @pytest.mark.parametrize("counts,N,K", [
     ([0, 1, 63, 64, 65, 127, 128, 129, 0], 264, 64),          # edges of both tile heights, a ragged last column tile
