@@ -397,8 +397,11 @@ bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cu
   if (g_few_rows >= 2) return true;
   // The 256-row tiles do 1.48 PFLOP/s inside a K step, the largest tile here 0.9: they win where they fill the chip
   // (150 rows per expert of 4096 / 14336: 225 and 225 us there, 306 and 278 here; 1024 rows of 768 / 3072, FFN1: 67 and
-  // 80), and lose where a few of them cannot (figures at the top).  Both priced in microseconds for evenly popular experts.  M tiles of an expert: the ceiling, which a load
-  // within two standard deviations of a whole number of tiles may miss by one either way.
+  // 80), and lose where a few of them cannot (figures at the top; FFN2 of 16 experts of 2048 / 8192, 121 and 200 rows
+  // each: 165 and 180 us there, 151 and 158 here).  Of 360 GEMMs timed in both forms (14 widths and numbers of
+  // experts, 32 to 512 rows each) the rule takes one that is over 5 % slower in 18; with a cut that costs 35 us however
+  // many tiles are cut it did in 35.  Both priced in microseconds for evenly popular experts.  M tiles of an expert: the
+  // ceiling, which a load within two standard deviations of a whole number of tiles may miss by one either way.
   const int used = E < max_rows ? E : max_rows;
   const double avg = static_cast<double>(max_rows) / used, sd = std::sqrt(avg), kt = K / kBK;
   auto near = [&](double gap) { return gap < 2 * sd ? 0.5 - 0.25 * gap / sd : 0.0; };
@@ -406,7 +409,7 @@ bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cu
     const double base = std::ceil(avg / bm);
     return used * (base + near(base * bm - avg) - (base > 1 ? near(avg - (base - 1) * bm) : 0.0));
   };
-  const double epi_us = epi == kFewPlain ? 3 : 6;
+  const double epi_us = epi == kFewPlain ? 4 : 8;
   double mine = 1e30;
   for (int rs = 0; rs < 2; ++rs)
     for (int cs = b_kn ? 1 : 0; cs < 3; ++cs) {
@@ -422,11 +425,11 @@ bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cu
   const double rounds = m_tiles(256) * ((N + 255) / 256) / cus, full = std::floor(rounds), part = rounds - full;
   double last = part > 0 ? tile : 0.0;
   if (part > 0 && kt >= 64 && part <= 0.5) {
-    const double cut = kt / std::fmin(std::floor(1 / part), 8.0) * 1.45 + 35;
+    const double cut = kt / std::fmin(std::floor(1 / part), 8.0) * 1.45 + 20 + 100 * part;   // more live tiles, more partial ones
     last = cut < tile ? cut : tile;
   }
   double big = full * tile + last;
-  big = (big > weights ? big : weights) + 6;
+  big = (big > weights ? big : weights) + 6 + 0.05 * weights;
   return mine < 0.95 * big;
 }
 
