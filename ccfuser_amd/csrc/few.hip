@@ -387,14 +387,12 @@ few_rows_kernel(FewArgs p) {
 
 }  // namespace
 
-int g_few_rows = 1;          // 0: never, 1: by the rule below, 2: always, 16 + i: always and with tile shape i
-
-bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cus) {
-  if (!g_few_rows || epi > kFewGeluKeep || (b_kn && epi == kFewGeluKeep) || cus < 8 || K % kBK || E > 1024) return false;
+bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn, int cus) {
+  if (!mode || epi > kFewGeluKeep || (b_kn && epi == kFewGeluKeep) || cus < 8 || K % kBK || E > 1024) return false;
   // the tile table holds kFewMaxRounds tiles per workgroup of the largest shape
   const long long worst = (static_cast<long long>(max_rows) / 128 + E) * ((N + 255) / 256);
   if (worst >= static_cast<long long>(kFewMaxRounds - 1) * cus) return false;
-  if (g_few_rows >= 2) return true;
+  if (mode >= 2) return true;
   // The 256-row tiles do 1.48 PFLOP/s inside a K step, the largest tile here 0.9: they win where they fill the chip
   // (150 rows per expert of 4096 / 14336: 225 and 225 us there, 306 and 278 here; 1024 rows of 768 / 3072, FFN1: 67 and
   // 80), and lose where a few of them cannot (figures at the top; FFN2 of 16 experts of 2048 / 8192, 121 and 200 rows
@@ -433,8 +431,8 @@ bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cu
   return mine < 0.95 * big;
 }
 
-int few_rows_gemm(FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {
-  p.force = g_few_rows >= 16 ? g_few_rows & 15 : -1;
+int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {
+  p.force = mode >= 16 ? mode & 15 : -1;
   void (*kernel)(FewArgs) = b_kn ? (epi == kFewPlain ? few_rows_kernel<kFewPlain, true> : few_rows_kernel<kFewGelu, true>)
                                  : (epi == kFewPlain ? few_rows_kernel<kFewPlain, false>
                                                      : (epi == kFewGelu ? few_rows_kernel<kFewGelu, false> : few_rows_kernel<kFewGeluKeep, false>));

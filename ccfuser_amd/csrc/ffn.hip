@@ -1144,20 +1144,22 @@ int g_wgrad_transpose = 0;   // 1: weight gradients always on transposed copies 
 int g_split_tail = 1;        // 0: the last round of tiles is not cut along K
 constexpr int kSplitTailMinKT = 64;
 int g_split_tail_min_kt = kSplitTailMinKT;
-int g_split_max_parts = 8;
+constexpr int kSplitMaxParts = 8;
+int g_split_max_parts = kSplitMaxParts;
 int g_fused_combine = 0;     // 1: top-2 layers add the gate-weighted expert outputs in the second GEMM's epilogue
 constexpr int kSkinnyPct = 70;
 int g_skinny_pct = kSkinnyPct;       // a K step of a skinny tile in percent of a 256-row tile's (plan model); 0: no skinny tiles
 int g_skinny_positions = 0;  // skinny ranges inside the persistent launch: 0 = a point per round of tiles, 2 = in front of / behind all tiles
 int g_split_inside = 1;      // 1: the parts of a split last round run inside the persistent launch, 0: as a launch of their own
 int g_skinny_tail = 0;       // 0: skinny tiles never run as a launch of their own
+int g_few_rows = 1;          // few rows per expert as tiles of 64 or 128 rows (few.hip): the modes of few_rows_fits()
 
 // The tuning knobs a grouped GEMM's plan and launches depend on, read once per call: the plan
 // and the kernels that consume it must agree even if another thread calls ccf_set_option
 // between the routing stage (which builds the plans of the layer's forward call) and the GEMMs.
 GemmOptions current_options() {
   return GemmOptions{g_variant, g_split_tail, g_split_tail_min_kt, g_split_max_parts, g_skinny_pct, g_fused_combine,
-                     g_skinny_tail, g_few_rows};
+                     g_skinny_tail, g_split_inside, g_few_rows};
 }
 
 // The kernels of one family of epilogues: `first` and `second` are two epilogue forms, each as
@@ -1307,7 +1309,8 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
 // Few rows per expert: the kernel of few.hip, unless a knob asks for a form of the 256-row tiles.
 bool use_few_rows(int max_rows, int E, int N, int K, int epi, bool b_kn, const GemmOptions &opt) {
   return opt.few_rows && opt.variant == kDefaultVariant && opt.skinny_pct == kSkinnyPct && opt.split_tail == 1 &&
-         opt.split_tail_min_kt == kSplitTailMinKT && few_rows_fits(max_rows, E, N, K, epi, b_kn, persistent_grid());
+         opt.split_tail_min_kt == kSplitTailMinKT && opt.split_max_parts == kSplitMaxParts && opt.skinny_tail == 0 &&
+         opt.split_inside == 1 && few_rows_fits(opt.few_rows, max_rows, E, N, K, epi, b_kn, persistent_grid());
 }
 
 // plan_ready: the plan (and the split list) of this very call was already built in `region`
@@ -1338,10 +1341,11 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
               "%s: operands must be 16-byte aligned", what);
   CCF_REQUIRE(!(gelu && row_scale), CCF_ERR_ARG, "%s: the GELU epilogue takes no row scale", what);
   if (max_rows == 0) return CCF_OK;
-  if (use_few_rows(max_rows, E, N, K, epi, b_kn, opt ? *opt : current_options()))
-    return few_rows_gemm(FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1}, epi,
+  const GemmOptions options = opt ? *opt : current_options();
+  if (use_few_rows(max_rows, E, N, K, epi, b_kn, options))
+    return few_rows_gemm(options.few_rows, FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1}, epi,
                          b_kn, persistent_grid(), stream, what);
-  const GemmSetup gs = setup_gemm(max_rows, E, N, K, epi, b_kn, workspace, region, opt ? *opt : current_options());
+  const GemmSetup gs = setup_gemm(max_rows, E, N, K, epi, b_kn, workspace, region, options);
   const Launch &v = *gs.v;
   const bool second = gs.second, split = gs.split;
   const int grid = gs.grid;
@@ -1381,7 +1385,7 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
     const long long g = (split || gs.skinny || grid < wgs) ? grid : wgs;
     // the parts of a split last round: run by the persistent workgroups themselves behind their tiles (the
     // four-wavefront kernels; part i is workgroup i's), else by a launch of their own
-    const bool parts_inside = split && g_split_inside && gs.v != &kVariants[kFwd8Variant];
+    const bool parts_inside = split && options.split_inside && gs.v != &kVariants[kFwd8Variant];
     p.tail_inside = parts_inside ? 1 : 0;
     hipLaunchKernelGGL(second ? v.persistent_gelu : v.persistent_plain, dim3(static_cast<unsigned>(g)),
                        dim3(v.threads), 0, stream, p, static_cast<int>(wgs / 8));

@@ -495,7 +495,7 @@ __device__ inline void build_plan(const PlanReq &rq, const int32_t *__restrict__
 // ffn.hip
 // Snapshot of the tuning knobs (ccf_set_option) that a grouped GEMM's plan and launches depend on.
 struct GemmOptions {
-  int variant, split_tail, split_tail_min_kt, split_max_parts, skinny_pct, fused_combine, skinny_tail, few_rows;
+  int variant, split_tail, split_tail_min_kt, split_max_parts, skinny_pct, fused_combine, skinny_tail, split_inside, few_rows;
 };
 GemmOptions forward_options();
 bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *workspace, const GemmOptions &opt,
@@ -549,9 +549,9 @@ struct FewArgs {
   int max_rows, E, N, K;
   int force;                 // tile shape, or -1: chosen by the kernel; filled in by few_rows_gemm
 };
-bool few_rows_fits(int max_rows, int E, int N, int K, int epi, bool b_kn, int cus);
-int few_rows_gemm(FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what);
-extern int g_few_rows;
+// mode: GemmOptions::few_rows (0: never, 1: by the rule, 2: always, 16 + i: always and with tile shape i)
+bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn, int cus);
+int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what);
 
 // most entries of a table of per-run expert counts that the routing stage takes from the gate kernel
 long long route_rows_max_ints();

@@ -565,6 +565,24 @@ def test_few_rows_kernel(shape, counts, N, K):
     assert O.mean_rel_err(got[2].cpu(), plain.cpu()) <= MEAN_REL
 
 
+@pytest.mark.parametrize("knob,value,default", [("gemm_variant", 3, -1), ("split_tail", 0, 1), ("split_parts", 2, 8),
+                                                ("skinny", 0, 1), ("skinny_tail", 1, 0), ("split_inside", 0, 1)])
+def test_tile_knobs_select_the_256_row_tiles(knob, value, default):
+    """A knob of the 256-row tiles away from its default takes a GEMM of few rows back to them: the launch with a
+    plan (``persistent_wgs`` is 0 where no plan is used)."""
+    from ccfuser_amd import ops
+    R, E, d, f = 512, 8, 256, 1024
+    ws = ops.ffn_workspace(R, E, d, f, torch.empty(1, device="cuda")).zero_()
+    form = lambda: [ops.ffn_plan_info(ws, R, E, d, f, which)["persistent_wgs"] for which in (1, 2)]
+    assert form() == [0, 0]
+    ops.set_option(knob, value)
+    try:
+        assert all(n > 0 for n in form())
+    finally:
+        ops.set_option(knob, default)
+    assert form() == [0, 0]
+
+
 def test_ffn_special_cases():
     """Closed forms: zero weights give the bias path; a single expert is a dense MLP."""
     from ccfuser_amd import ops
