@@ -18,7 +18,7 @@ Weight layouts: the forward calls receive ``weight.transpose(-2, -1).contiguous(
 i.e. [E, K, N] (mix_moe/mix_moe/linear.py:74, 129), the backward calls the stored
 ``weight.contiguous()``, [E, out, in] (linear.py:103, 162).  A square weight
 (d_model == d_ffn) cannot be told apart by shape: the forward calls always take it
-as the reference's [E, K, N] and transpose it back.
+as the reference's [E, K, N].
 """
 from __future__ import annotations
 
@@ -57,18 +57,21 @@ def cpy_data2tensor(data: List[int], tensor: torch.Tensor) -> None:
 
 def _weight_form(weight: torch.Tensor, n_out: int, k_in: int):
     """(weight, is_kn): the reference passes ``weight.transpose(-2, -1).contiguous()``, i.e. [E, K, N]
-    (mix_moe/mix_moe/linear.py:74), which the GEMM reads as it is; a tensor already in [E, N, K] is used as
-    well.  Transposing the weights back first took 549 of 1069 us of a layer of 16 experts, 1024 / 4096, and
-    8192 tokens."""
+    (mix_moe/mix_moe/linear.py:74), which the GEMM reads as it is; a tensor already in [E, N, K], or an [E, K, N]
+    view of one, is used as [E, N, K].  Transposing the weights first takes 549 us for 16 experts of 1024 / 4096."""
     if weight.dim() != 3:
         raise ValueError("expert weight must be 3-D")
     if tuple(weight.shape[1:]) == (n_out, k_in) and n_out != k_in:
         return weight.contiguous(), False
     if tuple(weight.shape[1:]) == (k_in, n_out):
-        if k_in * n_out >= 1 << 31:                  # the [K, N] loads index an expert's weight with 31 bits
-            return weight.transpose(-2, -1).contiguous(), False
-        weight = weight.contiguous()
-        return (weight if weight.data_ptr() % 16 == 0 else weight.clone()), True
+        stored = weight.transpose(-2, -1)
+        if stored.is_contiguous():                   # a view of the stored [E, N, K] weight: used without a copy
+            weight, kn = stored, False
+        elif k_in * n_out >= 1 << 31:                # the [K, N] loads index an expert's weight with 31 bits
+            weight, kn = stored.contiguous(), False
+        else:
+            weight, kn = weight.contiguous(), True
+        return (weight if weight.data_ptr() % 16 == 0 else weight.clone()), kn
     raise ValueError(f"expert weight {tuple(weight.shape)} matches neither [E,{k_in},{n_out}] nor [E,{n_out},{k_in}]")
 
 

@@ -100,3 +100,32 @@ def test_integration_guide_constructor_example_is_valid():
     assert m, "the guide no longer shows the constructor call"
     mlp = eval(m.group(1), {"MixMOETransformerMLP": MixMOETransformerMLP})
     assert mlp.experts.htoh4.weight.shape[1:] == (14336, 4096) and mlp.top_k == 2
+
+
+@pytest.mark.parametrize("E,n_out,k_in", [(3, 16, 24), (2, 24, 24), (1, 8, 64)])
+def test_expert_weights_are_copied_only_where_no_kernel_reads_them(E, n_out, k_in):
+    """[E, K, N] weights, [E, N, K] ones and transposed views of them keep their memory; anything else is made
+    contiguous.  Either way the values are those of the [E, K, N] weight."""
+    from ccfuser_amd.mix_moe_hip import _weight_form
+    stored = torch.randn(E, n_out, k_in).half()
+    kn = stored.transpose(-2, -1).contiguous()
+
+    def form(weight, is_kn, memory_of=None):
+        w, got = _weight_form(weight, n_out, k_in)
+        assert got == is_kn and w.is_contiguous() and w.data_ptr() % 16 == 0
+        assert torch.equal(w, kn if is_kn else stored)
+        assert memory_of is None or w.data_ptr() == memory_of.data_ptr()
+
+    form(kn, True, kn)
+    form(stored.transpose(-2, -1), False, stored)
+    if n_out != k_in:
+        form(stored, False, stored)
+    wide = torch.zeros(E, k_in, n_out + 3).half()
+    wide[..., :n_out] = kn
+    form(wide[..., :n_out], True)                          # columns of a wider tensor
+    odd = torch.empty(kn.numel() + 1).half()[1:].view(kn.shape).copy_(kn)
+    form(odd, True)                                        # 2 bytes off any 16-byte boundary
+    odd = torch.empty(kn.numel() + 1).half()[1:].view(stored.shape).copy_(stored)
+    form(odd.transpose(-2, -1), False)
+    with pytest.raises(ValueError):
+        _weight_form(torch.zeros(E, n_out + 8, k_in).half(), n_out, k_in)
