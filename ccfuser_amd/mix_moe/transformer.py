@@ -71,13 +71,16 @@ class BlockInfos(dict):
 def _any_requires_grad(module):
     """``any(p.requires_grad for p in module.parameters())`` without the generators over names, which cost more host
     time than the launches of a small layer."""
-    todo = [module]
+    todo, seen = [module], {module}                      # a module may be reached twice, or contain one that holds it
     while todo:
         m = todo.pop()
         for p in m._parameters.values():
             if p is not None and p.requires_grad:
                 return True
-        todo.extend(c for c in m._modules.values() if c is not None)
+        for c in m._modules.values():
+            if c is not None and c not in seen:
+                seen.add(c)
+                todo.append(c)
     return False
 
 

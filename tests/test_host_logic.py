@@ -129,3 +129,24 @@ def test_expert_weights_are_copied_only_where_no_kernel_reads_them(E, n_out, k_i
     form(odd.transpose(-2, -1), False)
     with pytest.raises(ValueError):
         _weight_form(torch.zeros(E, n_out + 8, k_in).half(), n_out, k_in)
+
+
+@pytest.mark.timeout(20)
+def test_parameter_walk_visits_every_module_once():
+    """``_any_requires_grad`` agrees with ``parameters()``, also where modules are shared or refer back to the one that
+    holds them."""
+    from ccfuser_amd.mix_moe.transformer import _any_requires_grad
+    root = torch.nn.Sequential(torch.nn.Linear(2, 2), torch.nn.Sequential(torch.nn.Linear(2, 2), torch.nn.ReLU()))
+    shared = torch.nn.Linear(2, 2, bias=False)
+    root[1].add_module("shared", shared)
+    root.add_module("again", shared)
+    root.register_parameter("none", None)
+    root[1].add_module("holder", root)                     # a cycle
+    for p in root.parameters():
+        p.requires_grad_(False)
+    assert not _any_requires_grad(root)
+    for p in root.parameters():
+        p.requires_grad_(True)
+        assert _any_requires_grad(root) and _any_requires_grad(root[1])
+        p.requires_grad_(False)
+    assert not _any_requires_grad(root)
