@@ -429,7 +429,9 @@ int route_impl(const int64_t *gate_idx, int n_flat, int E, int top_k, int capaci
   int32_t *chunk_cnt = static_cast<int32_t *>(ws);
   // the table of counts: the gate's rows, or one row per chunk from the hist launch
   int nrows = nchunk, rows_per_chunk = 1;
-  const bool self_count = gate_row_len == 0 && !cum_inout && nchunk <= kSelfChunks && nchunk <= g_route_rows_max / E;
+  // (not where workgroups would count indices that another one replaces by idx_kept)
+  const bool in_place = idx_kept == gate_idx && nchunk + n_plans > 1;
+  const bool self_count = gate_row_len == 0 && !cum_inout && nchunk <= kSelfChunks && nchunk <= g_route_rows_max / E && !in_place;
   if (gate_row_len > 0) {
     CCF_REQUIRE(kChunk % gate_row_len == 0 && !cum_inout, CCF_ERR_ARG, "route: rows of %d indices do not tile a chunk", gate_row_len);
     nrows = (n_flat + gate_row_len - 1) / gate_row_len;

@@ -196,7 +196,7 @@ int ccf_assign_pos(int32_t *cum_count, const int64_t *gate_idx, int n_flat,
  *   src_row int32 [n_flat] or NULL  pos[j] / top_k  (row of x to read)
  *   dst_row int32 [n_flat] or NULL  pos[j]          (row of y_flat to write)
  *   inv_pos int32 [n_flat] or NULL  j for kept flat index i, else -1
- *   idx_kept int64 [n_flat] or NULL gate_idx with dropped entries set to -1
+ *   idx_kept int64 [n_flat] or NULL gate_idx with dropped entries set to -1 (may be gate_idx itself)
  */
 int ccf_route(const int64_t *gate_idx, int n_flat, int num_expert, int top_k,
               int capacity, int32_t *counts, int32_t *offsets, int64_t *pos,

@@ -509,6 +509,27 @@ def test_route_of_few_indices(n, E, capacity):
         assert torch.equal(got[k][:m], v[:m]), k
 
 
+@pytest.mark.parametrize("n", [1000, 1500, 2048, 5000])
+def test_route_in_place(n):
+    """``idx_kept`` written over the indices themselves: every index is counted before any is replaced."""
+    from ccfuser_amd import _lib, ops
+    E, capacity = 8, n // 20
+    idx = dev(torch.randint(0, E, (n,), generator=torch.Generator().manual_seed(n)))
+    ref = ops.route(idx, E, 1, capacity)
+    got = {k: torch.empty_like(v) for k, v in ref.items()}
+    got["idx_kept"] = idx.clone()
+    nbytes = _lib.lib().ccf_route_workspace_bytes(n, E)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    _lib.call("ccf_route", got["idx_kept"].data_ptr(), n, E, 1, capacity, *[got[k].data_ptr() for k in
+              ("counts", "offsets", "pos", "src_row", "dst_row", "inv_pos", "idx_kept")], ws.data_ptr(), nbytes,
+              torch.cuda.current_stream().cuda_stream)
+    kept = int(ref["offsets"][-1])
+    assert kept < n
+    for k, v in ref.items():
+        m = kept if k in ("pos", "src_row", "dst_row") else v.numel()
+        assert torch.equal(got[k][:m], v[:m]), k
+
+
 @pytest.mark.parametrize("shape", range(6))
 @pytest.mark.parametrize("counts,N,K", [
     ([0, 1, 63, 64, 65, 127, 128, 129, 0], 264, 64),          # edges of both tile heights, a ragged last column tile
