@@ -385,7 +385,40 @@ few_rows_kernel(FewArgs p) {
   static_for<0, kFewShapes>(go);
 }
 
+double upper_tail(double z) { return 0.5 * std::erfc(z * 0.70710678118654752); }
+
 }  // namespace
+
+TileCount m_tiles(int max_rows, int E, int bm) {
+  const int used = E < max_rows ? E : max_rows;
+  const double avg = static_cast<double>(max_rows) / used, sd = std::sqrt(avg * (1.0 - 1.0 / used));
+  if (sd == 0) return {used * std::ceil(avg / bm), 0.0};
+  // tiles of an expert: the sum over j of (rows > j bm)
+  const double first = std::floor((avg - 5 * sd) / bm);
+  const int j0 = first > 0 ? static_cast<int>(first) : 0;
+  double m = j0, m2 = static_cast<double>(j0) * j0;
+  for (int j = j0;; ++j) {
+    const double p = upper_tail((static_cast<double>(j) * bm + 0.5 - avg) / sd);
+    if (p < 1e-4) break;
+    m += p;
+    m2 += (2.0 * j + 1) * p;
+  }
+  return {used * m, used * (m2 > m * m ? m2 - m * m : 0.0)};
+}
+
+SkinnyCount skinny_tiles(int max_rows, int E) {
+  const int used = E < max_rows ? E : max_rows;
+  const double avg = static_cast<double>(max_rows) / used, sd = std::sqrt(avg * (1.0 - 1.0 / used));
+  const auto at_most = [&](double x) { return sd > 0 ? 1 - upper_tail((x + 0.5 - avg) / sd) : (avg <= x ? 1.0 : 0.0); };
+  const int j0 = avg > 5 * sd ? static_cast<int>((avg - 5 * sd) / 256) : 0, j1 = static_cast<int>((avg + 5 * sd) / 256);
+  double full = 0, skinny = 0;
+  for (int j = j0; j <= j1; ++j) {
+    const double whole = at_most(256.0 * j), one = at_most(256.0 * j + 64), two = at_most(256.0 * j + 128);
+    full += j * (two - at_most(256.0 * j - 1)) + (j + 1) * (at_most(256.0 * j + 256 - 1) - two);
+    skinny += (one - whole) + 2 * (two - one);
+  }
+  return {used * full, used * skinny};
+}
 
 bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn, int cus) {
   if (!mode || epi > kFewGeluKeep || (b_kn && epi == kFewGeluKeep) || cus < 8 || K % kBK || E > 1024) return false;

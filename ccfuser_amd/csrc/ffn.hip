@@ -1256,6 +1256,22 @@ struct GemmSetup {
   PlanReq req;
 };
 
+// Whether fewer 256-row tiles than workgroups are worth cutting along K: if they fill about half of the CUs and less
+// (10 % more, for loads that are not quite even), or if the remainder rows as skinny tiles leave no more than half.  The
+// plan decides by the experts' real loads; this only keeps the reduction launch away from calls that it cannot help
+// (FFN2 of 8 experts of 2304 / 8192, 400 rows each, 144 tiles: 169 us without the reduction launch, 175 with it) or would
+// not pay in (of 2560 / 8960, 300 rows each, 80 tiles cut in three and 80 skinny ones: 177 us uncut, 195 cut; of 3072 /
+// 11008: 228 and 263).
+bool few_tiles_cut(int max_rows, int E, int n_tiles_n, int k_tiles, int epi_cost, int cus) {
+  const double half = 0.5 * cus;
+  if (m_tiles(max_rows, E, Cfg5::BM).mean * n_tiles_n <= 1.1 * half) return true;
+  const SkinnyCount sk = skinny_tiles(max_rows, E);
+  const double full = sk.full * n_tiles_n;
+  if (full > half) return false;
+  const double parts = full > 0 ? fmin(floor(cus / full), 8.0) : 8.0;
+  return k_tiles / parts + kSplitFixed + sk.skinny * n_tiles_n * k_tiles / cus * kSkAloneStepPct / 100 + kSkInsideFixed < k_tiles + epi_cost;
+}
+
 GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void *workspace, int region,
                      const GemmOptions &opt) {
   GemmSetup g;
@@ -1287,13 +1303,16 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   // the last, partly filled round is cut along K and spread over all workgroups (forward forms;
   // worth its two small launches only where a tile is long: K of 4096 and more)
   // A launch with a split round or skinny tiles has all CUs' workgroups, also where the plan has fewer entries: few
-  // tiles are where cutting them along K pays most.  One token, top-2 of 8 experts, 4096 / 14336: FFN2's 32 tiles
-  // 235 us on 32 workgroups, 52 us cut over 256.
-  g.split = opt.split_tail && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 8 &&
+  // tiles are where cutting them along K pays most (one token, top-2 of 8 experts, 4096 / 14336: FFN2's 32 tiles 235 us
+  // on 32 workgroups, 52 us cut over 256).  Where they cannot be cut, the reduction launch is for nothing: see below.
+  const bool few_entries = g.grid > g.wgs;
+  const bool cut_pays = !few_entries || (kt_all >= opt.split_tail_min_kt &&
+                                         few_tiles_cut(max_rows, E, n_tiles_n, kt_all, gelu ? kEpiCostGelu : kEpiCostPlain, g.grid));
+  g.split = opt.split_tail && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 8 && cut_pays &&
             g.grid <= kTailMaxParts && v.bm == Cfg5::BM && v.bn == Cfg5::BN && K / 64 >= opt.split_tail_min_kt;
   // remainder rows as skinny tiles: forward epilogues of the persistent 256 x 256 kernel (either weight layout)
   g.skinny = opt.skinny_pct != 0 && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 64 &&
-             (g.grid <= g.wgs || K / 64 >= opt.split_tail_min_kt) &&   // few short tiles: not worth the reduction launch
+             cut_pays &&
              v.bm == Cfg5::BM && v.bn == Cfg5::BN && v.persistent_plain && (!wide || g.split);
   // skinny tiles may be cut along K (partial tiles in the split scratch, summed by the reduction launch) at any K,
   // also where the last round of 256-row tiles is not split
@@ -1302,7 +1321,8 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   static_assert(plan_bm_ok(Cfg5::BM) && plan_bm_ok(Cfg8::BM), "build_plan shifts by the tile height");
   g.req = PlanReq{v.bm, max_tiles, max_rows, n_tiles_n, g.split ? g.grid / 8 : 0, K / 64, opt.split_max_parts, g.plan,
                   (g.split || g.cut) ? g.tail : nullptr, g.skinny ? g.skinny_list : nullptr, g.grid,
-                  gelu ? kEpiCostGelu : kEpiCostPlain, opt.skinny_pct, g.cut && opt.skinny_tail, !wide};
+                  gelu ? kEpiCostGelu : kEpiCostPlain, opt.skinny_pct, g.cut && opt.skinny_tail, !wide,
+                  few_entries ? kSkAloneStepPct : kSkInsideStepPct};
   return g;
 }
 
@@ -1421,7 +1441,7 @@ PlanReq wgrad_plan_request(int E, int M, int N, int32_t *workspace) {
   int32_t *plan = reinterpret_cast<int32_t *>(reinterpret_cast<char *>(workspace) + kTailBytes);
   const int max_rows = E * M;
   return PlanReq{Cfg5::BM, max_tiles_for(max_rows, E, Cfg5::BM), max_rows, (N + Cfg5::BN - 1) / Cfg5::BN, 0, 0, 0, plan,
-                 nullptr, nullptr, 0, 0, 0, 0, 0};
+                 nullptr, nullptr, 0, 0, 0, 0, 0, 0};
 }
 
 // C[e*M + m, n] = sum over k in [k_seg[e], k_seg[e+1]) of A[m, k] * B[n, k]: the weight

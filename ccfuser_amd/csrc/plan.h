@@ -106,6 +106,10 @@ struct FastDiv {
   }
 };
 
+// Cost of a last round that is cut along K beyond its parts' K steps, in K steps: two more launches, pipeline fill, the
+// reduction (measured).
+constexpr int kSplitFixed = 28;
+
 // Time, in K steps of a 256-row tile, that F tiles of k_tiles K steps and an epilogue worth
 // `epi` K steps take on spx workgroups: whole rounds, then the last, partly filled round, which
 // is cut along K when the request allows it (same rule as the split below).
@@ -122,7 +126,7 @@ __device__ inline int rounds_cost(int F, int spx, int k_tiles, int epi, bool may
       S = S > k_tiles / 4 ? k_tiles / 4 : S;
       S = (S >= 2 && 8 * r * S <= 256) ? S : 0;
     }
-    cost += S ? FastDiv(S).div(k_tiles) + 28 : k_tiles + epi;    // 28: two more launches, pipeline fill, the reduction (measured)
+    cost += S ? FastDiv(S).div(k_tiles) + kSplitFixed : k_tiles + epi;
   }
   return cost;
 }
@@ -170,6 +174,7 @@ struct PlanReq {
                     // the persistent launch (both need `tail`)
   int sk_tail_ok;   // the skinny tiles may run as a launch of their own (the caller launches the kernels for it)
   int sk_beside_ok; // they may run in workgroups of the persistent launch (its four-wavefront form only)
+  int inside_pct;   // a K step of a skinny tile inside the persistent launch, in percent of one of a 256-row tile
 };
 
 // A K step of a skinny tile, in percent of a 256-row tile's, when the whole chip runs skinny tiles
@@ -177,9 +182,10 @@ struct PlanReq {
 // (Measured on 4096 x 4096 x 14336 layers, 80 and 280 skinny tiles, 70 K steps per workgroup: ~100 K steps'
 // worth of time for the launch of its own with its reduction, ~80 inside the persistent launch.)
 constexpr int kSkTailStepPct = 115, kSkTailFixed = 16;
-// The same when the ranges run inside the persistent launch, half of the chip at a time beside 256-row tiles.
-constexpr int kSkInsideStepPct = 105, kSkInsideFixed = 8;
-
+// The same when the ranges run inside the persistent launch, half of the chip at a time beside 256-row tiles; and where
+// the launch has fewer tiles than CUs, whose ranges run with nothing beside them (18 launches of 64 to 128 tiles and 24 to
+// 100 skinny tiles: 137 to 220 % of a step).
+constexpr int kSkInsideStepPct = 105, kSkInsideFixed = 8, kSkAloneStepPct = 160;
 // Most tiles a range of q consecutive K steps can touch when a tile has k_tiles steps.
 __host__ __device__ inline int sk_tail_segments(int q, int k_tiles) { return (q - 1 + k_tiles - 1) / k_tiles + 1; }
 
@@ -288,7 +294,7 @@ __device__ inline void build_plan(const PlanReq &rq, const int32_t *__restrict__
           cost += (q_c * kSkTailStepPct + 99) / 100 + kSkTailFixed;
           ok = ok && q_c > 0 && rq.sk_tail_ok;
         } else if (cand == kSkinnyMaxWgs + 2) {
-          cost += (q_c * kSkInsideStepPct + 99) / 100 + kSkInsideFixed;
+          cost += (q_c * rq.inside_pct + 99) / 100 + kSkInsideFixed;
           ok = ok && q_c > 0 && rq.sk_beside_ok;
         }
         cost = cost < (1 << 26) ? cost : (1 << 26);
@@ -535,6 +541,17 @@ int blocks_with_plans(const int64_t *pos, int n_pos, int top_k, int n_tokens, co
                       const int32_t *lens, const int32_t *starts, int n_blocks, int block_size, int num_expert,
                       int32_t *counts, int32_t *offsets, int32_t *token_rows, int32_t *flat_rows, hipStream_t stream,
                       const PlanReq *plans, int n_plans);
+// few.hip: mean and variance of the number of M tiles of bm rows when max_rows rows fall on E evenly popular experts
+// (an expert's rows: a binomial variable, by its normal approximation)
+struct TileCount {
+  double mean, var;
+};
+TileCount m_tiles(int max_rows, int E, int bm);
+// The same loads: mean number of 256-row M tiles and of 64-row ones when remainders of up to 128 rows are skinny tiles
+struct SkinnyCount {
+  double full, skinny;
+};
+SkinnyCount skinny_tiles(int max_rows, int E);
 // few.hip: the forward GEMMs of few rows per expert.  C[c_rows[j]] = epilogue(A[a_rows[j]] * B[e]^T + bias[e]) for the
 // rows offsets[e] <= j < offsets[e+1]; the forms are those of the grouped GEMM's epilogues 0, 1 and 2.
 constexpr int kFewPlain = 0, kFewGelu = 1, kFewGeluKeep = 2;

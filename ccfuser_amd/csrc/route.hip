@@ -449,7 +449,7 @@ int route_impl(const int64_t *gate_idx, int n_flat, int E, int top_k, int capaci
                        counts, offsets, cum_inout);
     if (int rc = check_launch("scan_kernel")) return rc;
   }
-  const PlanReq none{0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  const PlanReq none{};
   const size_t pos_lds = sizeof(int) * (static_cast<size_t>(kSub + (sum_rows ? 3 : 0)) * E + 1);
   if (pos_lds > 32768) {
     // with the plan builder's static arrays the kernel passes 64 KB of LDS for many experts
@@ -666,7 +666,7 @@ namespace {
 int launch_segments(const int32_t *seg_start, const int32_t *seg_len, const int32_t *seg_expert, int n_seg, int E,
                     int total_rows, int32_t *counts, int32_t *offsets, int32_t *rows, const SegBlocks &blk,
                     hipStream_t stream, const PlanReq *plans, int n_plans) {
-  const PlanReq none{0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  const PlanReq none{};
   const int plan_wgs = 8;
   int row_wgs = (n_seg + kSegThreads / 64 - 1) / (kSegThreads / 64);
   row_wgs = row_wgs < 1 ? 1 : (row_wgs > 512 ? 512 : row_wgs);

@@ -610,6 +610,35 @@ def test_few_tiles_of_a_long_contraction(counts):
     close(gx, torch.cat([a[e_of.cuda() == e].float() @ w1[e].float() for e in range(E)]))
 
 
+@pytest.mark.parametrize("E,rows,N,K,cut", [(16, 300, 1536, 6144, False), (8, 300, 2560, 8960, False),
+                                            (8, 400, 2304, 8192, False), (8, 20, 512, 4160, True), (4, 230, 4096, 4096, True)])
+def test_tiles_for_most_compute_units_need_no_reduction(E, rows, N, K, cut):
+    """With fewer plan entries than compute units a contraction of 4096 and more is cut along K, which takes a
+    reduction launch, only where its tiles fill about half of the units or less.  Such a call writes the header of its
+    list of parts, at the start of the first GEMM's workspace; any other leaves it alone."""
+    from ccfuser_amd import ops
+    _say(f"cut or not E={E} rows={rows} N={N} K={K}")
+    n = E * rows
+    off = (torch.arange(E + 1) * rows).to(torch.int32).cuda()
+    g = torch.Generator(device="cuda").manual_seed(n)
+    a = torch.randn(n, K, generator=g, device="cuda").half()
+    w = (torch.randn(E, N, K, generator=g, device="cuda") * 0.02).half()
+    b = torch.randn(E, N, generator=g, device="cuda").half()
+    ws = ops.ffn_workspace(n, E, K, N, a).fill_(0x55)
+    ops.set_option("few_rows", 0)
+    try:
+        y = ops.ffn1(a, None, off, n, w, b, workspace=ws)
+        info = ops.ffn_plan_info(ws, n, E, K, N, 1)
+    finally:
+        ops.set_option("few_rows", 1)
+    assert info["worst_case_tiles"] < info["persistent_wgs"]
+    assert bool((ws[:8] != 0x55).any()) == cut
+    assert (info["split_tiles"] + info["skinny_tiles"] > 0) == cut, info
+    ref = torch.cat([a[e * rows:(e + 1) * rows].float() @ w[e].float().t() + b[e].float() for e in range(E)])
+    ref = torch.nn.functional.gelu(ref)
+    assert float((y.float() - ref).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(ref.abs().max()) + 1e-4
+
+
 @pytest.mark.parametrize("T,d,f,E,k,bs,stored", [(1, 64, 192, 4, 2, 64, False), (333, 320, 832, 5, 2, 64, False),
                                                   (700, 256, 256, 3, 1, 32, False), (900, 512, 1024, 8, 2, 64, True),
                                                   (60, 4160, 512, 2, 2, 64, False)])
