@@ -19,8 +19,8 @@
 // Bound by streaming the weights from HBM at 5.3 - 5.7 TB/s where they are large, by the latency of a few dependent
 // steps where they are small.  FFN1 / FFN2 including their plan and reduction launches, 256-row tiles -> here:
 // 8 experts of 4096 / 14336, 32 rows each: 205 -> 165 and 176 -> 172 us, 83 rows each: 213 -> 191 and 201 -> 177;
-// 4 experts of 256 / 1024, 128 rows each: 20 -> 10 and 28 -> 10; 8 experts of 768 / 3072, 500 rows each: 44 -> 43 and
-// 70 -> 38; 16 experts of 1024 / 4096, 64 rows each: 37 -> 28 and 53 -> 31.
+// 4 experts of 256 / 1024, 128 rows each: 20 -> 10 and 28 -> 10; FFN2 of 8 experts of 768 / 3072, 500 rows
+// each: 70 -> 38; 16 experts of 1024 / 4096, 64 rows each: 37 -> 28 and 53 -> 31.
 #include "ccf_common.h"
 #include "gelu.h"
 #include "gemm_tile.h"
@@ -35,8 +35,10 @@ constexpr int kFewThreads = 512;
 constexpr int kFewLds = 163840;
 constexpr int kFewMaxRounds = 64;      // most tiles of a workgroup: one per lane of the tile table
 constexpr int kBK = 64;
-// A K step of 64 by tile shape [rows 64, 128][columns 64, 128, 256] in microseconds, operands in L2 (measured)
-constexpr double kFewStepUs[2][3] = {{0.36, 0.45, 0.80}, {0.42, 0.62, 1.20}};
+// A K step of 64 and an epilogue (GELU, plain) by tile shape, in microseconds: fitted to 2520 timed launches of all
+// shapes where the weights' bytes do not bound them, 4 to 9 % off each
+constexpr double kFewStepUs[6] = {0.274, 0.415, 0.705, 0.408, 0.600, 0.900};
+constexpr double kFewEpiUs[2][6] = {{1.3, 2.2, 3.2, 2.7, 5.5, 8.7}, {0.8, 0.6, 0.5, 1.7, 3.3, 5.7}};
 
 // Tile of 16 TM rows x 32 DB columns, 64 K elements per stage.  Eight wavefronts, 2 along the rows (wavefront half m
 // holds the 16-row blocks m, m + 2, ...) x 4 along the columns (16 NB columns each): two wavefronts per SIMD, so one's
@@ -306,8 +308,9 @@ few_rows_kernel(FewArgs p) {
     m64 += __shfl_xor(m64, off, 64);
     m128 += __shfl_xor(m128, off, 64);
   }
-  // price the shapes, one per lane: rounds of tiles times the rows of both operands that a K step loads (of the
-  // measured shapes the best, or within 4 % of it, in every case above)
+  // price the shapes, one per lane: rounds of tiles times the rows of both operands that a K step loads.  Of 2520 timed
+  // launches this takes a shape that is over 5 % slower than the best one in 120, on average 0.8 %; kFewStepUs did
+  // so in 49, but was up to 14 % slower than this choice where most experts' rows end just past a tile.
   const int slots = gridDim.x >> 3;                                 // workgroups per XCD
   const int ci = lane < kFewShapes ? lane : 0;
   const int rsel = ci / 3, csel = ci - 3 * rsel;
@@ -385,7 +388,9 @@ few_rows_kernel(FewArgs p) {
   static_for<0, kFewShapes>(go);
 }
 
-double upper_tail(double z) { return 0.5 * std::erfc(z * 0.70710678118654752); }
+// P(X > z) of a standard normal variable, within 2e-4: the rule below is on the host path of every GEMM, and an exp
+// takes a third of an erfc's time.
+double upper_tail(double z) { return 1 / (1 + std::exp(z * (1.5976 + 0.07056 * z * z))); }
 
 }  // namespace
 
@@ -404,6 +409,20 @@ TileCount m_tiles(int max_rows, int E, int bm) {
     m2 += (2.0 * j + 1) * p;
   }
   return {used * m, used * (m2 > m * m ? m2 - m * m : 0.0)};
+}
+
+// Mean of ceil(M tiles * n_col / cus): the rounds that the workgroups of cus CUs take.
+static double mean_rounds(const TileCount &t, int n_col, int cus) {
+  const double sd = std::sqrt(t.var), per = static_cast<double>(cus) / n_col;     // M tiles of a round
+  if (sd < 0.2) return std::ceil(t.mean / per - 1e-9);
+  const double first = std::floor((t.mean - 4 * sd) / per);
+  double rounds = first > 0 ? first : 0;
+  for (double r = rounds;; r += 1) {
+    const double p = upper_tail((std::floor(r * per) + 0.5 - t.mean) / sd);       // more M tiles than r rounds hold
+    if (p < 1e-3) break;
+    rounds += p;
+  }
+  return rounds;
 }
 
 SkinnyCount skinny_tiles(int max_rows, int E) {
@@ -426,42 +445,52 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
   const long long worst = (static_cast<long long>(max_rows) / 128 + E) * ((N + 255) / 256);
   if (worst >= static_cast<long long>(kFewMaxRounds - 1) * cus) return false;
   if (mode >= 2) return true;
-  // The 256-row tiles do 1.48 PFLOP/s inside a K step, the largest tile here 0.9: they win where they fill the chip
-  // (150 rows per expert of 4096 / 14336: 225 and 225 us there, 306 and 278 here; 1024 rows of 768 / 3072, FFN1: 67 and
-  // 80), and lose where a few of them cannot (figures at the top; FFN2 of 16 experts of 2048 / 8192, 121 and 200 rows
-  // each: 165 and 180 us there, 151 and 158 here).  Of 360 GEMMs timed in both forms (14 widths and numbers of
-  // experts, 32 to 512 rows each) the rule takes one that is over 5 % slower in 18; with a cut that costs 35 us however
-  // many tiles are cut it did in 35.  Both priced in microseconds for evenly popular experts.  M tiles of an expert: the
-  // ceiling, which a load within two standard deviations of a whole number of tiles may miss by one either way.
-  const int used = E < max_rows ? E : max_rows;
-  const double avg = static_cast<double>(max_rows) / used, sd = std::sqrt(avg), kt = K / kBK;
-  auto near = [&](double gap) { return gap < 2 * sd ? 0.5 - 0.25 * gap / sd : 0.0; };
-  auto m_tiles = [&](int bm) {
-    const double base = std::ceil(avg / bm);
-    return used * (base + near(base * bm - avg) - (base > 1 ? near(avg - (base - 1) * bm) : 0.0));
-  };
-  const double epi_us = epi == kFewPlain ? 4 : 8;
-  double mine = 1e30;
-  for (int rs = 0; rs < 2; ++rs)
-    for (int cs = b_kn ? 1 : 0; cs < 3; ++cs) {
-      const int bm = 64 << rs, bn = 64 << cs;
-      const double rounds = std::ceil(m_tiles(bm) * ((N + bn - 1) / bn) / cus);
-      const double t = rounds * (kt * kFewStepUs[rs][cs] + epi_us * bm * bn / 32768);
-      mine = t < mine ? t : mine;
-    }
-  const double weights = 2.0 * used * N * K / 5.5e6;                // every weight once, from HBM
-  mine = (mine > weights ? mine : weights) + 6;
-  // 256 x 256 tiles: 1.45 us a K step and the epilogue; a last round of at most half the CUs is cut along K
-  const double tile = kt * 1.45 + (epi == kFewPlain ? 7 : 13);
-  const double rounds = m_tiles(256) * ((N + 255) / 256) / cus, full = std::floor(rounds), part = rounds - full;
-  double last = part > 0 ? tile : 0.0;
-  if (part > 0 && kt >= 64 && part <= 0.5) {
-    const double cut = kt / std::fmin(std::floor(1 / part), 8.0) * 1.45 + 20 + 100 * part;   // more live tiles, more partial ones
-    last = cut < tile ? cut : tile;
+  // Where either is far ahead nothing is priced (0.3 to 0.8 us): three rounds of 256-row tiles waste too little for
+  // smaller tiles to win, and a quarter of a round makes a single one of 128 x 128 tiles at most.
+  const int n_tiles_n = (N + 255) / 256;
+  if (static_cast<long long>(max_rows / 256) * n_tiles_n >= 3ll * cus) return false;
+  if (K < 64 * kBK && 4 * (static_cast<long long>(max_rows) / 256 + E) * n_tiles_n <= cus) return true;
+  // The 256-row tiles do 1.48 PFLOP/s inside a K step, the largest tile here 1.2: they win where they fill the chip
+  // (FFN1 / FFN2, 256-row tiles and here: 8 experts of 3072 / 11008, 256 rows each: 184 and 230, 1024 rows of 768 / 3072:
+  // 67 and 80 us), and lose where a few of them cannot (figures at the top; FFN2 of 16 experts of 2048 / 8192, 121 and
+  // 200 rows each: 165 and 180 us there, 151 and 158 here).  Both forms are priced in microseconds for evenly popular
+  // experts.  Their loads scatter, so a launch whose tiles fill a round, or two, just so may take one more: rounds are
+  // an expectation over the tile counts.  Of 840 GEMMs timed in both forms (28 widths and numbers of experts, 32 to 700
+  // rows each, means over three loads) the rule takes one that is over 4 % slower in 45, most of them by staying with the
+  // 256-row tiles; rounding an expected count up did so in 57 and was up to 27 % slower than the 256-row tiles.
+  // The weights, once, from HBM at 5.5 TB/s overlap with the steps, but not fully.
+  const double used = E < max_rows ? E : max_rows, kt = K / kBK, weights = 2.0 * used * N * K / 5.5e6;
+  const TileCount mt[2] = {m_tiles(max_rows, E, 64), m_tiles(max_rows, E, 128)};
+  double key = 1e300, steps = 0;                                    // the shape that the kernel will choose
+  for (int i = b_kn ? 1 : 0; i < kFewShapes; ++i) {
+    if (b_kn && i % 3 == 0) continue;
+    const int bm = 64 << (i / 3), bn = 64 << (i % 3);
+    const double rounds = mean_rounds(mt[i / 3], (N + bn - 1) / bn, cus);
+    if (rounds * (bm + bn) >= key) continue;
+    key = rounds * (bm + bn);
+    steps = rounds * (kt * kFewStepUs[i] + kFewEpiUs[epi == kFewPlain][i]);
   }
-  double big = full * tile + last;
-  big = (big > weights ? big : weights) + 6 + 0.05 * weights;
-  return mine < 0.95 * big;
+  const double mine = std::sqrt(steps * steps + weights * weights) + 5;
+  // 256 x 256 tiles: 1.02 us a K step (1.2 to 1.45 with the whole chip at it, which this range never has) and the
+  // epilogue; a last round of at most half the CUs is cut along K
+  const TileCount big_mt = m_tiles(max_rows, E, 256);
+  const double tile = kt * 1.02 + (epi == kFewPlain ? 5 : 15);
+  if (kt >= 64) {
+    const double rounds = big_mt.mean * n_tiles_n / cus, full = std::floor(rounds), part = rounds - full;
+    double last = part > 0 ? tile : 0.0;
+    if (part > 0 && part <= 0.5) {
+      // the parts' steps, the reduction, and the partial tiles: fewer of them, and of their rows, with one or two rows
+      // per expert (FFN2 of one token, top-2 of 8 experts of 4096 / 14336: 51 us cut, 60 here)
+      const double rows = std::fmin(max_rows / used / 8, 1.0);
+      const double cut = kt / std::fmin(std::floor(1 / part), 8.0) * 1.02 + 10 + 25 * rows + 42 * part;
+      last = cut < tile ? cut : tile;
+    }
+    steps = full * tile + last;
+  } else {
+    steps = mean_rounds(big_mt, n_tiles_n, cus) * tile;
+  }
+  const double big = std::sqrt(steps * steps + weights * weights) + 5;
+  return mine < 1.02 * big;
 }
 
 int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {

@@ -604,6 +604,32 @@ def test_tile_knobs_select_the_256_row_tiles(knob, value, default):
     assert form() == [0, 0]
 
 
+@pytest.mark.parametrize("E,rows,d,f,which,few", [
+    # FFN1 / FFN2 in microseconds, 256-row tiles against tiles of few rows
+    (8, 256, 3072, 11008, 1, False),      # 184, 230
+    (16, 128, 1536, 6144, 1, False),      # 100, 110
+    (32, 128, 768, 3072, 1, False),       # 56, 62
+    (16, 256, 1024, 4096, 1, False),      # 68, 72
+    (4, 256, 3584, 12096, 1, False),      # 133, 154
+    (4, 300, 2048, 8192, 2, False),       # 68, 81
+    (2, 1, 4096, 14336, 2, False),        # 51, 60
+    (2, 1, 4096, 14336, 1, True),         # 53, 38
+    (8, 32, 4096, 14336, 1, True),        # 207, 179
+    (8, 32, 4096, 14336, 2, True),        # 197, 175
+    (4, 128, 256, 1024, 2, True),         # 29, 10
+    (16, 64, 1024, 4096, 1, True),        # 38, 29
+    (8, 110, 4096, 12288, 2, True),       # 234, 187
+    (8, 230, 1024, 4096, 1, True),        # 44, 40
+])
+def test_few_row_rule_takes_the_faster_form(E, rows, d, f, which, few):
+    """The form that a GEMM of evenly loaded experts runs in, at sizes where the other one measured slower
+    (``persistent_wgs`` is 0 where no plan is used)."""
+    from ccfuser_amd import ops
+    R = E * rows
+    ws = ops.ffn_workspace(R, E, d, f, torch.empty(1, device="cuda")).zero_()
+    assert (ops.ffn_plan_info(ws, R, E, d, f, which)["persistent_wgs"] == 0) == few
+
+
 def test_ffn_special_cases():
     """Closed forms: zero weights give the bias path; a single expert is a dense MLP."""
     from ccfuser_amd import ops
