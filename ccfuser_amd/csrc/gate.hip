@@ -610,7 +610,7 @@ gate_stream_kernel(const half_t *__restrict__ x, const half_t *__restrict__ wg, 
 // * Rows are 80 bytes apart: the eight rows that a read touches start 20 banks apart, none in conflict.
 // * Behind a round of parts their sums meet in LDS and are added in ascending order onto the running sums.
 //
-// TT shrinks with the tokens, so that there is a workgroup per CU from 2048 tokens on, EE with the experts.
+// TT shrinks with the tokens, so that 2049 and 4097 tokens still make 129 workgroups, EE with the experts.
 // 8192 tokens x 2048, 64 experts, top-2: 66 us, 988 us as one wavefront per token whose lanes each walked
 // rows of their own (and left the selection to one lane).
 constexpr int kF32StageK = 16;                     // K elements of a stage
@@ -780,6 +780,65 @@ int launch_gate_f32_experts(const float *x, const float *wg, const float *bg, in
   return launch(x, wg, bg, tokens, d, E, k, idx_out, score_out, logits_out, stream);
 }
 
+// The same for few tokens where those tiles leave most of their lanes or wavefronts idle: one to three experts of a
+// wide model (tiles have eight at least), or many experts of a narrow one (its one or two parts make as many wavefronts,
+// which walk the experts' tiles one after the other).  One wavefront per token: a lane takes one (expert, part) pair at
+// a time and walks the part in ascending K, then the lanes add each expert's part sums in order.
+__global__ void __launch_bounds__(64)
+gate_f32_walk_kernel(const float *__restrict__ x, const float *__restrict__ wg, const float *__restrict__ bg,
+                     int d, int E, int k, int group, int64_t *__restrict__ idx_out,
+                     float *__restrict__ score_out, float *__restrict__ logits_out) {
+#pragma clang fp contract(off)
+  extern __shared__ float s_mem[];
+  const int lane = threadIdx.x, t = blockIdx.x;
+  const int nparts = (d + kPart - 1) / kPart;
+  float *s_logit = s_mem;                          // [E]
+  float *s_part = s_mem + E;                       // [group][nparts]: `group` experts at a time
+  const float *xrow = x + static_cast<size_t>(t) * d;
+  for (int e0 = 0; e0 < E; e0 += group) {
+    const int ne = (E - e0) < group ? (E - e0) : group;
+    for (int q = lane; q < ne * nparts; q += kWave) {   // part fastest: neighbours read neighbouring K
+      const int p = q % nparts;
+      const float *wrow = wg + static_cast<size_t>(e0 + q / nparts) * d;
+      const int k_end = (p + 1) * kPart < d ? (p + 1) * kPart : d;
+      float acc = 0.0f;
+      for (int kk = p * kPart; kk < k_end; kk += 4) {
+        const float4v xv = *reinterpret_cast<const float4v *>(xrow + kk);
+        const float4v wv = *reinterpret_cast<const float4v *>(wrow + kk);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float prod = xv[j] * wv[j];
+          acc = acc + prod;
+        }
+      }
+      s_part[q] = acc;
+    }
+    __syncthreads();
+    for (int g = lane; g < ne; g += kWave) {
+      float s = s_part[g * nparts];
+      for (int p = 1; p < nparts; ++p) s = s + s_part[g * nparts + p];
+      if (bg) s = s + bg[e0 + g];
+      s_logit[e0 + g] = s;
+      if (logits_out) logits_out[static_cast<size_t>(t) * E + e0 + g] = s;
+    }
+    __syncthreads();
+  }
+  if (lane == 0) {
+    Best<kMaxTopK> best;
+    best.clear();
+    for (int e = 0; e < E; ++e) best.offer(s_logit[e], e, k);
+    best.write<float>(t, k, idx_out, score_out);
+  }
+}
+
+// Microseconds of the tiles and of a wavefront per token: 256 tokens of 4096, 1 expert: 12 and 8, 2: 12 and 9 (3: the
+// tiles; of 8192: 22 and 20); 256 of 128, 33 experts: 15 and 12, 128: 37 and 28, 512: 140 and 94; of 256, 200: 60 and 55.
+// More tokens fill the chip with either: 2048 of 128, 128 experts 37 and 53; 1024 of 256, 256: 69 and 86.
+bool gate_f32_walks(int tokens, int d, int E) {
+  if (E <= 3) return tokens * static_cast<long long>(E) <= 1024 && d > (E < 3 ? 2048 : 6144) && d <= 8192 * kPart;   // (LDS)
+  return (E > 32 && d <= kPart && tokens <= (E > 64 ? 1024 : 512)) || (E > 128 && d <= 2 * kPart && tokens <= 512);
+}
+
 }  // namespace
 }  // namespace ccf
 
@@ -801,6 +860,16 @@ int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int 
   CCF_REQUIRE(aligned16(x) && aligned16(wg), CCF_ERR_ARG, "gate: x and wg must be 16-byte aligned");
   if (tokens == 0) return CCF_OK;
   const int nparts = (d_model + kPart - 1) / kPart;
+  if (dtype == CCF_F32 && gate_f32_walks(tokens, d_model, tot_expert)) {
+    // part sums of as many experts at a time as 32 KB hold
+    int group = 8192 / nparts;
+    group = group < 1 ? 1 : (group > tot_expert ? tot_expert : group);
+    const size_t lds = sizeof(float) * (static_cast<size_t>(tot_expert) + static_cast<size_t>(group) * nparts);
+    hipLaunchKernelGGL(gate_f32_walk_kernel, dim3(tokens), dim3(64), lds, as_stream(stream), static_cast<const float *>(x),
+                       static_cast<const float *>(wg), static_cast<const float *>(bg), d_model, tot_expert, top_k, group,
+                       idx_out, static_cast<float *>(score_out), static_cast<float *>(logits_out));
+    return check_launch("gate_f32_walk_kernel");
+  }
   if (dtype == CCF_F32) {
     auto launch = tokens > 4096 ? launch_gate_f32_experts<4>
                                 : (tokens > 2048 ? launch_gate_f32_experts<2> : launch_gate_f32_experts<1>);

@@ -71,6 +71,24 @@ def test_gate_fp32_tiles(T, d, E, k):
     assert torch.equal(idx2.cpu(), O.naive_gate(x, wg, None, k)[0])
 
 
+@pytest.mark.parametrize("T,d,E,k", [(1, 4096, 1, 1), (512, 2056, 2, 2), (513, 2056, 2, 1), (341, 6152, 3, 3), (342, 6152, 3, 2), (300, 128, 33, 2), (513, 128, 33, 2),
+                                     (1024, 64, 130, 2), (1025, 64, 130, 2), (40, 256, 200, 8), (100, 264, 130, 2),
+                                     (5, 136, 1024, 2), (33, 8, 64, 1)])
+def test_gate_fp32_wavefront_per_token(T, d, E, k):
+    """Both sides of each line between a wavefront per token and the tiles: the oracle's bits, with and without a
+    bias."""
+    from ccfuser_amd import ops
+    _say(f"fp32 gate T={T} d={d} E={E} k={k}")
+    g = torch.Generator().manual_seed(T + d + E)
+    x, wg, bg = torch.randn(T, d, generator=g), torch.randn(E, d, generator=g) * 0.05, torch.randn(E, generator=g) * 0.05
+    for b in (bg, None):
+        idx_ref, score_ref, logits_ref = O.naive_gate(x, wg, b, k)
+        idx, score, logits = ops.gate_topk_softmax(dev(x), dev(wg), None if b is None else dev(b), k, return_logits=True)
+        assert torch.equal(logits.cpu(), logits_ref), "logits differ bitwise"
+        assert torch.equal(idx.cpu(), idx_ref), "expert choice differs"
+        assert torch.allclose(score.cpu(), score_ref, rtol=1e-5, atol=1e-7)
+
+
 _GATE_CASES = {}
 
 
