@@ -42,3 +42,12 @@ def workloads():
         return cache[key]
 
     return get
+
+
+@pytest.fixture(params=[1, 0], ids=["by_rule", "256_row_tiles"])
+def gemm_form(request):
+    """Runs a test twice: GEMMs of few rows per expert in the form that the library picks, and in 256-row tiles."""
+    from ccfuser_amd import ops
+    ops.set_option("few_rows", request.param)
+    yield request.param
+    ops.set_option("few_rows", 1)

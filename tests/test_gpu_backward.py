@@ -38,6 +38,7 @@ def _case(T, d, f, E, k, seed, skew=False):
     return p
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("T,d,f,E,k,cap,skew,seed", [
     (300, 256, 512, 4, 2, -1, False, 0),
     (512, 512, 256, 8, 2, 100, False, 1),     # capacity drops slots
@@ -270,6 +271,7 @@ def _ffn_backward_stages(T, d, f, E, k, cap, skew, seed):
     _close(gb1_2, gb1_ref2, "grad_b1 through the GELU")
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("T,d,f,E,k,cf,seed", [
     (384, 256, 512, 4, 2, None, 10),
     (512, 256, 512, 8, 2, 1.0, 11),          # capacity factor 1.0 drops slots
@@ -410,6 +412,7 @@ def _random_shapes(count, seed):
     return out
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("T,d,f,E,k,cap,seed", _random_shapes(10, 4242))
 def test_ffn_backward_random_shapes(T, d, f, E, k, cap, seed):
     """Widths from 64 to 640 in steps of 64 (one K tile, partial M and N tiles, both weight

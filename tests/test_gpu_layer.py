@@ -35,6 +35,7 @@ def _check_layer(wl, out, routing, ref):
     assert ma <= MAX_ABS and mr <= MEAN_REL
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("name,rows", [
     ("c1_tiny", None),          # 512 tokens, run in fp16 on the GPU (the reference's GPU path is fp16 only)
     ("c2_gshard", 1024),        # capacity 1.25 with drops
@@ -74,6 +75,7 @@ def test_golden_layer_fixture():
     assert O.max_abs_err(out.cpu(), ref) <= MAX_ABS and O.mean_rel_err(out.cpu(), ref) <= MEAN_REL
 
 
+@pytest.mark.usefixtures("gemm_form")
 def test_mirrored_module_staged_equals_fused(workloads):
     """MixMOETransformerMLP through process_data + MixMOE.forward (the reference's
     call sequence) gives the same bits as the single fused call, and the async
@@ -117,6 +119,7 @@ def test_mirrored_module_staged_equals_fused(workloads):
     mlp.close()
 
 
+@pytest.mark.usefixtures("gemm_form")
 def test_extension_class_with_reference_block_arrays(workloads):
     """mix_moe_cuda.MixMOE.first_gemm_forward / second_gemm_forward / forward called
     with the reference's argument lists (pybind.cpp:39-58): [E,K,N] weights and the
@@ -152,6 +155,7 @@ def test_extension_class_with_reference_block_arrays(workloads):
     assert O.max_abs_err(y2.cpu(), y_ref) <= MAX_ABS
 
 
+@pytest.mark.usefixtures("gemm_form")
 def test_extension_class_backward_with_reference_block_arrays(workloads):
     """mix_moe_cuda.MixMOE.first_gemm_backward / second_gemm_backward called the way
     MixMOELinear1/2.backward call them (linear.py:103, 162; pybind.cpp:56-57): stored
@@ -219,6 +223,7 @@ def test_extension_class_backward_with_reference_block_arrays(workloads):
                                t["b2"].cuda(), pos, *blocks)
 
 
+@pytest.mark.usefixtures("gemm_form")
 def test_ep_share_segments(workloads):
     """One GPU's expert-parallel share at reduced rows: (start, len, expert) triples."""
     from ccfuser_amd import ops
@@ -485,11 +490,12 @@ def test_fused_call_equals_stage_by_stage_calls(workloads, name, rows, variant):
         ops.set_option("gemm_variant", -1)
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("T,d,f,E,k", [(2048, 64, 128, 600, 2), (4096, 128, 64, 1024, 1), (300, 64, 64, 37, 4),
                                        (1000, 128, 64, 20, 3), (5000, 256, 64, 8, 8)])
 def test_fused_layer_with_many_experts(T, d, f, E, k):
-    """Most experts get a handful of rows or none; the routing launch builds the tile plans with
-    eight workgroups per plan and needs more than 64 KB of LDS past 512 experts.  The cases also
+    """Most experts get a handful of rows or none; in 256-row tiles the routing launch builds the tile plans
+    with eight workgroups per plan and needs more than 64 KB of LDS past 512 experts.  The cases also
     cover the ways the routing stage gets its counts: from the gate kernel's workgroups (top-k
     a power of two, small table), from its own histogram launch (1024 experts; top-3)."""
     from ccfuser_amd import ops
@@ -522,6 +528,7 @@ def _random_layer_shapes(count, seed):
     return shapes + [(1, 64, 64, 1, 1, -1, 9100), (257, 832, 320, 3, 3, 100, 9101)]
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("T,d,f,E,k,cap,seed", _random_layer_shapes(12, 777))
 def test_fused_layer_random_shapes(T, d, f, E, k, cap, seed):
     """Shapes drawn at random (1-3000 tokens, widths any multiple of 64 up to 768 x 1024, 1-40
@@ -547,12 +554,12 @@ def test_fused_layer_random_shapes(T, d, f, E, k, cap, seed):
     assert torch.equal(fused, _staged_forward(ops, args, E, k, cap))
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("T,d,f,E,k", [(1, 256, 1024, 8, 2), (2, 512, 512, 8, 2), (48, 256, 1024, 16, 2),
                                        (97, 1024, 256, 32, 2), (130, 256, 512, 4, 2), (64, 320, 832, 32, 1)])
 def test_fused_layer_with_a_few_rows_per_expert(T, d, f, E, k):
-    """Fewer rows than 64 per expert: every expert is a skinny M tile of its own, more of them than
-    64-row blocks fit the rows (the list of skinny tiles is sized by experts, not by rows).  Against
-    the oracle, the staged path bit for bit, and a second call bit for bit."""
+    """Fewer rows than 64 per expert, in either form, against the oracle, the staged path bit for bit, and a
+    second call bit for bit."""
     from ccfuser_amd import ops
     _say(f"few rows per expert T={T} d={d} f={f} E={E} k={k}")
     g = torch.Generator().manual_seed(100 * T + d)
@@ -577,10 +584,61 @@ def test_fused_layer_with_a_few_rows_per_expert(T, d, f, E, k):
     assert torch.equal(out, ops.combine(y, score.view(-1), k, m["inv_pos"]))
 
 
+@pytest.mark.parametrize("T,d,f,E,k,which", [(32, 256, 1024, 64, 1, (1,)), (16, 256, 4160, 16, 2, (1, 2)),
+                                             (3, 512, 4096, 32, 4, (1, 2)), (100, 4096, 1024, 64, 2, (1,))])
+def test_skinny_list_with_more_tiles_than_blocks_of_rows(T, d, f, E, k, which):
+    """A few rows per expert, forced into skinny tiles that are cut along K: every expert with rows is a skinny M tile of
+    its own, more of them than 64-row blocks fit the rows, so the list of skinny tiles is sized by experts, not by rows
+    (in the layer call the plan of the second GEMM lies behind the first one's list).  Against the oracle, and two
+    calls bit for bit."""
+    from ccfuser_amd import ops
+    _say(f"skinny list T={T} d={d} f={f} E={E} k={k}")
+    g = torch.Generator().manual_seed(T + f)
+    r = lambda *s, sc=1.0: (torch.randn(*s, generator=g) * sc).half()
+    cpu = (r(T, d), r(E, d, sc=0.05), r(E, sc=0.02), r(E, f, d, sc=0.02), r(E, f, sc=0.02), r(E, d, f, sc=0.02), r(E, d, sc=0.02))
+    ref = O.moe_layer_forward(*cpu, k, capacity=-1)
+    args = [a.cuda() for a in cpu]
+    x, wg, bg, w1, b1, w2, b2 = args
+    n = T * k
+    ops.set_option("skinny", -6)
+    try:
+        out = ops.moe_forward(*args, k)
+        again = ops.moe_forward(*args, k)
+        m = ops.route(ops.gate_topk_softmax(x, wg, bg, k)[0].view(-1), E, k)
+        ws = ops.ffn_workspace(n, E, d, f, x).zero_()
+        h = ops.ffn1(x, m["src_row"], m["offsets"], n, w1, b1, workspace=ws)
+        ops.ffn2(h, m["dst_row"], m["offsets"], n, w2, b2, torch.empty(n, d, dtype=torch.float16, device="cuda"), workspace=ws)
+        for w in which:
+            n_cols = -(-(f if w == 1 else d) // 256)
+            assert ops.ffn_plan_info(ws, n, E, d, f, w)["skinny_tiles"] > -(-n // 64) * n_cols, w
+    finally:
+        ops.set_option("skinny", 1)
+    assert O.max_abs_err(out.cpu(), ref["out"]) <= MAX_ABS and O.mean_rel_err(out.cpu(), ref["out"]) <= MEAN_REL
+    assert torch.equal(out, again)
+
+
+def test_one_token_takes_the_cut_tiles_of_a_long_contraction():
+    """Two rows, 16 tiles each of a contraction over 14336: by default the 256-row launch with fewer plan entries than
+    compute units, its tiles cut along K, against fp32 (bound: see below)."""
+    from ccfuser_amd import ops
+    E, n, K, N = 2, 2, 14336, 4096
+    g = torch.Generator(device="cuda").manual_seed(3)
+    h = torch.randn(n, K, generator=g, device="cuda").half()
+    w = (torch.randn(E, N, K, generator=g, device="cuda") * 0.02).half()
+    b = torch.randn(E, N, generator=g, device="cuda").half()
+    off = torch.tensor([0, 1, 2], dtype=torch.int32, device="cuda")
+    ws = ops.ffn_workspace(n, E, N, K, h).zero_()
+    y = ops.ffn2(h, None, off, n, w, b, torch.empty(n, N, dtype=torch.float16, device="cuda"), workspace=ws)
+    info = ops.ffn_plan_info(ws, n, E, N, K, 2)
+    assert info["split_tiles"] + info["skinny_tiles"] > 0 and info["worst_case_tiles"] < info["persistent_wgs"], info
+    ref = torch.stack([h[e].float() @ w[e].float().t() + b[e].float() for e in range(E)])
+    assert float((y.float() - ref).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(ref.abs().max()) + 1e-4
+
+
 @pytest.mark.parametrize("counts", [[1], [5, 0, 70], [300, 17, 129, 64], [0, 513, 0, 256]])
-def test_few_tiles_of_a_long_contraction(counts):
-    """Fewer plan entries than compute units, each a contraction over 4160: cut along K over all of them, as
-    skinny tiles or as the split last round.  Both products, the pre-activation form and the input gradient on
+def test_few_tiles_of_a_long_contraction(counts, gemm_form):
+    """Fewer plan entries than compute units, each a contraction over 4160; in 256-row tiles: cut along K over all of
+    them, as skinny tiles or as the split last round.  Both products, the pre-activation form and the input gradient on
     the stored [K][N] weight, against fp32 (fp16 results of sums of 4160 products of order 1e-2: half an fp16
     step of the result, 2^-11, plus 4160 * 2^-24 relative for the order of the sums)."""
     from ccfuser_amd import ops
@@ -597,7 +655,10 @@ def test_few_tiles_of_a_long_contraction(counts):
     def close(got, want):
         assert float((got.float() - want).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(want.abs().max()) + 1e-4
 
-    y = ops.ffn2(a, None, off, n, w, b, torch.empty(n, N, dtype=torch.float16, device="cuda"))
+    ws = ops.ffn_workspace(n, E, N, K, a).zero_()
+    y = ops.ffn2(a, None, off, n, w, b, torch.empty(n, N, dtype=torch.float16, device="cuda"), workspace=ws)
+    info = ops.ffn_plan_info(ws, n, E, N, K, 2)
+    assert gemm_form or info["split_tiles"] + info["skinny_tiles"] > 0, info
     close(y, ref)
     assert torch.equal(y, ops.ffn2(a, None, off, n, w, b, torch.empty_like(y)))
     close(ops.ffn1(a, None, off, n, w, b), torch.nn.functional.gelu(ref))
@@ -639,6 +700,7 @@ def test_tiles_for_most_compute_units_need_no_reduction(E, rows, N, K, cut):
     assert float((y.float() - ref).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(ref.abs().max()) + 1e-4
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("T,d,f,E,k,bs,stored", [(1, 64, 192, 4, 2, 64, False), (333, 320, 832, 5, 2, 64, False),
                                                   (700, 256, 256, 3, 1, 32, False), (900, 512, 1024, 8, 2, 64, True),
                                                   (60, 4160, 512, 2, 2, 64, False)])
@@ -675,6 +737,55 @@ def test_block_arrays_on_kn_weights(T, d, f, E, k, bs, stored):
     # a block count below the arrays' length, and none: rows that no block covers are zero
     part = mix_moe_hip.MixMOE(1, T, E, k, d, f, bs, *kn, b1, b2).forward(x, m["pos"], *blocks[:4], 0, 0)
     assert part.shape == want.shape and not part.any()
+
+
+@pytest.mark.parametrize("T,d,f,E", [(3000, 1088, 1344, 24), (1500, 1344, 832, 40), (2000, 320, 4160, 12)])
+def test_block_arrays_in_256_row_tiles(T, d, f, E):
+    """``MixMOE.forward`` on [E, K, N] weights with the tile plans that the regrouping launch builds, at widths that
+    are no multiple of the column tile: without any cut the bits of the staged calls on [E, N, K] weights, the same
+    with skinny tiles beside the others; with the plan's own choice, with skinny tiles cut along K and with the last
+    round cut as well, those results within two fp16 steps of the largest.  Every mix of weight layouts."""
+    from ccfuser_amd import mix_moe_hip, ops
+    k, bs = 2, 64
+    _say(f"block arrays in 256-row tiles T={T} d={d} f={f} E={E}")
+    g = torch.Generator().manual_seed(T + d)
+    r = lambda *s, sc=1.0: (torch.randn(*s, generator=g) * sc).half().cuda()
+    x, w1, b1, w2, b2 = r(T, d), r(E, f, d, sc=0.05), r(E, f), r(E, d, f, sc=0.05), r(E, d)
+    m = ops.route(torch.randint(0, E, (T * k,), generator=g).cuda(), E, k)
+    plan = ops.plan_blocks(m["counts"], T * k, bs)
+    total, remote = plan["block_nums"].tolist()
+    blocks = (plan["expert_ids"], plan["ranks"], plan["lens"], plan["start_addrs"], total, remote)
+    kn = [w.transpose(-2, -1).contiguous() for w in (w1, w2)]
+
+    def forward(first, second, **knobs):
+        for name, value in dict(dict(few_rows=0, skinny=1, split_tail=1), **knobs).items():
+            ops.set_option(name, value)
+        try:
+            return mix_moe_hip.MixMOE(1, T, E, k, d, f, bs, first, second, b1, b2).forward(x, m["pos"], *blocks)
+        finally:
+            for name in ("few_rows", "skinny", "split_tail"):
+                ops.set_option(name, 1)
+
+    off = dict(skinny=0, split_tail=0)
+    plain = forward(*kn, **off)
+    for name, value in dict(off, few_rows=0).items():
+        ops.set_option(name, value)
+    try:
+        h = ops.ffn1(x, m["src_row"], m["offsets"], T * k, w1, b1)
+        staged = ops.ffn2(h, m["dst_row"], m["offsets"], T * k, w2, b2, torch.empty_like(plain))
+    finally:
+        for name in ("few_rows", "skinny", "split_tail"):
+            ops.set_option(name, 1)
+    assert torch.equal(plain, staged)
+    assert torch.equal(plain, forward(w1, kn[1], **off)) and torch.equal(plain, forward(kn[0], w2, **off))
+    assert torch.equal(plain, forward(*kn, skinny=-2, split_tail=0))
+    most = float(plain.float().abs().max())
+    for knobs in ({}, dict(skinny=-6, split_tail=0), dict(skinny=-6, split_tail=2), dict(skinny=0, split_tail=2)):
+        got = forward(*kn, **knobs)
+        assert float((got.float() - plain.float()).abs().max()) <= 2.0 ** -9 * most, knobs
+        assert torch.equal(got, forward(*kn, **knobs)), knobs
+        if knobs.get("skinny") == -6:
+            assert not torch.equal(got, plain), knobs       # summed in another order: the cut form ran
 
 
 def _forced_plan_cases(count, seed):

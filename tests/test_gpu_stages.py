@@ -433,6 +433,7 @@ def _ffn_case(R, d, f, E, seed, skew=False):
     return x, w1, b1, w2, b2, e_of_row
 
 
+@pytest.mark.usefixtures("gemm_form")
 @pytest.mark.parametrize("variant", [0, 1, 2, 3])
 @pytest.mark.parametrize("R,d,f,E,skew,seed", [
     (512, 256, 1024, 4, False, 0),
@@ -648,6 +649,7 @@ def test_few_row_rule_takes_the_faster_form(E, rows, d, f, which, few):
     assert (ops.ffn_plan_info(ws, R, E, d, f, which)["persistent_wgs"] == 0) == few
 
 
+@pytest.mark.usefixtures("gemm_form")
 def test_ffn_special_cases():
     """Closed forms: zero weights give the bias path; a single expert is a dense MLP."""
     from ccfuser_amd import ops
