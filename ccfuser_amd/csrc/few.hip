@@ -1,9 +1,9 @@
 // Grouped GEMM of few rows per expert for gfx950: decoding batches, short prompts, small layers.
 //
 // The 256-row tiles of ffn.hip leave most of the chip idle there: 32 rows per expert fill an eighth of a
-// tile, and a layer of a few hundred rows makes a few dozen tiles for 256 CUs.  This kernel has tiles of 32,
-// 64 or 128 rows by 64, 128 or 256 columns, picks among them on the device from the experts' row counts, and
-// runs all of K in one workgroup: no plan launch in front, no partial tiles, no reduction behind.
+// tile, and a layer of a few hundred rows makes a few dozen tiles for 256 CUs.  This kernel has tiles of 64
+// or 128 rows by 64, 128 or 256 columns, picks among them on the device from the experts' row counts, and runs
+// all of K in one workgroup: no plan launch in front, no partial tiles, no reduction behind.
 //
 //   * every workgroup derives its own tiles from the offsets (a scan over the experts and one binary search
 //     per tile), so the launch stands alone;

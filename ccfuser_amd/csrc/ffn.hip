@@ -92,13 +92,13 @@ __device__ __forceinline__ int tile_row_to_local(int r, int rows) {
   return RingFor<Cfg, false>::local_row(r, rows);
 }
 
+// First column (of eight) that a load of a [K][N] operand fetches: past the matrix, the last eight again.
+__device__ __forceinline__ int kn_column(int c, int N) { return c < N - 8 ? c : N - 8; }
+
 // Global source of every tile load of this lane for the tile of plan entry
 // `ent`: K element 0 of the (clamped) A row and B row, at this lane's K chunk.
 // Padded A rows re-read the tile's last real row, B rows past N the last row.
 // tid: threadIdx.x, or fresh_tid() where what is derived from it must not be kept from an earlier call.
-// First column (of eight) that a load of a [K][N] operand fetches: past the matrix, the last eight again.
-__device__ __forceinline__ int kn_column(int c, int N) { return c < N - 8 ? c : N - 8; }
-
 template <class Cfg, bool kSeg = false, bool kKN = false>
 __device__ __forceinline__ void tile_sources(const GroupedArgs &p, const int4v ent,
                                              const half_t *(&a_src)[Cfg::A_DMA],

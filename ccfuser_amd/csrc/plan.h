@@ -552,13 +552,13 @@ struct SkinnyCount {
   double full, skinny;
 };
 SkinnyCount skinny_tiles(int max_rows, int E);
-// few.hip: the forward GEMMs of few rows per expert.  C[c_rows[j]] = epilogue(A[a_rows[j]] * B[e]^T + bias[e]) for the
-// rows offsets[e] <= j < offsets[e+1]; the forms are those of the grouped GEMM's epilogues 0, 1 and 2.
+// few.hip: the forward and input-gradient GEMMs of few rows per expert.  C[c_rows[j]] = epilogue(A[a_rows[j]] * B[e]^T +
+// bias[e]) for the rows offsets[e] <= j < offsets[e+1]; the forms are those of the grouped GEMM's epilogues 0, 1 and 2.
 constexpr int kFewPlain = 0, kFewGelu = 1, kFewGeluKeep = 2;
 struct FewArgs {
   const half_t *A;
   const int32_t *a_rows;     // or NULL (identity)
-  const half_t *B, *bias;    // [E, N, K], [E, N] or NULL
+  const half_t *B, *bias;    // [E, N, K] or, for the [K][N] forms, [E, K, N]; [E, N] or NULL
   half_t *C, *C2;            // C2: pre-activations in expert order (kFewGeluKeep)
   const int32_t *c_rows;     // or NULL (identity)
   const half_t *row_scale;   // or NULL
