@@ -396,6 +396,7 @@ double upper_tail(double z) { return 1 / (1 + std::exp(z * (1.5976 + 0.07056 * z
 
 TileCount m_tiles(int max_rows, int E, int bm) {
   const int used = E < max_rows ? E : max_rows;
+  if (used <= 0) return {0.0, 0.0};
   const double avg = static_cast<double>(max_rows) / used, sd = std::sqrt(avg * (1.0 - 1.0 / used));
   if (sd == 0) return {used * std::ceil(avg / bm), 0.0};
   // tiles of an expert: the sum over j of (rows > j bm)
@@ -404,7 +405,7 @@ TileCount m_tiles(int max_rows, int E, int bm) {
   double m = j0, m2 = static_cast<double>(j0) * j0;
   for (int j = j0;; ++j) {
     const double p = upper_tail((static_cast<double>(j) * bm + 0.5 - avg) / sd);
-    if (p < 1e-4) break;
+    if (!(p >= 1e-4)) break;
     m += p;
     m2 += (2.0 * j + 1) * p;
   }
@@ -419,7 +420,7 @@ static double mean_rounds(const TileCount &t, int n_col, int cus) {
   double rounds = first > 0 ? first : 0;
   for (double r = rounds;; r += 1) {
     const double p = upper_tail((std::floor(r * per) + 0.5 - t.mean) / sd);       // more M tiles than r rounds hold
-    if (p < 1e-3) break;
+    if (!(p >= 1e-3)) break;
     rounds += p;
   }
   return rounds;
@@ -427,6 +428,7 @@ static double mean_rounds(const TileCount &t, int n_col, int cus) {
 
 SkinnyCount skinny_tiles(int max_rows, int E) {
   const int used = E < max_rows ? E : max_rows;
+  if (used <= 0) return {0.0, 0.0};
   const double avg = static_cast<double>(max_rows) / used, sd = std::sqrt(avg * (1.0 - 1.0 / used));
   const auto at_most = [&](double x) { return sd > 0 ? 1 - upper_tail((x + 0.5 - avg) / sd) : (avg <= x ? 1.0 : 0.0); };
   const int j0 = avg > 5 * sd ? static_cast<int>((avg - 5 * sd) / 256) : 0, j1 = static_cast<int>((avg + 5 * sd) / 256);
@@ -440,7 +442,8 @@ SkinnyCount skinny_tiles(int max_rows, int E) {
 }
 
 bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn, int cus) {
-  if (!mode || epi > kFewGeluKeep || (b_kn && epi == kFewGeluKeep) || cus < 8 || K % kBK || E > 1024) return false;
+  if (!mode || epi > kFewGeluKeep || (b_kn && epi == kFewGeluKeep) || cus < 8 || K % kBK || E <= 0 || E > 1024 || max_rows <= 0)
+    return false;
   // the tile table holds kFewMaxRounds tiles per workgroup of the largest shape
   const long long worst = (static_cast<long long>(max_rows) / 128 + E) * ((N + 255) / 256);
   if (worst >= static_cast<long long>(kFewMaxRounds - 1) * cus) return false;

@@ -402,6 +402,20 @@ def test_backward_without_rows():
     assert gx.shape == (0, d) and float(gw1.abs().max()) == 0.0 and float(gb1.abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("E,d,f", [(3, 4160, 64), (70, 64, 512), (3, 64, 4160)])
+def test_backward_without_rows_of_a_long_contraction(E, d, f):
+    """No rows at sizes where the form of the input-gradient GEMM, or a cut along K, is decided by an estimate."""
+    from ccfuser_amd import ops
+    offsets = torch.zeros(E + 1, dtype=torch.int32, device="cuda")
+    empty = lambda n: torch.empty(0, n, dtype=torch.float16, device="cuda")
+    w2 = torch.ones(E, d, f, dtype=torch.float16, device="cuda")
+    ga, gw, gb = ops.ffn2_backward(empty(d), empty(f), None, offsets, 0, w2)
+    assert ga.shape == (0, f) and not gw.any() and not gb.any()
+    w1 = torch.ones(E, f, d, dtype=torch.float16, device="cuda")
+    gx, gw, gb = ops.ffn1_backward(empty(f), empty(d), None, None, offsets, 0, w1, 0)
+    assert gx.shape == (0, d) and not gw.any() and not gb.any()
+
+
 def _random_shapes(count, seed):
     g = torch.Generator().manual_seed(seed)
     r = lambda lo, hi: int(torch.randint(lo, hi + 1, (1,), generator=g))
