@@ -474,8 +474,8 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
     steps = rounds * (kt * kFewStepUs[i] + kFewEpiUs[epi == kFewPlain][i]);
   }
   const double mine = std::sqrt(steps * steps + weights * weights) + 5;
-  // 256 x 256 tiles: 1.02 us a K step (1.2 to 1.45 with the whole chip at it, which this range never has) and the
-  // epilogue; a last round of at most half the CUs is cut along K
+  // 256 x 256 tiles: 1.02 us a K step and the epilogue, fitted with the weights beside them (a step alone measures 1.2 to
+  // 1.45 us); a last round of at most half the CUs is cut along K
   const TileCount big_mt = m_tiles(max_rows, E, 256);
   const double tile = kt * 1.02 + (epi == kFewPlain ? 5 : 15);
   if (kt >= 64) {
