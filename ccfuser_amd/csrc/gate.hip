@@ -20,7 +20,8 @@
 // per K element.  The blocks of an instruction are independent products, so a
 // block is either another group of tokens or the same tokens on another part
 // of K ("slot"): few tokens still fill the machine.  fp32 inputs keep multiply
-// and add separate (two roundings) and run on the vector unit.
+// and add separate (two roundings): both on the vector unit, or with many tokens
+// the multiplies as MFMAs onto zero.
 #include "ccf_common.h"
 #include "mfma_f32.h"
 
@@ -611,7 +612,7 @@ gate_stream_kernel(const half_t *__restrict__ x, const half_t *__restrict__ wg, 
 // * Behind a round of parts their sums meet in LDS and are added in ascending order onto the running sums.
 //
 // TT shrinks with the tokens, so that 2049 and 4097 tokens still make 129 workgroups, EE with the experts.
-// 8192 tokens x 2048, 64 experts, top-2: 66 us, 988 us as one wavefront per token whose lanes each walked
+// 4096 tokens x 2048, 64 experts, top-2: 42 us; 8192 tokens: 66 us, 988 us as one wavefront per token whose lanes each walked
 // rows of their own (and left the selection to one lane).
 constexpr int kF32StageK = 16;                     // K elements of a stage
 constexpr int kF32Row = kF32StageK + 4;            // row stride in LDS, floats
@@ -775,9 +776,189 @@ int launch_gate_f32(const float *x, const float *wg, const float *bg, int tokens
 template <int TT>
 int launch_gate_f32_experts(const float *x, const float *wg, const float *bg, int tokens, int d, int E, int k,
                             int64_t *idx_out, float *score_out, float *logits_out, hipStream_t stream) {
-  auto launch = E <= 8 ? launch_gate_f32<TT, 1> : (E <= 16 ? launch_gate_f32<TT, 2>
-                                                           : (E <= 32 ? launch_gate_f32<TT, 4> : launch_gate_f32<TT, 8>));
+  auto launch = E <= 8 ? launch_gate_f32<TT, 1> : (E <= 16 ? launch_gate_f32<TT, 2> : launch_gate_f32<TT, 4>);
+  if constexpr (TT < 4) {                          // more tokens of more than 32 experts: gate_f32_on_mfma()
+    if (E > 32) launch = launch_gate_f32<TT, 8>;
+  }
   return launch(x, wg, bg, tokens, d, E, k, idx_out, score_out, logits_out, stream);
+}
+
+// The same order with the products on the matrix cores: fma(x, w, 0) of a K = 1 MFMA is the rounded product, subnormal
+// ones included, for 2048 token-expert pairs in 64 cycles, and the vector unit has one addition per product left
+// instead of two instructions.  (A product of -0 comes out as +0, which no running sum can tell: it starts at +0 and is
+// never -0.)  The two do not overlap, not even from two wavefronts of a SIMD: a step takes 30 ns for the MFMA and 40
+// for its 32 additions, against 80 for 64 vector instructions, and two LDS reads feed 32 of them instead of three.
+//
+// * A wavefront computes 32 tokens x 64 experts (64 x 32, 64 x 16 for fewer experts) over one part of K, one product
+//   tile ahead of the additions; the wavefronts of a workgroup take different parts of the same tile.
+// * Operands come in stages of 16 K elements through the wavefront's own LDS, as above, into one buffer: a
+//   wavefront's LDS accesses happen in order, so its writes of the next stage land behind its reads of this one.
+//   The last stage of a part loads the first of the wavefront's next part.
+// * Eight threads select a token's experts (one per token: 4 us of 64 experts).
+//
+// 8192 tokens x 2048, 64 experts, top-2: 64 -> 49 us; x 4096: 116 -> 92; 32768 x 2048, 32 experts: 141 -> 96.
+template <int N, int WE>
+struct GateF32Mfma {
+  static constexpr int WT = 64 / N * N * N / WE;   // tokens of a tile
+  static constexpr int ROWS = WT + WE;
+  static constexpr int LOADS = (ROWS + 15) / 16;
+  static constexpr int BUF = LOADS * 16 * kF32Row;
+  static constexpr int LD = WE + 1;
+  static constexpr int REGION = BUF > WT * LD ? BUF : WT * LD;           // a wavefront's LDS, floats
+};
+
+template <int N, int WE, int KS>
+__global__ void __launch_bounds__(kMaxWaves * 64)
+gate_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__ wg, const float *__restrict__ bg,
+                     int tokens, int d, int E, int k, int64_t *__restrict__ idx_out,
+                     float *__restrict__ score_out, float *__restrict__ logits_out) {
+#pragma clang fp contract(off)
+  using C = GateF32Mfma<N, WE>;
+  using M = Mfma<N>;
+  extern __shared__ float s_mem[];
+  const int waves = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  float *region = s_mem + static_cast<size_t>(wave) * C::REGION;
+  float *s_logit = s_mem + static_cast<size_t>(waves) * C::REGION;       // [WT][LD] running sums, then logits
+  const int t0 = blockIdx.x * C::WT;
+  const int nparts = (d + kPart - 1) / kPart;
+  const int l_row = lane >> 2, l_piece = lane & 3;                       // as a loader
+  // as a reader: the instruction's blocks are other tokens, or the same tokens and other experts
+  const int my_t = WE == N ? lane : lane % N;
+  const int my_e = C::WT + (WE == N ? lane % N : lane);
+  // as a selector: 8 threads per token, every eighth expert each, where there are as many threads
+  const int per = static_cast<int>(blockDim.x) >= 8 * C::WT ? 8 : 1;
+  const int sel_t = threadIdx.x / per, sel_e = threadIdx.x % per;
+  typename M::Acc zero;
+#pragma unroll
+  for (int v = 0; v < M::kRegs; ++v) zero[v] = 0.0f;
+  Best<KS> best;
+  best.clear();
+  for (int e0 = 0; e0 < E; e0 += WE) {
+    // this lane's rows of the tile's tokens, then of its experts (past the end: a repeated row, never used)
+    const float *xb = x + static_cast<size_t>(t0) * d, *wb = wg + static_cast<size_t>(e0) * d;
+    unsigned src[C::LOADS];
+#pragma unroll
+    for (int i = 0; i < C::LOADS; ++i) {
+      const int r = 16 * i + l_row - (16 * i < C::WT ? 0 : C::WT);
+      const int most = (16 * i < C::WT ? tokens - t0 : E - e0) - 1;
+      src[i] = static_cast<unsigned>(r < most ? r : most) * d + l_piece * 4;
+    }
+    float4v reg[C::LOADS];
+    // K past the part's end reads as zero, which adds nothing
+    auto fetch = [&](int kk, int k_hi) {
+      const bool in = kk + l_piece * 4 < k_hi;                           // d is a multiple of 8
+#pragma unroll
+      for (int i = 0; i < C::LOADS; ++i) {
+        const float4v none = {0.0f, 0.0f, 0.0f, 0.0f};
+        reg[i] = in ? *reinterpret_cast<const float4v *>((16 * i < C::WT ? xb : wb) + (src[i] + static_cast<unsigned>(kk))) : none;
+      }
+    };
+    if (wave < nparts) fetch(wave * kPart, d);
+    for (int p0 = 0; p0 < nparts; p0 += waves) {
+      const int part = p0 + wave;
+      if (part < nparts) {                                               // uniform per wavefront
+        const int k_lo = part * kPart;
+        const int k_hi = k_lo + kPart < d ? k_lo + kPart : d;
+        float acc[M::kRegs];
+#pragma unroll
+        for (int v = 0; v < M::kRegs; ++v) acc[v] = 0.0f;
+        for (int kk = k_lo; kk < k_hi; kk += kF32StageK) {
+#pragma unroll
+          for (int i = 0; i < C::LOADS; ++i)
+            *reinterpret_cast<float4v *>(region + (16 * i + l_row) * kF32Row + l_piece * 4) = reg[i];
+          // the next stage, at the part's end the first of this wavefront's next part
+          const int next = kk + kF32StageK < k_hi ? kk + kF32StageK : k_lo + waves * kPart;
+          if (next < d) fetch(next, d);
+          asm volatile("" ::: "memory");                                 // the loads stay ahead of the arithmetic
+          const float *xr = region + my_t * kF32Row, *wr = region + my_e * kF32Row;
+          float4v xv[2], wv[2];
+          xv[0] = *reinterpret_cast<const float4v *>(xr);
+          wv[0] = *reinterpret_cast<const float4v *>(wr);
+          typename M::Acc prod[2];
+          prod[0] = M::run(xv[0][0], wv[0][0], zero);
+#pragma unroll
+          for (int q = 0; q < kF32StageK; ++q) {
+            const int c = q >> 2, n = q + 1;
+            if ((q & 3) == 0 && c + 1 < kF32StageK / 4) {
+              xv[(c + 1) & 1] = *reinterpret_cast<const float4v *>(xr + 4 * (c + 1));
+              wv[(c + 1) & 1] = *reinterpret_cast<const float4v *>(wr + 4 * (c + 1));
+            }
+            // the next products are issued ahead of these additions, and stay there (left alone, the compiler puts
+            // them among the additions, which then wait)
+            if (n < kF32StageK) prod[n & 1] = M::run(xv[(n >> 2) & 1][n & 3], wv[(n >> 2) & 1][n & 3], zero);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < M::kRegs; ++v) {
+              acc[v] = acc[v] + prod[q & 1][v];
+              asm volatile("" : "+v"(acc[v]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          asm volatile("" ::: "memory");
+        }
+#pragma unroll
+        for (int v = 0; v < M::kRegs; ++v) {
+          const int b = M::block(v) * N, row = M::row(v, lane), col = lane % N;
+          region[(WE == N ? b + row : row) * C::LD + (WE == N ? col : b + col)] = acc[v];
+        }
+      }
+      __syncthreads();
+      const int np = nparts - p0 < waves ? nparts - p0 : waves;
+      const bool last = p0 + waves >= nparts;
+      for (int o = threadIdx.x; o < C::WT * WE; o += blockDim.x) {
+        const int t = o / WE, e = o % WE;
+        const int at = t * C::LD + e;
+        float s = p0 == 0 ? s_mem[at] : s_logit[at] + s_mem[at];
+        for (int w = 1; w < np; ++w) s = s + s_mem[static_cast<size_t>(w) * C::REGION + at];
+        if (last && e0 + e < E) {
+          if (bg) s = s + bg[e0 + e];
+          if (logits_out && t0 + t < tokens) logits_out[static_cast<size_t>(t0 + t) * E + e0 + e] = s;
+        }
+        s_logit[at] = s;
+      }
+      __syncthreads();
+    }
+    if (sel_t < C::WT) {
+      const int ne = (E - e0) < WE ? (E - e0) : WE;
+      for (int e = sel_e; e < ne; e += per) best.offer(s_logit[sel_t * C::LD + e], e0 + e, k);
+    }
+    // the next tile's logits are written behind the barrier that follows its first round's part sums
+  }
+  // lists of disjoint experts: (logit, expert) is a strict order, so it does not matter in which order they are offered
+  for (int off = 1; off < per; off <<= 1) {
+    float ov[KS];
+    int oid[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      ov[s] = __shfl_xor(best.v[s], off, 64);
+      oid[s] = __shfl_xor(best.id[s], off, 64);
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      if (s < k && oid[s] != INT_MAX) best.offer(ov[s], oid[s], k);
+  }
+  if (sel_t < C::WT && sel_e == 0 && t0 + sel_t < tokens) best.template write<float>(t0 + sel_t, k, idx_out, score_out);
+}
+
+template <int N, int WE>
+int launch_gate_f32_mfma(const float *x, const float *wg, const float *bg, int tokens, int d, int E, int k, int64_t *idx_out,
+                         float *score_out, float *logits_out, hipStream_t stream) {
+  using C = GateF32Mfma<N, WE>;
+  const int nparts = (d + kPart - 1) / kPart;
+  const int waves = nparts < kMaxWaves ? nparts : kMaxWaves;
+  const size_t lds = sizeof(float) * (static_cast<size_t>(waves) * C::REGION + C::WT * C::LD);
+  static_assert(sizeof(float) * (kMaxWaves * C::REGION + C::WT * C::LD) <= 160 * 1024, "LDS of a CU");
+  auto kern = k <= 2 ? gate_f32_mfma_kernel<N, WE, 2> : gate_f32_mfma_kernel<N, WE, kMaxTopK>;
+  if (lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       static_cast<int>(lds));
+    if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate: LDS attribute: %s", hipGetErrorString(e));
+  }
+  hipLaunchKernelGGL(kern, dim3((tokens + C::WT - 1) / C::WT), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
+                     idx_out, score_out, logits_out);
+  return check_launch("gate_f32_mfma_kernel");
 }
 
 // The same for few tokens where those tiles leave most of their lanes or wavefronts idle: one to three experts of a
@@ -839,6 +1020,18 @@ bool gate_f32_walks(int tokens, int d, int E) {
   return (E > 32 && d <= kPart && tokens <= (E > 64 ? 1024 : 512)) || (E > 128 && d <= 2 * kPart && tokens <= 512);
 }
 
+// Where the products run as MFMAs, in microseconds (vector unit, MFMA).  More than 32 experts: at 4097 tokens, where the
+// vector unit's tiles grow to 32 tokens as well, 64 experts of 256: 32, 29; of 2048: 55, 43; of 7168: 157, 135 (4096
+// tokens of 2048: 42, 46).  Up to 32 experts the tiles are twice as tall (8192 tokens of 2048, 32 experts: 39, 48; 8193:
+// 61, 43) and want six parts of K (24576 of 512, 32 experts: 28, 28; 8193: 19, 24), and a second round of
+// workgroups more of them (24576 tokens of 768, 32 experts: 46, 53; of 2048: 101, 86).  16 experts of a very wide model
+// are bound by reading the tokens (16384 of 7168, 9 experts: 119, 126).
+bool gate_f32_on_mfma(int tokens, int d, int E) {
+  if (E > 32) return tokens > 4096;
+  if (E <= 8 || tokens <= 8192 || d <= 5 * kPart) return false;
+  return (tokens <= 16384 || d >= 12 * kPart) && (E > 16 || d <= 4096);
+}
+
 }  // namespace
 }  // namespace ccf
 
@@ -869,6 +1062,13 @@ int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int 
                        static_cast<const float *>(wg), static_cast<const float *>(bg), d_model, tot_expert, top_k, group,
                        idx_out, static_cast<float *>(score_out), static_cast<float *>(logits_out));
     return check_launch("gate_f32_walk_kernel");
+  }
+  if (dtype == CCF_F32 && gate_f32_on_mfma(tokens, d_model, tot_expert)) {
+    auto launch = tot_expert <= 16 ? launch_gate_f32_mfma<16, 16>
+                                   : (tot_expert <= 32 ? launch_gate_f32_mfma<32, 32> : launch_gate_f32_mfma<32, 64>);
+    return launch(static_cast<const float *>(x), static_cast<const float *>(wg), static_cast<const float *>(bg), tokens,
+                  d_model, tot_expert, top_k, idx_out, static_cast<float *>(score_out), static_cast<float *>(logits_out),
+                  as_stream(stream));
   }
   if (dtype == CCF_F32) {
     auto launch = tokens > 4096 ? launch_gate_f32_experts<4>

@@ -71,6 +71,25 @@ def test_gate_fp32_tiles(T, d, E, k):
     assert torch.equal(idx2.cpu(), O.naive_gate(x, wg, None, k)[0])
 
 
+@pytest.mark.parametrize("scale", [1.0, 1e-20])
+@pytest.mark.parametrize("T,d,E,k", [(4097, 8, 33, 2), (4127, 136, 64, 8), (4128, 1160, 70, 1), (8193, 648, 9, 2), (8256, 768, 16, 3),
+                                     (8257, 1064, 17, 1), (16385, 1536, 32, 2)])
+def test_gate_fp32_products_as_mfmas(T, d, E, k, scale):
+    """Many tokens: the fp32 gate's products on the matrix cores, fewer parts of K than wavefronts and more, ragged in
+    every direction, zeros of both signs, and operands whose products are subnormal or vanish: the oracle's bits."""
+    from ccfuser_amd import ops
+    _say(f"fp32 gate on MFMAs T={T} d={d} E={E} k={k} scale={scale}")
+    g = torch.Generator().manual_seed(T + d + E)
+    x, wg = torch.randn(T, d, generator=g) * scale, torch.randn(E, d, generator=g) * scale
+    x[:, ::7], wg[::3, 1::5] = -0.0, 0.0
+    bg = torch.randn(E, generator=g) * scale * scale
+    idx_ref, score_ref, logits_ref = O.naive_gate(x, wg, bg, k)
+    idx, score, logits = ops.gate_topk_softmax(dev(x), dev(wg), dev(bg), k, return_logits=True)
+    assert torch.equal(logits.cpu().view(torch.int32), logits_ref.view(torch.int32)), "logits differ bitwise"
+    assert torch.equal(idx.cpu(), idx_ref), "expert choice differs"
+    assert torch.allclose(score.cpu(), score_ref, rtol=1e-5, atol=1e-7)
+
+
 @pytest.mark.parametrize("T,d,E,k", [(1, 4096, 1, 1), (512, 2056, 2, 2), (513, 2056, 2, 1), (341, 6152, 3, 3), (342, 6152, 3, 2), (300, 128, 33, 2), (513, 128, 33, 2),
                                      (1024, 64, 130, 2), (1025, 64, 130, 2), (40, 256, 200, 8), (100, 264, 130, 2),
                                      (5, 136, 1024, 2), (33, 8, 64, 1)])
