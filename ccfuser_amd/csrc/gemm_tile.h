@@ -380,6 +380,14 @@ struct Ring16Mainloop {
   // states; this is 32).
   static __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n s_nop 15" ::: "memory"); }
 
+  // Order of a full substep's blocks: along strips of two row blocks, up and down, so that consecutive MFMAs share an
+  // operand and each is used again two MFMAs later at the latest.
+  static constexpr int path_row(int i) { return 2 * (i / (2 * TN)) + ((i ^ (i >> 1)) & 1); }
+  static constexpr int path_col(int i) {
+    const int j = i % (2 * TN) / 2;
+    return (i / (2 * TN)) & 1 ? TN - 1 - j : j;
+  }
+
   // One substep: PER_SUB MFMAs on fragment buffer SUB; interleaved with them the
   // reads of the NEXT substep's fragments (LDS addresses ra, rb) into the other
   // buffer and the tile loads into the slot at byte offset ws.
@@ -405,19 +413,27 @@ struct Ring16Mainloop {
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    static_for<0, TM>([&](auto T) {
-      constexpr int tm = T.value;
-      // one (wavefront-uniform) branch per row block, not per MFMA
-      if (FULL || tm < live_m) {
-        static_for<0, TN>([&](auto J) {
-          constexpr int tn = J.value;
-          mfma16<tm * TN + tn>(b[SUB][tn], a[AS][tm]);
-          behind(std::integral_constant<int, tm * TN + tn>{});
-        });
-      } else {
-        static_for<0, TN>([&](auto J) { behind(std::integral_constant<int, tm * TN + J.value>{}); });
-      }
-    });
+    if constexpr (FULL && !ROLL_A) {
+      static_for<0, PER_SUB>([&](auto II) {
+        constexpr int tm = path_row(II.value), tn = path_col(II.value);
+        mfma16<tm * TN + tn>(b[SUB][tn], a[AS][tm]);
+        behind(II);
+      });
+    } else {
+      static_for<0, TM>([&](auto T) {
+        constexpr int tm = T.value;
+        // one (wavefront-uniform) branch per row block, not per MFMA
+        if (FULL || tm < live_m) {
+          static_for<0, TN>([&](auto J) {
+            constexpr int tn = J.value;
+            mfma16<tm * TN + tn>(b[SUB][tn], a[AS][tm]);
+            behind(std::integral_constant<int, tm * TN + tn>{});
+          });
+        } else {
+          static_for<0, TN>([&](auto J) { behind(std::integral_constant<int, tm * TN + J.value>{}); });
+        }
+      });
+    }
   }
 
   // K tile kt in ring phase ph; k2 / kb2: element offset from the A / B sources of the K
