@@ -19,7 +19,7 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "libccfuser_moe.so"
 PROBE_LIB = HERE / "libccfuser_probe.so"
-SOURCES = ["api.hip", "gate.hip", "route.hip", "rows.hip", "bwd.hip", "few.hip", "ffn.hip"]
+SOURCES = ["api.hip", "gate.hip", "route.hip", "rows.hip", "bwd.hip", "few.hip", "thin.hip", "ffn.hip"]
 PROBE_SOURCES = ["probe.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -447,7 +447,7 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
   // the tile table holds kFewMaxRounds tiles per workgroup of the largest shape
   const long long worst = (static_cast<long long>(max_rows) / 128 + E) * ((N + 255) / 256);
   if (worst >= static_cast<long long>(kFewMaxRounds - 1) * cus) return false;
-  if (mode >= 2) return true;
+  if (mode >= 2 || thin_rows_fits(mode, max_rows, E, N, K, epi, b_kn)) return true;
   // Where either is far ahead nothing is priced (0.3 to 0.8 us): three rounds of 256-row tiles waste too little for
   // smaller tiles to win, and a quarter of a round makes a single one of 128 x 128 tiles at most.
   const int n_tiles_n = (N + 255) / 256;
@@ -497,6 +497,7 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
 }
 
 int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {
+  if (thin_rows_fits(mode, p.max_rows, p.E, p.N, p.K, epi, b_kn)) return thin_rows_gemm(p, epi, stream, what);
   p.force = mode >= 16 ? mode & 15 : -1;
   void (*kernel)(FewArgs) = b_kn ? (epi == kFewPlain ? few_rows_kernel<kFewPlain, true> : few_rows_kernel<kFewGelu, true>)
                                  : (epi == kFewPlain ? few_rows_kernel<kFewPlain, false>

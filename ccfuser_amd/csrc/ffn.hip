@@ -1730,8 +1730,8 @@ extern "C" int ccf_set_option(const char *name, int value) {
     return CCF_OK;
   }
   if (!strcmp(name, "few_rows")) {
-    CCF_REQUIRE((value >= 0 && value <= 2) || (value >= 16 && value < 22), CCF_ERR_ARG,
-                "set_option: few_rows %d is neither 0..2 nor 16..21", value);
+    CCF_REQUIRE((value >= 0 && value <= 3) || (value >= 16 && value < 22), CCF_ERR_ARG,
+                "set_option: few_rows %d is neither 0..3 nor 16..21", value);
     g_few_rows = value;
     return CCF_OK;
   }

@@ -566,7 +566,11 @@ struct FewArgs {
   int max_rows, E, N, K;
   int force;                 // tile shape, or -1: chosen by the kernel; filled in by few_rows_gemm
 };
-// mode: GemmOptions::few_rows (0: never, 1: by the rule, 2: always, 16 + i: always and with tile shape i)
+// thin.hip: at most 32 rows in all (the two epilogues without a kept pre-activation, [E, N, K] weights)
+bool thin_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn);
+int thin_rows_gemm(const FewArgs &p, int epi, hipStream_t stream, const char *what);
+// mode: GemmOptions::few_rows (0: never, 1: by the rule, 2: always, 3: always, in the form of thin.hip where that can,
+// 16 + i: always and with tile shape i)
 bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn, int cus);
 int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what);
 

@@ -80,8 +80,11 @@ const char *ccf_last_error(void);
  *                     2: half of the workgroups in front of all their tiles, half behind)
  *   "few_rows"        1 (default): a forward or input-gradient GEMM whose 256-row tiles would leave most of the
  *                     chip idle (few rows per expert, small layers) runs as tiles of 64 or 128 rows in a kernel that
- *                     needs no plan; 0 = never, 2 = always, 16..21 = always, and with that tile shape.  The knobs
- *                     above apply to the 256-row tiles: with any of the first six away from its default, they are used
+ *                     needs no plan, at most 32 rows in all and a long contraction in one that cuts K over the
+ *                     wavefronts of a workgroup; 0 = never, 2 = always in tiles of 64 or 128 rows, 16..21 = always, and
+ *                     with that tile shape, 3 = cut over the wavefronts wherever that can be (at most 32 rows, [E, N, K]
+ *                     weights), else as 2.  The knobs above apply to the 256-row tiles: with any of the first six away
+ *                     from its default, they are used
  *   "fused_combine"   0/1 (default 0): ccf_moe_forward with top_k = 2 adds the gate-weighted expert outputs
  *                     into the output in the second GEMM's epilogue (packed fp16 atomic adds onto zeros)
  *                     instead of running the combine pass; measured slower, kept for comparison
@@ -302,6 +305,7 @@ size_t ccf_ffn_workspace_bytes(int max_rows, int num_expert, int d_model, int d_
  *   [4] skinny tiles per XCD, [5] K steps per workgroup when they are cut along K: > 0 as a launch of their
  *       own, < 0 inside the persistent launch, 0 = not cut
  *   [6] workgroups of the persistent launch (0 = one workgroup per tile), [7] worst-case tile count
+ * A GEMM of few rows (option "few_rows") has no plan: all zeros.
  */
 int ccf_ffn_plan_info(const void *workspace, int max_rows, int num_expert, int d_model, int d_ffn,
                       int which, int32_t *info, ccf_stream_t stream);

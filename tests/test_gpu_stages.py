@@ -568,6 +568,57 @@ def test_route_in_place(n):
         assert torch.equal(got[k][:m], v[:m]), k
 
 
+@pytest.mark.parametrize("counts,N,K,pad", [
+    ([1], 8, 64, 0),                                          # fewer K tiles than wavefronts, half a column tile
+    ([1, 0, 1], 264, 448, 0),                                 # seven wavefronts with a K tile; a ragged last column tile
+    ([0, 16, 0, 0], 40, 576, 0),                              # a full row block, nine K tiles
+    ([17, 0, 15], 24, 1088, 0),                               # two row blocks, one row in the second
+    ([0] * 70 + [3, 0, 1] + [0] * 60 + [2], 136, 1024, 9),    # experts over several passes of the search, spare rows
+    ([1] * 32, 16, 2112, 0),
+    ([0, 0], 16, 64, 4),                                      # no rows
+])
+def test_thin_rows_kernel(counts, N, K, pad):
+    """K cut over the wavefronts of a workgroup for a few rows in all, through row indices, both epilogues: the fp32
+    product within the error of the sums and one rounding to fp16, and a second call bit for bit; rows no index
+    points at stay as they are."""
+    from ccfuser_amd import ops
+    _say(f"thin rows counts={len(counts)} N={N} K={K}")
+    E, R = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(N + K)
+    x = dev(torch.randn(R + 9, K, generator=g).half())
+    w = dev((torch.randn(E, N, K, generator=g) * K ** -0.5).half())
+    b = dev(torch.randn(E, N, generator=g).half())
+    off = dev(torch.tensor([0] + counts).cumsum(0).int())
+    src = dev(torch.cat([torch.randperm(R + 9, generator=g)[:R], torch.zeros(pad, dtype=torch.int64)]).int())
+    dst = dev(torch.cat([torch.randperm(R + 3, generator=g)[:R], torch.zeros(pad, dtype=torch.int64)]).int())
+    scale = dev(torch.rand(R + pad, generator=g).half())
+
+    def outputs():
+        y = torch.full((R + 3 + pad, N), 7.0, dtype=torch.float16, device="cuda")
+        return (ops.ffn1(x, src, off, R + pad, w, b, gelu=True, out=y.clone(), dst_row=dst),
+                ops.ffn2(x, dst, off, R + pad, w, b, y.clone(), src_row=src, row_scale=scale))
+
+    ops.set_option("few_rows", 3)
+    try:
+        got, again = outputs(), outputs()
+    finally:
+        ops.set_option("few_rows", 1)
+    e_of = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).cuda()
+    xs, rows = x[src[:R].long()].double(), dst[:R].long()
+    pre = torch.empty(R, N, dtype=torch.float64, device="cuda")
+    for e in e_of.unique().tolist():
+        pre[e_of == e] = xs[e_of == e] @ w[e].double().t() + b[e].double()
+    refs = (torch.nn.functional.gelu(pre), pre * scale[:R, None].double())
+    for out, second, ref in zip(got, again, refs):
+        assert torch.equal(out, second)
+        # K additions in fp32 of terms whose magnitudes sum to K^0.5 or so, the GELU's 6e-5, half a step of fp16
+        tol = K * 2.0 ** -24 * K ** 0.5 + 6e-5
+        assert ((out[rows].double() - ref).abs() <= tol + 2.0 ** -11 * ref.abs()).all()
+        rest = torch.ones(out.shape[0], dtype=torch.bool, device="cuda")
+        rest[rows] = False
+        assert (out[rest] == 7.0).all()
+
+
 @pytest.mark.parametrize("shape", range(6))
 @pytest.mark.parametrize("counts,N,K", [
     ([0, 1, 63, 64, 65, 127, 128, 129, 0], 264, 64),          # edges of both tile heights, a ragged last column tile
