@@ -37,14 +37,30 @@ constexpr int kPadK = 256;            // shortest K range the persistent GEMM ta
 //   cnt = -1 for blocks past k_seg[E]
 __global__ void __launch_bounds__(1024)
 kseg_kernel(const int32_t *__restrict__ offsets, int E, int max_rows, int seg_rows, int n_blk,
-            int32_t *__restrict__ k_seg, int32_t *__restrict__ row_off,
+            int32_t *__restrict__ k_seg, int32_t *__restrict__ row_off,   // row_off: may be null
             int32_t *__restrict__ blk_row0, int32_t *__restrict__ blk_cnt, int32_t *__restrict__ row_lo,
-            half_t *__restrict__ zero_row, PlanReq rows_plan, int rows_plan_wgs, PlanReq w_plan, int w_plan_wgs) {
-  // workgroups behind the first build the tile plans of the call's two GEMMs
+            half_t *__restrict__ zero_row, SetupJobs jobs) {
+  // workgroups behind the first build the tile plans of the call's GEMMs, the last ones clear the unused slots' gradients
   if (blockIdx.x > 0) {
-    const int b = static_cast<int>(blockIdx.x) - 1;
-    if (b < rows_plan_wgs) build_plan(rows_plan, offsets, E, b, rows_plan_wgs);
-    else build_plan(w_plan, nullptr, E, b - rows_plan_wgs, w_plan_wgs, seg_rows);
+    int b = static_cast<int>(blockIdx.x) - 1;
+    const int n = jobs.plan_wgs;
+    if (b < jobs.n_rows * n) {
+      if (b < n) build_plan(jobs.rows_plan[0], offsets, E, b, n);
+      else build_plan(jobs.rows_plan[1], offsets, E, b - n, n);
+      return;
+    }
+    b -= jobs.n_rows * n;
+    if (jobs.w_experts > 0) {
+      if (b < n) {
+        build_plan(jobs.w_plan, nullptr, jobs.w_experts, b, n, seg_rows);
+        return;
+      }
+      b -= n;
+    }
+    const half8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int r = 0; r < 4; ++r)
+      for (size_t c = static_cast<size_t>(b) * 1024 + threadIdx.x; c < jobs.zero[r].chunks; c += static_cast<size_t>(jobs.zero_wgs) * 1024)
+        reinterpret_cast<half8 *>(jobs.zero[r].dst)[c] = z;
     return;
   }
   __shared__ int s_k[1025];
@@ -72,8 +88,10 @@ kseg_kernel(const int32_t *__restrict__ offsets, int E, int max_rows, int seg_ro
   }
   if (t <= E && t < 1024) k_seg[t] = s_k[t];
   if (t == 0) k_seg[E] = s_k[E];
-  if (t <= E && t < 1024) row_off[t] = t * seg_rows;
-  if (t == 0) row_off[E] = E * seg_rows;
+  if (row_off) {
+    if (t <= E && t < 1024) row_off[t] = t * seg_rows;
+    if (t == 0) row_off[E] = E * seg_rows;
+  }
   const int total_blk = s_k[E] / kTile;
   if (t < E) {
     const int b0 = s_k[t] / kTile, nb = padded / kTile;
@@ -125,13 +143,13 @@ transpose_weights_kernel(const half_t *__restrict__ in, half_t *__restrict__ out
 // kT false: nothing is transposed; the (gathered) rows go to out_t as a row-major [rows, C] matrix in sorted
 // row order (out_t NULL: nowhere), and the pass is a row gather and / or the partial sums.
 template <bool kGelu, bool kT>
-__global__ void __launch_bounds__(256)
-transpose_rows_kernel(half_t *in, const int32_t *__restrict__ rows,
-                      const int32_t *__restrict__ blk_row0, const int32_t *__restrict__ blk_cnt,
-                      int C, int ld_t, half_t *__restrict__ out_t, float *__restrict__ partial,
-                      const half_t *__restrict__ pre) {
+__device__ __forceinline__ void
+rows_block(half_t *in, const int32_t *__restrict__ rows,
+           const int32_t *__restrict__ blk_row0, const int32_t *__restrict__ blk_cnt,
+           int C, int ld_t, half_t *__restrict__ out_t, float *__restrict__ partial,
+           const half_t *__restrict__ pre, int c_tile) {
   __shared__ half_t tile[kTile][kTile + 8];
-  const int b = blockIdx.x, c0 = blockIdx.y * kTile;
+  const int b = blockIdx.x, c0 = c_tile * kTile;
   const int cnt = blk_cnt[b];
   if (cnt < 0) return;                              // past the last expert's range: never read
   const int row0 = blk_row0[b];
@@ -178,11 +196,42 @@ transpose_rows_kernel(half_t *in, const int32_t *__restrict__ rows,
   }
 }
 
+template <bool kGelu, bool kT>
+__global__ void __launch_bounds__(256)
+transpose_rows_kernel(half_t *in, const int32_t *__restrict__ rows,
+                      const int32_t *__restrict__ blk_row0, const int32_t *__restrict__ blk_cnt,
+                      int C, int ld_t, half_t *__restrict__ out_t, float *__restrict__ partial,
+                      const half_t *__restrict__ pre) {
+  rows_block<kGelu, kT>(in, rows, blk_row0, blk_cnt, C, ld_t, out_t, partial, pre, blockIdx.y);
+}
+
+// The gathers of two matrices of one width: the column tiles of the second behind those of the first, which also leaves
+// the partial sums of its columns.
+__global__ void __launch_bounds__(256)
+gather_pair_kernel(const half_t *__restrict__ first, const int32_t *__restrict__ first_rows, half_t *__restrict__ first_out,
+                   float *__restrict__ partial, const half_t *__restrict__ second, const int32_t *__restrict__ second_rows,
+                   half_t *__restrict__ second_out, const int32_t *__restrict__ blk_row0,
+                   const int32_t *__restrict__ blk_cnt, int C) {
+  const int tiles = C / kTile;
+  const bool lead = static_cast<int>(blockIdx.y) < tiles;
+  rows_block<false, false>(const_cast<half_t *>(lead ? first : second), lead ? first_rows : second_rows, blk_row0, blk_cnt, C, 0,
+                           lead ? first_out : second_out, lead ? partial : nullptr, nullptr,
+                           lead ? blockIdx.y : blockIdx.y - tiles);
+}
+
 // grad_bias[e][c] = sum of partial[b][c] over expert e's blocks, in block order.
 __global__ void __launch_bounds__(256)
 bias_reduce_kernel(const float *__restrict__ partial, const int32_t *__restrict__ k_seg, int C,
-                   half_t *__restrict__ grad_bias) {
-  const int e = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
+                   half_t *__restrict__ grad_bias, const float *__restrict__ partial2, int C2, half_t *__restrict__ grad_bias2) {
+  const int e = blockIdx.x;
+  int y = blockIdx.y;
+  if (y >= (C + 255) / 256) {                          // the second layer's columns
+    y -= (C + 255) / 256;
+    partial = partial2;
+    C = C2;
+    grad_bias = grad_bias2;
+  }
+  const int c = y * 256 + threadIdx.x;
   if (c >= C) return;
   const int b0 = k_seg[e] / kTile, b1 = k_seg[e + 1] / kTile;
   float s = 0.0f;
@@ -262,14 +311,17 @@ int padded_rows(int max_rows, int E) {
 
 int launch_kseg(const int32_t *offsets, int E, int max_rows, int seg_rows, int n_blk, int32_t *k_seg,
                 int32_t *row_off, int32_t *blk_row0, int32_t *blk_cnt, int32_t *row_lo, half_t *zero_row,
-                const PlanReq *rows_plan, const PlanReq *w_plan, hipStream_t stream) {
+                SetupJobs jobs, hipStream_t stream) {
   // a wavefront per expert at least, 4 to 8 workgroups: wavefronts beyond the experts share their entries
-  const int per_plan = (E + 15) / 16 > 8 ? 8 : ((E + 15) / 16 < 4 ? 4 : (E + 15) / 16);
-  const int na = rows_plan ? per_plan : 0, nb = w_plan ? per_plan : 0;
-  const PlanReq none{};
-  hipLaunchKernelGGL(kseg_kernel, dim3(1 + na + nb), dim3(1024), 0, stream, offsets, E, max_rows, seg_rows,
-                     n_blk, k_seg, row_off, blk_row0, blk_cnt, row_lo, zero_row, rows_plan ? *rows_plan : none, na,
-                     w_plan ? *w_plan : none, nb);
+  const int most = jobs.w_experts > E ? jobs.w_experts : E;
+  jobs.plan_wgs = (most + 15) / 16 > 8 ? 8 : ((most + 15) / 16 < 4 ? 4 : (most + 15) / 16);
+  size_t chunks = 0;
+  for (const ZeroReq &z : jobs.zero) chunks += z.chunks;
+  chunks = (chunks + 4 * 1024 - 1) / (4 * 1024);                  // 64 KB a workgroup, up to two per CU
+  jobs.zero_wgs = static_cast<int>(chunks < 512 ? chunks : 512);
+  const int wgs = 1 + (jobs.n_rows + (jobs.w_experts > 0 ? 1 : 0)) * jobs.plan_wgs + jobs.zero_wgs;
+  hipLaunchKernelGGL(kseg_kernel, dim3(wgs), dim3(1024), 0, stream, offsets, E, max_rows, seg_rows,
+                     n_blk, k_seg, row_off, blk_row0, blk_cnt, row_lo, zero_row, jobs);
   return check_launch("kseg_kernel");
 }
 
@@ -300,10 +352,18 @@ int launch_transpose_rows(const half_t *in, const int32_t *rows, const int32_t *
   return check_launch("transpose_rows_kernel");
 }
 
+int launch_gather_pair(const half_t *first, const int32_t *first_rows, half_t *first_out, float *partial,
+                       const half_t *second, const int32_t *second_rows, half_t *second_out, const int32_t *blk_row0,
+                       const int32_t *blk_cnt, int n_blk, int C, hipStream_t stream) {
+  hipLaunchKernelGGL(gather_pair_kernel, dim3(n_blk, 2 * (C / kTile)), dim3(256), 0, stream, first, first_rows, first_out,
+                     partial, second, second_rows, second_out, blk_row0, blk_cnt, C);
+  return check_launch("gather_pair_kernel");
+}
+
 int launch_bias_reduce(const float *partial, const int32_t *k_seg, int E, int C, half_t *grad_bias,
-                       hipStream_t stream) {
-  hipLaunchKernelGGL(bias_reduce_kernel, dim3(E, (C + 255) / 256), dim3(256), 0, stream, partial,
-                     k_seg, C, grad_bias);
+                       hipStream_t stream, const float *partial2, int C2, half_t *grad_bias2) {
+  hipLaunchKernelGGL(bias_reduce_kernel, dim3(E, (C + 255) / 256 + (C2 + 255) / 256), dim3(256), 0, stream, partial,
+                     k_seg, C, grad_bias, partial2, C2, grad_bias2);
   return check_launch("bias_reduce_kernel");
 }
 

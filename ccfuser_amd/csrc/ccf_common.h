@@ -46,8 +46,15 @@ int launch_transpose_weights(const half_t *in, half_t *out, int E, int R, int C,
 int launch_transpose_rows(const half_t *in, const int32_t *rows, const int32_t *blk_row0,
                           const int32_t *blk_cnt, int n_blk, int C, int ld_t, half_t *out_t,
                           float *partial, hipStream_t stream, const half_t *gelu_pre_inplace, bool transposed);
+int launch_gather_pair(const half_t *first, const int32_t *first_rows, half_t *first_out, float *partial,
+                       const half_t *second, const int32_t *second_rows, half_t *second_out, const int32_t *blk_row0,
+                       const int32_t *blk_cnt, int n_blk, int C, hipStream_t stream);
 int launch_bias_reduce(const float *partial, const int32_t *k_seg, int E, int C, half_t *grad_bias,
-                       hipStream_t stream);
+                       hipStream_t stream, const float *partial2 = nullptr, int C2 = 0, half_t *grad_bias2 = nullptr);
+
+// rows.hip: score null: every weight is one
+int launch_combine(const half_t *y_flat, const half_t *score, const int32_t *inv_pos, half_t *out, int tokens, int top_k,
+                   int hidden, hipStream_t stream);
 
 // gate.hip
 int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int d_model, int tot_expert, int top_k,

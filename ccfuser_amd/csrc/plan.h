@@ -519,12 +519,23 @@ int ffn2_forward_combine(const void *h, const int32_t *token_row, const int32_t 
                          int max_rows, int num_expert, int d_model, int d_ffn, const void *w2, const void *b2,
                          const void *score, void *out, void *workspace, size_t workspace_bytes, hipStream_t stream,
                          const GemmOptions *planned);
-// bwd.hip: the padded K ranges and row blocks of a backward call; the same launch builds the tile plan of its
-// input-gradient GEMM (`rows_plan`, from the offsets) and of its weight-gradient GEMM (`w_plan`: every expert
-// has seg_rows output rows) when given.
+// A range that a launch clears beside its own work: 16-byte chunks at a 16-byte aligned address.
+struct ZeroReq {
+  void *dst;
+  size_t chunks;
+};
+// bwd.hip: the padded K ranges and row blocks of a backward call.  The same launch builds up to two tile plans of
+// input-gradient GEMMs (from the offsets), one of a weight-gradient GEMM (w_experts > 0: that many experts of seg_rows
+// output rows) and clears four ranges.
+struct SetupJobs {
+  PlanReq rows_plan[2], w_plan;
+  int n_rows, w_experts;
+  ZeroReq zero[4];
+  int plan_wgs, zero_wgs;    // filled in by launch_kseg
+};
 int launch_kseg(const int32_t *offsets, int E, int max_rows, int seg_rows, int n_blk, int32_t *k_seg,
                 int32_t *row_off, int32_t *blk_row0, int32_t *blk_cnt, int32_t *row_lo, half_t *zero_row,
-                const PlanReq *rows_plan, const PlanReq *w_plan, hipStream_t stream);
+                SetupJobs jobs, hipStream_t stream);
 
 // route.hip: ccf_route(), whose last launch also builds n_plans (0..2) tile plans from the offsets.  gate_row_len > 0:
 // the head of the workspace already holds the gate kernel's counts, one row per gate_row_len flat indices.

@@ -48,7 +48,7 @@ combine_kernel(const half_t *__restrict__ y_flat, const half_t *__restrict__ sco
       if (s < kk) {
         const size_t flat = t * kk + s;
         if (!inv_pos || inv_pos[flat] >= 0) {
-          const float g = static_cast<float>(score[flat]);
+          const float g = score ? static_cast<float>(score[flat]) : 1.0f;
           const half8 v = reinterpret_cast<const half8 *>(y_flat)[flat * chunks_per_row + col];
 #pragma unroll
           for (int j = 0; j < 8; ++j) acc[j] += g * static_cast<float>(v[j]);
@@ -87,6 +87,20 @@ int row_move(const void *in, void *out, const int32_t *pos, int pos_len, int hid
 }
 
 }  // namespace
+
+int launch_combine(const half_t *y, const half_t *g, const int32_t *inv_pos, half_t *o, int tokens, int top_k, int hidden,
+                   hipStream_t st) {
+  if (tokens == 0) return CCF_OK;
+  const int cpr = hidden / 8;
+  const int grid = grid_for(static_cast<size_t>(tokens) * cpr);
+  if (top_k == 1)
+    hipLaunchKernelGGL(combine_kernel<1>, dim3(grid), dim3(kThreads), 0, st, y, g, inv_pos, o, tokens, top_k, cpr);
+  else if (top_k == 2)
+    hipLaunchKernelGGL(combine_kernel<2>, dim3(grid), dim3(kThreads), 0, st, y, g, inv_pos, o, tokens, top_k, cpr);
+  else
+    hipLaunchKernelGGL(combine_kernel<0>, dim3(grid), dim3(kThreads), 0, st, y, g, inv_pos, o, tokens, top_k, cpr);
+  return check_launch("combine_kernel");
+}
 }  // namespace ccf
 
 extern "C" int ccf_local_scatter(const void *in, void *out, const int32_t *pos, int pos_len,
@@ -107,18 +121,6 @@ extern "C" int ccf_combine(const void *y_flat, const void *score, const int32_t 
   CCF_REQUIRE(top_k >= 1 && top_k <= 8, CCF_ERR_SHAPE, "combine: top_k=%d outside 1..8", top_k);
   CCF_REQUIRE(hidden % 8 == 0, CCF_ERR_SHAPE, "combine: hidden=%d is not a multiple of 8", hidden);
   CCF_REQUIRE(aligned16(y_flat) && aligned16(out), CCF_ERR_ARG, "combine: rows must be 16-byte aligned");
-  if (tokens == 0) return CCF_OK;
-  const int cpr = hidden / 8;
-  const int grid = grid_for(static_cast<size_t>(tokens) * cpr);
-  const half_t *y = static_cast<const half_t *>(y_flat);
-  const half_t *g = static_cast<const half_t *>(score);
-  half_t *o = static_cast<half_t *>(out);
-  hipStream_t st = as_stream(stream);
-  if (top_k == 1)
-    hipLaunchKernelGGL(combine_kernel<1>, dim3(grid), dim3(kThreads), 0, st, y, g, inv_pos, o, tokens, top_k, cpr);
-  else if (top_k == 2)
-    hipLaunchKernelGGL(combine_kernel<2>, dim3(grid), dim3(kThreads), 0, st, y, g, inv_pos, o, tokens, top_k, cpr);
-  else
-    hipLaunchKernelGGL(combine_kernel<0>, dim3(grid), dim3(kThreads), 0, st, y, g, inv_pos, o, tokens, top_k, cpr);
-  return check_launch("combine_kernel");
+  return launch_combine(static_cast<const half_t *>(y_flat), static_cast<const half_t *>(score), inv_pos,
+                        static_cast<half_t *>(out), tokens, top_k, hidden, as_stream(stream));
 }

@@ -167,6 +167,10 @@ class MixMOEFusedFFN(Function):
         input_buf, w1, w2, act, h_pre, src_row, dst_row, offsets, inv_pos = ctx.saved_tensors
         max_rows, n_flat, may_drop = ctx.sizes
         E = offsets.numel() - 1
+        if inv_pos is not None and n_flat == max_rows:
+            grad_in, grad_w1, grad_b1, grad_w2, grad_b2 = ops.ffn_backward_pair(
+                grad_y.contiguous(), input_buf, act, h_pre, src_row, dst_row, inv_pos, offsets, w1.detach(), w2.detach())
+            return grad_in, None, None, grad_w1, grad_b1, grad_w2, grad_b2
         grad_w2, grad_b2 = _param_grads(w2, E)
         grad_act, _, _ = ops.ffn2_backward(grad_y.contiguous(), act, dst_row, offsets, max_rows,
                                            w2.detach()[:E], grad_w2[:E], grad_b2[:E], may_drop=may_drop)

@@ -122,6 +122,41 @@ def gate_backward_products(score: torch.Tensor, grad_score: torch.Tensor, idx: t
     return g_x, g_w, g_b
 
 
+def ffn_backward_pair(grad_y_flat: torch.Tensor, x: torch.Tensor, act: torch.Tensor, h_pre: torch.Tensor,
+                      src_row: torch.Tensor, dst_row: torch.Tensor, inv_pos: torch.Tensor, offsets: torch.Tensor,
+                      w1: torch.Tensor, w2: torch.Tensor):
+    """(grad_x [T, d], grad_w1, grad_b1, grad_w2, grad_b2) of ``ffn1_keep`` and ``ffn2`` over all slots of the T tokens:
+    ``ffn2_backward``, ``ffn1_backward`` through the GELU and the sum of a token's slots in one call.  The weights may
+    hold more experts than ``offsets``; the gradients of those are zero."""
+    _check(grad_y_flat, "grad_y_flat", dtype=torch.float16, ndim=2)
+    _check(x, "x", dtype=torch.float16, ndim=2)
+    _check(act, "act", dtype=torch.float16, ndim=2)
+    _check(h_pre, "h_pre", dtype=torch.float16, ndim=2)
+    _check(w1, "ffn1 weight", dtype=torch.float16, ndim=3)
+    _check(w2, "ffn2 weight", dtype=torch.float16, ndim=3)
+    for t, nm in ((src_row, "src_row"), (dst_row, "dst_row"), (inv_pos, "inv_pos"), (offsets, "offsets")):
+        _check(t, nm, dtype=torch.int32, ndim=1)
+    slots, f, d = w1.shape
+    T, n = x.shape[0], inv_pos.numel()
+    E = offsets.numel() - 1
+    top_k = n // T if T else 1
+    if tuple(w2.shape) != (slots, d, f) or E < 1 or E > slots or x.shape[1] != d or T * top_k != n or \
+            tuple(grad_y_flat.shape) != (n, d) or tuple(act.shape) != (n, f) or tuple(h_pre.shape) != (n, f) or \
+            src_row.numel() < n or dst_row.numel() < n:
+        raise ValueError("ffn_backward_pair: sizes do not match")
+    dev = x.device
+    grad_x = torch.empty(T, d, dtype=torch.float16, device=dev)
+    grad_w1, grad_w2 = torch.empty_like(w1), torch.empty_like(w2)
+    grad_b1 = torch.empty(slots, f, dtype=torch.float16, device=dev)
+    grad_b2 = torch.empty(slots, d, dtype=torch.float16, device=dev)
+    with _on(x):
+        ws = _workspace(_lib.lib().ccf_ffn_backward_pair_workspace_bytes(n, E, d, f), x)
+        _lib.call("ccf_ffn_backward_pair", _ptr(grad_y_flat), _ptr(x), _ptr(act), _ptr(h_pre), _ptr(src_row), _ptr(dst_row),
+                  _ptr(inv_pos), _ptr(offsets), T, top_k, E, slots, d, f, _ptr(w1), _ptr(w2), _ptr(grad_x), _ptr(grad_w1),
+                  _ptr(grad_b1), _ptr(grad_w2), _ptr(grad_b2), _ptr(ws), ws.numel(), _stream(x))
+    return grad_x, grad_w1, grad_b1, grad_w2, grad_b2
+
+
 def gate_products_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``gate_backward_products`` takes these operands."""
     return (x.dtype == torch.float16 and weight.dtype == torch.float16 and x.is_contiguous() and weight.is_contiguous()

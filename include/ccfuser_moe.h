@@ -536,6 +536,26 @@ int ccf_ffn1_backward_gelu(void *grad_act, const void *h_pre, const void *x, con
                            void *grad_x_flat, void *grad_w1, void *grad_b1, void *workspace,
                            size_t workspace_bytes, ccf_stream_t stream);
 
+/*
+ * Backward of both expert layers of a training step in one call: ccf_ffn2_backward, ccf_ffn1_backward_gelu and the sum of
+ * a token's slots (mix_moe/csrc/mix_moe.h:300-388, 439-505, with the GeluBackward between them, and the index_add_ at
+ * 359-365), which share their launches where the widths are multiples of 256.  max_rows is tokens * top_k.
+ *   grad_y_flat fp16 [tokens*top_k, d_model]  flat token order
+ *   x           fp16 [tokens, d_model], act and h_pre fp16 [tokens*top_k, d_ffn] from ccf_ffn1_forward_keep
+ *   src_row, dst_row, inv_pos, offsets  from ccf_route
+ *   grad_x      fp16 [tokens, d_model]  out
+ *   grad_w1, grad_b1, grad_w2, grad_b2  fp16, out, with expert_slots >= num_expert leading entries: those from num_expert
+ *               on become zero
+ */
+size_t ccf_ffn_backward_pair_workspace_bytes(int max_rows, int num_expert, int d_model, int d_ffn);
+/* See above (mix_moe/csrc/mix_moe.h:300-388, 439-505). */
+int ccf_ffn_backward_pair(const void *grad_y_flat, const void *x, const void *act, const void *h_pre,
+                          const int32_t *src_row, const int32_t *dst_row, const int32_t *inv_pos,
+                          const int32_t *offsets, int tokens, int top_k, int num_expert, int expert_slots,
+                          int d_model, int d_ffn, const void *w1, const void *w2, void *grad_x, void *grad_w1,
+                          void *grad_b1, void *grad_w2, void *grad_b2, void *workspace, size_t workspace_bytes,
+                          ccf_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

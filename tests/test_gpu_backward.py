@@ -441,3 +441,41 @@ def test_zero_tails(E, first, shape):
     ops.zero_tails(a, b, first)
     for t in (a, b):
         assert (t[:first] == 1).all() and (t[first:] == 0).all()
+
+
+@pytest.mark.usefixtures("gemm_form")
+@pytest.mark.parametrize("T,k,d,f,E,slots,capacity", [
+    (700, 2, 256, 512, 4, 7, -1),           # both weight gradients in one launch, fewer tiles than compute units
+    (700, 2, 512, 256, 4, 4, 90),           # wider input, dropped slots, no unused slot
+    (1999, 2, 768, 3072, 8, 11, -1),        # more than one round of tiles
+    (33, 1, 256, 256, 16, 19, -1),          # experts without rows, square widths
+    (1, 2, 256, 256, 3, 6, -1),
+    (300, 3, 256, 768, 1, 2, -1),           # one expert, three slots a token
+    (300, 2, 320, 704, 4, 7, 100),          # widths that are no multiples of 256: the layers one after the other
+    (70, 2, 256, 256, 520, 521, -1),        # more experts than one plan holds twice
+])
+def test_backward_of_both_layers_in_one_call(T, k, d, f, E, slots, capacity):
+    """Gradients of both expert layers from one call: the bits of the two layers' own calls and the sum over a token's
+    slots, unused slots zero."""
+    from ccfuser_amd import ops
+    print(f"backward pair T={T} k={k} d={d} f={f} E={E} slots={slots} capacity={capacity}", flush=True)
+    g = torch.Generator().manual_seed(T + d)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.1).half().cuda()
+    k_eff = min(k, E)
+    idx = torch.rand(T, E, generator=g).topk(k_eff, dim=-1).indices
+    if k_eff < k:
+        idx = idx.repeat(1, k)[:, :k]
+    r = ops.route(idx.reshape(-1).contiguous().cuda(), E, k, capacity)
+    n = T * k
+    x, gy = rnd(T, d), rnd(n, d)
+    w1, b1, w2 = rnd(slots, f, d), rnd(slots, f), rnd(slots, d, f)
+    act, pre = ops.ffn1_keep(x, r["src_row"], r["offsets"], n, w1[:E], b1[:E])
+    torch.full((slots, f, d), float("nan"), dtype=torch.float16, device="cuda")          # freed at once
+    got = ops.ffn_backward_pair(gy, x, act, pre, r["src_row"], r["dst_row"], r["inv_pos"], r["offsets"], w1, w2)
+    ga, gw2, gb2 = ops.ffn2_backward(gy, act, r["dst_row"], r["offsets"], n, w2[:E])
+    gf, gw1, gb1 = ops.ffn1_backward(ga, x, r["src_row"], r["dst_row"], r["offsets"], n, w1[:E], n, h_pre=pre)
+    gx = ops.combine(gf, torch.ones(n, dtype=torch.float16, device="cuda"), k, r["inv_pos"])
+    for name, a, b in zip(("x", "w1", "b1", "w2", "b2"), got, (gx, gw1, gb1, gw2, gb2)):
+        tail = a[b.shape[0]:]
+        assert torch.equal(a[:b.shape[0]], b), name
+        assert torch.equal(tail, torch.zeros_like(tail)), name
