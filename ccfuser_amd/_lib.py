@@ -57,6 +57,7 @@ SIGNATURES = {
     "ccf_segments_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "ccf_moe_ffn_segments": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "ccf_blocks_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "ccf_gate_route": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "ccf_ffn_backward_pair_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "ccf_ffn_backward_pair": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "ccf_moe_ffn_blocks": (_i, [_p, _i, _p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _i, _p, _i, _p, _p, _i, _p, _p, _p, _sz, _p]),

@@ -243,6 +243,26 @@ extern "C" int ccf_moe_forward(const void *x, const void *wg, const void *bg, co
   return CCF_OK;
 }
 
+// The gate and the routing of its choice: the gate's counts spare the routing a launch of its own to count the indices.
+extern "C" int ccf_gate_route(const void *x, const void *wg, const void *bg, int tokens, int d_model, int num_expert,
+                              int top_k, int dtype, int capacity, int64_t *idx, void *score, int32_t *counts,
+                              int32_t *offsets, int64_t *pos, int32_t *src_row, int32_t *dst_row, int32_t *inv_pos,
+                              int64_t *idx_kept, void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
+  using namespace ccf;
+  CCF_REQUIRE(tokens >= 0 && top_k >= 1 && static_cast<long long>(tokens) * top_k < (1ll << 31), CCF_ERR_SHAPE,
+              "gate_route: tokens*top_k too large");
+  const int n = tokens * top_k;
+  CCF_REQUIRE(workspace && workspace_bytes >= ccf_route_workspace_bytes(n, num_expert), CCF_ERR_WORKSPACE,
+              "gate_route: workspace of %zu bytes needed, %zu given", ccf_route_workspace_bytes(n, num_expert), workspace_bytes);
+  int gate_tokens = 0;
+  const bool pow2_k = (top_k & (top_k - 1)) == 0;     // a workgroup's flat indices tile the routing's chunks
+  if (int rc = gate_forward(x, wg, bg, tokens, d_model, num_expert, top_k, dtype, idx, score, nullptr, stream,
+                            pow2_k ? static_cast<int32_t *>(workspace) : nullptr, route_rows_max_ints(), &gate_tokens))
+    return rc;
+  return route_with_plans(idx, n, num_expert, top_k, capacity, counts, offsets, pos, src_row, dst_row, inv_pos, idx_kept,
+                          workspace, workspace_bytes, as_stream(stream), nullptr, 0, gate_tokens * top_k);
+}
+
 extern "C" size_t ccf_segments_workspace_bytes(int total_rows, int n_seg, int num_expert,
                                                int d_model, int d_ffn) {
   if (total_rows < 0 || n_seg < 0 || num_expert <= 0 || d_model <= 0 || d_ffn <= 0) return 0;

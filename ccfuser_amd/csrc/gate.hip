@@ -104,6 +104,22 @@ struct Best {
   }
 };
 
+// Leaves how many of the workgroup's token slots chose each expert, for the routing stage: the selection threads hold the
+// ids, so the routing needs no pass of its own over idx to count them.  `row`: E ints of LDS that nothing else uses from
+// here on; `mine`: this thread holds a token's list.  All threads of the workgroup call it, behind a barrier.  A list
+// that NaN logits left short has entries that are no expert.
+template <int KS>
+__device__ inline void leave_counts(const Best<KS> &best, bool mine, int k, int E, int *row, int32_t *__restrict__ wg_cnt) {
+  for (int e = threadIdx.x; e < E; e += blockDim.x) row[e] = 0;
+  __syncthreads();
+  if (mine) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      if (s < k && best.id[s] < E) atomicAdd(&row[best.id[s]], 1);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += blockDim.x) wg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = row[e];
+}
 
 // fp16 gate.  An MFMA has 64 / N blocks; with S = 1 << LS slots, block b of a wavefront is
 // token block b / S on slot b % S, so a wavefront covers TW = (64 / N / S) * N tokens and
@@ -336,21 +352,8 @@ gate_mfma_kernel(const half_t *__restrict__ x, const half_t *__restrict__ wg, co
   }
   if (threadIdx.x < TW && t0 + threadIdx.x < tokens)
     best.template write<half_t>(t0 + threadIdx.x, k, idx_out, score_out);
-  if (wg_cnt) {
-    // How many of this workgroup's token slots chose each expert, for the routing stage: the
-    // selection threads hold the ids, so the routing needs no pass of its own over idx to count
-    // them.  The wavefronts' regions are free since the last barrier.
-    int *row = reinterpret_cast<int *>(s_mem);
-    for (int e = threadIdx.x; e < E; e += blockDim.x) row[e] = 0;
-    __syncthreads();
-    if (threadIdx.x < TW && t0 + threadIdx.x < tokens) {
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-        if (s < k) atomicAdd(&row[best.id[s]], 1);
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < E; e += blockDim.x) wg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = row[e];
-  }
+  // the wavefronts' regions are free since the last barrier
+  if (wg_cnt) leave_counts<KS>(best, threadIdx.x < TW && t0 + threadIdx.x < tokens, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
 }
 
 // fp16 gate for many tokens: every wavefront works alone.  It takes TW tokens through all of
@@ -584,18 +587,8 @@ gate_stream_kernel(const half_t *__restrict__ x, const half_t *__restrict__ wg, 
     if (lane < TW && t0 + lane < tokens) best.template write<half_t>(t0 + lane, k, idx_out, score_out);
   }
   if (wg_cnt) {
-    // expert counts of the workgroup's kStreamWaves * TW tokens, as in gate_mfma_kernel
     __syncthreads();
-    int *row = reinterpret_cast<int *>(s_mem);
-    for (int e = threadIdx.x; e < E; e += blockDim.x) row[e] = 0;
-    __syncthreads();
-    if (lane < TW && t0 + lane < tokens) {
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-        if (s < k) atomicAdd(&row[best.id[s]], 1);
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < E; e += blockDim.x) wg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = row[e];
+    leave_counts<KS>(best, lane < TW && t0 + lane < tokens, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
   }
 }
 
@@ -636,7 +629,7 @@ template <int TT, int EE, int KS>
 __global__ void __launch_bounds__(kMaxWaves * 64)
 gate_f32_kernel(const float *__restrict__ x, const float *__restrict__ wg, const float *__restrict__ bg,
                 int tokens, int d, int E, int k, int64_t *__restrict__ idx_out,
-                float *__restrict__ score_out, float *__restrict__ logits_out) {
+                float *__restrict__ score_out, float *__restrict__ logits_out, int32_t *__restrict__ wg_cnt) {
 #pragma clang fp contract(off)
   using C = GateF32Tile<TT, EE>;
   extern __shared__ float s_mem[];
@@ -752,11 +745,13 @@ gate_f32_kernel(const float *__restrict__ x, const float *__restrict__ wg, const
     // the next tile's logits are written behind the barrier that follows its first round's part sums
   }
   if (threadIdx.x < C::WT && t0 + threadIdx.x < tokens) best.template write<float>(t0 + threadIdx.x, k, idx_out, score_out);
+  static_assert(C::REGION >= (EE >= 8 ? 1024 : 8 * EE), "a count per expert");
+  if (wg_cnt) leave_counts<KS>(best, threadIdx.x < C::WT && t0 + threadIdx.x < tokens, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
 }
 
 template <int TT, int EE>
 int launch_gate_f32(const float *x, const float *wg, const float *bg, int tokens, int d, int E, int k, int64_t *idx_out,
-                    float *score_out, float *logits_out, hipStream_t stream) {
+                    float *score_out, float *logits_out, hipStream_t stream, int32_t *wg_cnt, long long max_cnt, int *tokens_per_wg) {
   using C = GateF32Tile<TT, EE>;
   const int nparts = (d + kPart - 1) / kPart;
   const int waves = nparts < kMaxWaves ? nparts : kMaxWaves;
@@ -768,19 +763,23 @@ int launch_gate_f32(const float *x, const float *wg, const float *bg, int tokens
                                        static_cast<int>(lds));
     if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate: LDS attribute: %s", hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(kern, dim3((tokens + C::WT - 1) / C::WT), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
-                     idx_out, score_out, logits_out);
+  const int wgs = (tokens + C::WT - 1) / C::WT;
+  if (static_cast<long long>(wgs) * E > max_cnt) wg_cnt = nullptr;
+  if (wg_cnt && tokens_per_wg) *tokens_per_wg = C::WT;
+  hipLaunchKernelGGL(kern, dim3(wgs), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
+                     idx_out, score_out, logits_out, wg_cnt);
   return check_launch("gate_f32_kernel");
 }
 
 template <int TT>
 int launch_gate_f32_experts(const float *x, const float *wg, const float *bg, int tokens, int d, int E, int k,
-                            int64_t *idx_out, float *score_out, float *logits_out, hipStream_t stream) {
+                            int64_t *idx_out, float *score_out, float *logits_out, hipStream_t stream, int32_t *wg_cnt,
+                            long long max_cnt, int *tokens_per_wg) {
   auto launch = E <= 8 ? launch_gate_f32<TT, 1> : (E <= 16 ? launch_gate_f32<TT, 2> : launch_gate_f32<TT, 4>);
   if constexpr (TT < 4) {                          // more tokens of more than 32 experts: gate_f32_on_mfma()
     if (E > 32) launch = launch_gate_f32<TT, 8>;
   }
-  return launch(x, wg, bg, tokens, d, E, k, idx_out, score_out, logits_out, stream);
+  return launch(x, wg, bg, tokens, d, E, k, idx_out, score_out, logits_out, stream, wg_cnt, max_cnt, tokens_per_wg);
 }
 
 // The same order with the products on the matrix cores: fma(x, w, 0) of a K = 1 MFMA is the rounded product, subnormal
@@ -811,7 +810,7 @@ template <int N, int WE, int KS>
 __global__ void __launch_bounds__(kMaxWaves * 64)
 gate_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__ wg, const float *__restrict__ bg,
                      int tokens, int d, int E, int k, int64_t *__restrict__ idx_out,
-                     float *__restrict__ score_out, float *__restrict__ logits_out) {
+                     float *__restrict__ score_out, float *__restrict__ logits_out, int32_t *__restrict__ wg_cnt) {
 #pragma clang fp contract(off)
   using C = GateF32Mfma<N, WE>;
   using M = Mfma<N>;
@@ -939,12 +938,15 @@ gate_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__ wg, 
     for (int s = 0; s < KS; ++s)
       if (s < k && oid[s] != INT_MAX) best.offer(ov[s], oid[s], k);
   }
-  if (sel_t < C::WT && sel_e == 0 && t0 + sel_t < tokens) best.template write<float>(t0 + sel_t, k, idx_out, score_out);
+  const bool mine = sel_t < C::WT && sel_e == 0 && t0 + sel_t < tokens;
+  if (mine) best.template write<float>(t0 + sel_t, k, idx_out, score_out);
+  static_assert(C::REGION >= (WE >= 64 ? 1024 : WE), "a count per expert");
+  if (wg_cnt) leave_counts<KS>(best, mine, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
 }
 
 template <int N, int WE>
 int launch_gate_f32_mfma(const float *x, const float *wg, const float *bg, int tokens, int d, int E, int k, int64_t *idx_out,
-                         float *score_out, float *logits_out, hipStream_t stream) {
+                         float *score_out, float *logits_out, hipStream_t stream, int32_t *wg_cnt, long long max_cnt, int *tokens_per_wg) {
   using C = GateF32Mfma<N, WE>;
   const int nparts = (d + kPart - 1) / kPart;
   const int waves = nparts < kMaxWaves ? nparts : kMaxWaves;
@@ -956,8 +958,11 @@ int launch_gate_f32_mfma(const float *x, const float *wg, const float *bg, int t
                                        static_cast<int>(lds));
     if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate: LDS attribute: %s", hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(kern, dim3((tokens + C::WT - 1) / C::WT), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
-                     idx_out, score_out, logits_out);
+  const int wgs = (tokens + C::WT - 1) / C::WT;
+  if (static_cast<long long>(wgs) * E > max_cnt) wg_cnt = nullptr;
+  if (wg_cnt && tokens_per_wg) *tokens_per_wg = C::WT;
+  hipLaunchKernelGGL(kern, dim3(wgs), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
+                     idx_out, score_out, logits_out, wg_cnt);
   return check_launch("gate_f32_mfma_kernel");
 }
 
@@ -1036,7 +1041,7 @@ bool gate_f32_on_mfma(int tokens, int d, int E) {
 }  // namespace ccf
 
 namespace ccf {
-// The gate; with wg_cnt (room for max_cnt ints) the fp16 kernel also leaves, per workgroup, how many of
+// The gate; with wg_cnt (room for max_cnt ints) the tiled kernels also leave, per workgroup, how many of
 // its token slots chose each expert ([workgroups][tot_expert], a workgroup covering *tokens_per_wg
 // consecutive tokens), when that table fits; *tokens_per_wg = 0 says it was not written.
 int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int d_model, int tot_expert, int top_k,
@@ -1068,14 +1073,14 @@ int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int 
                                    : (tot_expert <= 32 ? launch_gate_f32_mfma<32, 32> : launch_gate_f32_mfma<32, 64>);
     return launch(static_cast<const float *>(x), static_cast<const float *>(wg), static_cast<const float *>(bg), tokens,
                   d_model, tot_expert, top_k, idx_out, static_cast<float *>(score_out), static_cast<float *>(logits_out),
-                  as_stream(stream));
+                  as_stream(stream), wg_cnt, max_cnt, tokens_per_wg);
   }
   if (dtype == CCF_F32) {
     auto launch = tokens > 4096 ? launch_gate_f32_experts<4>
                                 : (tokens > 2048 ? launch_gate_f32_experts<2> : launch_gate_f32_experts<1>);
     return launch(static_cast<const float *>(x), static_cast<const float *>(wg), static_cast<const float *>(bg), tokens,
                   d_model, tot_expert, top_k, idx_out, static_cast<float *>(score_out), static_cast<float *>(logits_out),
-                  as_stream(stream));
+                  as_stream(stream), wg_cnt, max_cnt, tokens_per_wg);
   }
   // Tile and slots.  With S slots a wavefront covers 64 / S tokens, so S grows while there
   // are fewer than four workgroups per CU and K has parts for the slots.

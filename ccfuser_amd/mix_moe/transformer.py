@@ -4,6 +4,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from .gates import NaiveGate
 from .layers import MixMOE
 from .linear import FMoELinear, MixMOEFusedFFN, MixMOEInstance, MixMOELinear1, MixMOELinear2
 
@@ -152,9 +153,11 @@ class AsyncExpertAssignment:
         ``pos`` has tokens*top_k entries; the first ``offsets[-1]`` are valid."""
         if world_size != 1:
             raise NotImplementedError("single-GPU build: world_size must be 1")
-        gate_top_k_idx, gate_score = gate(attn_inp)
-        top_k = gate_top_k_idx.shape[-1]
-        r = ops.route(gate_top_k_idx.reshape(-1), num_expert, top_k, self.capacity)
+        if isinstance(gate, NaiveGate) and num_expert == gate.tot_expert and gate.calls_forward_only():
+            _, gate_score, r = gate.forward_with_routing(attn_inp, self.capacity)
+        else:
+            gate_top_k_idx, gate_score = gate(attn_inp)
+            r = ops.route(gate_top_k_idx.reshape(-1), num_expert, gate_top_k_idx.shape[-1], self.capacity)
         infos = BlockInfos(offsets=r["offsets"], counts=r["counts"], src_row=r["src_row"],
                            dst_row=r["dst_row"], inv_pos=r["inv_pos"], idx_kept=r["idx_kept"],
                            max_rows=r["pos"].numel(), n_flat=r["pos"].numel(),

@@ -194,6 +194,18 @@ def assign_pos(cum_count: torch.Tensor, gate: torch.Tensor, pos: torch.Tensor) -
             pos.copy_(full[: pos.numel()])
 
 
+def _routing_buffers(n: int, num_expert: int, dev) -> Dict[str, torch.Tensor]:
+    return {
+        "counts": torch.empty(num_expert, dtype=torch.int32, device=dev),
+        "offsets": torch.empty(num_expert + 1, dtype=torch.int32, device=dev),
+        "pos": torch.empty(n, dtype=torch.int64, device=dev),
+        "src_row": torch.empty(n, dtype=torch.int32, device=dev),
+        "dst_row": torch.empty(n, dtype=torch.int32, device=dev),
+        "inv_pos": torch.empty(n, dtype=torch.int32, device=dev),
+        "idx_kept": torch.empty(n, dtype=torch.int64, device=dev),
+    }
+
+
 def route(gate_idx: torch.Tensor, num_expert: int, top_k: int, capacity: int = -1) -> Dict[str, torch.Tensor]:
     """Counts, offsets, deterministic pos and the row maps, all on the device.
 
@@ -203,15 +215,7 @@ def route(gate_idx: torch.Tensor, num_expert: int, top_k: int, capacity: int = -
     _check(gate_idx, "gate_idx", dtype=torch.int64)
     n = gate_idx.numel()
     dev = gate_idx.device
-    out = {
-        "counts": torch.empty(num_expert, dtype=torch.int32, device=dev),
-        "offsets": torch.empty(num_expert + 1, dtype=torch.int32, device=dev),
-        "pos": torch.empty(n, dtype=torch.int64, device=dev),
-        "src_row": torch.empty(n, dtype=torch.int32, device=dev),
-        "dst_row": torch.empty(n, dtype=torch.int32, device=dev),
-        "inv_pos": torch.empty(n, dtype=torch.int32, device=dev),
-        "idx_kept": torch.empty(n, dtype=torch.int64, device=dev),
-    }
+    out = _routing_buffers(n, num_expert, dev)
     with _on(gate_idx):
         ws = _workspace(_lib.lib().ccf_route_workspace_bytes(n, num_expert), gate_idx)
         _lib.call("ccf_route", _ptr(gate_idx), n, int(num_expert), int(top_k), int(capacity),
@@ -219,6 +223,32 @@ def route(gate_idx: torch.Tensor, num_expert: int, top_k: int, capacity: int = -
                   _ptr(out["dst_row"]), _ptr(out["inv_pos"]), _ptr(out["idx_kept"]), _ptr(ws),
                   ws.numel(), _stream(gate_idx))
     return out
+
+
+def gate_route(x: torch.Tensor, wg: torch.Tensor, bg: Optional[torch.Tensor], top_k: int, capacity: int = -1):
+    """(idx, score, routing): ``gate_topk_softmax`` and ``route`` on its choice in one call, one launch less where the
+    gate leaves counts that ``route`` would have to make."""
+    _check(x, "x", ndim=2)
+    if x.dtype not in (torch.float16, torch.float32):
+        raise TypeError(f"gate input must be float16 or float32, got {x.dtype}")
+    _check(wg, "gate weight", dtype=x.dtype, ndim=2)
+    if bg is not None:
+        _check(bg, "gate bias", dtype=x.dtype, ndim=1)
+    T, d = x.shape
+    E = wg.shape[0]
+    if wg.shape[1] != d or (bg is not None and bg.shape[0] != E):
+        raise ValueError("gate weight/bias shapes do not match the input")
+    dev, n = x.device, T * top_k
+    idx = torch.empty(T, top_k, dtype=torch.int64, device=dev)
+    score = torch.empty(T, top_k, dtype=x.dtype, device=dev)
+    r = _routing_buffers(n, E, dev)
+    with _on(x):
+        ws = _workspace(_lib.lib().ccf_route_workspace_bytes(n, E), x)
+        _lib.call("ccf_gate_route", _ptr(x), _ptr(wg), _ptr(bg), T, d, E, int(top_k),
+                  CCF_F16 if x.dtype == torch.float16 else CCF_F32, int(capacity), _ptr(idx), _ptr(score),
+                  _ptr(r["counts"]), _ptr(r["offsets"]), _ptr(r["pos"]), _ptr(r["src_row"]), _ptr(r["dst_row"]),
+                  _ptr(r["inv_pos"]), _ptr(r["idx_kept"]), _ptr(ws), ws.numel(), _stream(x))
+    return idx, score, r
 
 
 def route_static(gate_idx: torch.Tensor, num_expert: int, top_k: int, capacity: int = -1,

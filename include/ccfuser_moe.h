@@ -367,6 +367,17 @@ int ccf_moe_forward(const void *x, const void *wg, const void *bg,
                     void *workspace, size_t workspace_bytes, ccf_stream_t stream);
 
 /*
+ * ccf_gate_topk_softmax and ccf_route on its choice in one call (NaiveGate.forward,
+ * mix_moe/mix_moe/gates/naive_gate.py:31-45, then AsyncExpertAssignment.process_data,
+ * mix_moe/mix_moe/transformer.py:102-145): the gate leaves counts that the routing would otherwise make.  idx
+ * [tokens*top_k] is the gate's choice, idx_kept the one after the capacity limit; workspace as ccf_route's.
+ */
+int ccf_gate_route(const void *x, const void *wg, const void *bg, int tokens, int d_model, int num_expert,
+                   int top_k, int dtype, int capacity, int64_t *idx, void *score, int32_t *counts,
+                   int32_t *offsets, int64_t *pos, int32_t *src_row, int32_t *dst_row, int32_t *inv_pos,
+                   int64_t *idx_kept, void *workspace, size_t workspace_bytes, ccf_stream_t stream);
+
+/*
  * Profiling hook (no counterpart in the reference).  Gives up to six hipEvent_t
  * handles; every later ccf_moe_forward on this thread records them on its
  * stream: [0] before the gate, then after the gate, the count/scan/pos, FFN1,

@@ -978,3 +978,68 @@ def test_mfma_probe_runs_and_counts_its_flop():
         if const:
             assert not out.any()
     assert probe.ccf_probe_mfma(0, iters, 1, out.data_ptr(), C.byref(flop), None) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("T,d,E,k,capacity", [
+    (1, 128, 8, 2, -1),                    # one workgroup of one token
+    (333, 192, 4, 1, 20),                  # few experts: counts one at a time, capacity limit
+    (1999, 768, 8, 2, -1),
+    (515, 64, 3, 3, -1),                   # slots that do not tile the routing's chunks: counted by the routing
+    (8192, 256, 64, 2, 300),               # the longest table there is room for in fp32
+    (8193, 128, 64, 1, -1),                # one workgroup more than that
+    (4096, 128, 36, 2, -1),                # four counts a load, experts that do not divide a wavefront
+    (6000, 64, 9, 4, -1),                  # a long table of odd width
+    (200, 64, 600, 2, -1),                 # more experts than threads
+    (700, 4096, 2, 1, -1),                 # fp32: a wavefront per token, which leaves no counts
+])
+def test_gate_with_routing_is_the_gate_then_the_routing(T, d, E, k, capacity, dtype):
+    """One call for both: the bits of the gate alone and of the routing on its choice; rows of NaN choose nothing."""
+    from ccfuser_amd import ops
+    _say(f"gate_route T={T} d={d} E={E} k={k} capacity={capacity} {dtype}")
+    g = torch.Generator().manual_seed(T + E)
+    x = torch.randn(T, d, generator=g)
+    if T > 100:
+        x[7] = float("nan")
+    x, wg, bg = [t.to(dtype).cuda() for t in (x, torch.randn(E, d, generator=g) * 0.1, torch.randn(E, generator=g))]
+    idx, score, r = ops.gate_route(x, wg, bg, k, capacity)
+    idx0, score0 = ops.gate_topk_softmax(x, wg, bg, k)
+    r0 = ops.route(idx0.reshape(-1), E, k, capacity)
+    assert torch.equal(idx, idx0) and torch.equal(score.nan_to_num(3.0), score0.nan_to_num(3.0))
+    n = int(r0["offsets"][-1])
+    for name in ("counts", "offsets", "inv_pos", "idx_kept"):
+        assert torch.equal(r[name], r0[name]), name
+    for name in ("pos", "src_row", "dst_row"):
+        assert torch.equal(r[name][:n], r0[name][:n]), name
+
+
+def test_gate_hooks_run_where_the_routing_goes_with_the_gate():
+    """A gate with a hook, a subclass and another number of experts are called as modules, the gate itself is not."""
+    from ccfuser_amd.mix_moe.gates import NaiveGate
+    from ccfuser_amd.mix_moe.transformer import AsyncExpertAssignment
+    with torch.device("cuda"):
+        gate = NaiveGate(64, 4, 1, 2).half()
+    x = torch.randn(50, 64, dtype=torch.float16, device="cuda")
+    assign = AsyncExpertAssignment(0, 1, 0, 4, 50)
+    pos0, score0, infos0 = assign.process_data(gate, x, 4, 1)
+    assert gate.calls_forward_only() and gate.has_loss
+    seen = []
+    handle = gate.register_forward_hook(lambda m, a, out: seen.append(out[0].shape))
+    pos1, score1, infos1 = assign.process_data(gate, x, 4, 1)
+    handle.remove()
+    assert seen == [torch.Size([50, 2])]
+
+    class Mine(NaiveGate):
+        def forward(self, inp, return_all_scores=False):
+            seen.append("mine")
+            return super().forward(inp, return_all_scores)
+    with torch.device("cuda"):
+        mine = Mine(64, 4, 1, 2).half()
+    mine.load_state_dict(gate.state_dict())
+    pos2, score2, infos2 = assign.process_data(mine, x, 4, 1)
+    assert seen[-1] == "mine"
+    wide = assign.process_data(gate, x, 6, 1)[2]
+    assert wide["counts"].numel() == 6 and torch.equal(wide["counts"][:4], infos0["counts"])
+    n = int(infos0["offsets"][-1])
+    for pos, score, infos in ((pos1, score1, infos1), (pos2, score2, infos2)):
+        assert torch.equal(pos[:n], pos0[:n]) and torch.equal(score, score0) and torch.equal(infos["inv_pos"], infos0["inv_pos"])
