@@ -254,6 +254,10 @@ extern "C" int ccf_gate_route(const void *x, const void *wg, const void *bg, int
   const int n = tokens * top_k;
   CCF_REQUIRE(workspace && workspace_bytes >= ccf_route_workspace_bytes(n, num_expert), CCF_ERR_WORKSPACE,
               "gate_route: workspace of %zu bytes needed, %zu given", ccf_route_workspace_bytes(n, num_expert), workspace_bytes);
+  if (idx && score && counts && offsets && pos && src_row && dst_row && inv_pos && idx_kept &&
+      gate_route_tiny_fits(tokens, d_model, num_expert, top_k, dtype, x, wg))
+    return gate_route_tiny(x, wg, bg, tokens, d_model, num_expert, top_k, capacity, idx, score, counts, offsets, pos, src_row,
+                           dst_row, inv_pos, idx_kept, as_stream(stream));
   int gate_tokens = 0;
   const bool pow2_k = (top_k & (top_k - 1)) == 0;     // a workgroup's flat indices tile the routing's chunks
   if (int rc = gate_forward(x, wg, bg, tokens, d_model, num_expert, top_k, dtype, idx, score, nullptr, stream,

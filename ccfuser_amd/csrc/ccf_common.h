@@ -61,6 +61,12 @@ int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int 
                  int dtype, int64_t *idx_out, void *score_out, void *logits_out, ccf_stream_t stream,
                  int32_t *wg_cnt, long long max_cnt, int *tokens_per_wg);
 
+// the gate and the routing of a few tokens as one launch; _fits: all pointers below must be given
+bool gate_route_tiny_fits(int tokens, int d, int E, int k, int dtype, const void *x, const void *wg);
+int gate_route_tiny(const void *x, const void *wg, const void *bg, int tokens, int d, int E, int k, int capacity, int64_t *idx,
+                    void *score, int32_t *counts, int32_t *offsets, int64_t *pos, int32_t *src_row, int32_t *dst_row,
+                    int32_t *inv_pos, int64_t *idx_kept, hipStream_t stream);
+
 // tuning knobs set through ccf_set_option()
 extern int g_gate_waves, g_gate_slots, g_gate_stream;   // gate.hip
 extern int g_route_rows_max;             // route.hip

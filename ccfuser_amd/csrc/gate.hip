@@ -24,6 +24,7 @@
 // the multiplies as MFMAs onto zero.
 #include "ccf_common.h"
 #include "mfma_f32.h"
+#include "plan.h"
 
 #include <limits.h>
 #include <type_traits>
@@ -1037,10 +1038,241 @@ bool gate_f32_on_mfma(int tokens, int d, int E) {
   return (tokens <= 16384 || d >= 12 * kPart) && (E > 16 || d <= 4096);
 }
 
+// fp16 gate of few tokens.  The MFMA tiles above have 16 tokens at least, and the 1024 instructions that 16 tokens of 4096
+// and 16 experts take keep the one CU that has them busy for 4 us, the conversions of their operands for as long again.
+// Here a thread walks one part of K of one expert for one token as a chain of 128 fused multiply-adds: the same chain, the
+// same bits, and with 8 experts of 4096 four wavefronts, whose 256 chains run side by side.
+//
+// * A workgroup holds all expert rows and the rows of `group` tokens in LDS, fetched by direct loads that are all on their
+//   way at once, and takes `wg_tokens` tokens, `group` at a time.  A part is 16 chunks of 16 bytes; chunk c of part i sits
+//   at c ^ (i % 16), applied on the global side, so that lanes on neighbouring parts read other banks.
+// * The part sums meet in LDS, a thread per token and expert adds them in part order, and one per token selects.
+// * With `route` (one workgroup, at most 64 indices) the routing of the choice follows: a lane per index.
+//
+// Microseconds, MFMA tiles and here (the gate alone): see gate_f16_walks().
+struct TinyRoute {
+  int32_t *counts, *offsets;                       // counts null: no routing
+  int64_t *pos;
+  int32_t *src_row, *dst_row, *inv_pos;
+  int64_t *idx_kept;
+  int capacity;
+};
+constexpr int kTinyIndices = 64;
+constexpr int kTinyBatches = 2;     // most turns of the one workgroup that gates and routes
+
+// LDS of a workgroup, in bytes: expert rows, token rows, part sums, logits, biases, counts, routed indices
+struct WalkLds {
+  int x, part, logit, bias, row, idx, bytes;
+};
+__host__ __device__ inline WalkLds walk_lds(int E, int nparts, int group) {
+  WalkLds l;
+  l.x = (E * nparts * 256 + 1023) / 1024 * 1024;
+  l.part = l.x + (group * nparts * 256 + 1023) / 1024 * 1024;
+  l.logit = l.part + 4 * group * E * (nparts + 1);
+  l.bias = l.logit + 4 * group * (E + 1);
+  l.row = l.bias + 4 * E;
+  l.idx = l.row + 4 * E;
+  l.bytes = l.idx + 4 * 2 * kTinyIndices;
+  return l;
+}
+
+template <int KS>
+__global__ void __launch_bounds__(512)
+gate_walk_kernel(const half_t *__restrict__ x, const half_t *__restrict__ wg, const half_t *__restrict__ bg,
+                 int tokens, int d, int E, int k, int group, int wg_tokens, int64_t *__restrict__ idx_out,
+                 half_t *__restrict__ score_out, half_t *__restrict__ logits_out, int32_t *__restrict__ wg_cnt,
+                 TinyRoute route) {
+  extern __shared__ __attribute__((aligned(1024))) char s_raw[];
+  const int nparts = (d + kPart - 1) / kPart, chains = E * nparts;
+  const WalkLds at = walk_lds(E, nparts, group);
+  float *s_part = reinterpret_cast<float *>(s_raw + at.part), *s_logit = reinterpret_cast<float *>(s_raw + at.logit);
+  float *s_bias = reinterpret_cast<float *>(s_raw + at.bias);
+  int *s_row = reinterpret_cast<int *>(s_raw + at.row), *s_idx = reinterpret_cast<int *>(s_raw + at.idx);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+  const FastDiv by_parts(nparts), by_chains(chains), by_experts(E);
+
+  // `rows` rows of base from row `first` on (past `last` that one again) into LDS at byte `to`
+  auto fetch = [&](const half_t *base, int first, int rows, int last, int to) {
+    const int parts = rows * nparts;
+    for (int s0 = wave * 64; s0 < parts * 16; s0 += waves * 64) {
+      const int s = s0 + lane, i = s >> 4, part = i < parts ? i : parts - 1;
+      const int r = by_parts.div(part);
+      const int row = first + r < last ? first + r : last;
+      const int kk = (part - r * nparts) * kPart + (((s & 15) ^ (i & 15)) << 3);
+      const half_t *src = base + static_cast<size_t>(row) * d + (kk < d ? kk : 0);       // past the end of K: never used
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                       (__attribute__((address_space(3))) void *)(s_raw + to + s0 * 16), 16, 0, 0);
+    }
+  };
+  fetch(wg, 0, E, E - 1, 0);
+  for (int e = tid; e < E; e += blockDim.x) {
+    s_bias[e] = bg ? static_cast<float>(bg[e]) : 0.0f;
+    s_row[e] = 0;
+  }
+  const int g = by_chains.div(tid), chain = tid - g * chains;
+  const int e_of = by_parts.div(chain), p_of = chain - e_of * nparts;
+  const bool full = d % kPart == 0;
+  const int t_first = blockIdx.x * wg_tokens;
+  for (int t0 = t_first; t0 < t_first + wg_tokens && t0 < tokens; t0 += group) {
+    fetch(x, t0, group, tokens - 1, at.x);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (g < group) {
+      const int xi = g * nparts + p_of;
+      const char *wr = s_raw + chain * 256, *xr = s_raw + at.x + xi * 256;
+      const int len = d - p_of * kPart;            // K elements left for this part
+      float acc = 0.0f;
+      auto walk = [&](auto FULL) {
+#pragma unroll
+        for (int c = 0; c < kPart / 8; ++c) {
+          const half8 wv = *reinterpret_cast<const half8 *>(wr + ((c ^ (chain & 15)) << 4));
+          const half8 xv = *reinterpret_cast<const half8 *>(xr + ((c ^ (xi & 15)) << 4));
+          if (decltype(FULL)::value || c * 8 < len) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc = __builtin_fmaf(static_cast<float>(xv[j]), static_cast<float>(wv[j]), acc);
+          }
+        }
+      };
+      if (full) walk(std::true_type{});
+      else walk(std::false_type{});
+      s_part[(g * E + e_of) * (nparts + 1) + p_of] = acc;
+    }
+    __syncthreads();
+    for (int i = tid; i < group * E; i += blockDim.x) {
+      const int gi = by_experts.div(i), e = i - gi * E;
+      const float *ps = s_part + i * (nparts + 1);
+      float t = ps[0];
+#pragma unroll 8
+      for (int p = 1; p < nparts; ++p) t = t + ps[p];
+      if (bg) t = t + s_bias[e];
+      t = round_to<half_t>(t);
+      if (logits_out && t0 + gi < tokens) logits_out[static_cast<size_t>(t0 + gi) * E + e] = static_cast<half_t>(t);
+      s_logit[gi * (E + 1) + e] = t;
+    }
+    __syncthreads();
+    if (tid < group && t0 + tid < tokens) {
+      Best<KS> best;
+      best.clear();
+#pragma unroll 8
+      for (int e = 0; e < E; ++e) best.offer(s_logit[tid * (E + 1) + e], e, k);
+      best.template write<half_t>(t0 + tid, k, idx_out, score_out);
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        if (s < k) {
+          if (wg_cnt && best.id[s] < E) atomicAdd(&s_row[best.id[s]], 1);
+          if (route.counts) s_idx[(t0 + tid) * k + s] = best.id[s];
+        }
+    }
+    // the next tokens' rows land behind every thread's reads of these; their logits two barriers further on
+  }
+  if (wg_cnt) {
+    __syncthreads();
+    for (int e = tid; e < E; e += blockDim.x) wg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = s_row[e];
+  }
+  if (!route.counts) return;
+  // The routing, as pos_kernel does it: ranks in index order, the capacity, then the experts' starts.  A list that NaN
+  // logits left short has entries that are no expert.
+  int *s_kept = s_idx + kTinyIndices;
+  const int n = tokens * k;
+  __syncthreads();
+  int e = INT_MAX, rank = 0;
+  if (tid < n) {
+    e = s_idx[tid];
+    for (int q = 0; q < tid; ++q) rank += s_idx[q] == e;
+    const bool kept = e < E && (route.capacity < 0 || rank < route.capacity);
+    s_kept[tid] = kept ? e : INT_MAX;
+  }
+  __syncthreads();
+  if (tid < n) {
+    const bool kept = s_kept[tid] < E;
+    int j = rank;
+    for (int q = 0; q < n; ++q) j += s_kept[q] < e;
+    if (kept) {
+      route.pos[j] = tid;
+      route.src_row[j] = tid / k;
+      route.dst_row[j] = tid;
+    }
+    route.inv_pos[tid] = kept ? j : -1;
+    route.idx_kept[tid] = kept ? e : -1;
+  }
+  for (int c = tid; c <= E; c += blockDim.x) {
+    int start = 0, count = 0;
+    for (int q = 0; q < n; ++q) {
+      start += s_kept[q] < c;
+      count += s_kept[q] == c;
+    }
+    route.offsets[c] = start;
+    if (c < E) route.counts[c] = count;
+  }
+}
+
+// (a knob away from its default asks for a form of the MFMA tiles)
+bool gate_default_shape() { return g_gate_slots == 0 && g_gate_waves == kMaxWaves && g_gate_stream == -1; }
+
+// Tokens that a workgroup of gate_walk_kernel takes at a time, 0: not a case for it.  The expert rows fit in LDS, and all
+// workgroups are on the chip at once: a second round loads the expert rows again and loses to the MFMA tiles.  Microseconds
+// (MFMA tiles, here): 8 experts of 4096, 1 token 11.4, 5.8, 333 tokens 12.0, 7.2, 512 (one round) 11.7, 7.4, 1024 12.4,
+// 13.2; of 2048, 1536 (one round) 8.9, 7.0, 2048 9.0, 10.5; of 768, 8192 (one round) 11.8, 10.1, 16384 13.4, 15.9; 16
+// experts of 1024, 2048 (one round) 8.7, 8.5, 4096 9.2, 14.8; 32 of 768, 768 (one round) 11.9, 8.1, 1536 12.0, 13.5; 4 of
+// 256, 512 8.6, 4.0.
+int gate_f16_walk_group(int tokens, int d, int E) {
+  constexpr int kCus = 256, kLds = 160 * 1024, kMaxLds = 150 * 1024, kWgsPerCu = 8;
+  const int nparts = (d + kPart - 1) / kPart;
+  if (static_cast<long long>(E) * nparts > 512) return 0;
+  const int chains = E * nparts;
+  int group = 1;
+  while (2 * group * chains <= 256 && group < tokens) group *= 2;
+  const int lds = walk_lds(E, nparts, group).bytes;
+  if (lds > kMaxLds) return 0;
+  const int per_cu = kLds / lds < kWgsPerCu ? kLds / lds : kWgsPerCu;
+  return (tokens + group - 1) / group <= kCus * per_cu ? group : 0;
+}
+
+int launch_gate_walk(const half_t *x, const half_t *wg, const half_t *bg, int tokens, int d, int E, int k, int group,
+                     int64_t *idx_out, half_t *score_out, half_t *logits_out, hipStream_t stream, int32_t *wg_cnt,
+                     long long max_cnt, int *tokens_per_wg, const TinyRoute &route) {
+  const int nparts = (d + kPart - 1) / kPart, chains = E * nparts;
+  const int threads = chains * group > 256 ? 512 : 256;
+  const int wg_tokens = route.counts ? (tokens + group - 1) / group * group : group;
+  const int wgs = (tokens + wg_tokens - 1) / wg_tokens;
+  if (static_cast<long long>(wgs) * E > max_cnt) wg_cnt = nullptr;
+  if (wg_cnt && tokens_per_wg) *tokens_per_wg = wg_tokens;
+  const int lds = walk_lds(E, nparts, group).bytes;
+  auto kern = k == 1 ? gate_walk_kernel<1> : (k == 2 ? gate_walk_kernel<2> : gate_walk_kernel<kMaxTopK>);
+  if (lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate: LDS attribute: %s", hipGetErrorString(e));
+  }
+  hipLaunchKernelGGL(kern, dim3(wgs), dim3(threads), lds, stream, x, wg, bg, tokens, d, E, k, group, wg_tokens, idx_out, score_out,
+                     logits_out, wg_cnt, route);
+  return check_launch("gate_walk_kernel");
+}
+
 }  // namespace
 }  // namespace ccf
 
 namespace ccf {
+// Gate and routing of a few tokens as one launch, by a workgroup that takes its tokens in two turns at most.  Microseconds
+// as two launches (gate in MFMA tiles, then in walks; both with 5 of routing) and as one: 8 experts of 4096, 1 token 16.3,
+// 10.8, 6.7, 2 (two turns) 16.5, 11.1, 9.9, 3 16.4, 11.1, 12.9; of 768, 8 (two turns) 12.4, 9.9, 8.7; 32 of 1024, 1 17.8,
+// 11.6, 8.7.
+bool gate_route_tiny_fits(int tokens, int d, int E, int k, int dtype, const void *x, const void *wg) {
+  if (dtype != CCF_F16 || tokens <= 0 || d <= 0 || d % 8 || E <= 0 || E > 512 || k < 1 || k > kMaxTopK || k > E || !x || !wg ||
+      !aligned16(x) || !aligned16(wg) || static_cast<long long>(tokens) * k > kTinyIndices || !gate_default_shape())
+    return false;
+  const int group = gate_f16_walk_group(tokens, d, E);
+  return group > 0 && tokens <= kTinyBatches * group;
+}
+
+int gate_route_tiny(const void *x, const void *wg, const void *bg, int tokens, int d, int E, int k, int capacity, int64_t *idx,
+                    void *score, int32_t *counts, int32_t *offsets, int64_t *pos, int32_t *src_row, int32_t *dst_row,
+                    int32_t *inv_pos, int64_t *idx_kept, hipStream_t stream) {
+  return launch_gate_walk(static_cast<const half_t *>(x), static_cast<const half_t *>(wg), static_cast<const half_t *>(bg), tokens, d,
+                          E, k, gate_f16_walk_group(tokens, d, E), idx, static_cast<half_t *>(score), nullptr, stream, nullptr, 0,
+                          nullptr, TinyRoute{counts, offsets, pos, src_row, dst_row, inv_pos, idx_kept, capacity});
+}
+
 // The gate; with wg_cnt (room for max_cnt ints) the tiled kernels also leave, per workgroup, how many of
 // its token slots chose each expert ([workgroups][tot_expert], a workgroup covering *tokens_per_wg
 // consecutive tokens), when that table fits; *tokens_per_wg = 0 says it was not written.
@@ -1082,6 +1314,11 @@ int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int 
                   d_model, tot_expert, top_k, idx_out, static_cast<float *>(score_out), static_cast<float *>(logits_out),
                   as_stream(stream), wg_cnt, max_cnt, tokens_per_wg);
   }
+  const int group = gate_default_shape() ? gate_f16_walk_group(tokens, d_model, tot_expert) : 0;
+  if (group > 0)
+    return launch_gate_walk(static_cast<const half_t *>(x), static_cast<const half_t *>(wg), static_cast<const half_t *>(bg), tokens,
+                            d_model, tot_expert, top_k, group, idx_out, static_cast<half_t *>(score_out),
+                            static_cast<half_t *>(logits_out), as_stream(stream), wg_cnt, max_cnt, tokens_per_wg, TinyRoute{});
   // Tile and slots.  With S slots a wavefront covers 64 / S tokens, so S grows while there
   // are fewer than four workgroups per CU and K has parts for the slots.
   const int n = tot_expert > 16 ? 32 : 16;

@@ -151,6 +151,35 @@ def test_gate_launch_shapes(slots, waves, stream, T, d, E, k):
     assert (score.cpu().float() - score_ref.float()).abs().max() <= 1e-3
 
 
+@pytest.mark.parametrize("T,d,E,k", [
+    (1, 8, 1, 1), (3, 136, 5, 3), (40, 200, 9, 8),         # one short part, a part and a bit, more lists than two
+    (333, 4096, 8, 2), (512, 4096, 8, 1), (513, 4096, 8, 2),         # one round of workgroups, one workgroup more
+    (5, 8192, 8, 2), (5, 8200, 8, 2),                      # as many chains as threads, one part more (MFMA tiles)
+    (9, 4096, 16, 2), (2, 128, 512, 2), (2, 128, 513, 2),  # 512 chains of other shapes
+    (100, 64, 3, 1), (2000, 768, 8, 2), (700, 1032, 7, 2), # several tokens at a time, ragged groups and parts
+    (64, 32768, 1, 1), (64, 32768, 2, 1),                  # very long rows: LDS of a workgroup
+])
+def test_gate_of_few_tokens(T, d, E, k):
+    """A thread per token, expert and part of K, and the sizes around it: the oracle's bits, with and without a bias,
+    and what the MFMA tiles give."""
+    from ccfuser_amd import ops
+    _say(f"gate of few tokens T={T} d={d} E={E} k={k}")
+    x, wg, bg, idx_ref, score_ref, logits_ref = _gate_case(T, d, E, k)
+    idx, score, logits = ops.gate_topk_softmax(dev(x), dev(wg), dev(bg), k, return_logits=True)
+    assert torch.equal(logits.cpu(), logits_ref), "logits differ bitwise"
+    assert torch.equal(idx.cpu(), idx_ref), "expert choice differs"
+    assert (score.cpu().float() - score_ref.float()).abs().max() <= 1e-3
+    bare = ops.gate_topk_softmax(dev(x), dev(wg), None, k, return_logits=True)
+    ops.set_option("gate_stream", 0)
+    try:
+        tiles = ops.gate_topk_softmax(dev(x), dev(wg), dev(bg), k, return_logits=True)
+        bare_tiles = ops.gate_topk_softmax(dev(x), dev(wg), None, k, return_logits=True)
+    finally:
+        ops.set_option("gate_stream", -1)
+    for a, b in zip((idx, score, logits, *bare), (*tiles, *bare_tiles)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("stream", [0, 1])
 @pytest.mark.parametrize("E,k", [(32, 2), (8, 1), (70, 3)])
 def test_gate_logits_that_are_nothing_but_rounding_error(E, k, stream):
@@ -992,6 +1021,10 @@ def test_mfma_probe_runs_and_counts_its_flop():
     (6000, 64, 9, 4, -1),                  # a long table of odd width
     (200, 64, 600, 2, -1),                 # more experts than threads
     (700, 4096, 2, 1, -1),                 # fp32: a wavefront per token, which leaves no counts
+    (2, 4096, 8, 2, -1), (3, 4096, 8, 2, -1),        # fp16: gate and routing as one launch in two turns, one token more
+    (8, 768, 8, 2, 3), (9, 768, 8, 2, 0),            # the same at four tokens a turn, capacity limits
+    (32, 256, 4, 2, 9), (33, 256, 4, 2, -1),         # 64 indices, and more
+    (7, 136, 9, 8, 4), (21, 8, 3, 3, -1), (1, 512, 128, 8, -1),
 ])
 def test_gate_with_routing_is_the_gate_then_the_routing(T, d, E, k, capacity, dtype):
     """One call for both: the bits of the gate alone and of the routing on its choice; rows of NaN choose nothing."""
