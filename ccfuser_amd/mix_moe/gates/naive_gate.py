@@ -85,11 +85,11 @@ class NaiveGate(BaseGate):
 
     def _choose(self, inp, return_all_scores, capacity=None, routing=None):
         lead = inp.shape[:-1]
-        x = inp.reshape(-1, inp.shape[-1])
+        x = inp if inp.dim() == 2 else inp.reshape(-1, inp.shape[-1])
         if not x.is_contiguous():
             x = x.contiguous()
         res = _GateFunction.apply(x, self.gate.weight, self.gate.bias, self.top_k, return_all_scores, capacity, routing)
-        idx = res[0].view(*lead, self.top_k)
+        idx = res[0] if len(lead) == 1 else res[0].view(*lead, self.top_k)
         score = res[1]                                   # [(B*L), top_k], as the reference returns it
         # dummy loss, on the input's device (naive_gate.py:41): a fresh leaf over a zero made once per
         # device, so that the forward pays no fill kernel for it

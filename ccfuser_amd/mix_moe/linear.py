@@ -47,6 +47,14 @@ def _param_grads(weight, E):
     return grad_w, grad_b
 
 
+def _pair(weight, bias, E):
+    """Weight and bias for a call that uses their first E experts (``spare_experts``): as they are, since a slice costs as
+    much host time as a launch, or the slices where only those are contiguous."""
+    if weight.is_contiguous() and bias.is_contiguous() and weight.shape[0] == bias.shape[0]:
+        return weight, bias
+    return weight.detach()[:E], bias.detach()[:E]
+
+
 def _routing(pos, block_infos, top_k_hint=None):
     """(src_row, dst_row, offsets, max_rows, n_flat) for the grouped GEMMs."""
     if "offsets" in block_infos:                      # planned by this package: all on device
@@ -67,8 +75,8 @@ class MixMOELinear1(Function):
         ctx.save_for_backward(input_buf, weight, src_row, dst_row, offsets,
                               moe_inp_block_infos.get("inv_pos"))
         ctx.sizes = (max_rows, n_flat, bool(fuse_gelu), bool(moe_inp_block_infos.get("may_drop", True)))
-        return ops.ffn1(input_buf, src_row, offsets, max_rows, weight.detach()[:E],
-                        bias.detach()[:E], gelu=bool(fuse_gelu))
+        return ops.ffn1(input_buf, src_row, offsets, max_rows, *_pair(weight, bias, E), gelu=bool(fuse_gelu),
+                        spare_experts=True)
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -105,8 +113,7 @@ class MixMOELinear2(Function):
         y = alloc(n_flat, d, dtype=input_buf.dtype, device=input_buf.device)
         ctx.save_for_backward(input_buf, weight, dst_row, offsets)
         ctx.sizes = (max_rows, bool(moe_inp_block_infos.get("may_drop", True)))
-        return ops.ffn2(input_buf, dst_row, offsets, max_rows, weight.detach()[:E],
-                        bias.detach()[:E], y)
+        return ops.ffn2(input_buf, dst_row, offsets, max_rows, *_pair(weight, bias, E), y, spare_experts=True)
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -153,10 +160,10 @@ class MixMOEFusedFFN(Function):
         src_row, dst_row, offsets, max_rows, n_flat = _routing(pos, moe_inp_block_infos)
         E = offsets.numel() - 1
         may_drop = bool(moe_inp_block_infos.get("may_drop", True))
-        act, h_pre = ops.ffn1_keep(input_buf, src_row, offsets, max_rows, w1.detach()[:E], b1.detach()[:E])
+        act, h_pre = ops.ffn1_keep(input_buf, src_row, offsets, max_rows, *_pair(w1, b1, E), spare_experts=True)
         y = (torch.zeros if may_drop else torch.empty)(n_flat, w2.shape[1], dtype=input_buf.dtype,
                                                        device=input_buf.device)
-        ops.ffn2(act, dst_row, offsets, max_rows, w2.detach()[:E], b2.detach()[:E], y)
+        ops.ffn2(act, dst_row, offsets, max_rows, *_pair(w2, b2, E), y, spare_experts=True)
         ctx.save_for_backward(input_buf, w1, w2, act, h_pre, src_row, dst_row, offsets,
                               moe_inp_block_infos.get("inv_pos"))
         ctx.sizes = (max_rows, n_flat, may_drop)

@@ -6,7 +6,7 @@ import torch.nn as nn
 from .. import ops
 from .gates import NaiveGate
 from .layers import MixMOE
-from .linear import FMoELinear, MixMOEFusedFFN, MixMOEInstance, MixMOELinear1, MixMOELinear2
+from .linear import FMoELinear, MixMOEFusedFFN, MixMOEInstance, MixMOELinear1, MixMOELinear2, _pair
 
 _COMPAT_KEYS = ("expert_ids", "local_expert_id_indexs", "ranks", "lens", "start_addrs",
                 "remote_block_num", "total_block_num", "expert_block_ids", "expert_block_id_idxs")
@@ -243,7 +243,9 @@ class MixMOETransformerMLP(MixMOE):
 
     def forward(self, inp: torch.Tensor):
         original_shape = inp.shape
-        inp = inp.reshape(-1, self.d_model)
+        rows = len(original_shape) == 2 and original_shape[1] == self.d_model        # no view to take, nor to differentiate
+        if not rows:
+            inp = inp.reshape(-1, self.d_model)
         if inp.dtype != torch.float16:
             raise TypeError("moe input data type must be float 16")
         if not inp.is_contiguous():
@@ -257,13 +259,12 @@ class MixMOETransformerMLP(MixMOE):
         elif self.fused and self.experts._gelu_is_fusable() and not (
                 torch.is_grad_enabled() and (inp.requires_grad or _any_requires_grad(self))):
             ex = self.experts
-            with torch.no_grad():
-                lin, up, down = self.gate.gate, ex.htoh4, ex.h4toh
-                output = ops.moe_forward(inp, lin.weight, lin.bias, up.weight[:E], up.bias[:E], down.weight[:E],
-                                         down.bias[:E], self.top_k, self._capacity(inp.shape[0]))
+            lin, up, down = self.gate.gate, ex.htoh4, ex.h4toh
+            output = ops.moe_forward(inp, lin.weight, lin.bias, *_pair(up.weight, up.bias, E), *_pair(down.weight, down.bias, E),
+                                     self.top_k, self._capacity(inp.shape[0]), spare_experts=True)
         else:
             self.async_expert_assign.capacity = self._capacity(inp.shape[0])
             pos, gate_score, infos = self.async_expert_assign.process_data(
                 self.gate, inp, self.num_expert, self.world_size)
             output = super().forward(inp, pos, gate_score, infos)
-        return output.reshape(original_shape)
+        return output if rows else output.reshape(original_shape)

@@ -383,8 +383,9 @@ def _check_expert(w: torch.Tensor, b: torch.Tensor, name: str, kn: bool = False)
 def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor, max_rows: int,
          w1: torch.Tensor, b1: torch.Tensor, gelu: bool = True,
          out: Optional[torch.Tensor] = None, dst_row: Optional[torch.Tensor] = None,
-         workspace: Optional[torch.Tensor] = None, w_kn: bool = False) -> torch.Tensor:
-    """h [max_rows, f] (or ``out``); rows nothing maps to are left as they were.  ``w_kn``: the weight is
+         workspace: Optional[torch.Tensor] = None, w_kn: bool = False, spare_experts: bool = False) -> torch.Tensor:
+    """h [max_rows, f] (or ``out``); rows nothing maps to are left as they were.  ``spare_experts``: the weight may
+    hold more experts than ``offsets``, the first of which are used.  ``w_kn``: the weight is
     stored [E, d, f] (input width first)."""
     if x.dtype != torch.float16:
         raise TypeError("moe input data type must be float 16")
@@ -392,6 +393,8 @@ def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor
     _check_expert(w1, b1, "ffn1", w_kn)
     _check(offsets, "offsets", dtype=torch.int32, ndim=1)
     E, f, d = (w1.shape[0], w1.shape[2], w1.shape[1]) if w_kn else w1.shape
+    if spare_experts and 0 < offsets.numel() - 1 < E:
+        E = offsets.numel() - 1
     if x.shape[1] != d or offsets.numel() != E + 1:
         raise ValueError("ffn1: x/offsets do not match the weight shape")
     if src_row is not None:
@@ -416,13 +419,15 @@ def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor
 
 
 def ffn1_keep(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor, max_rows: int,
-              w1: torch.Tensor, b1: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+              w1: torch.Tensor, b1: torch.Tensor, spare_experts: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
     """(act, h_pre), both [max_rows, f]: ``ffn1`` with the GELU, keeping the pre-activation
-    for the backward."""
+    for the backward.  ``spare_experts`` as in ``ffn1``."""
     _check(x, "x", dtype=torch.float16, ndim=2)
     _check_expert(w1, b1, "ffn1")
     _check(offsets, "offsets", dtype=torch.int32, ndim=1)
     E, f, d = w1.shape
+    if spare_experts and 0 < offsets.numel() - 1 < E:
+        E = offsets.numel() - 1
     if x.shape[1] != d or offsets.numel() != E + 1:
         raise ValueError("ffn1_keep: x/offsets do not match the weight shape")
     if src_row is not None:
@@ -444,14 +449,16 @@ def ffn2(h: torch.Tensor, dst_row: Optional[torch.Tensor], offsets: torch.Tensor
          w2: torch.Tensor, b2: torch.Tensor, y: torch.Tensor,
          row_scale: Optional[torch.Tensor] = None,
          src_row: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None,
-         w_kn: bool = False) -> torch.Tensor:
+         w_kn: bool = False, spare_experts: bool = False) -> torch.Tensor:
     """Writes ``y[dst_row[j]]`` for the routed rows and returns ``y``.  ``w_kn``: the weight is stored
-    [E, f, d] (input width first)."""
+    [E, f, d] (input width first).  ``spare_experts`` as in ``ffn1``."""
     _check(h, "h", dtype=torch.float16, ndim=2)
     _check_expert(w2, b2, "ffn2", w_kn)
     _check(offsets, "offsets", dtype=torch.int32, ndim=1)
     _check(y, "y", dtype=torch.float16, ndim=2)
     E, d, f = (w2.shape[0], w2.shape[2], w2.shape[1]) if w_kn else w2.shape
+    if spare_experts and 0 < offsets.numel() - 1 < E:
+        E = offsets.numel() - 1
     if h.shape[1] != f or offsets.numel() != E + 1 or y.shape[1] != d:
         raise ValueError("ffn2: h/offsets/y do not match the weight shape")
     if src_row is not None:
@@ -611,8 +618,9 @@ def ffn1_backward(grad_h: torch.Tensor, x: torch.Tensor, src_row: Optional[torch
 
 # ------------------------------------------------------- the whole layer
 def moe_forward(x, wg, bg, w1, b1, w2, b2, top_k: int, capacity: int = -1,
-                return_routing: bool = False, workspace: Optional[torch.Tensor] = None):
-    """The fused layer forward: out [T, d] fp16 (and the routing tensors on request)."""
+                return_routing: bool = False, workspace: Optional[torch.Tensor] = None, spare_experts: bool = False):
+    """The fused layer forward: out [T, d] fp16 (and the routing tensors on request).  ``spare_experts``: the expert
+    weights may hold more experts than the gate scores, the first of which are used."""
     if x.dtype != torch.float16:
         raise TypeError("moe input data type must be float 16")
     _check(x, "x", dtype=torch.float16, ndim=2)
@@ -622,8 +630,9 @@ def moe_forward(x, wg, bg, w1, b1, w2, b2, top_k: int, capacity: int = -1,
     _check_expert(w1, b1, "ffn1")
     _check_expert(w2, b2, "ffn2")
     T, d = x.shape
-    E, f, d1 = w1.shape
-    if d1 != d or tuple(w2.shape) != (E, d, f) or tuple(wg.shape) != (E, d):
+    slots, f, d1 = w1.shape
+    E = wg.shape[0] if spare_experts and wg.shape[0] < slots else slots
+    if d1 != d or tuple(w2.shape) != (slots, d, f) or tuple(wg.shape) != (E, d):
         raise ValueError("moe_forward: weight shapes do not match (one GPU: the gate scores the local experts)")
     dev = x.device
     out = torch.empty(T, d, dtype=x.dtype, device=dev)

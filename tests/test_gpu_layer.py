@@ -835,3 +835,42 @@ def test_fused_layer_random_shapes_with_forced_plans(T, d, f, E, k, skinny, sk_t
     _say(f"  counts={ref['counts'].tolist()} max_abs={ma:.3e} mean_rel={mr:.3e}")
     assert ma <= MAX_ABS and mr <= MEAN_REL
     assert torch.equal(fused, again)
+
+
+@pytest.mark.parametrize("slots", [4, 7])
+def test_weights_of_more_experts_than_the_gate_scores(slots):
+    """The first experts of larger weights: refused unless asked for, then the bits of the slices; a module whose
+    parameters are contiguous only as slices takes those."""
+    from ccfuser_amd import ops
+    from ccfuser_amd.mix_moe import MixMOETransformerMLP
+    E, d, f, T = 4, 128, 256, 300
+    g = torch.Generator().manual_seed(slots)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.1).half().cuda()
+    x, wg, bg, w = rnd(T, d), rnd(E, d), rnd(E), [rnd(slots, f, d), rnd(slots, f), rnd(slots, d, f), rnd(slots, d)]
+    ref = ops.moe_forward(x, wg, bg, *[t[:E] for t in w], 2)
+    assert torch.equal(ref, ops.moe_forward(x, wg, bg, *w, 2, spare_experts=True))
+    r = ops.route(torch.randint(0, E, (2 * T,), generator=g).cuda(), E, 2)
+    rows = (x, r["src_row"], r["offsets"], 2 * T)
+    h, pre = ops.ffn1_keep(*rows, *w[:2], spare_experts=True)
+    assert torch.equal(h, ops.ffn1(*rows, w[0][:E], w[1][:E]))
+    y = [torch.zeros(2 * T, d, dtype=torch.float16, device="cuda") for _ in range(2)]
+    ops.ffn2(h, r["dst_row"], r["offsets"], 2 * T, *w[2:], y[0], spare_experts=True)
+    ops.ffn2(h, r["dst_row"], r["offsets"], 2 * T, w[2][:E], w[3][:E], y[1])
+    assert torch.equal(*y)
+    if slots > E:
+        for call in (lambda: ops.moe_forward(x, wg, bg, *w, 2), lambda: ops.ffn1(*rows, *w[:2]), lambda: ops.ffn1_keep(*rows, *w[:2]),
+                     lambda: ops.ffn2(h, r["dst_row"], r["offsets"], 2 * T, *w[2:], y[0])):
+            with pytest.raises(ValueError):
+                call()
+    with pytest.raises(ValueError):                         # fewer experts than the gate scores
+        ops.moe_forward(x, wg, bg, *[t[:E - 1] for t in w], 2, spare_experts=True)
+    # one expert of three slots, the slots far apart in memory: only a slice of the first is contiguous
+    with torch.device("cuda"):
+        mlp = MixMOETransformerMLP("naive", {"num_local_expert": 1, "hidden_size": f}, d, 0, 1, total_batch_size=T, top_k=1,
+                                   popular_expert_num=2).half().requires_grad_(False)
+    ref = mlp(x)
+    for lin in (mlp.experts.htoh4, mlp.experts.h4toh):
+        wide = torch.empty(3, 2, *lin.weight.shape[1:], dtype=torch.float16, device="cuda")
+        wide[:, 0] = lin.weight
+        lin.weight = torch.nn.Parameter(wide[:, 0], requires_grad=False)
+    assert not mlp.experts.htoh4.weight.is_contiguous() and torch.equal(mlp(x), ref)
