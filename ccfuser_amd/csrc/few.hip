@@ -123,14 +123,29 @@ __device__ __forceinline__ void few_frags_kn(half8 (&a)[TMW], half8 (&b)[NB], ui
 // the row (the layout of the 256-row tiles' main loop, gemm_tile.h).
 __device__ __forceinline__ int few_kn_swz(int row) { return (row & 3) | (((row >> 3) & 1) << 2); }
 
+// lds_dma16 with the non-temporal hint, for weights that one tile reads once: 6.2 TB/s from HBM instead of 5.5.  Weights
+// that several M tiles share, or that a next call finds in the 256 MB Infinity Cache, do better without: the hint is for a
+// tile that has its expert to itself, in a GEMM of 160 MB of weights and more (a layer's two are 320 then).  Microseconds
+// of FFN1 / FFN2, without and with it, six layers one after the other: 8 experts of 4096 / 14336, 83 rows each 184, 184
+// and 176, 167; 16 of 2048 / 8192, 100 rows 140, 134 and 138, 119; 8 of 2560 / 8960, 100 rows 113, 101 and 108, 96; one
+// layer of 8 of 2048 / 8192 again and again 47, 47 and 66, 54 (its FFN1 alone, 268 MB; in a layer nothing is found again).
+// A layer of 128 tokens, 8 experts of 4096 / 14336: 356 -> 333 us.
+constexpr double kStreamBytes = 160e6;
+__device__ __forceinline__ void lds_dma16_nt(const void *gptr, lds_char *lds_wave_base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)gptr,
+                                   (__attribute__((address_space(3))) void *)lds_wave_base, 16, 0, 2);
+}
+
 // One lane's tile table entry.
 struct FewTile {
   int e, row0, rows, n0;
+  int alone;               // no other tile reads these weights
 };
 
 __device__ __forceinline__ FewTile tile_at(const FewTile &mine, int r) {
   return FewTile{__builtin_amdgcn_readlane(mine.e, r), __builtin_amdgcn_readlane(mine.row0, r),
-                 __builtin_amdgcn_readlane(mine.rows, r), __builtin_amdgcn_readlane(mine.n0, r)};
+                 __builtin_amdgcn_readlane(mine.rows, r), __builtin_amdgcn_readlane(mine.n0, r),
+                 __builtin_amdgcn_readlane(mine.alone, r)};
 }
 
 // The workgroup's `nr` (>= 1) tiles, one after the other.  mine: lane r holds tile r.
@@ -164,9 +179,11 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
   // 1024 (8 j + wave) of the operand's part of the stage: eight 128-byte rows, or 1024 / (2 BN) K rows of a [K][N] tile.
   const half_t *a_src[C::A_DMA], *b_src[C::B_DMA];
   int it = 0, ik = 0;
+  bool stream = false;                                             // the weights being loaded are read once
   const size_t b_step = kKN ? static_cast<size_t>(kBK) * p.N : kBK;
   auto sources = [&](const FewTile &t) {
     const half_t *Be = p.B + static_cast<size_t>(t.e) * p.N * p.K;
+    stream = p.stream && t.alone;
 #pragma unroll
     for (int j = 0; j < C::A_DMA; ++j) {
       const int r = (j * 8 + wave) * 8 + (lane >> 3);
@@ -192,8 +209,13 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
     lds_char *base = lds + stage * C::STAGE;
 #pragma unroll
     for (int j = 0; j < C::A_DMA; ++j) lds_dma16(a_src[j], base + (j * 8 + wave) * 1024);
+    if (stream) {
 #pragma unroll
-    for (int j = 0; j < C::B_DMA; ++j) lds_dma16(b_src[j], base + C::A_BYTES + (j * 8 + wave) * 1024);
+      for (int j = 0; j < C::B_DMA; ++j) lds_dma16_nt(b_src[j], base + C::A_BYTES + (j * 8 + wave) * 1024);
+    } else {
+#pragma unroll
+      for (int j = 0; j < C::B_DMA; ++j) lds_dma16(b_src[j], base + C::A_BYTES + (j * 8 + wave) * 1024);
+    }
     if (ik + 1 < KT) {
       ++ik;
 #pragma unroll
@@ -377,6 +399,7 @@ few_rows_kernel(FewArgs p) {
     mine.row0 = s_off[lo] + r0;
     mine.rows = cnt - r0 < bm ? cnt - r0 : bm;
     mine.n0 = ct << (6 + cs);
+    mine.alone = mts == 1;
   }
   __syncthreads();                                                  // the tables have been read
   lds_char *lds = (lds_char *)buf;
@@ -499,6 +522,7 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
 int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {
   if (thin_rows_fits(mode, p.max_rows, p.E, p.N, p.K, epi, b_kn)) return thin_rows_gemm(p, epi, stream, what);
   p.force = mode >= 16 ? mode & 15 : -1;
+  p.stream = 2.0 * (p.E < p.max_rows ? p.E : p.max_rows) * p.N * p.K >= kStreamBytes;
   void (*kernel)(FewArgs) = b_kn ? (epi == kFewPlain ? few_rows_kernel<kFewPlain, true> : few_rows_kernel<kFewGelu, true>)
                                  : (epi == kFewPlain ? few_rows_kernel<kFewPlain, false>
                                                      : (epi == kFewGelu ? few_rows_kernel<kFewGelu, false> : few_rows_kernel<kFewGeluKeep, false>));

@@ -1076,3 +1076,37 @@ def test_gate_hooks_run_where_the_routing_goes_with_the_gate():
     n = int(infos0["offsets"][-1])
     for pos, score, infos in ((pos1, score1, infos1), (pos2, score2, infos2)):
         assert torch.equal(pos[:n], pos0[:n]) and torch.equal(score, score0) and torch.equal(infos["inv_pos"], infos0["inv_pos"])
+
+
+@pytest.mark.parametrize("kn", [False, True])
+@pytest.mark.parametrize("counts", [[64, 1], [60, 200], [0, 128]])
+def test_few_rows_of_large_weights(counts, kn):
+    """Weights large enough for non-temporal loads, an expert of one M tile beside none, another or one of several: the
+    bits of the 256-row tiles."""
+    from ccfuser_amd import ops
+    E, d, f = 2, 4096, 10304                                # 169 MB each way, a last column tile that is not full
+    R = sum(counts)
+    _say(f"few rows of large weights {counts} kn={kn}")
+    g = torch.Generator(device="cuda").manual_seed(R)
+    rnd = lambda *s: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, 0.05, generator=g)
+    off = torch.tensor([0, counts[0], R], dtype=torch.int32, device="cuda")
+    x, h = rnd(R, d), rnd(R, f)
+    w1, w2 = (rnd(E, d, f), rnd(E, f, d)) if kn else (rnd(E, f, d), rnd(E, d, f))
+    b1, b2 = rnd(E, f), rnd(E, d)
+    rows = torch.randperm(R, generator=torch.Generator().manual_seed(R)).int().cuda()
+
+    def both():
+        y = torch.zeros(R, d, dtype=torch.float16, device="cuda")
+        return ops.ffn1(x, rows, off, R, w1, b1, w_kn=kn), ops.ffn2(h, rows, off, R, w2, b2, y, w_kn=kn)
+
+    ops.set_option("few_rows", 2)
+    try:
+        got = both()
+        for name, value in (("few_rows", 0), ("split_tail", 0), ("skinny", 0)):
+            ops.set_option(name, value)
+        ref = both()
+    finally:
+        for name, value in (("few_rows", 1), ("split_tail", 1), ("skinny", 1)):
+            ops.set_option(name, value)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
