@@ -259,9 +259,16 @@ extern "C" int ccf_gate_route(const void *x, const void *wg, const void *bg, int
     return gate_route_tiny(x, wg, bg, tokens, d_model, num_expert, top_k, capacity, idx, score, counts, offsets, pos, src_row,
                            dst_row, inv_pos, idx_kept, as_stream(stream));
   int gate_tokens = 0;
-  const bool pow2_k = (top_k & (top_k - 1)) == 0;     // a workgroup's flat indices tile the routing's chunks
+  // Counts from the gate where the routing would launch a count of its own or count two chunks of 1024 indices, and where
+  // adding them up is no longer than that: a table of at most 8192 of them, or one per index (443 tokens, top-2, 64 experts
+  // of 256, with the gate's counts and without: 22.8 and 20.0 us; 700: 23.4 and 23.5; 2000 in fp32, a table of 16000: 31.6
+  // and 29.6; 8192 of 2048, 64 experts, a table of 16384: 55.7 and 58.9).  top_k a power of two: a workgroup's flat indices
+  // tile the routing's chunks.
+  const bool counted = (top_k & (top_k - 1)) == 0 && n > 1024;
+  const long long most = n > 8192 ? n : 8192;
   if (int rc = gate_forward(x, wg, bg, tokens, d_model, num_expert, top_k, dtype, idx, score, nullptr, stream,
-                            pow2_k ? static_cast<int32_t *>(workspace) : nullptr, route_rows_max_ints(), &gate_tokens))
+                            counted ? static_cast<int32_t *>(workspace) : nullptr,
+                            most < route_rows_max_ints() ? most : route_rows_max_ints(), &gate_tokens))
     return rc;
   return route_with_plans(idx, n, num_expert, top_k, capacity, counts, offsets, pos, src_row, dst_row, inv_pos, idx_kept,
                           workspace, workspace_bytes, as_stream(stream), nullptr, 0, gate_tokens * top_k);
