@@ -149,7 +149,7 @@ __device__ __forceinline__ FewTile tile_at(const FewTile &mine, int r) {
 }
 
 // The workgroup's `nr` (>= 1) tiles, one after the other.  mine: lane r holds tile r.
-template <class C, int kEpi, bool kKN>
+template <class C, int kEpi, bool kKN, bool kStream>
 __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, int nr, lds_char *lds) {
   constexpr int TMW = C::TMW, NB = C::NB, S = C::STAGES;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -183,7 +183,7 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
   const size_t b_step = kKN ? static_cast<size_t>(kBK) * p.N : kBK;
   auto sources = [&](const FewTile &t) {
     const half_t *Be = p.B + static_cast<size_t>(t.e) * p.N * p.K;
-    stream = p.stream && t.alone;
+    stream = kStream && t.alone;
 #pragma unroll
     for (int j = 0; j < C::A_DMA; ++j) {
       const int r = (j * 8 + wave) * 8 + (lane >> 3);
@@ -209,7 +209,7 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
     lds_char *base = lds + stage * C::STAGE;
 #pragma unroll
     for (int j = 0; j < C::A_DMA; ++j) lds_dma16(a_src[j], base + (j * 8 + wave) * 1024);
-    if (stream) {
+    if (kStream && stream) {
 #pragma unroll
       for (int j = 0; j < C::B_DMA; ++j) lds_dma16_nt(b_src[j], base + C::A_BYTES + (j * 8 + wave) * 1024);
     } else {
@@ -304,7 +304,9 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
 // Candidate tile shapes: index = 3 * (rows: 0 = 64, 1 = 128) + (columns: 0 = 64, 1 = 128, 2 = 256).
 constexpr int kFewShapes = 6;
 
-template <int kEpi, bool kKN>
+// kStream: the weights are large (a form of its own: the choice by tile in the loads of small ones cost 0.4 us of 36, two
+// short launches of more code)
+template <int kEpi, bool kKN, bool kStream>
 __global__ void __launch_bounds__(kFewThreads)
 few_rows_kernel(FewArgs p) {
   __shared__ __attribute__((aligned(1024))) char buf[kFewLds];
@@ -406,7 +408,7 @@ few_rows_kernel(FewArgs p) {
   auto go = [&](auto CI) {
     constexpr int i = CI.value;
     if constexpr (!kKN || i % 3 > 0)
-      if (shape == i) few_run<FewCfg<4 << (i / 3), 2 << (i % 3)>, kEpi, kKN>(p, mine, nr, lds);
+      if (shape == i) few_run<FewCfg<4 << (i / 3), 2 << (i % 3)>, kEpi, kKN, kStream>(p, mine, nr, lds);
   };
   static_for<0, kFewShapes>(go);
 }
@@ -522,10 +524,14 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
 int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {
   if (thin_rows_fits(mode, p.max_rows, p.E, p.N, p.K, epi, b_kn)) return thin_rows_gemm(p, epi, stream, what);
   p.force = mode >= 16 ? mode & 15 : -1;
-  p.stream = 2.0 * (p.E < p.max_rows ? p.E : p.max_rows) * p.N * p.K >= kStreamBytes;
-  void (*kernel)(FewArgs) = b_kn ? (epi == kFewPlain ? few_rows_kernel<kFewPlain, true> : few_rows_kernel<kFewGelu, true>)
-                                 : (epi == kFewPlain ? few_rows_kernel<kFewPlain, false>
-                                                     : (epi == kFewGelu ? few_rows_kernel<kFewGelu, false> : few_rows_kernel<kFewGeluKeep, false>));
+  const bool large = 2.0 * (p.E < p.max_rows ? p.E : p.max_rows) * p.N * p.K >= kStreamBytes;
+  const auto pick = [&](auto S_) -> void (*)(FewArgs) {
+    constexpr bool S = decltype(S_)::value;
+    if (b_kn) return epi == kFewPlain ? few_rows_kernel<kFewPlain, true, S> : few_rows_kernel<kFewGelu, true, S>;
+    return epi == kFewPlain ? few_rows_kernel<kFewPlain, false, S>
+                            : (epi == kFewGelu ? few_rows_kernel<kFewGelu, false, S> : few_rows_kernel<kFewGeluKeep, false, S>);
+  };
+  void (*kernel)(FewArgs) = large ? pick(std::true_type{}) : pick(std::false_type{});
   hipLaunchKernelGGL(kernel, dim3(cus), dim3(kFewThreads), 0, stream, p);
   return check_launch(what);
 }

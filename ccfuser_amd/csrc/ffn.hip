@@ -1398,7 +1398,7 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
   if (max_rows == 0) return CCF_OK;
   const GemmOptions options = opt ? *opt : current_options();
   if (use_few_rows(max_rows, E, N, K, epi, b_kn, options))
-    return few_rows_gemm(options.few_rows, FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1, false}, epi,
+    return few_rows_gemm(options.few_rows, FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1}, epi,
                          b_kn, persistent_grid(), stream, what);
   const GemmSetup gs = setup_gemm(max_rows, E, N, K, epi, b_kn, workspace, region, options);
   const Launch &v = *gs.v;

@@ -576,7 +576,6 @@ struct FewArgs {
   const int32_t *offsets;
   int max_rows, E, N, K;
   int force;                 // tile shape, or -1: chosen by the kernel; filled in by few_rows_gemm
-  bool stream;               // weights that one tile reads are loaded as non-temporal; filled in by few_rows_gemm
 };
 // thin.hip: at most 32 rows in all (the two epilogues without a kept pre-activation, [E, N, K] weights)
 bool thin_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn);
