@@ -174,7 +174,8 @@ class MixMOEFusedFFN(Function):
         input_buf, w1, w2, act, h_pre, src_row, dst_row, offsets, inv_pos = ctx.saved_tensors
         max_rows, n_flat, may_drop = ctx.sizes
         E = offsets.numel() - 1
-        if inv_pos is not None and n_flat == max_rows:
+        if inv_pos is not None and n_flat == max_rows and w1.shape[0] == w2.shape[0] and \
+                w1.is_contiguous() and w2.is_contiguous():          # else only their first experts may be
             grad_in, grad_w1, grad_b1, grad_w2, grad_b2 = ops.ffn_backward_pair(
                 grad_y.contiguous(), input_buf, act, h_pre, src_row, dst_row, inv_pos, offsets, w1.detach(), w2.detach())
             return grad_in, None, None, grad_w1, grad_b1, grad_w2, grad_b2

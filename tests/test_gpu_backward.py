@@ -479,3 +479,27 @@ def test_backward_of_both_layers_in_one_call(T, k, d, f, E, slots, capacity):
         tail = a[b.shape[0]:]
         assert torch.equal(a[:b.shape[0]], b), name
         assert torch.equal(tail, torch.zeros_like(tail)), name
+
+
+def test_backward_with_parameters_that_are_contiguous_only_as_slices():
+    """One expert of three slots that lie apart in memory: the layers' own calls on the slice, the gradients of the
+    contiguous parameter."""
+    from ccfuser_amd.mix_moe import MixMOETransformerMLP
+    d, f, T = 256, 512, 100
+    grads = []
+    for apart in (False, True):
+        torch.manual_seed(0)
+        with torch.device("cuda"):
+            mlp = MixMOETransformerMLP("naive", {"num_local_expert": 1, "hidden_size": f}, d, 0, 1, total_batch_size=T, top_k=1,
+                                       popular_expert_num=2).half()
+        if apart:
+            for lin in (mlp.experts.htoh4, mlp.experts.h4toh):
+                wide = torch.empty(3, 2, *lin.weight.shape[1:], dtype=torch.float16, device="cuda")
+                wide[:, 0] = lin.weight.detach()
+                lin.weight = torch.nn.Parameter(wide[:, 0])
+            assert not mlp.experts.htoh4.weight.is_contiguous()
+        x = torch.randn(T, d, dtype=torch.float16, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).requires_grad_(True)
+        mlp(x).backward(torch.ones(T, d, dtype=torch.float16, device="cuda"))
+        grads.append({"x": x.grad, **{n: p.grad[:1] for n, p in mlp.named_parameters() if n.startswith("experts")}})
+    for name, g in grads[0].items():
+        assert torch.equal(g, grads[1][name]), name
