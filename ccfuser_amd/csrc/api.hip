@@ -187,12 +187,10 @@ extern "C" int ccf_moe_forward(const void *x, const void *wg, const void *bg, co
   int rc;
   mark_stage(0, st);
   // the gate's selection threads also leave per-workgroup expert counts in the routing workspace when that
-  // table is small and a workgroup's flat indices tile the routing chunks (top_k a power of two): the
-  // routing stage is then one launch
+  // table is small and its rows tile the routing's chunks: the routing stage is then one launch
   int gate_tokens = 0;
-  const bool pow2_k = (top_k & (top_k - 1)) == 0;
   if ((rc = gate_forward(x, wg, bg, tokens, d_model, num_expert, top_k, CCF_F16, w.idx, w.score, nullptr, stream,
-                         pow2_k ? reinterpret_cast<int32_t *>(w.route_ws) : nullptr, route_rows_max_ints(), &gate_tokens)))
+                         reinterpret_cast<int32_t *>(w.route_ws), route_rows_max_ints(), &gate_tokens)))
     return rc;
   mark_stage(1, st);
   // the tile plans of both GEMMs are built by two more workgroups of the routing stage's last
@@ -262,9 +260,8 @@ extern "C" int ccf_gate_route(const void *x, const void *wg, const void *bg, int
   // Counts from the gate where the routing would launch a count of its own or count two chunks of 1024 indices, and where
   // adding them up is no longer than that: a table of at most 8192 of them, or one per index (443 tokens, top-2, 64 experts
   // of 256, with the gate's counts and without: 22.8 and 20.0 us; 700: 23.4 and 23.5; 2000 in fp32, a table of 16000: 31.6
-  // and 29.6; 8192 of 2048, 64 experts, a table of 16384: 55.7 and 58.9).  top_k a power of two: a workgroup's flat indices
-  // tile the routing's chunks.
-  const bool counted = (top_k & (top_k - 1)) == 0 && n > 1024;
+  // and 29.6; 8192 of 2048, 64 experts, a table of 16384: 55.7 and 58.9).
+  const bool counted = n > 1024;
   const long long most = n > 8192 ? n : 8192;
   if (int rc = gate_forward(x, wg, bg, tokens, d_model, num_expert, top_k, dtype, idx, score, nullptr, stream,
                             counted ? static_cast<int32_t *>(workspace) : nullptr,

@@ -56,6 +56,9 @@ int launch_bias_reduce(const float *partial, const int32_t *k_seg, int E, int C,
 int launch_combine(const half_t *y_flat, const half_t *score, const int32_t *inv_pos, half_t *out, int tokens, int top_k,
                    int hidden, hipStream_t stream);
 
+// Flat indices of a workgroup of the routing stage: rows of the gate's counts tile runs of that many.
+constexpr int kRouteChunk = 1024;
+
 // gate.hip
 int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int d_model, int tot_expert, int top_k,
                  int dtype, int64_t *idx_out, void *score_out, void *logits_out, ccf_stream_t stream,

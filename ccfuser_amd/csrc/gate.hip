@@ -122,6 +122,13 @@ __device__ inline void leave_counts(const Best<KS> &best, bool mine, int k, int 
   for (int e = threadIdx.x; e < E; e += blockDim.x) wg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = row[e];
 }
 
+// Whether a gate of `wgs` workgroups of `wg_tokens` tokens leaves them: the table fits, and its rows tile the routing's
+// chunks.  256 tokens of the stream form with eight experts each do not, nor does a top_k that is no power of two: the
+// routing counts for itself then.
+bool counts_fit(const int32_t *wg_cnt, long long wgs, int E, int wg_tokens, int k, long long max_cnt) {
+  return wg_cnt && wgs * E <= max_cnt && kRouteChunk % (wg_tokens * k) == 0;
+}
+
 // fp16 gate.  An MFMA has 64 / N blocks; with S = 1 << LS slots, block b of a wavefront is
 // token block b / S on slot b % S, so a wavefront covers TW = (64 / N / S) * N tokens and
 // S parts of K at a time, and the wavefronts of a workgroup (all on the same TW tokens)
@@ -765,7 +772,7 @@ int launch_gate_f32(const float *x, const float *wg, const float *bg, int tokens
     if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate: LDS attribute: %s", hipGetErrorString(e));
   }
   const int wgs = (tokens + C::WT - 1) / C::WT;
-  if (static_cast<long long>(wgs) * E > max_cnt) wg_cnt = nullptr;
+  if (!counts_fit(wg_cnt, wgs, E, C::WT, k, max_cnt)) wg_cnt = nullptr;
   if (wg_cnt && tokens_per_wg) *tokens_per_wg = C::WT;
   hipLaunchKernelGGL(kern, dim3(wgs), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
                      idx_out, score_out, logits_out, wg_cnt);
@@ -960,7 +967,7 @@ int launch_gate_f32_mfma(const float *x, const float *wg, const float *bg, int t
     if (e != hipSuccess) return fail(CCF_ERR_HIP, "gate: LDS attribute: %s", hipGetErrorString(e));
   }
   const int wgs = (tokens + C::WT - 1) / C::WT;
-  if (static_cast<long long>(wgs) * E > max_cnt) wg_cnt = nullptr;
+  if (!counts_fit(wg_cnt, wgs, E, C::WT, k, max_cnt)) wg_cnt = nullptr;
   if (wg_cnt && tokens_per_wg) *tokens_per_wg = C::WT;
   hipLaunchKernelGGL(kern, dim3(wgs), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
                      idx_out, score_out, logits_out, wg_cnt);
@@ -1236,7 +1243,7 @@ int launch_gate_walk(const half_t *x, const half_t *wg, const half_t *bg, int to
   const int threads = chains * group > 256 ? 512 : 256;
   const int wg_tokens = route.counts ? (tokens + group - 1) / group * group : group;
   const int wgs = (tokens + wg_tokens - 1) / wg_tokens;
-  if (static_cast<long long>(wgs) * E > max_cnt) wg_cnt = nullptr;
+  if (!counts_fit(wg_cnt, wgs, E, wg_tokens, k, max_cnt)) wg_cnt = nullptr;
   if (wg_cnt && tokens_per_wg) *tokens_per_wg = wg_tokens;
   const int lds = walk_lds(E, nparts, group).bytes;
   auto kern = k == 1 ? gate_walk_kernel<1> : (k == 2 ? gate_walk_kernel<2> : gate_walk_kernel<kMaxTopK>);
@@ -1275,7 +1282,8 @@ int gate_route_tiny(const void *x, const void *wg, const void *bg, int tokens, i
 
 // The gate; with wg_cnt (room for max_cnt ints) the tiled kernels also leave, per workgroup, how many of
 // its token slots chose each expert ([workgroups][tot_expert], a workgroup covering *tokens_per_wg
-// consecutive tokens), when that table fits; *tokens_per_wg = 0 says it was not written.
+// consecutive tokens), when that table is one that the routing can use (counts_fit); *tokens_per_wg = 0 says
+// it was not written.
 int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int d_model, int tot_expert, int top_k,
                  int dtype, int64_t *idx_out, void *score_out, void *logits_out, ccf_stream_t stream,
                  int32_t *wg_cnt, long long max_cnt, int *tokens_per_wg) {
@@ -1348,7 +1356,7 @@ int gate_forward(const void *x, const void *wg, const void *bg, int tokens, int 
                                       (stream_form ? 0 : static_cast<size_t>(tw) * (n + 1)));
   CCF_REQUIRE(lds <= 160 * 1024, CCF_ERR_SHAPE, "gate: %zu bytes of LDS needed", lds);
   dim3 grid((tokens + wg_tokens - 1) / wg_tokens), block(waves * 64);
-  if (wg_cnt && static_cast<long long>(grid.x) * tot_expert <= max_cnt) {
+  if (counts_fit(wg_cnt, grid.x, tot_expert, wg_tokens, top_k, max_cnt)) {
     if (tokens_per_wg) *tokens_per_wg = wg_tokens;
   } else {
     wg_cnt = nullptr;

@@ -40,8 +40,8 @@ int g_route_rows_max = 16384;   // largest table of counts (entries) that the po
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPasses = 4;                       // indices per thread
-constexpr int kChunk = kThreads * kPasses;       // flat indices per workgroup
+constexpr int kChunk = kRouteChunk;              // flat indices per workgroup
+constexpr int kPasses = kChunk / kThreads;       // indices per thread
 constexpr int kSub = kPasses * (kThreads / 64);  // wavefront passes per chunk
 constexpr int kMaxExpert = 1024;
 // Most chunks whose indices every workgroup of the pos launch counts itself instead of a hist launch in front of it.

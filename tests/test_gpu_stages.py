@@ -1046,6 +1046,28 @@ def test_gate_with_routing_is_the_gate_then_the_routing(T, d, E, k, capacity, dt
         assert torch.equal(r[name][:n], r0[name][:n]), name
 
 
+@pytest.mark.parametrize("T,E,k", [(65536, 32, 8), (65537, 17, 8), (131075, 8, 8), (65536, 32, 4), (65536, 20, 5)])
+def test_gate_workgroups_of_more_indices_than_a_routing_chunk(T, E, k):
+    """Gate workgroups of 256 tokens: eight experts each are 2048 indices, twice a chunk of the routing, which then counts
+    for itself; four fill a chunk.  Gate with routing and the layer call against the gate, then the routing."""
+    from ccfuser_amd import ops
+    _say(f"gate rows longer than a chunk T={T} E={E} k={k}")
+    d = f = 64
+    g = torch.Generator(device="cuda").manual_seed(T + k)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device="cuda") * 0.1).half()
+    x, wg, bg = rnd(T, d), rnd(E, d), rnd(E)
+    idx0, score0 = ops.gate_topk_softmax(x, wg, bg, k)
+    r0 = ops.route(idx0.reshape(-1), E, k)
+    idx, score, r = ops.gate_route(x, wg, bg, k)
+    assert torch.equal(idx, idx0) and torch.equal(score, score0)
+    for name in ("counts", "offsets", "pos", "src_row", "dst_row", "inv_pos", "idx_kept"):
+        assert torch.equal(r[name], r0[name]), name
+    _, m = ops.moe_forward(x, wg, bg, rnd(E, f, d), rnd(E, f), rnd(E, d, f), rnd(E, d), k, return_routing=True)
+    for name in ("counts", "offsets", "pos"):
+        assert torch.equal(m[name], r0[name]), name
+    assert torch.equal(m["idx"].view(-1), idx0.view(-1)) and torch.equal(m["score"].view(-1), score0.view(-1))
+
+
 def test_gate_hooks_run_where_the_routing_goes_with_the_gate():
     """A gate with a hook, a subclass and another number of experts are called as modules, the gate itself is not."""
     from ccfuser_amd.mix_moe.gates import NaiveGate
