@@ -631,8 +631,9 @@ def moe_forward(x, wg, bg, w1, b1, w2, b2, top_k: int, capacity: int = -1,
     _check_expert(w2, b2, "ffn2")
     T, d = x.shape
     slots, f, d1 = w1.shape
-    E = wg.shape[0] if spare_experts and wg.shape[0] < slots else slots
-    if d1 != d or tuple(w2.shape) != (slots, d, f) or tuple(wg.shape) != (E, d):
+    E = wg.shape[0] if spare_experts else slots
+    fits = min(slots, w2.shape[0]) >= E if spare_experts else w2.shape[0] == E      # either weight may have its own spares
+    if d1 != d or not fits or tuple(w2.shape[1:]) != (d, f) or tuple(wg.shape) != (E, d):
         raise ValueError("moe_forward: weight shapes do not match (one GPU: the gate scores the local experts)")
     dev = x.device
     out = torch.empty(T, d, dtype=x.dtype, device=dev)

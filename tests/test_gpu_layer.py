@@ -874,3 +874,31 @@ def test_weights_of_more_experts_than_the_gate_scores(slots):
         wide[:, 0] = lin.weight
         lin.weight = torch.nn.Parameter(wide[:, 0], requires_grad=False)
     assert not mlp.experts.htoh4.weight.is_contiguous() and torch.equal(mlp(x), ref)
+
+
+@pytest.mark.parametrize("which", ["weight_slots", "bias_slots", "one_apart"])
+def test_spare_experts_of_one_layer_only(which):
+    """Expert parameters of a module whose two layers hold different numbers of spare experts, whose bias has none, or
+    of which only one layer's is contiguous as a whole: the bits of the module as it was made."""
+    from ccfuser_amd.mix_moe import MixMOETransformerMLP
+    E, d, f, T = (1 if which == "one_apart" else 4), 128, 256, 300
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        mlp = MixMOETransformerMLP("naive", {"num_local_expert": E, "hidden_size": f}, d, 0, 1, total_batch_size=T, top_k=1,
+                                   popular_expert_num=2).half().requires_grad_(False)
+    x = torch.randn(T, d, dtype=torch.float16, device="cuda")
+    ref = mlp(x)
+    frozen = lambda t: torch.nn.Parameter(t, requires_grad=False)
+    lin = mlp.experts.h4toh
+    if which == "one_apart":
+        wide = torch.empty(3, 2, *lin.weight.shape[1:], dtype=torch.float16, device="cuda")
+        wide[:, 0] = lin.weight
+        lin.weight = frozen(wide[:, 0])
+        assert not lin.weight.is_contiguous()
+    else:
+        lin.bias = frozen(lin.bias[:E].clone())
+        if which == "weight_slots":
+            lin.weight = frozen(lin.weight[:E].clone())
+    assert torch.equal(mlp(x), ref)
+    mlp.fused = False
+    assert torch.equal(mlp(x), ref)
