@@ -153,7 +153,7 @@ class AsyncExpertAssignment:
         ``pos`` has tokens*top_k entries; the first ``offsets[-1]`` are valid."""
         if world_size != 1:
             raise NotImplementedError("single-GPU build: world_size must be 1")
-        if isinstance(gate, NaiveGate) and num_expert == gate.tot_expert and gate.calls_forward_only():
+        if isinstance(gate, NaiveGate) and gate.calls_forward_only() and gate.gate.weight.shape[0] == num_expert:
             _, gate_score, r = gate.forward_with_routing(attn_inp, self.capacity)
         else:
             gate_top_k_idx, gate_score = gate(attn_inp)

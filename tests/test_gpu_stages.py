@@ -1100,6 +1100,26 @@ def test_gate_hooks_run_where_the_routing_goes_with_the_gate():
         assert torch.equal(pos[:n], pos0[:n]) and torch.equal(score, score0) and torch.equal(infos["inv_pos"], infos0["inv_pos"])
 
 
+@pytest.mark.parametrize("scored", [3, 6])
+def test_gate_that_scores_another_number_of_experts_is_called_as_a_module(scored):
+    """A router whose linear layer was replaced: the routing goes over the caller's experts, and a choice beyond them is
+    nobody's."""
+    from ccfuser_amd import ops
+    from ccfuser_amd.mix_moe.gates import NaiveGate
+    from ccfuser_amd.mix_moe.transformer import AsyncExpertAssignment
+    with torch.device("cuda"):
+        gate = NaiveGate(64, 4, 1, 2).half()
+        gate.gate = torch.nn.Linear(64, scored).half()
+    x = torch.randn(500, 64, dtype=torch.float16, device="cuda")
+    pos, score, infos = AsyncExpertAssignment(0, 1, 0, 4, 500).process_data(gate, x, 4, 1)
+    idx, score0 = gate(x)
+    r = ops.route(idx.reshape(-1), 4, 2)
+    n = int(r["offsets"][-1])
+    assert torch.equal(score, score0) and torch.equal(pos[:n], r["pos"][:n])
+    for name in ("counts", "offsets", "inv_pos", "idx_kept"):
+        assert torch.equal(infos[name], r[name]), name
+
+
 @pytest.mark.parametrize("kn", [False, True])
 @pytest.mark.parametrize("counts", [[64, 1], [60, 200], [0, 128]])
 def test_few_rows_of_large_weights(counts, kn):
