@@ -63,6 +63,8 @@ SIGNATURES = {
     "ccf_moe_ffn_blocks": (_i, [_p, _i, _p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _i, _p, _i, _p, _p, _i, _p, _p, _p, _sz, _p]),
     "ccf_ffn1_forward_kn": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _i, _p, _p, _sz, _p]),
     "ccf_ffn2_forward_kn": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _p, _sz, _p]),
+    "ccf_ffn1_forward_opts": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _i, _i, _p, _p, _sz, _p]),
+    "ccf_ffn2_forward_opts": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _p, _i, _p, _p, _sz, _p]),
 }
 
 

@@ -125,12 +125,15 @@ __device__ __forceinline__ int few_kn_swz(int row) { return (row & 3) | (((row >
 
 // lds_dma16 with the non-temporal hint, for weights that one tile reads once: 6.2 TB/s from HBM instead of 5.5.  Weights
 // that several M tiles share, or that a next call finds in the 256 MB Infinity Cache, do better without: the hint is for a
-// tile that has its expert to itself, in a GEMM of 160 MB of weights and more (a layer's two are 320 then).  Microseconds
-// of FFN1 / FFN2, without and with it, six layers one after the other: 8 experts of 4096 / 14336, 83 rows each 184, 184
-// and 176, 167; 16 of 2048 / 8192, 100 rows 140, 134 and 138, 119; 8 of 2560 / 8960, 100 rows 113, 101 and 108, 96; one
-// layer of 8 of 2048 / 8192 again and again 47, 47 and 66, 54 (its FFN1 alone, 268 MB; in a layer nothing is found again).
+// tile that has its expert to itself where 320 MB pass before its weights are read again.  The kernel counts the experts
+// that have rows; a layer's two products alternate, so each is half of that.  Microseconds without and with the hint:
+//   a layer's two, again and again, 4 to 83 rows per expert: 8 experts with rows of 2304 / 8192 (302 MB each way) 124, 113;
+//     of 4096 / 14336 334, 309; 16 of 2048 / 8192 245, 229; 4 of 2560 / 8192 (168 MB each) 78, 74, of 2304 / 8192 (151)
+//     69, 69, of 2048 / 8192 (134) 62, 73; 2 of 4096 / 14336 (235) 141, 135, 1 of them (117) 85, 102
+//   FFN1 alone: 8 of 2048 / 8192 (268 MB) 47, 66, of 2304 / 8192 (302) 51, 52, of 2560 / 8192 (336) 61, 57; 2 of 4096 /
+//     14336 (235) 40, 54, 4 of them (470) 111, 105
 // A layer of 128 tokens, 8 experts of 4096 / 14336: 356 -> 333 us.
-constexpr double kStreamBytes = 160e6;
+constexpr double kStreamBytes = 320e6;
 __device__ __forceinline__ void lds_dma16_nt(const void *gptr, lds_char *lds_wave_base) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)gptr,
                                    (__attribute__((address_space(3))) void *)lds_wave_base, 16, 0, 2);
@@ -321,11 +324,13 @@ few_rows_kernel(FewArgs p) {
   __syncthreads();
   // M tiles of each height over all experts (every wavefront for itself)
   int m64 = 0, m128 = 0;
-  for (int e = lane; e < E; e += 64) {
-    int cnt = s_off[e + 1] - s_off[e];
+  int used = 0;                                                     // experts with rows
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    int cnt = e0 + lane < E ? s_off[e0 + lane + 1] - s_off[e0 + lane] : 0;
     cnt = cnt > 0 ? cnt : 0;
     m64 += (cnt + 63) >> 6;
     m128 += (cnt + 127) >> 7;
+    if constexpr (kStream) used += __popcll(__ballot(cnt > 0));
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
@@ -408,7 +413,12 @@ few_rows_kernel(FewArgs p) {
   auto go = [&](auto CI) {
     constexpr int i = CI.value;
     if constexpr (!kKN || i % 3 > 0)
-      if (shape == i) few_run<FewCfg<4 << (i / 3), 2 << (i % 3)>, kEpi, kKN, kStream>(p, mine, nr, lds);
+      if (shape == i) {
+        // two loops, not one that chooses: FFN2 of 64 rows of one of 16 experts of 2048 / 8192 takes 40 us, 46 with the
+        // choice at every load (42 with the hint, 38 in the form of small weights)
+        if (kStream && used >= p.stream_experts) few_run<FewCfg<4 << (i / 3), 2 << (i % 3)>, kEpi, kKN, kStream>(p, mine, nr, lds);
+        else few_run<FewCfg<4 << (i / 3), 2 << (i % 3)>, kEpi, kKN, false>(p, mine, nr, lds);
+      }
   };
   static_for<0, kFewShapes>(go);
 }
@@ -521,10 +531,12 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
   return mine < 1.02 * big;
 }
 
-int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what) {
+int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, bool in_layer, int cus, hipStream_t stream, const char *what) {
   if (thin_rows_fits(mode, p.max_rows, p.E, p.N, p.K, epi, b_kn)) return thin_rows_gemm(p, epi, stream, what);
   p.force = mode >= 16 ? mode & 15 : -1;
-  const bool large = 2.0 * (p.E < p.max_rows ? p.E : p.max_rows) * p.N * p.K >= kStreamBytes;
+  const double experts = std::ceil((in_layer ? kStreamBytes / 2 : kStreamBytes) / (2.0 * p.N * p.K));
+  const bool large = experts <= (p.E < p.max_rows ? p.E : p.max_rows);
+  p.stream_experts = large ? static_cast<int>(experts) : INT_MAX;
   const auto pick = [&](auto S_) -> void (*)(FewArgs) {
     constexpr bool S = decltype(S_)::value;
     if (b_kn) return epi == kFewPlain ? few_rows_kernel<kFewPlain, true, S> : few_rows_kernel<kFewGelu, true, S>;

@@ -1374,7 +1374,8 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
                  int N, int K, const half_t *B, const half_t *bias, int epi, half_t *C,
                  const int32_t *c_rows, const half_t *row_scale, void *workspace, hipStream_t stream,
                  const char *what, bool b_kn = false, half_t *C2 = nullptr, int region = 0,
-                 bool plan_ready = false, const GemmOptions *opt = nullptr, const int32_t *scale_rows = nullptr) {
+                 bool plan_ready = false, const GemmOptions *opt = nullptr, const int32_t *scale_rows = nullptr,
+                 bool in_layer = true) {
   CCF_REQUIRE(A && offsets && B && C && workspace, CCF_ERR_ARG, "%s: null pointer", what);
   const bool gelu = epi != kEpiPlain && epi != kEpiCombine;
   CCF_REQUIRE(epi >= kEpiPlain && epi <= kEpiCombine &&
@@ -1398,8 +1399,8 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
   if (max_rows == 0) return CCF_OK;
   const GemmOptions options = opt ? *opt : current_options();
   if (use_few_rows(max_rows, E, N, K, epi, b_kn, options))
-    return few_rows_gemm(options.few_rows, FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1}, epi,
-                         b_kn, persistent_grid(), stream, what);
+    return few_rows_gemm(options.few_rows, FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1, 0}, epi,
+                         b_kn, in_layer, persistent_grid(), stream, what);
   const GemmSetup gs = setup_gemm(max_rows, E, N, K, epi, b_kn, workspace, region, options);
   const Launch &v = *gs.v;
   const bool second = gs.second, split = gs.split;
@@ -1883,7 +1884,7 @@ bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *wo
 int ffn1_forward(const void *x, const int32_t *src_row, const int32_t *dst_row, const int32_t *offsets,
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w1, const void *b1,
                  int apply_gelu, void *h, void *workspace, size_t workspace_bytes, hipStream_t stream,
-                 const GemmOptions *planned, bool w_kn) {
+                 const GemmOptions *planned, bool w_kn, bool in_layer) {
   const bool plan_ready = planned != nullptr;
   const size_t need = ccf_ffn_workspace_bytes(max_rows, num_expert, d_model, d_ffn);
   CCF_REQUIRE(workspace && workspace_bytes >= need, CCF_ERR_WORKSPACE,
@@ -1891,13 +1892,13 @@ int ffn1_forward(const void *x, const int32_t *src_row, const int32_t *dst_row, 
   return grouped_gemm(static_cast<const half_t *>(x), src_row, offsets, max_rows, num_expert, d_ffn,
                       d_model, static_cast<const half_t *>(w1), static_cast<const half_t *>(b1),
                       apply_gelu != 0 ? kEpiGelu : kEpiPlain, static_cast<half_t *>(h), dst_row, nullptr,
-                      workspace, stream, "ffn1", w_kn, nullptr, 0, plan_ready && apply_gelu != 0, planned);
+                      workspace, stream, "ffn1", w_kn, nullptr, 0, plan_ready && apply_gelu != 0, planned, nullptr, in_layer);
 }
 
 int ffn2_forward(const void *h, const int32_t *src_row, const int32_t *dst_row, const int32_t *offsets,
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w2, const void *b2,
                  const void *row_scale, void *y, void *workspace, size_t workspace_bytes,
-                 hipStream_t stream, const GemmOptions *planned, bool w_kn) {
+                 hipStream_t stream, const GemmOptions *planned, bool w_kn, bool in_layer) {
   const bool plan_ready = planned != nullptr;
   const size_t need = ccf_ffn_workspace_bytes(max_rows, num_expert, d_model, d_ffn);
   CCF_REQUIRE(workspace && workspace_bytes >= need, CCF_ERR_WORKSPACE,
@@ -1905,7 +1906,7 @@ int ffn2_forward(const void *h, const int32_t *src_row, const int32_t *dst_row, 
   return grouped_gemm(static_cast<const half_t *>(h), src_row, offsets, max_rows, num_expert, d_model,
                       d_ffn, static_cast<const half_t *>(w2), static_cast<const half_t *>(b2), kEpiPlain,
                       static_cast<half_t *>(y), dst_row, static_cast<const half_t *>(row_scale),
-                      workspace, stream, "ffn2", w_kn, nullptr, 1, plan_ready, planned);
+                      workspace, stream, "ffn2", w_kn, nullptr, 1, plan_ready, planned, nullptr, in_layer);
 }
 
 // FFN2 with the combine in its epilogue: out[token_row[j]] += (h[j] * w2[e]^T + b2[e]) * score[flat_row[j]].
@@ -1925,12 +1926,32 @@ int ffn2_forward_combine(const void *h, const int32_t *token_row, const int32_t 
 
 }  // namespace ccf
 
+extern "C" int ccf_ffn1_forward_opts(const void *x, const int32_t *src_row, const int32_t *dst_row,
+                                     const int32_t *offsets, int max_rows, int num_expert, int d_model,
+                                     int d_ffn, const void *w1, const void *b1, int apply_gelu, int opts, void *h,
+                                     void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
+  using namespace ccf;
+  CCF_REQUIRE(!(opts & ~(CCF_FFN_KN | CCF_FFN_IN_LAYER)), CCF_ERR_ARG, "ffn1: options %d", opts);
+  return ffn1_forward(x, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w1, b1, apply_gelu, h, workspace,
+                      workspace_bytes, as_stream(stream), nullptr, (opts & CCF_FFN_KN) != 0, (opts & CCF_FFN_IN_LAYER) != 0);
+}
+
+extern "C" int ccf_ffn2_forward_opts(const void *h, const int32_t *src_row, const int32_t *dst_row,
+                                     const int32_t *offsets, int max_rows, int num_expert, int d_model,
+                                     int d_ffn, const void *w2, const void *b2, const void *row_scale, int opts,
+                                     void *y, void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
+  using namespace ccf;
+  CCF_REQUIRE(!(opts & ~(CCF_FFN_KN | CCF_FFN_IN_LAYER)), CCF_ERR_ARG, "ffn2: options %d", opts);
+  return ffn2_forward(h, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w2, b2, row_scale, y, workspace,
+                      workspace_bytes, as_stream(stream), nullptr, (opts & CCF_FFN_KN) != 0, (opts & CCF_FFN_IN_LAYER) != 0);
+}
+
 extern "C" int ccf_ffn1_forward(const void *x, const int32_t *src_row, const int32_t *dst_row,
                                 const int32_t *offsets, int max_rows, int num_expert, int d_model,
                                 int d_ffn, const void *w1, const void *b1, int apply_gelu, void *h,
                                 void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
-  return ccf::ffn1_forward(x, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w1, b1,
-                           apply_gelu, h, workspace, workspace_bytes, ccf::as_stream(stream), nullptr);
+  return ccf_ffn1_forward_opts(x, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w1, b1, apply_gelu, 0, h,
+                               workspace, workspace_bytes, stream);
 }
 
 extern "C" int ccf_ffn2_forward(const void *h, const int32_t *src_row, const int32_t *dst_row,
@@ -1938,8 +1959,8 @@ extern "C" int ccf_ffn2_forward(const void *h, const int32_t *src_row, const int
                                 int d_ffn, const void *w2, const void *b2, const void *row_scale,
                                 void *y, void *workspace, size_t workspace_bytes,
                                 ccf_stream_t stream) {
-  return ccf::ffn2_forward(h, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w2, b2,
-                           row_scale, y, workspace, workspace_bytes, ccf::as_stream(stream), nullptr);
+  return ccf_ffn2_forward_opts(h, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w2, b2, row_scale, 0, y,
+                               workspace, workspace_bytes, stream);
 }
 
 // The same on weights stored [E, K, N], as the reference hands them to its extension (linear.py:74, 129).
@@ -1947,17 +1968,16 @@ extern "C" int ccf_ffn1_forward_kn(const void *x, const int32_t *src_row, const 
                                    const int32_t *offsets, int max_rows, int num_expert, int d_model,
                                    int d_ffn, const void *w1, const void *b1, int apply_gelu, void *h,
                                    void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
-  return ccf::ffn1_forward(x, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w1, b1,
-                           apply_gelu, h, workspace, workspace_bytes, ccf::as_stream(stream), nullptr, true);
+  return ccf_ffn1_forward_opts(x, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w1, b1, apply_gelu,
+                               CCF_FFN_KN, h, workspace, workspace_bytes, stream);
 }
 
 extern "C" int ccf_ffn2_forward_kn(const void *h, const int32_t *src_row, const int32_t *dst_row,
                                    const int32_t *offsets, int max_rows, int num_expert, int d_model,
                                    int d_ffn, const void *w2, const void *b2, const void *row_scale,
-                                   void *y, void *workspace, size_t workspace_bytes,
-                                   ccf_stream_t stream) {
-  return ccf::ffn2_forward(h, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w2, b2,
-                           row_scale, y, workspace, workspace_bytes, ccf::as_stream(stream), nullptr, true);
+                                   void *y, void *workspace, size_t workspace_bytes, ccf_stream_t stream) {
+  return ccf_ffn2_forward_opts(h, src_row, dst_row, offsets, max_rows, num_expert, d_model, d_ffn, w2, b2, row_scale,
+                               CCF_FFN_KN, y, workspace, workspace_bytes, stream);
 }
 
 extern "C" int ccf_ffn_plan_info(const void *workspace, int max_rows, int num_expert, int d_model, int d_ffn,

@@ -510,11 +510,11 @@ int ffn1_forward(const void *x, const int32_t *src_row, const int32_t *dst_row, 
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w1, const void *b1,
                  int apply_gelu, void *h, void *workspace, size_t workspace_bytes, hipStream_t stream,
                  const GemmOptions *planned,    // planned: the options the plan in the workspace was built under, or NULL
-                 bool w_kn = false);
+                 bool w_kn = false, bool in_layer = true);     // in_layer: see few_rows_gemm
 int ffn2_forward(const void *h, const int32_t *src_row, const int32_t *dst_row, const int32_t *offsets,
                  int max_rows, int num_expert, int d_model, int d_ffn, const void *w2, const void *b2,
                  const void *row_scale, void *y, void *workspace, size_t workspace_bytes,
-                 hipStream_t stream, const GemmOptions *planned, bool w_kn = false);
+                 hipStream_t stream, const GemmOptions *planned, bool w_kn = false, bool in_layer = true);
 int ffn2_forward_combine(const void *h, const int32_t *token_row, const int32_t *flat_row, const int32_t *offsets,
                          int max_rows, int num_expert, int d_model, int d_ffn, const void *w2, const void *b2,
                          const void *score, void *out, void *workspace, size_t workspace_bytes, hipStream_t stream,
@@ -576,6 +576,7 @@ struct FewArgs {
   const int32_t *offsets;
   int max_rows, E, N, K;
   int force;                 // tile shape, or -1: chosen by the kernel; filled in by few_rows_gemm
+  int stream_experts;        // so many experts with rows and more: their weights are not kept; filled in by few_rows_gemm
 };
 // thin.hip: at most 32 rows in all (the two epilogues without a kept pre-activation, [E, N, K] weights)
 bool thin_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn);
@@ -583,7 +584,9 @@ int thin_rows_gemm(const FewArgs &p, int epi, hipStream_t stream, const char *wh
 // mode: GemmOptions::few_rows (0: never, 1: by the rule, 2: always, 3: always, in the form of thin.hip where that can,
 // 16 + i: always and with tile shape i)
 bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn, int cus);
-int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, int cus, hipStream_t stream, const char *what);
+// in_layer: before these weights are read again, as many bytes pass as they have (the layer's other product, or the weight
+// gradient)
+int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, bool in_layer, int cus, hipStream_t stream, const char *what);
 
 // most entries of a table of per-run expert counts that the routing stage takes from the gate kernel
 long long route_rows_max_ints();

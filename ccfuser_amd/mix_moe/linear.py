@@ -76,7 +76,7 @@ class MixMOELinear1(Function):
                               moe_inp_block_infos.get("inv_pos"))
         ctx.sizes = (max_rows, n_flat, bool(fuse_gelu), bool(moe_inp_block_infos.get("may_drop", True)))
         return ops.ffn1(input_buf, src_row, offsets, max_rows, *_pair(weight, bias, E), gelu=bool(fuse_gelu),
-                        spare_experts=True)
+                        spare_experts=True, in_layer=True)
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -113,7 +113,7 @@ class MixMOELinear2(Function):
         y = alloc(n_flat, d, dtype=input_buf.dtype, device=input_buf.device)
         ctx.save_for_backward(input_buf, weight, dst_row, offsets)
         ctx.sizes = (max_rows, bool(moe_inp_block_infos.get("may_drop", True)))
-        return ops.ffn2(input_buf, dst_row, offsets, max_rows, *_pair(weight, bias, E), y, spare_experts=True)
+        return ops.ffn2(input_buf, dst_row, offsets, max_rows, *_pair(weight, bias, E), y, spare_experts=True, in_layer=True)
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -163,7 +163,7 @@ class MixMOEFusedFFN(Function):
         act, h_pre = ops.ffn1_keep(input_buf, src_row, offsets, max_rows, *_pair(w1, b1, E), spare_experts=True)
         y = (torch.zeros if may_drop else torch.empty)(n_flat, w2.shape[1], dtype=input_buf.dtype,
                                                        device=input_buf.device)
-        ops.ffn2(act, dst_row, offsets, max_rows, *_pair(w2, b2, E), y, spare_experts=True)
+        ops.ffn2(act, dst_row, offsets, max_rows, *_pair(w2, b2, E), y, spare_experts=True, in_layer=True)
         ctx.save_for_backward(input_buf, w1, w2, act, h_pre, src_row, dst_row, offsets,
                               moe_inp_block_infos.get("inv_pos"))
         ctx.sizes = (max_rows, n_flat, may_drop)

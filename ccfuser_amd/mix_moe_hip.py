@@ -132,7 +132,7 @@ class MixMOE:
         M = int(total_block_num) * self._block_size
         ffn1_out = torch.zeros(M, self._ffn_hidden_size, dtype=inp.dtype, device=inp.device)
         ops.ffn1(inp.contiguous(), a_rows, offsets, M, w, bias.contiguous(), gelu=False,
-                 out=ffn1_out, dst_row=rows, w_kn=kn)
+                 out=ffn1_out, dst_row=rows, w_kn=kn, in_layer=True)
         merged_input = inp[src_of_padded] * valid[:, None].to(inp.dtype)
         return [merged_input, ffn1_out]
 
@@ -145,7 +145,8 @@ class MixMOE:
         c_rows = flat_of_padded[rows.long()].to(torch.int32)
         M = int(total_block_num) * self._block_size
         output = torch.zeros(pos.numel(), self._hidden_size, dtype=ffn1_out.dtype, device=ffn1_out.device)
-        ops.ffn2(ffn1_out.contiguous(), c_rows, offsets, M, w, bias.contiguous(), output, src_row=rows, w_kn=kn)
+        ops.ffn2(ffn1_out.contiguous(), c_rows, offsets, M, w, bias.contiguous(), output, src_row=rows, w_kn=kn,
+                 in_layer=True)
         return [ffn1_out, output]
 
     def forward(self, inp, pos, expert_ids, ranks, expert_lens, start_addrs, total_block_num,

@@ -16,6 +16,7 @@ import torch
 from . import _lib
 
 CCF_F16, CCF_F32 = 0, 1
+CCF_FFN_KN, CCF_FFN_IN_LAYER = 1, 2
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -383,10 +384,12 @@ def _check_expert(w: torch.Tensor, b: torch.Tensor, name: str, kn: bool = False)
 def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor, max_rows: int,
          w1: torch.Tensor, b1: torch.Tensor, gelu: bool = True,
          out: Optional[torch.Tensor] = None, dst_row: Optional[torch.Tensor] = None,
-         workspace: Optional[torch.Tensor] = None, w_kn: bool = False, spare_experts: bool = False) -> torch.Tensor:
+         workspace: Optional[torch.Tensor] = None, w_kn: bool = False, spare_experts: bool = False,
+         in_layer: bool = False) -> torch.Tensor:
     """h [max_rows, f] (or ``out``); rows nothing maps to are left as they were.  ``spare_experts``: the weight may
     hold more experts than ``offsets``, the first of which are used.  ``w_kn``: the weight is
-    stored [E, d, f] (input width first)."""
+    stored [E, d, f] (input width first).  ``in_layer``: ``ffn2`` on weights of the same size comes before the next
+    call on these (how large weights are loaded; the results are the same)."""
     if x.dtype != torch.float16:
         raise TypeError("moe input data type must be float 16")
     _check(x, "x", dtype=torch.float16, ndim=2)
@@ -413,8 +416,8 @@ def ffn1(x: torch.Tensor, src_row: Optional[torch.Tensor], offsets: torch.Tensor
         raise ValueError("ffn1: output buffer too small")
     with _on(x):
         ws = workspace if workspace is not None else ffn_workspace(max_rows, E, d, f, x)
-        _lib.call("ccf_ffn1_forward_kn" if w_kn else "ccf_ffn1_forward", _ptr(x), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
-                  _ptr(w1), _ptr(b1), int(bool(gelu)), _ptr(h), _ptr(ws), ws.numel(), _stream(x))
+        _lib.call("ccf_ffn1_forward_opts", _ptr(x), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
+                  _ptr(w1), _ptr(b1), int(bool(gelu)), (CCF_FFN_KN if w_kn else 0) | (CCF_FFN_IN_LAYER if in_layer else 0), _ptr(h), _ptr(ws), ws.numel(), _stream(x))
     return h
 
 
@@ -449,9 +452,9 @@ def ffn2(h: torch.Tensor, dst_row: Optional[torch.Tensor], offsets: torch.Tensor
          w2: torch.Tensor, b2: torch.Tensor, y: torch.Tensor,
          row_scale: Optional[torch.Tensor] = None,
          src_row: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None,
-         w_kn: bool = False, spare_experts: bool = False) -> torch.Tensor:
+         w_kn: bool = False, spare_experts: bool = False, in_layer: bool = False) -> torch.Tensor:
     """Writes ``y[dst_row[j]]`` for the routed rows and returns ``y``.  ``w_kn``: the weight is stored
-    [E, f, d] (input width first).  ``spare_experts`` as in ``ffn1``."""
+    [E, f, d] (input width first).  ``spare_experts`` and ``in_layer`` as in ``ffn1``."""
     _check(h, "h", dtype=torch.float16, ndim=2)
     _check_expert(w2, b2, "ffn2", w_kn)
     _check(offsets, "offsets", dtype=torch.int32, ndim=1)
@@ -477,8 +480,8 @@ def ffn2(h: torch.Tensor, dst_row: Optional[torch.Tensor], offsets: torch.Tensor
         _check(row_scale, "row_scale", dtype=torch.float16, ndim=1)
     with _on(h):
         ws = workspace if workspace is not None else ffn_workspace(max_rows, E, d, f, h)
-        _lib.call("ccf_ffn2_forward_kn" if w_kn else "ccf_ffn2_forward", _ptr(h), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
-                  _ptr(w2), _ptr(b2), _ptr(row_scale), _ptr(y), _ptr(ws), ws.numel(), _stream(h))
+        _lib.call("ccf_ffn2_forward_opts", _ptr(h), _ptr(src_row), _ptr(dst_row), _ptr(offsets), int(max_rows), E, d, f,
+                  _ptr(w2), _ptr(b2), _ptr(row_scale), (CCF_FFN_KN if w_kn else 0) | (CCF_FFN_IN_LAYER if in_layer else 0), _ptr(y), _ptr(ws), ws.numel(), _stream(h))
     return y
 
 

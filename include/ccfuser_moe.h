@@ -446,6 +446,30 @@ int ccf_ffn2_forward_kn(const void *h, const int32_t *src_row,
                         void *y, void *workspace, size_t workspace_bytes,
                         ccf_stream_t stream);
 
+/*
+ * ccf_ffn1_forward / ccf_ffn2_forward (mix_moe/csrc/mix_moe.h:236-298, 390-437)
+ * with options, a sum of
+ *   CCF_FFN_KN        the weight is stored [E, K, N]
+ *   CCF_FFN_IN_LAYER  the call is one of a layer's two products, which alternate:
+ *                     large weights are read past the last-level cache from half
+ *                     the size on that a call repeated by itself needs for that
+ * The results do not depend on the second.
+ */
+enum { CCF_FFN_KN = 1, CCF_FFN_IN_LAYER = 2 };
+int ccf_ffn1_forward_opts(const void *x, const int32_t *src_row,
+                          const int32_t *dst_row, const int32_t *offsets,
+                          int max_rows, int num_expert, int d_model, int d_ffn,
+                          const void *w1, const void *b1, int apply_gelu,
+                          int opts, void *h, void *workspace,
+                          size_t workspace_bytes, ccf_stream_t stream);
+/* See above (mix_moe/csrc/mix_moe.h:390-437). */
+int ccf_ffn2_forward_opts(const void *h, const int32_t *src_row,
+                          const int32_t *dst_row, const int32_t *offsets,
+                          int max_rows, int num_expert, int d_model, int d_ffn,
+                          const void *w2, const void *b2, const void *row_scale,
+                          int opts, void *y, void *workspace,
+                          size_t workspace_bytes, ccf_stream_t stream);
+
 /* ------------------------------------------------------------ backward */
 
 /*

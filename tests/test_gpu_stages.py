@@ -1152,3 +1152,36 @@ def test_few_rows_of_large_weights(counts, kn):
             ops.set_option(name, value)
     for a, b in zip(got, ref):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kn", [False, True])
+@pytest.mark.parametrize("counts", [[64, 0, 0, 0], [0, 5, 60, 0], [20, 1, 40, 64], [0, 200, 3, 0]])
+def test_few_rows_of_large_weights_by_experts_with_rows(counts, kn):
+    """Experts of 84 MB, of which non-temporal loads want four with rows, or two of a layer's alternating products: on
+    both sides of either number the bits of the 256-row tiles."""
+    from ccfuser_amd import ops
+    E, d, f = 4, 4096, 10304
+    R = sum(counts)
+    _say(f"few rows by experts with rows {counts} kn={kn}")
+    g = torch.Generator(device="cuda").manual_seed(R)
+    rnd = lambda *s: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, 0.05, generator=g)
+    off = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    x, h = rnd(R, d), rnd(R, f)
+    w1, w2 = (rnd(E, d, f), rnd(E, f, d)) if kn else (rnd(E, f, d), rnd(E, d, f))
+    b1, b2 = rnd(E, f), rnd(E, d)
+
+    def both(in_layer):
+        y = torch.zeros(R, d, dtype=torch.float16, device="cuda")
+        return ops.ffn1(x, None, off, R, w1, b1, w_kn=kn, in_layer=in_layer), ops.ffn2(h, None, off, R, w2, b2, y, w_kn=kn, in_layer=in_layer)
+
+    ops.set_option("few_rows", 2)
+    try:
+        got = both(False) + both(True)
+        for name, value in (("few_rows", 0), ("split_tail", 0), ("skinny", 0)):
+            ops.set_option(name, value)
+        ref = both(False)
+    finally:
+        for name, value in (("few_rows", 1), ("split_tail", 1), ("skinny", 1)):
+            ops.set_option(name, value)
+    for a, b in zip(got, ref + ref):
+        assert torch.equal(a, b)
