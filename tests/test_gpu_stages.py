@@ -180,6 +180,42 @@ def test_gate_of_few_tokens(T, d, E, k):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("T", [1, 5, 70])
+@pytest.mark.parametrize("d,E,k", [(136, 9, 1), (136, 9, 2), (136, 9, 3), (64, 3, 3), (256, 8, 8), (64, 300, 5), (1024, 16, 8)])
+def test_gate_of_few_tokens_orders_ties_infinities_and_nan(T, d, E, k):
+    """Experts whose logits tie, are infinite or NaN, up to lists that NaN leave short, and rows of NaN: the choice, the
+    scores and the routing of the form for few tokens are those of the MFMA tiles and of the routing on its own."""
+    from ccfuser_amd import ops
+    _say(f"gate order T={T} d={d} E={E} k={k}")
+    g = torch.Generator().manual_seed(d + E)
+    x, wg = torch.randn(T, d, generator=g), torch.randn(E, d, generator=g) * 0.05
+    half = E // 2
+    wg[half:2 * half] = wg[:half]                                        # ties, in pairs
+    if T > 1:
+        x[1] = float("nan")
+    x, wg = x.half().cuda(), wg.half().cuda()
+    nan, inf = float("nan"), float("inf")
+    for bad in ([], [nan], [-inf], [inf], [-inf] * E, [nan] * E, [nan, -inf, inf, nan, -inf], [nan] * (E - 1), [nan] * (E - 2) + [-inf]):
+        bg = torch.zeros(E)
+        bad = bad[:E]
+        bg[torch.randperm(E, generator=g)[:len(bad)]] = torch.tensor(bad)
+        bg = bg.half().cuda()
+        got = ops.gate_topk_softmax(x, wg, bg, k, return_logits=True)
+        idx, score, routing = ops.gate_route(x, wg, bg, k, 2)
+        ops.set_option("gate_waves", 7)                                  # the MFMA tiles
+        try:
+            ref = ops.gate_topk_softmax(x, wg, bg, k, return_logits=True)
+        finally:
+            ops.set_option("gate_waves", 8)
+        for a, b in zip(got + (idx, score), ref + ref[:2]):
+            assert torch.equal(a.nan_to_num(3.0, 4.0, 5.0) if a.is_floating_point() else a, b.nan_to_num(3.0, 4.0, 5.0) if b.is_floating_point() else b)
+        r0 = ops.route(ref[0].reshape(-1), E, k, 2)
+        n = int(r0["offsets"][-1])
+        for name in ("counts", "offsets", "inv_pos", "idx_kept"):
+            assert torch.equal(routing[name], r0[name]), name
+        assert torch.equal(routing["pos"][:n], r0["pos"][:n])
+
+
 @pytest.mark.parametrize("stream", [0, 1])
 @pytest.mark.parametrize("E,k", [(32, 2), (8, 1), (70, 3)])
 def test_gate_logits_that_are_nothing_but_rounding_error(E, k, stream):
