@@ -324,14 +324,15 @@ few_rows_kernel(FewArgs p) {
   __syncthreads();
   // M tiles of each height over all experts (every wavefront for itself)
   int m64 = 0, m128 = 0;
-  int used = 0;                                                     // experts with rows
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    int cnt = e0 + lane < E ? s_off[e0 + lane + 1] - s_off[e0 + lane] : 0;
+  for (int e = lane; e < E; e += 64) {
+    int cnt = s_off[e + 1] - s_off[e];
     cnt = cnt > 0 ? cnt : 0;
     m64 += (cnt + 63) >> 6;
     m128 += (cnt + 127) >> 7;
-    if constexpr (kStream) used += __popcll(__ballot(cnt > 0));
   }
+  [[maybe_unused]] int used = 0;                                    // experts with rows
+  if constexpr (kStream)
+    for (int e0 = 0; e0 < E; e0 += 64) used += __popcll(__ballot(e0 + lane < E && s_off[e0 + lane + 1] > s_off[e0 + lane]));
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     m64 += __shfl_xor(m64, off, 64);
