@@ -107,19 +107,29 @@ struct Best {
 
 // Leaves how many of the workgroup's token slots chose each expert, for the routing stage: the selection threads hold the
 // ids, so the routing needs no pass of its own over idx to count them.  `row`: E ints of LDS that nothing else uses from
-// here on; `mine`: this thread holds a token's list.  All threads of the workgroup call it, behind a barrier.  A list
+// here on; `mine`: this thread holds a token's list.  All threads of the workgroup call it, behind a barrier; with
+// kFirstWave its first wavefront alone, which holds all lists, and the others make room for the next workgroup.  A list
 // that NaN logits left short has entries that are no expert.
-template <int KS>
+template <int KS, bool kFirstWave = false>
 __device__ inline void leave_counts(const Best<KS> &best, bool mine, int k, int E, int *row, int32_t *__restrict__ wg_cnt) {
-  for (int e = threadIdx.x; e < E; e += blockDim.x) row[e] = 0;
-  __syncthreads();
+  const int step = kFirstWave ? 64 : static_cast<int>(blockDim.x);
+  auto meet = [] {
+    if constexpr (kFirstWave) {                      // a wavefront's LDS accesses happen in order
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      __syncthreads();
+    }
+  };
+  for (int e = threadIdx.x; e < E; e += step) row[e] = 0;
+  meet();
   if (mine) {
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       if (s < k && best.id[s] < E) atomicAdd(&row[best.id[s]], 1);
   }
-  __syncthreads();
-  for (int e = threadIdx.x; e < E; e += blockDim.x) wg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = row[e];
+  meet();
+  for (int e = threadIdx.x; e < E; e += step) wg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = row[e];
 }
 
 // Whether a gate of `wgs` workgroups of `wg_tokens` tokens leaves them: the table fits, and its rows tile the routing's
@@ -754,7 +764,9 @@ gate_f32_kernel(const float *__restrict__ x, const float *__restrict__ wg, const
   }
   if (threadIdx.x < C::WT && t0 + threadIdx.x < tokens) best.template write<float>(t0 + threadIdx.x, k, idx_out, score_out);
   static_assert(C::REGION >= (EE >= 8 ? 1024 : 8 * EE), "a count per expert");
-  if (wg_cnt) leave_counts<KS>(best, threadIdx.x < C::WT && t0 + threadIdx.x < tokens, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
+  static_assert(C::WT <= 64, "lists in the first wavefront");
+  if (wg_cnt && threadIdx.x < 64)
+    leave_counts<KS, true>(best, threadIdx.x < C::WT && t0 + threadIdx.x < tokens, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
 }
 
 template <int TT, int EE>
