@@ -764,9 +764,11 @@ gate_f32_kernel(const float *__restrict__ x, const float *__restrict__ wg, const
   }
   if (threadIdx.x < C::WT && t0 + threadIdx.x < tokens) best.template write<float>(t0 + threadIdx.x, k, idx_out, score_out);
   static_assert(C::REGION >= (EE >= 8 ? 1024 : 8 * EE), "a count per expert");
+  // the first wavefront alone where a CU goes through several workgroups (as few as one of 8 tokens take 0.6 us longer with it)
+  constexpr bool kMany = TT == 4;
   static_assert(C::WT <= 64, "lists in the first wavefront");
-  if (wg_cnt && threadIdx.x < 64)
-    leave_counts<KS, true>(best, threadIdx.x < C::WT && t0 + threadIdx.x < tokens, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
+  if (wg_cnt && (!kMany || threadIdx.x < 64))
+    leave_counts<KS, kMany>(best, threadIdx.x < C::WT && t0 + threadIdx.x < tokens, k, E, reinterpret_cast<int *>(s_mem), wg_cnt);
 }
 
 template <int TT, int EE>
