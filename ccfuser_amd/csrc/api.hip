@@ -135,6 +135,17 @@ inline void mark_stage(int i, hipStream_t st) {
   if (i < g_stage_event_count && g_stage_events[i]) (void)hipEventRecord(g_stage_events[i], st);
 }
 
+// Largest table of counts that the gate leaves for the routing of n indices.  Up to 1024 indices the routing counts them in
+// its one launch itself, which is as long as adding up about 2048 counts; with more it needs a launch of its own, or
+// counts two chunks, and any table that it can add up is shorter.  Microseconds with the gate's counts and without, gate
+// and routing: 500 tokens of 4096, top-1 of 8 experts, 4000 counts 13.9, 13.5; 700 of 1024, 16 experts, 5600 counts 14.3,
+// 13.8; 64 of 1024, top-2 of 32, 2048 counts 14.9, 15.4; 2000 of 1024, 16 experts, 16000 counts 18.1, 19.4; 6000 of 2048,
+// 64 experts, 12032 counts 43.1, 45.5.
+long long gate_counts_max(int n) {
+  const long long most = route_rows_max_ints();
+  return n <= 1024 && most > 2048 ? 2048 : most;
+}
+
 bool sizes_ok(long long rows, int d, int f) {
   // row offsets are formed in 64 bits, but the row tables are int32
   return rows >= 0 && rows < (1ll << 31) && d > 0 && f > 0;
@@ -190,7 +201,7 @@ extern "C" int ccf_moe_forward(const void *x, const void *wg, const void *bg, co
   // table is small and its rows tile the routing's chunks: the routing stage is then one launch
   int gate_tokens = 0;
   if ((rc = gate_forward(x, wg, bg, tokens, d_model, num_expert, top_k, CCF_F16, w.idx, w.score, nullptr, stream,
-                         reinterpret_cast<int32_t *>(w.route_ws), route_rows_max_ints(), &gate_tokens)))
+                         reinterpret_cast<int32_t *>(w.route_ws), gate_counts_max(n), &gate_tokens)))
     return rc;
   mark_stage(1, st);
   // the tile plans of both GEMMs are built by two more workgroups of the routing stage's last
@@ -257,15 +268,8 @@ extern "C" int ccf_gate_route(const void *x, const void *wg, const void *bg, int
     return gate_route_tiny(x, wg, bg, tokens, d_model, num_expert, top_k, capacity, idx, score, counts, offsets, pos, src_row,
                            dst_row, inv_pos, idx_kept, as_stream(stream));
   int gate_tokens = 0;
-  // Counts from the gate where the routing would launch a count of its own or count two chunks of 1024 indices, and where
-  // adding them up is no longer than that: a table of at most 8192 of them, or one per index (443 tokens, top-2, 64 experts
-  // of 256, with the gate's counts and without: 22.8 and 20.0 us; 700: 23.4 and 23.5; 2000 in fp32, a table of 16000: 31.6
-  // and 29.6; 8192 of 2048, 64 experts, a table of 16384: 55.7 and 58.9).
-  const bool counted = n > 1024;
-  const long long most = n > 8192 ? n : 8192;
   if (int rc = gate_forward(x, wg, bg, tokens, d_model, num_expert, top_k, dtype, idx, score, nullptr, stream,
-                            counted ? static_cast<int32_t *>(workspace) : nullptr,
-                            most < route_rows_max_ints() ? most : route_rows_max_ints(), &gate_tokens))
+                            static_cast<int32_t *>(workspace), gate_counts_max(n), &gate_tokens))
     return rc;
   return route_with_plans(idx, n, num_expert, top_k, capacity, counts, offsets, pos, src_row, dst_row, inv_pos, idx_kept,
                           workspace, workspace_bytes, as_stream(stream), nullptr, 0, gate_tokens * top_k);

@@ -1056,6 +1056,9 @@ def test_mfma_probe_runs_and_counts_its_flop():
     (4096, 128, 36, 2, -1),                # four counts a load, experts that do not divide a wavefront
     (6000, 64, 9, 4, -1),                  # a long table of odd width
     (200, 64, 600, 2, -1),                 # more experts than threads
+    (700, 64, 300, 2, -1),                 # the same in a table of counts
+    (512, 256, 64, 2, -1), (513, 256, 64, 2, -1),    # 1024 indices, counted by the routing, and more
+    (64, 1024, 32, 2, -1), (65, 1024, 32, 2, -1),    # fp16: 2048 counts, and more than the routing takes for 1024 indices
     (700, 4096, 2, 1, -1),                 # fp32: a wavefront per token, which leaves no counts
     (2, 4096, 8, 2, -1), (3, 4096, 8, 2, -1),        # fp16: gate and routing as one launch in two turns, one token more
     (8, 768, 8, 2, 3), (9, 768, 8, 2, 0),            # the same at four tokens a turn, capacity limits
