@@ -150,20 +150,38 @@ thin_rows_kernel(FewArgs p, int n_col) {
 // Workgroups of 16 columns over all experts that may have rows.
 long long thin_wgs(int max_rows, int E, int N) { return static_cast<long long>((N + 15) / 16) * (E < max_rows ? E : max_rows); }
 
-}  // namespace
-
 // Two workgroups per CU at most: more of them are as many short ones, whose start costs more than their share of the
 // weights (tiles of few.hip and here: FFN1 of one token, top-2 of 4096 / 14336, 1792 workgroups, 38 and 55 us; FFN2 of 8
-// tokens of 1024 / 4096, 512 workgroups, 22 and 16; of 32 experts, 1024 workgroups, 22 and 25).  And eight wavefronts want
-// two K tiles each (K of 768, 384 workgroups: 8.4 and 9.7; of 1024, 128 workgroups: 8.8 and 7.4, 512 workgroups 9.7 and 9.9).
-// As many rows as experts and more of a K of 4096 and more stay with 256-row tiles that the plan cuts along K over the
-// chip, which is where that form is used and tested (8 rows of 8 experts of 1024 / 4096: 27 us there, 21 in tiles of
-// few.hip, 10 here).
+// tokens of 32 experts of 1024 / 4096, 1024 workgroups, 22 and 25).  And eight wavefronts want two K tiles each (K of 768,
+// 384 workgroups: 8.4 and 9.7).
+//
+// Within that, what takes the time here is the rounds of four K tiles that a wavefront has on their way, the rows of an
+// expert that each of them fetches again, and a second workgroup on the CU, so both forms are priced in microseconds.
+// Of 1295 GEMMs timed (K of 1024 to 4032, 1 to 32 experts, 64 to 512 workgroups, 1 to 32 rows) this takes the slower form
+// by over 2 % in one (3.6 %), and by over 3 % where it stays with few.hip in six (4.6 % at most).  Tiles of few.hip and
+// here: K of 1024, 256 workgroups, one expert: 16 rows 8.6 and 7.7, 32 rows 8.6 and 10.4; 512 workgroups, two experts: 2
+// rows 8.7 and 9.0, 32 rows 8.7 and 14.3; K of 2048, 512 workgroups, 8 experts: 16 rows 13.4 and 9.9; one: 32 rows 13.0
+// and 18.7.
+//
+// As many rows as experts and more of a K of 4096 and more are left to few.hip and to 256-row tiles that the plan cuts
+// along K over the chip.  The times do not cross there (8 rows of 8 experts of 1024 / 4096: 27 us in those tiles, 21 in
+// few.hip, 15 here; 2 of 2 of 4096 / 14336: 49, 59 and 37): the line keeps that form's calls as they were.
+bool thin_rows_pays(int max_rows, int E, int N, int K) {
+  const long long wgs = thin_wgs(max_rows, E, N);
+  if (K < 2 * kThinWaves * kThinK || wgs > 512 || (max_rows >= E && K >= 64 * kThinK)) return false;
+  const double rows = static_cast<double>(max_rows) / (E < max_rows ? E : max_rows);
+  const int rounds = (K + 4 * kThinWaves * kThinK - 1) / (4 * kThinWaves * kThinK);
+  const double here = 3.5 + (wgs <= 256 ? 1.0 : 2.5) * rounds * (2.1 + (max_rows > 16 ? 0.4 : 0.0) + 0.12 * rows);
+  return here < 4.5 + 0.265 * K / kThinK;
+}
+
+}  // namespace
+
 bool thin_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn) {
   if ((mode != 1 && mode != 3) || b_kn || epi > kFewGelu || K % kThinK || E <= 0 || E > 1024 || max_rows <= 0 ||
       max_rows > kThinMaxRows || thin_wgs(max_rows, E, N) >= (1ll << 24))
     return false;
-  return mode == 3 || (K >= 2 * kThinWaves * kThinK && thin_wgs(max_rows, E, N) <= 512 && (max_rows < E || K < 64 * kThinK));
+  return mode == 3 || thin_rows_pays(max_rows, E, N, K);
 }
 
 int thin_rows_gemm(const FewArgs &p, int epi, hipStream_t stream, const char *what) {

@@ -684,6 +684,40 @@ def test_thin_rows_kernel(counts, N, K, pad):
         assert (out[rest] == 7.0).all()
 
 
+@pytest.mark.parametrize("E,N,K,rows,thin", [
+    (4, 1024, 1024, 32, True), (4, 1024, 1024, 33, False),         # 32 rows in all
+    (4, 1024, 960, 16, False),                                     # two K tiles a wavefront
+    (8, 1024, 2048, 16, True), (8, 1040, 2048, 16, False),         # two workgroups a CU
+    (2, 4096, 1024, 2, False), (2, 2048, 1024, 2, True),           # two of few K tiles, one
+    (1, 4096, 1024, 16, True), (1, 4096, 1024, 32, False),         # rows of an expert
+    (1, 8192, 2048, 24, False), (1, 8192, 2048, 2, True),
+    (4, 1024, 4096, 3, True), (4, 1024, 4096, 4, False),           # fewer rows than experts of a long contraction
+])
+def test_thin_rows_rule_takes_the_faster_form(E, N, K, rows, thin):
+    """At most 32 rows: the form that cuts K over the wavefronts or tiles of few rows, told apart by the bits that their
+    orders of the sum leave; both against fp32."""
+    from ccfuser_amd import ops
+    _say(f"thin rule E={E} N={N} K={K} rows={rows}")
+    g = torch.Generator(device="cuda").manual_seed(N + K + rows)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    a, w, b = rnd(rows, K).half(), (rnd(E, N, K) * 0.02).half(), rnd(E, N).half()
+    counts = [rows // E + (e < rows % E) for e in range(E)]
+    off = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    out = {}
+    try:
+        for mode in (0, 1, 2, 3):
+            ops.set_option("few_rows", mode)
+            out[mode] = ops.ffn2(a, None, off, rows, w, b, torch.empty(rows, N, dtype=torch.float16, device="cuda"))
+    finally:
+        ops.set_option("few_rows", 1)
+    assert torch.equal(out[1], out[3]) == (thin or rows > 32)
+    if K < 4096:
+        assert torch.equal(out[1], out[2]) != thin
+    ref = torch.cat([a[off[e]:off[e + 1]].float() @ w[e].float().t() + b[e].float() for e in range(E)])
+    for y in out.values():
+        assert float((y.float() - ref).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(ref.abs().max()) + 1e-4
+
+
 @pytest.mark.parametrize("shape", range(6))
 @pytest.mark.parametrize("counts,N,K", [
     ([0, 1, 63, 64, 65, 127, 128, 129, 0], 264, 64),          # edges of both tile heights, a ragged last column tile
