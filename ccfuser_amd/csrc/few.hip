@@ -132,6 +132,7 @@ __device__ __forceinline__ int few_kn_swz(int row) { return (row & 3) | (((row >
 //     69, 69, of 2048 / 8192 (134) 62, 73; 2 of 4096 / 14336 (235) 141, 135, 1 of them (117) 85, 102
 //   FFN1 alone: 8 of 2048 / 8192 (268 MB) 47, 66, of 2304 / 8192 (302) 51, 52, of 2560 / 8192 (336) 61, 57; 2 of 4096 /
 //     14336 (235) 40, 54, 4 of them (470) 111, 105
+// (Alone, 83 rows each of 8 of 2048 / 8192 do better with it, 68 and 59 for FFN2: the line goes by bytes, not rows.)
 // A layer of 128 tokens, 8 experts of 4096 / 14336: 356 -> 333 us.
 constexpr double kStreamBytes = 320e6;
 __device__ __forceinline__ void lds_dma16_nt(const void *gptr, lds_char *lds_wave_base) {

@@ -610,21 +610,21 @@ gate_stream_kernel(const half_t *__restrict__ x, const half_t *__restrict__ wg, 
   }
 }
 
-// fp32 gate on the vector unit.  Each product is rounded before it is added, which no MFMA does, so the floor is
-// two vector instructions per product: 8192 tokens x 64 experts x 2048 are 33.6 M wavefront instructions, 33 K per
-// SIMD, ~40 us at the issue rate of a few wavefronts per SIMD.  What the kernel has to do is feed them:
+// fp32 gate on the vector unit.  Each product is rounded before it is added, which an accumulating MFMA does not do, so
+// the floor is two vector instructions per product: 4096 tokens x 64 experts x 2048 are 16.8 M wavefront instructions,
+// 16 K per SIMD, ~20 us at the issue rate of a few wavefronts per SIMD.  What the kernel has to do is feed them:
 //
 // * A wavefront computes a tile of 8 TT tokens x 8 EE experts over one part of K (lane l: tokens l / 8 + 8 i,
-//   experts l % 8 + 8 j), so four K elements of TT + EE rows read from LDS feed 8 TT EE instructions (12 reads for
-//   256 at the full tile).  The wavefronts of a workgroup take different parts of the same tile.
+//   experts l % 8 + 8 j), so four K elements of TT + EE rows read from LDS feed 8 TT EE instructions (8 reads for 128
+//   and 10 for 128 at the largest tiles, 32 x 32 and 16 x 64; more tokens of more than 32 experts are
+//   gate_f32_mfma_kernel's).  The wavefronts of a workgroup take different parts of the same tile.
 // * Operands come in stages of 16 K elements: four lanes per row fetch its 64 bytes a stage ahead into registers,
 //   which go into the other half of the wavefront's own LDS behind the stage's arithmetic: no barrier in the loop.
 // * Rows are 80 bytes apart: the eight rows that a read touches start 20 banks apart, none in conflict.
 // * Behind a round of parts their sums meet in LDS and are added in ascending order onto the running sums.
 //
 // TT shrinks with the tokens, so that 2049 and 4097 tokens still make 129 workgroups, EE with the experts.
-// 4096 tokens x 2048, 64 experts, top-2: 42 us; 8192 tokens: 66 us, 988 us as one wavefront per token whose lanes each walked
-// rows of their own (and left the selection to one lane).
+// 4096 tokens x 2048, 64 experts, top-2: 42 us; 8192 x 2048, 32 experts: 39 us.
 constexpr int kF32StageK = 16;                     // K elements of a stage
 constexpr int kF32Row = kF32StageK + 4;            // row stride in LDS, floats
 
@@ -1071,7 +1071,7 @@ bool gate_f32_on_mfma(int tokens, int d, int E) {
 //   more: as many rank them).
 // * With `route` (one workgroup, at most 64 indices) the routing of the choice follows: a lane per index.
 //
-// Microseconds, MFMA tiles and here (the gate alone): see gate_f16_walks().
+// Microseconds, MFMA tiles and here (the gate alone): see gate_f16_walk_group().
 struct TinyRoute {
   int32_t *counts, *offsets;                       // counts null: no routing
   int64_t *pos;

@@ -382,10 +382,9 @@ struct Ring16Mainloop {
 
   // Order of a substep's blocks: along strips of two row blocks, up and down, so that consecutive MFMAs share an operand
   // and take the other one from two MFMAs back or the next column.  Under load the chip runs at the clock that its power
-  // limit allows, and operands that stay switch less.  Register-only loops on random operands, PFLOP/s: both operands new
-  // each time 1.77, row block by row block 1.84, that as a serpentine 1.86, strips of two 1.89.  The layer of 8192
-  // tokens, 8 experts of 1024 / 4096: 356 -> 348 us; 16 experts on [E, K, N] weights 346 -> 334; a training step of 4096
-  // tokens of 4096 / 14336: 5695 -> 5640.
+  // limit allows, and operands that stay switch less.  Against row block by row block, the layer of 8192 tokens, 8 experts
+  // of 1024 / 4096: 356 -> 348 us; 16 experts on [E, K, N] weights 346 -> 334; a training step of 4096 tokens of 4096 /
+  // 14336: 5695 -> 5640; layers of 4096 / 14336 and of 2048 / 8192 by 1 %, which is their runs' spread.
   static constexpr int path_row(int i) { return 2 * (i / (2 * TN)) + ((i ^ (i >> 1)) & 1); }
   static constexpr int path_col(int i) {
     const int j = i % (2 * TN) / 2;

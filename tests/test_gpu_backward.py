@@ -453,6 +453,7 @@ def test_zero_tails(E, first, shape):
     (300, 3, 256, 768, 1, 2, -1),           # one expert, three slots a token
     (300, 2, 320, 704, 4, 7, 100),          # widths that are no multiples of 256: the layers one after the other
     (70, 2, 256, 256, 520, 521, -1),        # more experts than one plan holds twice
+    (70, 2, 256, 256, 512, 513, -1),        # as many as it holds
 ])
 def test_backward_of_both_layers_in_one_call(T, k, d, f, E, slots, capacity):
     """Gradients of both expert layers from one call: the bits of the two layers' own calls and the sum over a token's
