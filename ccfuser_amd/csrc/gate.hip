@@ -807,8 +807,9 @@ int launch_gate_f32_experts(const float *x, const float *wg, const float *bg, in
 // The same order with the products on the matrix cores: fma(x, w, 0) of a K = 1 MFMA is the rounded product, subnormal
 // ones included, for 2048 token-expert pairs in 64 cycles, and the vector unit has one addition per product left
 // instead of two instructions.  (A product of -0 comes out as +0, which no running sum can tell: it starts at +0 and is
-// never -0.)  The two do not overlap, not even from two wavefronts of a SIMD: a step takes 30 ns for the MFMA and 40
-// for its 32 additions, against 80 for 64 vector instructions, and two LDS reads feed 32 of them instead of three.
+// never -0.)  They come one after the other, also with two wavefronts on a SIMD: a step takes 30 ns for the MFMA and 40
+// for its 32 additions, against 80 for 64 vector instructions, and two LDS reads feed 32 of them instead of three.  (By the
+// counters of the 8192 tokens below the matrix pipe is busy 26 % of the time and the vector unit 45 to 60.)
 //
 // * A wavefront computes 32 tokens x 64 experts (64 x 32, 64 x 16 for fewer experts) over one part of K, one product
 //   tile ahead of the additions; the wavefronts of a workgroup take different parts of the same tile.
