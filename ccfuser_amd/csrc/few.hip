@@ -14,7 +14,8 @@
 //     this one).  One workgroup of eight wavefronts per CU: two workgroups of four with half of the LDS each
 //     measured the same at many tiles and up to a quarter slower at one tile per CU, whose weights then stream
 //     through a pipeline of half the depth;
-//   * accumulation runs over K in 32-wide steps in ascending order, as in the 256-row tiles: same bits.
+//   * accumulation runs over K in 32-wide steps in ascending order, as in the 256-row tiles: same bits (large weights by
+//     the rule start inside K and go around: starts_apart()).
 //
 // Bound by streaming the weights from HBM at 5.3 - 5.7 TB/s where they are large, by the latency of a few dependent
 // steps where they are small.  FFN1 / FFN2 including their plan and reduction launches, 256-row tiles -> here:
@@ -140,6 +141,28 @@ __device__ __forceinline__ void lds_dma16_nt(const void *gptr, lds_char *lds_wav
                                    (__attribute__((address_space(3))) void *)lds_wave_base, 16, 0, 2);
 }
 
+// Where the walk through K starts.  Rows of a [N][K] weight that are a multiple of 4 KB apart hold the same K at the same
+// place of their pages, and workgroups that all start at the first K tile stay at about the same K: their loads fall on a
+// few of the memory's channels at a time, on how few depends on where the weight happens to lie.  So where the weights
+// come from HBM a tile's 256 columns go around from one of 16 places, 256 bytes apart, and the 32 tiles that an XCD runs at
+// a time are spread over all of them.  The sum starts elsewhere (its error is the same) and depends on neither the tile's
+// shape nor the other rows.  Microseconds for a layer's two products without and with it, three places of the weights each:
+//   8 experts of 4096 / 14336, 32 rows each 367, 366, 348 and 287, 288, 288, 83 rows 420, 405, 385 and 339, 340, 340;
+//   two experts, one row each 101 and 90; 64 rows of 16 of 2048 / 8192 248 and 188, 40 rows of 8 110, 122, 122 and 93, 92, 92;
+//   40 rows of 16 of 1536 / 6144 127 and 114; 33 rows of 32 of 1024 / 4096 113 and 97; 64 rows of 8 of 3584 / 14336 307, 289
+// (with places by a hash of the columns 295, 344, 91, 194, 95, 114, 99, 289; all of K instead of 4 KB in small steps no better).
+// Not for weights that stay in the Infinity Cache (64 rows of 16 experts of 1024 / 4096, 134 MB: FFN2 alone 25.2 and 26.8),
+// not for several M tiles an expert (200 rows of 8 of 2048 / 8192: FFN2 alone 90 and 96), not for other row strides (33
+// rows of 32 of 1024 / 4096: FFN1, 2 KB, 51.7 and 53.9; these three with a hash).
+constexpr double kRotateBytes = 160e6;
+constexpr int kPlaces = 16, kPlaceStep = 2;        // K tiles of 128 bytes
+bool starts_apart(int max_rows, int E, int N, int K, bool b_kn) {
+  static_assert((kPlaces - 1) * kPlaceStep < 2048 / kBK, "a place inside the shortest K");
+  const int used = E < max_rows ? E : max_rows;
+  return !b_kn && K % 2048 == 0 && max_rows <= 128ll * used && 2.0 * used * N * K >= kRotateBytes;
+}
+__device__ __forceinline__ int first_k_tile(int e, int n0) { return kPlaceStep * (((n0 >> 8) + 3 * e) & (kPlaces - 1)); }
+
 // One lane's tile table entry.
 struct FewTile {
   int e, row0, rows, n0;
@@ -182,18 +205,20 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
   // The load side runs STAGES - 1 stages ahead: tile `it`, K tile `ik` of it.  Load j of a wavefront is 1 KB at
   // 1024 (8 j + wave) of the operand's part of the stage: eight 128-byte rows, or 1024 / (2 BN) K rows of a [K][N] tile.
   const half_t *a_src[C::A_DMA], *b_src[C::B_DMA];
-  int it = 0, ik = 0;
+  int it = 0, ik = 0, rot = 0;                                     // rot: the K tile that the walk starts with
   bool stream = false;                                             // the weights being loaded are read once
-  const size_t b_step = kKN ? static_cast<size_t>(kBK) * p.N : kBK;
+  const ptrdiff_t b_step = kKN ? static_cast<ptrdiff_t>(kBK) * p.N : kBK;
   auto sources = [&](const FewTile &t) {
     const half_t *Be = p.B + static_cast<size_t>(t.e) * p.N * p.K;
     stream = kStream && t.alone;
+    if constexpr (!kKN)
+      if (p.rotate) rot = first_k_tile(t.e, t.n0);
 #pragma unroll
     for (int j = 0; j < C::A_DMA; ++j) {
       const int r = (j * 8 + wave) * 8 + (lane >> 3);
       int g = t.row0 + (r < t.rows ? r : t.rows - 1);              // padded tile rows re-read the last real row
       if (p.a_rows) g = p.a_rows[g];
-      a_src[j] = p.A + static_cast<size_t>(g) * p.K + ((lane & 7) ^ swz<8>(r)) * 8;
+      a_src[j] = p.A + static_cast<size_t>(g) * p.K + rot * kBK + ((lane & 7) ^ swz<8>(r)) * 8;
     }
 #pragma unroll
     for (int j = 0; j < C::B_DMA; ++j) {
@@ -205,7 +230,7 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
       } else {
         const int r = (j * 8 + wave) * 8 + (lane >> 3);
         const int n = (t.n0 + r) < p.N ? (t.n0 + r) : p.N - 1;
-        b_src[j] = Be + static_cast<size_t>(n) * p.K + ((lane & 7) ^ swz<8>(r)) * 8;
+        b_src[j] = Be + static_cast<size_t>(n) * p.K + rot * kBK + ((lane & 7) ^ swz<8>(r)) * 8;
       }
     }
   };
@@ -222,10 +247,11 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
     }
     if (ik + 1 < KT) {
       ++ik;
+      const ptrdiff_t back = !kKN && ik + rot == KT ? static_cast<ptrdiff_t>(p.K) : 0;       // from the last K tile to the first
 #pragma unroll
-      for (int j = 0; j < C::A_DMA; ++j) a_src[j] += kBK;
+      for (int j = 0; j < C::A_DMA; ++j) a_src[j] += kBK - back;
 #pragma unroll
-      for (int j = 0; j < C::B_DMA; ++j) b_src[j] += b_step;
+      for (int j = 0; j < C::B_DMA; ++j) b_src[j] += b_step - back;
     } else if (it + 1 < nr) {
       ++it;
       ik = 0;
@@ -539,6 +565,7 @@ int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, bool in_layer, int cu
   const double experts = std::ceil((in_layer ? kStreamBytes / 2 : kStreamBytes) / (2.0 * p.N * p.K));
   const bool large = experts <= (p.E < p.max_rows ? p.E : p.max_rows);
   p.stream_experts = large ? static_cast<int>(experts) : INT_MAX;
+  p.rotate = mode == 1 && starts_apart(p.max_rows, p.E, p.N, p.K, b_kn);
   const auto pick = [&](auto S_) -> void (*)(FewArgs) {
     constexpr bool S = decltype(S_)::value;
     if (b_kn) return epi == kFewPlain ? few_rows_kernel<kFewPlain, true, S> : few_rows_kernel<kFewGelu, true, S>;

@@ -576,6 +576,7 @@ struct FewArgs {
   const int32_t *offsets;
   int max_rows, E, N, K;
   int force;                 // tile shape, or -1: chosen by the kernel; filled in by few_rows_gemm
+  int rotate;                // 1: column tiles start their walk through K at different places; filled in by few_rows_gemm
   int stream_experts;        // so many experts with rows and more: their weights are not kept; filled in by few_rows_gemm
 };
 // thin.hip: at most 32 rows in all (the two epilogues without a kept pre-activation, [E, N, K] weights)

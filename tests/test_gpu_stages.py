@@ -1258,3 +1258,46 @@ def test_few_rows_of_large_weights_by_experts_with_rows(counts, kn):
             ops.set_option(name, value)
     for a, b in zip(got, ref + ref):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("counts,N,K,apart", [
+    ([64, 1], 10304, 4096, True),              # 169 MB, a last column tile that is not full; one M tile each
+    ([100, 140], 6912, 6144, True),            # 170 MB; two M tiles of 128 rows for one of them
+    ([0, 33, 0], 20608, 4096, True),           # one expert with rows among three: their number is not known on the host
+    ([100, 157], 10304, 4096, False),          # more than 128 rows an expert on average
+    ([64, 1], 10304, 4160, False),             # rows that do not lie 4 KB apart
+    ([64, 1], 9728, 4096, False),              # 159 MB
+])
+def test_few_rows_of_weights_from_memory_start_at_places_of_their_own(counts, N, K, apart):
+    """By the rule, the column tiles of large [E, N, K] weights start inside K and go around: other bits than in ascending
+    order, and no further from the product in 64 bits (their errors' 2-norms within 5 %: both round about K sums of the
+    same terms, and then to fp16, which dominates).  The same bits from every epilogue, in a layer or alone, and from a
+    call with other rows beside them."""
+    from ccfuser_amd import ops
+    E, R = len(counts), sum(counts)
+    _say(f"starts apart {counts} N={N} K={K}")
+    g = torch.Generator(device="cuda").manual_seed(N + K + R)
+    rnd = lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, std, generator=g)
+    off = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    x, w, b = rnd(R, K), rnd(E, N, K, std=0.02), rnd(E, N)
+    ref = torch.cat([x[off[e]:off[e + 1]].double() @ w[e].double().t() + b[e].double() for e in range(E)])
+    new = lambda rows: torch.empty(rows, N, dtype=torch.float16, device="cuda")
+    out, h = {}, {}
+    try:
+        for mode in (2, 1):
+            ops.set_option("few_rows", mode)
+            out[mode] = ops.ffn2(x, None, off, R, w, b, new(R))
+            h[mode] = ops.ffn1(x, None, off, R, w, b)
+    finally:
+        ops.set_option("few_rows", 1)
+    assert torch.equal(out[1], out[2]) != apart and torch.equal(h[1], h[2]) != apart
+    err = {m: float((y.double() - ref).norm()) for m, y in out.items()}
+    assert err[1] <= 1.05 * err[2], err
+    assert torch.equal(out[1], ops.ffn2(x, None, off, R, w, b, new(R), in_layer=True))
+    act, pre = ops.ffn1_keep(x, None, off, R, w, b)
+    assert torch.equal(act, h[1]) and torch.equal(pre, out[1])
+    if apart and counts[1] > 1:                # the last expert's rows without one of them
+        e = max(i for i, c in enumerate(counts) if c)
+        fewer = off.clone()
+        fewer[e + 1:] -= 1
+        assert torch.equal(ops.ffn2(x, None, fewer, R - 1, w, b, new(R - 1)), out[1][:R - 1])
