@@ -50,75 +50,47 @@ struct FewCfg {
   static constexpr int A_DMA = TM / 4, B_DMA = DB / 2, LOADS = A_DMA + B_DMA;             // 1 KB loads per wavefront and stage
   static constexpr int A_BYTES = 16 * TM * kBK * 2, STAGE = A_BYTES + BN * kBK * 2;
   static constexpr int FIT = kFewLds / STAGE, STAGES = FIT > 8 ? 8 : FIT;
-  static_assert(TM % 4 == 0 && DB % 2 == 0 && STAGES >= 3 && (STAGES - 2) * LOADS < 63, "tile shape");
+  static_assert(TM % 4 == 0 && DB % 2 == 0 && STAGES >= 3 && (STAGES - 1) * LOADS < 63, "tile shape");
 };
 
-// One substep's fragments, waited for in the block that reads them: row blocks 32 rows (4096 bytes) apart, column
-// blocks 16 rows (2048 bytes) apart.
-template <int TMW, int NB>
-__device__ __forceinline__ void few_frags(half8 (&a)[TMW], half8 (&b)[NB], uint32_t ra, uint32_t rb);
-#define CCF_RD(o, base, off) "ds_read_b128 %" #o ", %" #base " offset:" #off "\n"
-#define CCF_LGKM "s_waitcnt lgkmcnt(0)"
-#define CCF_A2 "=&v"(a[0]), "=&v"(a[1])
-#define CCF_A4 CCF_A2, "=&v"(a[2]), "=&v"(a[3])
-#define CCF_B1 "=&v"(b[0])
-#define CCF_B2 CCF_B1, "=&v"(b[1])
-#define CCF_B4 CCF_B2, "=&v"(b[2]), "=&v"(b[3])
-#define CCF_FRAGS(TMW, NB, READS, ...)                                                                             \
-  template <>                                                                                                      \
-  __device__ __forceinline__ void few_frags<TMW, NB>(half8 (&a)[TMW], half8 (&b)[NB], uint32_t ra, uint32_t rb) { \
-    asm volatile(READS CCF_LGKM : __VA_ARGS__ : "v"(ra), "v"(rb) : "memory");                                      \
-  }
-CCF_FRAGS(2, 1, CCF_RD(0, 4, 0) CCF_RD(1, 3, 0) CCF_RD(2, 3, 4096), CCF_B1, CCF_A2)
-CCF_FRAGS(2, 2, CCF_RD(0, 5, 0) CCF_RD(1, 5, 2048) CCF_RD(2, 4, 0) CCF_RD(3, 4, 4096), CCF_B2, CCF_A2)
-CCF_FRAGS(2, 4, CCF_RD(0, 7, 0) CCF_RD(1, 7, 2048) CCF_RD(2, 7, 4096) CCF_RD(3, 7, 6144) CCF_RD(4, 6, 0) CCF_RD(5, 6, 4096),
-          CCF_B4, CCF_A2)
-CCF_FRAGS(4, 1, CCF_RD(0, 6, 0) CCF_RD(1, 5, 0) CCF_RD(2, 5, 4096) CCF_RD(3, 5, 8192) CCF_RD(4, 5, 12288), CCF_B1, CCF_A4)
-CCF_FRAGS(4, 2, CCF_RD(0, 7, 0) CCF_RD(1, 7, 2048) CCF_RD(2, 6, 0) CCF_RD(3, 6, 4096) CCF_RD(4, 6, 8192) CCF_RD(5, 6, 12288),
-          CCF_B2, CCF_A4)
-CCF_FRAGS(4, 4, CCF_RD(0, 9, 0) CCF_RD(1, 9, 2048) CCF_RD(2, 9, 4096) CCF_RD(3, 9, 6144) CCF_RD(4, 8, 0) CCF_RD(5, 8, 4096)
-                    CCF_RD(6, 8, 8192) CCF_RD(7, 8, 12288),
-          CCF_B4, CCF_A4)
-
-// The same for weights stored [K][N]: a column block's fragment is two transposing reads, K rows 0..3 and 4..7 of the
-// lane's eight (PITCH = 8 BN bytes apart), at the lane's address XOR 32 J.
-template <int TMW, int NB, int PITCH4>
-__device__ __forceinline__ void few_frags_kn(half8 (&a)[TMW], half8 (&b)[NB], uint32_t ra, uint32_t rb) {
-  static_assert((TMW == 2 || TMW == 4) && (NB == 2 || NB == 4), "written out below");
+// One K half's fragments of a wavefront: row blocks 32 rows (4096 bytes) apart, column blocks 16 rows (2048 bytes) apart.
+// For weights stored [K][N] (kKN) a column block's fragment is two transposing reads, K rows 0..3 and 4..7 of the lane's
+// eight (8 BN bytes apart), at the lane's address XOR 32 J.  read() leaves the reads in flight; ready() waits until at most
+// LATER reads that were issued behind them are, and ties the registers to the wait.
+template <class C, bool kKN>
+struct FewFrags {
+  static constexpr int TMW = C::TMW, NB = C::NB, READS = TMW + (kKN ? 2 : 1) * NB;
+  half8 a[TMW], b[NB];
   half4 lo[NB], hi[NB];
-#define CCF_TR(o, base) "ds_read_b64_tr_b16 %" #o ", %" #base "\n"
-#define CCF_TRH(o, base, off) "ds_read_b64_tr_b16 %" #o ", %" #base " offset:%" #off "\n"
-  if constexpr (NB == 2) {
-    if constexpr (TMW == 2)
-      asm volatile(CCF_TR(0, 7) CCF_TRH(1, 7, 9) CCF_TR(2, 8) CCF_TRH(3, 8, 9) CCF_RD(4, 6, 0) CCF_RD(5, 6, 4096) CCF_LGKM
-                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), CCF_A2
-                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "n"(PITCH4)
-                   : "memory");
-    else
-      asm volatile(CCF_TR(0, 9) CCF_TRH(1, 9, 11) CCF_TR(2, 10) CCF_TRH(3, 10, 11) CCF_RD(4, 8, 0) CCF_RD(5, 8, 4096)
-                   CCF_RD(6, 8, 8192) CCF_RD(7, 8, 12288) CCF_LGKM
-                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), CCF_A4
-                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "n"(PITCH4)
-                   : "memory");
-  } else {
-    if constexpr (TMW == 2)
-      asm volatile(CCF_TR(0, 11) CCF_TRH(1, 11, 15) CCF_TR(2, 12) CCF_TRH(3, 12, 15) CCF_TR(4, 13) CCF_TRH(5, 13, 15) CCF_TR(6, 14)
-                   CCF_TRH(7, 14, 15) CCF_RD(8, 10, 0) CCF_RD(9, 10, 4096) CCF_LGKM
-                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3]),
-                     CCF_A2
-                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "v"(rb ^ 64), "v"(rb ^ 96), "n"(PITCH4)
-                   : "memory");
-    else
-      asm volatile(CCF_TR(0, 13) CCF_TRH(1, 13, 17) CCF_TR(2, 14) CCF_TRH(3, 14, 17) CCF_TR(4, 15) CCF_TRH(5, 15, 17) CCF_TR(6, 16)
-                   CCF_TRH(7, 16, 17) CCF_RD(8, 12, 0) CCF_RD(9, 12, 4096) CCF_RD(10, 12, 8192) CCF_RD(11, 12, 12288) CCF_LGKM
-                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3]),
-                     CCF_A4
-                   : "v"(ra), "v"(rb), "v"(rb ^ 32), "v"(rb ^ 64), "v"(rb ^ 96), "n"(PITCH4)
-                   : "memory");
+  __device__ __forceinline__ void read(uint32_t ra, uint32_t rb) {
+    static_for<0, NB>([&](auto J) {
+      constexpr int j = J.value;
+      if constexpr (kKN) {
+        lo[j] = lds_read_tr_b64<0>(rb ^ (32 * j));
+        hi[j] = lds_read_tr_b64<8 * C::BN>(rb ^ (32 * j));
+      } else {
+        b[j] = lds_read_b128<2048 * j>(rb);
+      }
+    });
+    static_for<0, TMW>([&](auto I) { a[I.value] = lds_read_b128<4096 * I.value>(ra); });
   }
+  template <int LATER>
+  __device__ __forceinline__ void ready() {
+    static_assert(LATER < 15, "lgkmcnt has four bits");
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(LATER) : "memory");
 #pragma unroll
-  for (int i = 0; i < NB; ++i) b[i] = __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3, 4, 5, 6, 7);
-}
+    for (int j = 0; j < NB; ++j) {
+      if constexpr (kKN) {
+        asm volatile("" : "+v"(lo[j]), "+v"(hi[j]));
+        b[j] = __builtin_shufflevector(lo[j], hi[j], 0, 1, 2, 3, 4, 5, 6, 7);
+      } else {
+        asm volatile("" : "+v"(b[j]));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TMW; ++i) asm volatile("" : "+v"(a[i]));
+  }
+};
 
 // A [K][N] weight tile in LDS: 64 K rows of BN columns, the 32-byte chunks of each span of 128 columns XOR-swizzled by
 // the row (the layout of the 256-row tiles' main loop, gemm_tile.h).
@@ -202,7 +174,7 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
     }
   }
 
-  // The load side runs STAGES - 1 stages ahead: tile `it`, K tile `ik` of it.  Load j of a wavefront is 1 KB at
+  // The load side runs STAGES stages ahead: tile `it`, K tile `ik` of it.  Load j of a wavefront is 1 KB at
   // 1024 (8 j + wave) of the operand's part of the stage: eight 128-byte rows, or 1024 / (2 BN) K rows of a [K][N] tile.
   const half_t *a_src[C::A_DMA], *b_src[C::B_DMA];
   int it = 0, ik = 0, rot = 0;                                     // rot: the K tile that the walk starts with
@@ -260,8 +232,14 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
   };
   sources(tile_at(mine, 0));
 #pragma unroll
-  for (int s = 0; s < S - 1; ++s) issue(s);
+  for (int s = 0; s < S; ++s) issue(s);
 
+  // The fragments of a K half are read a half ahead of their use, so the barrier of a K step sits between its halves:
+  // behind it the next stage is complete, and everyone has read all of this one, which takes the load of S steps ahead.
+  FewFrags<C, kKN> f0, f1;
+  wait_vmcnt<(S - 1) * C::LOADS>();
+  block_barrier();
+  f0.read(a_off[0], b_off[0]);
   int stage = 0;
   for (int r = 0; r < nr; ++r) {
     const FewTile t = tile_at(mine, r);
@@ -271,28 +249,33 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
     for (int tm = 0; tm < TMW; ++tm)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) acc[tm][nb] = float4v{0, 0, 0, 0};
+    auto multiply = [&](const FewFrags<C, kKN> &f) {
+      static_for<0, TMW>([&](auto I) {
+        constexpr int tm = I.value;
+        if (2 * tm + wm < live) {                                  // uniform
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) acc[tm][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[nb], f.a[tm], acc[tm][nb], 0, 0, 0);
+        }
+      });
+    };
     for (int kt = 0; kt < KT; ++kt) {
-      // this step's stage has landed for this wavefront (the later ones may be in flight), then for all; behind
-      // the barrier everyone is also done with the stage of the step before, which takes the next load
-      wait_vmcnt<(S - 2) * C::LOADS>();
+      const int next = stage == S - 1 ? 0 : stage + 1;
+      const uint32_t so = stage * C::STAGE, sn = next * C::STAGE;
+      f1.read(so + a_off[1], so + b_off[1]);
+      f0.template ready<FewFrags<C, kKN>::READS>();
+      multiply(f0);
+      __builtin_amdgcn_sched_barrier(0);
+      f1.template ready<0>();
+      wait_vmcnt<(S - 2) * C::LOADS>();                            // the next stage has landed for this wavefront
       block_barrier();
-      issue(stage == 0 ? S - 1 : stage - 1);
-      const uint32_t so = stage * C::STAGE;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub) {
-        half8 a[TMW], b[NB];
-        if constexpr (kKN) few_frags_kn<TMW, NB, 8 * C::BN>(a, b, so + a_off[sub], so + b_off[sub]);
-        else few_frags<TMW, NB>(a, b, so + a_off[sub], so + b_off[sub]);
-        static_for<0, TMW>([&](auto I) {
-          constexpr int tm = I.value;
-          if (2 * tm + wm < live) {                                // uniform
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[tm][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[nb], a[tm], acc[tm][nb], 0, 0, 0);
-          }
-        });
-      }
-      stage = stage == S - 1 ? 0 : stage + 1;
+      issue(stage);
+      f0.read(sn + a_off[0], sn + b_off[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(f1);
+      __builtin_amdgcn_sched_barrier(0);
+      stage = next;
     }
+    f0.template ready<0>();                                        // the next tile's, or at the end nobody's
     // a lane holds one row and four consecutive columns of every block
     const half_t *bias_e = p.bias + static_cast<size_t>(t.e) * p.N;
     const int colb = t.n0 + wn * (16 * NB) + 4 * (lane >> 4);
