@@ -20,6 +20,8 @@
 #include "gelu.h"
 #include "plan.h"
 
+#include <cmath>
+
 namespace ccf {
 namespace {
 
@@ -1307,6 +1309,17 @@ bool few_tiles_cut(int max_rows, int E, int n_tiles_n, int k_tiles, int epi_cost
   return k_tiles / parts + kSplitFixed + sk.skinny * n_tiles_n * k_tiles / cus * kSkAloneStepPct / 100 + kSkInsideFixed < k_tiles + epi_cost;
 }
 
+// Whether the 256-row tiles of evenly popular experts fill one round of workgroups or less, most probably (two standard
+// deviations of their number): a remainder's tile then runs beside the others, and skinny tiles in its place take nothing
+// off but add a reduction launch, and their pricing to the plan's.  A training step of 1999 tokens of 768 / 3072, 8
+// experts, whose first product and its input gradient have about 220 tiles: 20 kernels of 318 us -> 18 of 307, the step on
+// a slow host 349 -> 340 us.
+bool fits_one_round(int max_rows, int E, int n_tiles_n, int cus) {
+  if (static_cast<long long>(max_rows / Cfg5::BM) * n_tiles_n > cus) return false;
+  const TileCount t = m_tiles(max_rows, E, Cfg5::BM);
+  return (t.mean + 2 * std::sqrt(t.var)) * n_tiles_n <= cus;
+}
+
 GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void *workspace, int region,
                      const GemmOptions &opt) {
   GemmSetup g;
@@ -1346,8 +1359,9 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   g.split = opt.split_tail && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 8 && cut_pays &&
             g.grid <= kTailMaxParts && v.bm == Cfg5::BM && v.bn == Cfg5::BN && K / 64 >= opt.split_tail_min_kt;
   // remainder rows as skinny tiles: forward epilogues of the persistent 256 x 256 kernel (either weight layout)
+  const bool one_round = !g.split && opt.skinny_pct > 0 && fits_one_round(max_rows, E, n_tiles_n, g.grid);
   g.skinny = opt.skinny_pct != 0 && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 64 &&
-             cut_pays &&
+             cut_pays && !one_round &&
              v.bm == Cfg5::BM && v.bn == Cfg5::BN && v.persistent_plain && (!wide || g.split);
   // skinny tiles may be cut along K (partial tiles in the split scratch, summed by the reduction launch) at any K,
   // also where the last round of 256-row tiles is not split

@@ -1301,3 +1301,37 @@ def test_few_rows_of_weights_from_memory_start_at_places_of_their_own(counts, N,
         fewer = off.clone()
         fewer[e + 1:] -= 1
         assert torch.equal(ops.ffn2(x, None, fewer, R - 1, w, b, new(R - 1)), out[1][:R - 1])
+
+
+@pytest.mark.parametrize("counts,N,K", [
+    ([513, 512, 511, 500, 257, 1, 0, 700], 3072, 768),       # remainders of one row, of none and of nearly a tile
+    ([300] * 8, 4096, 256),                                  # the shortest K, two tiles an expert: just a round
+    ([2040], 7168, 1024),
+])
+def test_one_round_of_tiles_has_no_skinny_tiles(counts, N, K):
+    """256-row tiles that fill a round at most need no reduction launch: both weight layouts and the form that keeps the
+    pre-activation against fp32 (sums of K terms, half an fp16 step), and the bits of the call without skinny tiles."""
+    from ccfuser_amd import ops
+    E, R = len(counts), sum(counts)
+    _say(f"one round {counts} N={N} K={K}")
+    g = torch.Generator(device="cuda").manual_seed(N + K + R)
+    rnd = lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, std, generator=g)
+    off = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    x, w, b = rnd(R, K), rnd(E, N, K, std=K ** -0.5), rnd(E, N)
+    kn = w.transpose(1, 2).contiguous()
+    ws = ops.ffn_workspace(R, E, K, N, x)
+    res = {}
+    try:
+        ops.set_option("few_rows", 0)
+        for skinny in (1, 0):
+            ops.set_option("skinny", skinny)
+            h = ops.ffn1(x, None, off, R, w, b, gelu=False, workspace=ws)
+            assert ops.ffn_plan_info(ws, R, E, K, N, 1)["skinny_tiles"] == 0
+            res[skinny] = (h, ops.ffn1(x, None, off, R, kn, b, gelu=False, w_kn=True), ops.ffn1_keep(x, None, off, R, w, b)[1])
+    finally:
+        ops.set_option("few_rows", 1)
+        ops.set_option("skinny", 1)
+    ref = torch.cat([x[off[e]:off[e + 1]].float() @ w[e].float().t() + b[e].float() for e in range(E)])
+    for a, c in zip(res[1], res[0]):
+        assert torch.equal(a, c)
+        assert float((a.float() - ref).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(ref.abs().max()) + 1e-4
