@@ -282,7 +282,7 @@ __device__ __forceinline__ void epilogue16(const GroupedArgs &p, int e, int row0
     half4 bv = {0, 0, 0, 0};
     if (p.bias && col[tn] < p.N) bv = *reinterpret_cast<const half4 *>(bias_e + col[tn]);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) bias_v[tn][c] = static_cast<float>(bv[c]);
+    for (int c = 0; c < 4; ++c) bias_v[tn][c] = (kEpi == kEpiGelu ? 0.5f : 1.0f) * static_cast<float>(bv[c]);
   }
   // Row data of all TM row blocks is looked up before the first accumulator is touched: one
   // memory round trip for the tile instead of one per row block (padded tile rows look up the
@@ -355,12 +355,17 @@ __device__ __forceinline__ void epilogue16(const GroupedArgs &p, int e, int row0
         if (kEpi == kEpiGeluGrad && col[tn] < p.N) pre = *reinterpret_cast<const half4 *>(row2 + col[tn]);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          float x = v[tn][c] + bias_v[tn][c];
-          if (kEpi == kEpiGeluGrad) {
-            x *= gelu_erf_grad(static_cast<float>(pre[c]));
+          float x;
+          if (kEpi == kEpiGelu) {
+            x = gelu_erf_of_twice(fmaf(v[tn][c], 0.5f, bias_v[tn][c]));   // FFN1: no row scale; half of the bias here
           } else {
-            if (kEpi == kEpiGeluKeep) pre[c] = static_cast<half_t>(x);
-            x = gelu_erf(x);                          // FFN1: no row scale
+            x = v[tn][c] + bias_v[tn][c];
+            if (kEpi == kEpiGeluKeep) {
+              pre[c] = static_cast<half_t>(x);
+              x = gelu_erf(x);
+            } else {
+              x *= gelu_erf_grad(static_cast<float>(pre[c]));
+            }
           }
           o[c] = static_cast<half_t>(x);
         }

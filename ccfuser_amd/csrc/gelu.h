@@ -5,44 +5,41 @@
 
 namespace ccf {
 
-// erf-form GELU, v * Phi(v) with Phi(v) = 0.5 + 0.5*erf(v/sqrt2) = 0.5 + u*Q(u^2), u = v
-// clamped to +-3*sqrt2 (beyond it 1 - erf < 2.3e-5).  0.5*erf(u/sqrt2) is an odd minimax
-// polynomial u*Q(u^2) of degree 8 in u^2, fitted on [0, 3] in z = u/sqrt2 with the 1/sqrt2
-// and the 0.5 folded into the coefficients.  Measured in fp32 against the exact function:
-// within 1.4e-5 for |v| <= 2, 5.9e-5 for |v| <= 8 (at -8 the result is -2e-5 instead of -0),
-// an eighth of the fp16 rounding step of a result of magnitude 1.  12 full-rate instructions
-// with the fp16 conversion and no transcendental (the library erff is ~40, the exp-based form
-// 15 plus rcp and exp at quarter rate); the FFN1 epilogue applies it to 256 values per lane
-// and tile and is bound by this arithmetic.
-__device__ __forceinline__ float gelu_erf(float v) {
-  const float u = __builtin_amdgcn_fmed3f(v, -4.2426406871192851464f, 4.2426406871192851464f);
-  const float t = u * u;
-  float q = 1.1253530e-10f * 0.5f;
-  q = fmaf(q, t, -1.0743734e-08f * 0.5f);
-  q = fmaf(q, t, 4.5365911e-07f * 0.5f);
-  q = fmaf(q, t, -1.1292428e-05f * 0.5f);
-  q = fmaf(q, t, 1.8718123e-04f * 0.5f);
-  q = fmaf(q, t, -2.2188006e-03f * 0.5f);
-  q = fmaf(q, t, 1.9636238e-02f * 0.5f);
-  q = fmaf(q, t, -1.3269384e-01f * 0.5f);
-  q = fmaf(q, t, 7.9780629e-01f * 0.5f);
-  return v * fmaf(u, q, 0.5f);
+// 1 - erfc(|v| / sqrt2) for h = v / 2.  erfc(sqrt2 |h|) is the eighth power of a polynomial of degree 5 in |h| that is 1 at
+// 0, kept within [0, 1]: the eighth root falls so slowly that degree 5 holds where erf itself, as u Q(u^2) on a clamped u,
+// took degree 17.  The absolute value and the clamp are modifiers of the instructions.  Exactly 1 beyond |v| of 6.2, and
+// for infinities (every partial sum then falls to -inf) and NaN.
+// (Coefficients: least maximum of (|v| + 1) times the error over |v| <= 9, by reweighted least squares.)
+__device__ __forceinline__ float erf_of_twice(float h) {
+  const float a = fabsf(h);
+  float q = -6.5160656e-03f;
+  q = fmaf(q, a, 3.3375409e-02f);
+  q = fmaf(q, a, -9.1669185e-03f);
+  q = fmaf(q, a, -1.3857770e-01f);
+  q = fmaf(q, a, -1.9951809e-01f);
+  q = __builtin_amdgcn_fmed3f(fmaf(q, a, 1.0f), 0.0f, 1.0f);
+  const float q2 = q * q, q4 = q2 * q2;
+  return fmaf(-q4, q4, 1.0f);
 }
 
-// Derivative of the erf GELU, Phi(v) + v*phi(v), with the same erf polynomial.
+// erf-form GELU of v = 2 h: h + |h| erf(|v| / sqrt2).  The caller has h for the price of v: half of a sum is one fused
+// multiply-add with half of the other addend.  Measured in fp32 against the exact function over all fp16 values: within
+// 3.4e-6 and within 4e-6 |v| (v * Phi(v) by the polynomial of degree 17: 5.5e-5 and 1.3e-5; below |v| = 0.1 that one
+// had 4e-6 |v| too).  NaN for -inf, as the exact form's -inf * 0.  Nine full-rate instructions, twelve before; the FFN1
+// epilogue applies it to 256 values per lane and tile and is bound by this arithmetic.
+__device__ __forceinline__ float gelu_erf_of_twice(float h) {
+  float g = fmaf(fabsf(h), erf_of_twice(h), h);
+  // rounded to fp32 in every kernel: fused with a conversion to fp16 behind it, as the compiler would have it in some of
+  // them, the instruction rounds once, and kernels that promise the same bits differ
+  asm("" : "+v"(g));
+  return g;
+}
+
+__device__ __forceinline__ float gelu_erf(float v) { return gelu_erf_of_twice(0.5f * v); }
+
+// Derivative of the erf GELU, Phi(v) + v*phi(v), with the same erf.
 __device__ __forceinline__ float gelu_erf_grad(float v) {
-  const float u = fminf(fabsf(v), 4.2426406871192851464f);
-  const float t = u * u;
-  float q = 1.1253530e-10f * 0.5f;
-  q = fmaf(q, t, -1.0743734e-08f * 0.5f);
-  q = fmaf(q, t, 4.5365911e-07f * 0.5f);
-  q = fmaf(q, t, -1.1292428e-05f * 0.5f);
-  q = fmaf(q, t, 1.8718123e-04f * 0.5f);
-  q = fmaf(q, t, -2.2188006e-03f * 0.5f);
-  q = fmaf(q, t, 1.9636238e-02f * 0.5f);
-  q = fmaf(q, t, -1.3269384e-01f * 0.5f);
-  q = fmaf(q, t, 7.9780629e-01f * 0.5f);
-  const float half_erf = copysignf(fminf(q * u, 0.5f), v);        // 0.5 * erf(v / sqrt2)
+  const float half_erf = copysignf(0.5f * erf_of_twice(0.5f * v), v);        // 0.5 * erf(v / sqrt2)
   // phi(v) = exp(-v^2/2) / sqrt(2 pi) = exp2(-v^2 * log2(e)/2) * 0.3989...
   const float pdf = 0.3989422804014327f * __builtin_amdgcn_exp2f(-0.72134752044448170368f * v * v);
   return fmaf(v, pdf, 0.5f + half_erf);
