@@ -46,8 +46,8 @@ constexpr int kPasses = kChunk / kThreads;       // indices per thread
 constexpr int kSub = kPasses * (kThreads / 64);  // wavefront passes per chunk
 constexpr int kMaxExpert = 1024;
 // Most chunks whose indices every workgroup of the pos launch counts itself instead of a hist launch in front of it.
-// Counting costs 2.3 us a chunk, a launch 4 (2 indices of 8 experts 7.0 -> 5.5 us, 1000: 8.9 -> 7.4, 2000: 9.6 -> 8.8,
-// 4000: 9.7 -> 11.5), and 4 us of host time less.
+// Counting another one's chunk costs 2.3 us, a launch 4 (2 indices of 8 experts 7.0 -> 5.5 us, 1000: 8.9 -> 7.4, 2000:
+// 9.6 -> 8.8, 4000: 9.7 -> 11.5; its own chunk counted twice over), and 4 us of host time less.
 constexpr int kSelfChunks = 2;
 constexpr int kRowsMaxInts = 32768;              // largest table of counts that the pos launch sums itself
 
@@ -185,32 +185,31 @@ pos_kernel(const int64_t *__restrict__ idx, int n, int E, int nbits, int top_k, 
            int64_t *__restrict__ idx_kept, int nchunk, int plan_wgs, PlanReq plan0, PlanReq plan1,
            const int32_t *__restrict__ rows, int nrows, int rows_per_chunk, int32_t *__restrict__ counts_out,
            int32_t *__restrict__ offsets_out, bool self_count) {
-  extern __shared__ int s_sub[];                 // [kSub][E], then with `rows`: [E] chunk base, [E] totals, [E + 1] offsets
+  extern __shared__ int s_sub[];                 // [kSub][E], then without a scan launch: [E] chunk base, [E] totals, [E + 1] offsets
   const bool is_plan = static_cast<int>(blockIdx.x) >= nchunk;
-  if (rows || self_count) {
-    // No scan launch: rows [nrows][E] hold counts of consecutive, equally long runs of flat
+  const bool sums = rows || self_count;          // no scan launch
+  const int own = blockIdx.x;
+  int *s_base = s_sub + kSub * E, *s_tot = s_base + E, *s_off = s_tot + E;
+  // This chunk's indices are requested first, and their wait falls together with the counts'; the experts' scan and that
+  // of the wavefront passes run side by side on different wavefronts.  The launch for 16384 indices of 64 experts in rows of
+  // 64 took 11.5 us with the four steps one behind the other, 8.1 so; 512 of four experts, whose one chunk was matched twice, 5.9 and
+  // 5.0 (rocprofv3).
+  int64_t raw[kPasses];
+  if (!is_plan) {
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int i = own * kChunk + p * kThreads + threadIdx.x;
+      raw[p] = i < n ? idx[i] : -1;
+    }
+  }
+  for (int i = (is_plan ? kSub * E : 0) + threadIdx.x; i < (sums ? kSub + 2 : kSub) * E; i += kThreads) s_sub[i] = 0;
+  __syncthreads();
+  if (rows) {
+    // Rows [nrows][E] hold counts of consecutive, equally long runs of flat
     // indices, rows_per_chunk of them per chunk.  Every workgroup adds up the rows in front of
     // its chunk (its rank base) and all rows (the experts' totals, hence the offsets).
-    int *s_base = s_sub + kSub * E, *s_tot = s_base + E, *s_off = s_tot + E;
-    for (int e = threadIdx.x; e < E; e += kThreads) { s_base[e] = 0; s_tot[e] = 0; }
-    __syncthreads();
-    const int first = is_plan ? 0 : static_cast<int>(blockIdx.x) * rows_per_chunk;   // rows in front of this chunk
-    if (self_count) {
-      // nor a hist launch: few chunks, whose indices every workgroup counts itself (first: chunks in front of this one)
-      for (int ch = 0; ch < nchunk; ++ch) {
-        int e_of[kPasses];
-#pragma unroll
-        for (int p = 0; p < kPasses; ++p) e_of[p] = load_expert(idx, ch * kChunk + p * kThreads + threadIdx.x, n, E);
-#pragma unroll
-        for (int p = 0; p < kPasses; ++p) {
-          const uint64_t peers = peers_of(e_of[p], e_of[p] >= 0, nbits);
-          if (e_of[p] >= 0 && (peers & lanes_below()) == 0) {
-            atomicAdd(&s_tot[e_of[p]], __popcll(peers));
-            if (ch < first) atomicAdd(&s_base[e_of[p]], __popcll(peers));
-          }
-        }
-      }
-    } else if (E % 4 == 0 && E <= 4 * kThreads && nrows * E > 4096 && (reinterpret_cast<uintptr_t>(rows) & 15) == 0) {
+    const int first = is_plan ? 0 : own * rows_per_chunk;          // rows in front of this chunk
+    if (E % 4 == 0 && E <= 4 * kThreads && nrows * E > 4096 && (reinterpret_cast<uintptr_t>(rows) & 15) == 0) {
       // a long table: four experts a load, which puts 16384 counts into 16 loads a thread, on the way together.  One count a
       // load, as below, waits for eight times eight of them: 16 us instead of 12 for 16384 indices of 64 experts in rows of
       // 64, whose hist launch (5 us) this table replaces.  (Short tables: the sums below meet in LDS less often.)
@@ -252,33 +251,82 @@ pos_kernel(const int64_t *__restrict__ idx, int n, int E, int nbits, int top_k, 
         s_base[e] = base;
       }
     }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      // capacity clamp and exclusive scan over experts by one wavefront, 64 at a time
-      int carry = 0;
-      const int lane = threadIdx.x;
-      for (int e0 = 0; e0 < E; e0 += 64) {
-        int v = 0;
-        if (e0 + lane < E) {
-          v = s_tot[e0 + lane];
-          v = (capacity >= 0 && v > capacity) ? capacity : v;
-          if (blockIdx.x == 0 && counts_out) counts_out[e0 + lane] = v;
-        }
-        int inc = v;
+  } else if (self_count) {
+    // nor a hist launch: few chunks, and every workgroup counts the other ones itself
+    for (int ch = 0; ch < nchunk; ++ch) {
+      if (ch == own) continue;
+      int e_of[kPasses];
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          int o = __shfl_up(inc, off, 64);
-          if (lane >= off) inc += o;
+      for (int p = 0; p < kPasses; ++p) e_of[p] = load_expert(idx, ch * kChunk + p * kThreads + threadIdx.x, n, E);
+#pragma unroll
+      for (int p = 0; p < kPasses; ++p) {
+        const uint64_t peers = peers_of(e_of[p], e_of[p] >= 0, nbits);
+        if (e_of[p] >= 0 && (peers & lanes_below()) == 0) {
+          atomicAdd(&s_tot[e_of[p]], __popcll(peers));
+          if (!is_plan && ch < own) atomicAdd(&s_base[e_of[p]], __popcll(peers));
         }
-        if (e0 + lane < E) s_off[e0 + lane] = carry + inc - v;
-        carry += __shfl(inc, 63, 64);
       }
-      if (lane == 0) s_off[E] = carry;
     }
-    __syncthreads();
+  }
+  const int wave = threadIdx.x >> 6;
+  int my_e[kPasses];
+  int my_rank[kPasses];
+  if (!is_plan) {
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int e = raw[p] >= 0 && raw[p] < E ? static_cast<int>(raw[p]) : -1;
+      const uint64_t peers = peers_of(e, e >= 0, nbits);
+      const uint64_t below = peers & lanes_below();
+      my_e[p] = e;
+      my_rank[p] = __popcll(below);
+      if (e >= 0 && below == 0) {
+        s_sub[(p * (kThreads / 64) + wave) * E + e] = __popcll(peers);
+        if (self_count) atomicAdd(&s_tot[e], __popcll(peers));
+      }
+    }
+  }
+  __syncthreads();
+  if (sums && threadIdx.x < 64) {
+    // capacity clamp and exclusive scan over experts by one wavefront, 64 at a time
+    int carry = 0;
+    const int lane = threadIdx.x;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      int v = 0;
+      if (e0 + lane < E) {
+        v = s_tot[e0 + lane];
+        v = (capacity >= 0 && v > capacity) ? capacity : v;
+        if (blockIdx.x == 0 && counts_out) counts_out[e0 + lane] = v;
+      }
+      int inc = v;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        int o = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += o;
+      }
+      if (e0 + lane < E) s_off[e0 + lane] = carry + inc - v;
+      carry += __shfl(inc, 63, 64);
+    }
+    if (lane == 0) s_off[E] = carry;
+  } else if (!is_plan) {
+    // exclusive running sum over the kSub wavefront passes, per expert (all read before the first is written: the compiler
+    // does not know that they are apart)
+    const int t0 = sums ? 64 : 0;
+    for (int e = threadIdx.x - t0; e < E; e += kThreads - t0) {
+      int run = sums ? s_base[e] : chunk_base[static_cast<size_t>(blockIdx.x) * E + e];
+      int v[kSub];
+#pragma unroll
+      for (int s = 0; s < kSub; ++s) v[s] = s_sub[s * E + e];
+#pragma unroll
+      for (int s = 0; s < kSub; ++s) {
+        s_sub[s * E + e] = run;
+        run += v[s];
+      }
+    }
+  }
+  __syncthreads();
+  if (sums) {
     if (blockIdx.x == 0)
       for (int e = threadIdx.x; e <= E; e += kThreads) offsets_out[e] = s_off[e];
-    chunk_base = nullptr;
     offsets = s_off;
   }
   // Workgroups past the chunks build the tile plans of the GEMMs that follow: the offsets are
@@ -288,34 +336,7 @@ pos_kernel(const int64_t *__restrict__ idx, int n, int E, int nbits, int top_k, 
     build_plan(r < plan_wgs ? plan0 : plan1, offsets, E, r % plan_wgs, plan_wgs);
     return;
   }
-  for (int i = threadIdx.x; i < kSub * E; i += kThreads) s_sub[i] = 0;
-  __syncthreads();
-  const int base = blockIdx.x * kChunk;
-  const int wave = threadIdx.x >> 6;
-  int my_e[kPasses];
-  int my_rank[kPasses];
-#pragma unroll
-  for (int p = 0; p < kPasses; ++p) {
-    const int i = base + p * kThreads + threadIdx.x;
-    const int e = load_expert(idx, i, n, E);
-    const uint64_t peers = peers_of(e, e >= 0, nbits);
-    const uint64_t below = peers & lanes_below();
-    my_e[p] = e;
-    my_rank[p] = __popcll(below);
-    if (e >= 0 && below == 0) s_sub[(p * (kThreads / 64) + wave) * E + e] = __popcll(peers);
-  }
-  __syncthreads();
-  // exclusive running sum over the kSub wavefront passes, per expert
-  for (int e = threadIdx.x; e < E; e += kThreads) {
-    int run = chunk_base ? chunk_base[static_cast<size_t>(blockIdx.x) * E + e] : s_sub[kSub * E + e];
-#pragma unroll
-    for (int s = 0; s < kSub; ++s) {
-      int v = s_sub[s * E + e];
-      s_sub[s * E + e] = run;
-      run += v;
-    }
-  }
-  __syncthreads();
+  const int base = own * kChunk;
 #pragma unroll
   for (int p = 0; p < kPasses; ++p) {
     const int i = base + p * kThreads + threadIdx.x;
