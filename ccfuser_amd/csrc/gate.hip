@@ -816,9 +816,12 @@ int launch_gate_f32_experts(const float *x, const float *wg, const float *bg, in
 // * Operands come in stages of 16 K elements through the wavefront's own LDS, as above, into one buffer: a
 //   wavefront's LDS accesses happen in order, so its writes of the next stage land behind its reads of this one.
 //   The last stage of a part loads the first of the wavefront's next part.
+// * LDS holds the part sums of two turns of the wavefronts (`turns`), so they meet at a barrier every second part: 8192
+//   tokens x 2048, 64 experts 50.7 -> 48.8 us, x 4096 89.1 -> 86.3; 30000 x 3000, 48 experts 253 -> 243.
 // * Eight threads select a token's experts (one per token: 4 us of 64 experts).
 //
-// 8192 tokens x 2048, 64 experts, top-2: 64 -> 49 us; x 4096: 116 -> 92; 32768 x 2048, 32 experts: 141 -> 96.
+// On the vector unit and so, first form: 8192 tokens x 2048, 64 experts, top-2: 64 and 49 us; x 4096: 116 and 92; 32768 x
+// 2048, 32 experts: 141 and 96.
 template <int N, int WE>
 struct GateF32Mfma {
   static constexpr int WT = 64 / N * N * N / WE;   // tokens of a tile
@@ -833,7 +836,7 @@ template <int N, int WE, int KS>
 __global__ void __launch_bounds__(kMaxWaves * 64)
 gate_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__ wg, const float *__restrict__ bg,
                      int tokens, int d, int E, int k, int64_t *__restrict__ idx_out,
-                     float *__restrict__ score_out, float *__restrict__ logits_out, int32_t *__restrict__ wg_cnt) {
+                     float *__restrict__ score_out, float *__restrict__ logits_out, int32_t *__restrict__ wg_cnt, int turns) {
 #pragma clang fp contract(off)
   using C = GateF32Mfma<N, WE>;
   using M = Mfma<N>;
@@ -841,8 +844,8 @@ gate_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__ wg, 
   const int waves = blockDim.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  float *region = s_mem + static_cast<size_t>(wave) * C::REGION;
-  float *s_logit = s_mem + static_cast<size_t>(waves) * C::REGION;       // [WT][LD] running sums, then logits
+  const int held = waves * turns;                                        // parts whose sums LDS holds at a time
+  float *s_logit = s_mem + static_cast<size_t>(held) * C::REGION;        // [WT][LD] running sums, then logits
   const int t0 = blockIdx.x * C::WT;
   const int nparts = (d + kPart - 1) / kPart;
   const int l_row = lane >> 2, l_piece = lane & 3;                       // as a loader
@@ -878,9 +881,9 @@ gate_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__ wg, 
       }
     };
     if (wave < nparts) fetch(wave * kPart, d);
-    for (int p0 = 0; p0 < nparts; p0 += waves) {
-      const int part = p0 + wave;
-      if (part < nparts) {                                               // uniform per wavefront
+    for (int p0 = 0; p0 < nparts; p0 += held) {
+      for (int part = p0 + wave; part < nparts && part < p0 + held; part += waves) {   // uniform per wavefront
+        float *region = s_mem + static_cast<size_t>(part - p0) * C::REGION;
         const int k_lo = part * kPart;
         const int k_hi = k_lo + kPart < d ? k_lo + kPart : d;
         float acc[M::kRegs];
@@ -927,13 +930,21 @@ gate_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__ wg, 
         }
       }
       __syncthreads();
-      const int np = nparts - p0 < waves ? nparts - p0 : waves;
-      const bool last = p0 + waves >= nparts;
+      const int np = nparts - p0 < held ? nparts - p0 : held;
+      const bool last = p0 + held >= nparts;
       for (int o = threadIdx.x; o < C::WT * WE; o += blockDim.x) {
         const int t = o / WE, e = o % WE;
         const int at = t * C::LD + e;
-        float s = p0 == 0 ? s_mem[at] : s_logit[at] + s_mem[at];
-        for (int w = 1; w < np; ++w) s = s + s_mem[static_cast<size_t>(w) * C::REGION + at];
+        float s = p0 == 0 ? 0.0f : s_logit[at];                          // (a part's sum is never -0)
+        int w = 0;
+        for (; w + kMaxWaves <= np; w += kMaxWaves) {                    // eight reads on their way
+          float part[kMaxWaves];
+#pragma unroll
+          for (int u = 0; u < kMaxWaves; ++u) part[u] = s_mem[static_cast<size_t>(w + u) * C::REGION + at];
+#pragma unroll
+          for (int u = 0; u < kMaxWaves; ++u) s = s + part[u];
+        }
+        for (; w < np; ++w) s = s + s_mem[static_cast<size_t>(w) * C::REGION + at];
         if (last && e0 + e < E) {
           if (bg) s = s + bg[e0 + e];
           if (logits_out && t0 + t < tokens) logits_out[static_cast<size_t>(t0 + t) * E + e0 + e] = s;
@@ -973,7 +984,11 @@ int launch_gate_f32_mfma(const float *x, const float *wg, const float *bg, int t
   using C = GateF32Mfma<N, WE>;
   const int nparts = (d + kPart - 1) / kPart;
   const int waves = nparts < kMaxWaves ? nparts : kMaxWaves;
-  const size_t lds = sizeof(float) * (static_cast<size_t>(waves) * C::REGION + C::WT * C::LD);
+  const auto lds_of = [&](int turns) { return sizeof(float) * (static_cast<size_t>(waves) * turns * C::REGION + C::WT * C::LD); };
+  // The 32-wide tiles' registers leave a CU one workgroup of eight wavefronts, which may as well have all of its LDS (not the
+  // 16-wide ones': two of them run side by side)
+  const int turns = N == 32 && nparts > waves && lds_of(2) <= 160 * 1024 ? 2 : 1;
+  const size_t lds = lds_of(turns);
   static_assert(sizeof(float) * (kMaxWaves * C::REGION + C::WT * C::LD) <= 160 * 1024, "LDS of a CU");
   auto kern = k <= 2 ? gate_f32_mfma_kernel<N, WE, 2> : gate_f32_mfma_kernel<N, WE, kMaxTopK>;
   if (lds > 65536) {
@@ -985,7 +1000,7 @@ int launch_gate_f32_mfma(const float *x, const float *wg, const float *bg, int t
   if (!counts_fit(wg_cnt, wgs, E, C::WT, k, max_cnt)) wg_cnt = nullptr;
   if (wg_cnt && tokens_per_wg) *tokens_per_wg = C::WT;
   hipLaunchKernelGGL(kern, dim3(wgs), dim3(waves * 64), lds, stream, x, wg, bg, tokens, d, E, k,
-                     idx_out, score_out, logits_out, wg_cnt);
+                     idx_out, score_out, logits_out, wg_cnt, turns);
   return check_launch("gate_f32_mfma_kernel");
 }
 

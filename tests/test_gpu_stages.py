@@ -73,7 +73,9 @@ def test_gate_fp32_tiles(T, d, E, k):
 
 @pytest.mark.parametrize("scale", [1.0, 1e-20])
 @pytest.mark.parametrize("T,d,E,k", [(4097, 8, 33, 2), (4127, 136, 64, 8), (4128, 1160, 70, 1), (8193, 648, 9, 2), (8256, 768, 16, 3),
-                                     (8257, 1064, 17, 1), (16385, 1536, 32, 2)])
+                                     (8257, 1064, 17, 1), (16385, 1536, 32, 2),
+                                     # part sums of two turns of the wavefronts at a time: 9, 16, 17 and 25 parts
+                                     (4097, 1032, 40, 2), (4130, 2048, 64, 2), (4099, 2056, 65, 2), (8200, 3080, 20, 1)])
 def test_gate_fp32_products_as_mfmas(T, d, E, k, scale):
     """Many tokens: the fp32 gate's products on the matrix cores, fewer parts of K than wavefronts and more, ragged in
     every direction, zeros of both signs, and operands whose products are subnormal or vanish: the oracle's bits."""
@@ -851,6 +853,30 @@ def test_ffn_special_cases():
     pre = ops.ffn1(dev(x), None, off, R, dev(w1), dev(b1), gelu=False)
     ref = x.float() @ w1[0].float().t() + b1.float()
     assert O.max_abs_err(pre.cpu(), ref) <= MAX_ABS
+
+
+@pytest.mark.usefixtures("gemm_form")
+@pytest.mark.parametrize("R", [4, 300])
+def test_gelu_of_every_fp16_value(R):
+    """Zero weights, every fp16 value as a bias: within the fp32 form's bound (4e-6 of the argument) and half an fp16
+    step of the exact function; infinities and NaN as the exact form has them; the same bits with the pre-activation kept."""
+    from ccfuser_amd import ops
+    d, f = 64, 65536
+    v = torch.arange(f, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    x, w = torch.ones(R, d, dtype=torch.float16), torch.zeros(1, f, d, dtype=torch.float16)
+    off = torch.tensor([0, R], dtype=torch.int32).cuda()
+    h = ops.ffn1(dev(x), None, off, R, dev(w), dev(v[None]), gelu=True)
+    kept, pre = ops.ffn1_keep(dev(x), None, off, R, dev(w), dev(v[None]))
+    bits = lambda t: t.nan_to_num(nan=7.0).view(torch.int16)
+    assert torch.equal(bits(h), bits(kept)) and torch.equal(bits(h), bits(h[:1].expand(R, f).contiguous()))
+    assert torch.equal(bits(pre[R - 1].cpu()), bits(v + 0.0))
+    got, u = h[R - 1].cpu().double(), v.double()
+    exact = 0.5 * u * torch.erfc(-u / 2.0 ** 0.5)
+    sane = torch.isfinite(u)
+    bound = 4e-6 * u.abs() + exact.abs() * 2.0 ** -11 + 2.0 ** -25
+    assert bool(((got - exact).abs() <= bound)[sane].all()), float(((got - exact).abs() / bound)[sane].max())
+    assert torch.equal(torch.isnan(got), torch.isnan(u) | (u == float("-inf")))
+    assert got[u == float("inf")] == float("inf")
 
 
 @pytest.mark.parametrize("inside", [1, 0])
