@@ -1544,7 +1544,10 @@ gate_bias_reduce_kernel(const float *__restrict__ partial, int n_wg, int E, half
 // writing grad_x.  Against the softmax kernel, its reduction and two library products, GPU time: 1000 tokens of 256, 16
 // experts 33 -> 16 us, 1999 of 768, 8: 22 -> 18, 4096 of 4096, 8: 42 -> 33, 32768 of 768, 8: 150 -> 65; and two launches
 // instead of four, the products' 15 us of host time each (1999 tokens, host included: 58 -> 23).  More than 16 experts
-// keep the products: the sums take so much LDS that a CU has one workgroup (8192 of 1024, 32: 47 against 57).
+// keep the products: the sums take so much LDS that a CU has one workgroup (8192 of 1024, 32: 47 against 57).  Since then eight
+// tokens' loads are ahead of their use and the reduction has no remainder loop: 1000 of 256, 16 experts 16.6 -> 14.0 us, 1999
+// of 768, 8: 18.7 -> 16.3, 4096 of 4096, 8: 33.1 -> 29.8, 32768 of 768, 8: 63.6 -> 56.4 (both launches, in a graph).  All 32 tokens'
+// loads of a run at once: 50 us for the 1999 tokens.
 //
 // A wavefront holds the values of 64 tokens in its lanes and broadcasts them through scalar registers; the expert
 // rows of wg sit in LDS, and the sums are plain reads and writes there (LDS float atomics run at ~190 cycles an
@@ -1602,14 +1605,17 @@ gate_products_kernel(const half_t *__restrict__ score, const half_t *__restrict_
         ex[j] = ex[j] >= 0 ? ex[j] : 0;              // nobody's choice: adds zero
       }
     }
-    constexpr int U = 8;                             // tokens whose loads leave together
-    for (int q0 = 0; q0 < n; q0 += U) {
-      half2v xv[U];
+    constexpr int U = 8;                             // tokens whose loads leave together, ahead of the eight before them
+    half2v xv[U], next[U];
+    const auto load = [&](half2v (&to)[U], int q0) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + u < n ? q0 + u : n - 1;
-        xv[u] = *reinterpret_cast<const half2v *>(x + static_cast<size_t>(base + q) * d + cc);
-      }
+      for (int u = 0; u < U; ++u) to[u] = *reinterpret_cast<const half2v *>(x + static_cast<size_t>(base + (q0 + u < n ? q0 + u : n - 1)) * d + cc);
+    };
+    load(next, 0);
+    for (int q0 = 0; q0 < n; q0 += U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) xv[u] = next[u];
+      load(next, q0 + U);                            // behind the last ones the last token again
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int q = q0 + u;
@@ -1644,6 +1650,20 @@ gate_products_kernel(const half_t *__restrict__ score, const half_t *__restrict_
   if (want_b && lane < E) partial_b[static_cast<size_t>(blockIdx.y) * E + lane] = bias;
 }
 
+// Sum of n values `ld` apart, in order, N loads on their way together: past the end the first one is read again and left out
+// (a remainder loop waits for each of its loads: 15 of 63).
+template <int N, class T, class Add>
+__device__ __forceinline__ void for_column(const T *col, size_t ld, int n, Add add) {
+  for (int r = 0; r < n; r += N) {
+    T v[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) v[u] = col[static_cast<size_t>(r + u < n ? r + u : 0) * ld];
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (r + u < n) add(v[u]);
+  }
+}
+
 // grad_wg (two columns per thread) and, in the workgroups behind them, grad_bias from the runs' partial sums, in order
 __global__ void __launch_bounds__(256)
 gate_products_reduce_kernel(const float *__restrict__ partial, const float *__restrict__ partial_b, int n_run, int E, int d,
@@ -1652,19 +1672,17 @@ gate_products_reduce_kernel(const float *__restrict__ partial, const float *__re
     const int e = threadIdx.x;
     if (e >= E) return;
     float acc = 0.0f;
-    for (int r = 0; r < n_run; ++r) acc += partial_b[static_cast<size_t>(r) * E + e];
+    for_column<32>(partial_b + e, E, n_run, [&](float v) { acc += v; });
     grad_bias[e] = static_cast<half_t>(acc);
     return;
   }
   const size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 2, n = static_cast<size_t>(E) * d;
   if (i >= n) return;
   float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll 16
-  for (int r = 0; r < n_run; ++r) {
-    const float2 v = *reinterpret_cast<const float2 *>(partial + static_cast<size_t>(r) * n + i);
+  for_column<32>(reinterpret_cast<const float2 *>(partial + i), n / 2, n_run, [&](const float2 &v) {
     a0 += v.x;
     a1 += v.y;
-  }
+  });
   *reinterpret_cast<half2v *>(grad_w + i) = half2v{static_cast<half_t>(a0), static_cast<half_t>(a1)};
 }
 
