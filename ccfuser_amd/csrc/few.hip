@@ -116,16 +116,21 @@ __device__ __forceinline__ void lds_dma16_nt(const void *gptr, lds_char *lds_wav
 // Where the walk through K starts.  Rows of a [N][K] weight that are a multiple of 4 KB apart hold the same K at the same
 // place of their pages, and workgroups that all start at the first K tile stay at about the same K: their loads fall on a
 // few of the memory's channels at a time, on how few depends on where the weight happens to lie.  So where the weights
-// come from HBM a tile's 256 columns go around from one of 16 places, 256 bytes apart, and the 32 tiles that an XCD runs at
-// a time are spread over all of them.  The sum starts elsewhere (its error is the same) and depends on neither the tile's
-// shape nor the other rows.  Microseconds for a layer's two products without and with it, three places of the weights each:
-//   8 experts of 4096 / 14336, 32 rows each 367, 366, 348 and 287, 288, 288, 83 rows 420, 405, 385 and 339, 340, 340;
-//   two experts, one row each 101 and 90; 64 rows of 16 of 2048 / 8192 248 and 188, 40 rows of 8 110, 122, 122 and 93, 92, 92;
-//   40 rows of 16 of 1536 / 6144 127 and 114; 33 rows of 32 of 1024 / 4096 113 and 97; 64 rows of 8 of 3584 / 14336 307, 289
-// (with places by a hash of the columns 295, 344, 91, 194, 95, 114, 99, 289; all of K instead of 4 KB in small steps no better).
-// Not for weights that stay in the Infinity Cache (64 rows of 16 experts of 1024 / 4096, 134 MB: FFN2 alone 25.2 and 26.8),
-// not for several M tiles an expert (200 rows of 8 of 2048 / 8192: FFN2 alone 90 and 96), not for other row strides (33
-// rows of 32 of 1024 / 4096: FFN1, 2 KB, 51.7 and 53.9; these three with a hash).
+// come from HBM a tile's 256 columns go around from one of 16 places, 256 bytes apart.  The sum starts elsewhere (its error is
+// the same), at a place that the column alone gives: not the tile's shape, nor the expert's slot, nor the other rows.
+// Microseconds for a layer's two products in ascending order and so, two places of the weights each:
+//   8 experts of 4096 / 14336, 32 rows each 313, 305 and 297, 296, 83 rows 347, 345 and 345, 344; two experts of it, one
+//   row each 113 and 102; 64 rows of 16 of 2048 / 8192 250, 253 and 198, 199, 40 rows of 8 126 and 99; 40 rows of 16 of
+//   1536 / 6144 127 and 119; 33 rows of 32 of 1024 / 4096 116, 112 and 105, 107; 64 rows of 8 of 3584 / 14336 314, 318 and 303.
+// The places are sums of the shifted column number, the best of 90 such over 11 layers: the column number itself falls in
+// with the channels' own pattern (those 16 of 2048 / 8192 206).  With 3 e added to it, places for every expert, 0 to 10 % faster
+// again where N is 2048 and less, whose few column ranges have few places (64 rows of 32 of 2048 / 2048: 146 ascending, 107
+// with 3 e, 117 here), the same at 4096 / 14336; but then an expert's results depend on its slot.
+// Not for weights that stay in the Infinity Cache (134 MB: 16 experts of 1024 / 4096, 64 rows each 68.1 and 68.0, 8 of 2048 / 4096
+// 65.7 and 66.0; 151 MB: 18 of 2048 / 2048 82 and 78), not for other row strides (5, 6, 7 and 10 KB, the first product of 8 experts
+// of 2560 / 10240, 3072 / 12288, 3584 / 14336, 5120 / 13824: 100.8, 118.9, 154.2, 214 and 100.8, 118.8, 154.7, 215), and not for several
+// M tiles an expert, where it wins and loses (200 rows of 8 of 2048 / 8192 183 and 174; 160 of 16 of 2048 / 6144, first product
+// 127 and 135).
 constexpr double kRotateBytes = 160e6;
 constexpr int kPlaces = 16, kPlaceStep = 2;        // K tiles of 128 bytes
 bool starts_apart(int max_rows, int E, int N, int K, bool b_kn) {
@@ -133,7 +138,10 @@ bool starts_apart(int max_rows, int E, int N, int K, bool b_kn) {
   const int used = E < max_rows ? E : max_rows;
   return !b_kn && K % 2048 == 0 && max_rows <= 128ll * used && 2.0 * used * N * K >= kRotateBytes;
 }
-__device__ __forceinline__ int first_k_tile(int e, int n0) { return kPlaceStep * (((n0 >> 8) + 3 * e) & (kPlaces - 1)); }
+__device__ __forceinline__ int first_k_tile(int n0) {
+  const int c = n0 >> 8;
+  return kPlaceStep * ((7 * c + 2 * (c >> 1) + 9 * (c >> 2) - (c >> 3) + 10 * (c >> 4)) & (kPlaces - 1));
+}
 
 // One lane's tile table entry.
 struct FewTile {
@@ -184,7 +192,7 @@ __device__ __forceinline__ void few_run(const FewArgs &p, const FewTile &mine, i
     const half_t *Be = p.B + static_cast<size_t>(t.e) * p.N * p.K;
     stream = kStream && t.alone;
     if constexpr (!kKN)
-      if (p.rotate) rot = first_k_tile(t.e, t.n0);
+      if (p.rotate) rot = first_k_tile(t.n0);
 #pragma unroll
     for (int j = 0; j < C::A_DMA; ++j) {
       const int r = (j * 8 + wave) * 8 + (lane >> 3);

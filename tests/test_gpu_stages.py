@@ -1329,6 +1329,30 @@ def test_few_rows_of_weights_from_memory_start_at_places_of_their_own(counts, N,
         assert torch.equal(ops.ffn2(x, None, fewer, R - 1, w, b, new(R - 1)), out[1][:R - 1])
 
 
+def test_places_of_a_sum_go_by_the_column_alone():
+    """Sums start where their column says: the same bits for an expert in another slot of the weights."""
+    from ccfuser_amd import ops
+    counts, N, K = [40, 24], 10304, 4096
+    E, R = len(counts), sum(counts)
+    _say("places by the column")
+    g = torch.Generator(device="cuda").manual_seed(R)
+    rnd = lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, std, generator=g)
+    x, w, b = rnd(R, K), rnd(E, N, K, std=0.02), rnd(E, N)
+
+    def product(x, counts, w, b):
+        off = torch.tensor([0] + counts).cumsum(0).int().cuda()
+        return ops.ffn2(x, None, off, len(x), w, b, torch.empty(len(x), N, dtype=torch.float16, device="cuda"))
+
+    out = product(x, counts, w, b)
+    ops.set_option("few_rows", 2)
+    try:
+        assert not torch.equal(out, product(x, counts, w, b))             # it is a call whose sums start inside K
+    finally:
+        ops.set_option("few_rows", 1)
+    swapped = product(torch.cat([x[40:], x[:40]]), counts[::-1], w.flip(0).contiguous(), b.flip(0).contiguous())
+    assert torch.equal(torch.cat([swapped[24:], swapped[:24]]), out)
+
+
 @pytest.mark.parametrize("counts,N,K", [
     ([513, 512, 511, 500, 257, 1, 0, 700], 3072, 768),       # remainders of one row, of none and of nearly a tile
     ([300] * 8, 4096, 256),                                  # the shortest K, two tiles an expert: just a round
