@@ -126,7 +126,9 @@ __device__ __forceinline__ void lds_dma16_nt(const void *gptr, lds_char *lds_wav
 // with the channels' own pattern (those 16 of 2048 / 8192 206).  With 3 e added to it, places for every expert, 0 to 10 % faster
 // again where N is 2048 and less, whose few column ranges have few places (64 rows of 32 of 2048 / 2048: 146 ascending, 107
 // with 3 e, 117 here), the same at 4096 / 14336; but then an expert's results depend on its slot.
-// Not for weights that stay in the Infinity Cache (134 MB: 16 experts of 1024 / 4096, 64 rows each 68.1 and 68.0, 8 of 2048 / 4096
+// Fewer rows than experts count as the others, so that a row's results are those of a larger call: the weights that they touch
+// may stay in the cache, where it makes no difference (one row of 8 of 4096 / 14336 78.7 and 78.8, 8 of 32 of 1024 / 4096 39.4 and
+// 39.2; four rows of the 8 202 and 147).  Not for weights that stay in the Infinity Cache anyhow (134 MB: 16 experts of 1024 / 4096, 64 rows each 68.1 and 68.0, 8 of 2048 / 4096
 // 65.7 and 66.0; 151 MB: 18 of 2048 / 2048 82 and 78), not for other row strides (5, 6, 7 and 10 KB, the first product of 8 experts
 // of 2560 / 10240, 3072 / 12288, 3584 / 14336, 5120 / 13824: 100.8, 118.9, 154.2, 214 and 100.8, 118.8, 154.7, 215), and not for several
 // M tiles an expert, where it wins and loses (200 rows of 8 of 2048 / 8192 183 and 174; 160 of 16 of 2048 / 6144, first product
@@ -135,8 +137,7 @@ constexpr double kRotateBytes = 160e6;
 constexpr int kPlaces = 16, kPlaceStep = 2;        // K tiles of 128 bytes
 bool starts_apart(int max_rows, int E, int N, int K, bool b_kn) {
   static_assert((kPlaces - 1) * kPlaceStep < 2048 / kBK, "a place inside the shortest K");
-  const int used = E < max_rows ? E : max_rows;
-  return !b_kn && K % 2048 == 0 && max_rows <= 128ll * used && 2.0 * used * N * K >= kRotateBytes;
+  return !b_kn && K % 2048 == 0 && max_rows <= 128ll * E && 2.0 * E * N * K >= kRotateBytes;
 }
 __device__ __forceinline__ int first_k_tile(int n0) {
   const int c = n0 >> 8;

@@ -83,9 +83,10 @@ const char *ccf_last_error(void);
  *                     needs no plan, at most 32 rows in all and a long contraction in one that cuts K over the
  *                     wavefronts of a workgroup; 0 = never, 2 = always in tiles of 64 or 128 rows, 16..21 = always, and
  *                     with that tile shape, 3 = cut over the wavefronts wherever that can be (at most 32 rows, [E, N, K]
- *                     weights), else as 2.  By the rule (1), column tiles of [E, N, K] weights that come from HBM, K a
- *                     multiple of 2048, start their sums at K places of their own; otherwise the sums of tiles of 64 or
- *                     128 rows are those of the 256-row tiles.  The knobs above apply to the 256-row tiles: with any of the first six away
+ *                     weights), else as 2.  By the rule (1), column tiles of [E, N, K] weights of 160 MB and more over all
+ *                     experts, K a multiple of 2048, at most 128 rows per expert on average, start their sums at K places of
+ *                     their own, which go by the column alone; otherwise the sums of tiles of 64 or 128 rows are those of
+ *                     the 256-row tiles.  The knobs above apply to the 256-row tiles: with any of the first six away
  *                     from its default, they are used
  *   "fused_combine"   0/1 (default 0): ccf_moe_forward with top_k = 2 adds the gate-weighted expert outputs
  *                     into the output in the second GEMM's epilogue (packed fp16 atomic adds onto zeros)

@@ -1353,6 +1353,25 @@ def test_places_of_a_sum_go_by_the_column_alone():
     assert torch.equal(torch.cat([swapped[24:], swapped[:24]]), out)
 
 
+def test_places_of_a_sum_for_fewer_rows_than_experts():
+    """Whether sums start inside K goes by the weights that are there, not by how many rows might touch them: a row has the
+    same bits alone in a call and beside others."""
+    from ccfuser_amd import ops
+    E, N, K = 2, 10304, 4096
+    _say("places with fewer rows than experts")
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, std, generator=g)
+    x, w, b = rnd(3, K), rnd(E, N, K, std=0.02), rnd(E, N)
+
+    def product(x, *counts):
+        off = torch.tensor([0, *counts]).cumsum(0).int().cuda()
+        return ops.ffn2(x, None, off, len(x), w, b, torch.empty(len(x), N, dtype=torch.float16, device="cuda"))
+
+    out = product(x, 2, 1)
+    for i, counts in enumerate(([1, 0], [1, 0], [0, 1])):
+        assert torch.equal(product(x[i:i + 1].contiguous(), *counts), out[i:i + 1]), i
+
+
 @pytest.mark.parametrize("counts,N,K", [
     ([513, 512, 511, 500, 257, 1, 0, 700], 3072, 768),       # remainders of one row, of none and of nearly a tile
     ([300] * 8, 4096, 256),                                  # the shortest K, two tiles an expert: just a round
