@@ -128,16 +128,20 @@ __device__ __forceinline__ void lds_dma16_nt(const void *gptr, lds_char *lds_wav
 // with 3 e, 117 here), the same at 4096 / 14336; but then an expert's results depend on its slot.
 // Fewer rows than experts count as the others, so that a row's results are those of a larger call: the weights that they touch
 // may stay in the cache, where it makes no difference (one row of 8 of 4096 / 14336 78.7 and 78.8, 8 of 32 of 1024 / 4096 39.4 and
-// 39.2; four rows of the 8 202 and 147).  Not for weights that stay in the Infinity Cache anyhow (134 MB: 16 experts of 1024 / 4096, 64 rows each 68.1 and 68.0, 8 of 2048 / 4096
-// 65.7 and 66.0; 151 MB: 18 of 2048 / 2048 82 and 78), not for other row strides (5, 6, 7 and 10 KB, the first product of 8 experts
-// of 2560 / 10240, 3072 / 12288, 3584 / 14336, 5120 / 13824: 100.8, 118.9, 154.2, 214 and 100.8, 118.8, 154.7, 215), and not for several
-// M tiles an expert, where it wins and loses (200 rows of 8 of 2048 / 8192 183 and 174; 160 of 16 of 2048 / 6144, first product
-// 127 and 135).
+// 39.2; four rows of the 8 202 and 147).
+// Not for weights that stay in the Infinity Cache anyhow (134 MB: 64 rows each of 16 of 1024 / 4096 68.1 and 68.0, of 8 of 2048 /
+// 4096 65.7 and 66.0; 151 MB: of 18 of 2048 / 2048 82 and 78), not for other row strides (5, 6, 7 and 10 KB, the first product of
+// 8 experts of 2560 / 10240, 3072 / 12288, 3584 / 14336, 5120 / 13824: 100.8, 118.9, 154.2, 214 and 100.8, 118.8, 154.7, 215),
+// and not for several M tiles an expert, where it wins and loses (200 rows of 8 of 2048 / 8192 183 and 174; 160 of 16 of 2048 /
+// 6144, first product, 127 and 135).
 constexpr double kRotateBytes = 160e6;
 constexpr int kPlaces = 16, kPlaceStep = 2;        // K tiles of 128 bytes
-bool starts_apart(int max_rows, int E, int N, int K, bool b_kn) {
+bool can_start_apart(int K) {
   static_assert((kPlaces - 1) * kPlaceStep < 2048 / kBK, "a place inside the shortest K");
-  return !b_kn && K % 2048 == 0 && max_rows <= 128ll * E && 2.0 * E * N * K >= kRotateBytes;
+  return K % 2048 == 0;
+}
+bool starts_apart(int max_rows, int E, int N, int K) {
+  return can_start_apart(K) && max_rows <= 128ll * E && 2.0 * E * N * K >= kRotateBytes;
 }
 __device__ __forceinline__ int first_k_tile(int n0) {
   const int c = n0 >> 8;
@@ -551,13 +555,14 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
   return mine < 1.02 * big;
 }
 
-int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, bool in_layer, int cus, hipStream_t stream, const char *what) {
+int few_rows_gemm(int mode, int places, FewArgs p, int epi, bool b_kn, bool in_layer, int cus, hipStream_t stream,
+                  const char *what) {
   if (thin_rows_fits(mode, p.max_rows, p.E, p.N, p.K, epi, b_kn)) return thin_rows_gemm(p, epi, stream, what);
   p.force = mode >= 16 ? mode & 15 : -1;
   const double experts = std::ceil((in_layer ? kStreamBytes / 2 : kStreamBytes) / (2.0 * p.N * p.K));
   const bool large = experts <= (p.E < p.max_rows ? p.E : p.max_rows);
   p.stream_experts = large ? static_cast<int>(experts) : INT_MAX;
-  p.rotate = mode == 1 && starts_apart(p.max_rows, p.E, p.N, p.K, b_kn);
+  p.rotate = places < 0 ? mode == 1 && starts_apart(p.max_rows, p.E, p.N, p.K) && !b_kn : places && can_start_apart(p.K) && !b_kn;
   const auto pick = [&](auto S_) -> void (*)(FewArgs) {
     constexpr bool S = decltype(S_)::value;
     if (b_kn) return epi == kFewPlain ? few_rows_kernel<kFewPlain, true, S> : few_rows_kernel<kFewGelu, true, S>;

@@ -1195,13 +1195,14 @@ int g_skinny_positions = 0;  // skinny ranges inside the persistent launch: 0 = 
 int g_split_inside = 1;      // 1: the parts of a split last round run inside the persistent launch, 0: as a launch of their own
 int g_skinny_tail = 0;       // 0: skinny tiles never run as a launch of their own
 int g_few_rows = 1;          // few rows per expert as tiles of 64 or 128 rows (few.hip): the modes of few_rows_fits()
+int g_few_places = -1;       // their sums start at K places of their own: -1 = by the rule of few.hip, 0 = never, 1 = wherever they can
 
 // The tuning knobs a grouped GEMM's plan and launches depend on, read once per call: the plan
 // and the kernels that consume it must agree even if another thread calls ccf_set_option
 // between the routing stage (which builds the plans of the layer's forward call) and the GEMMs.
 GemmOptions current_options() {
   return GemmOptions{g_variant, g_split_tail, g_split_tail_min_kt, g_split_max_parts, g_skinny_pct, g_fused_combine,
-                     g_skinny_tail, g_split_inside, g_few_rows};
+                     g_skinny_tail, g_split_inside, g_few_rows, g_few_places};
 }
 
 // The kernels of one family of epilogues: `first` and `second` are two epilogue forms, each as
@@ -1418,8 +1419,9 @@ int grouped_gemm(const half_t *A, const int32_t *a_rows, const int32_t *offsets,
   if (max_rows == 0) return CCF_OK;
   const GemmOptions options = opt ? *opt : current_options();
   if (use_few_rows(max_rows, E, N, K, epi, b_kn, options))
-    return few_rows_gemm(options.few_rows, FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1, 0}, epi,
-                         b_kn, in_layer, persistent_grid(), stream, what);
+    return few_rows_gemm(options.few_rows, options.few_places,
+                         FewArgs{A, a_rows, B, bias, C, C2, c_rows, row_scale, offsets, max_rows, E, N, K, -1, 0}, epi, b_kn,
+                         in_layer, persistent_grid(), stream, what);
   const GemmSetup gs = setup_gemm(max_rows, E, N, K, epi, b_kn, workspace, region, options);
   const Launch &v = *gs.v;
   const bool second = gs.second, split = gs.split;
@@ -1845,6 +1847,11 @@ extern "C" int ccf_set_option(const char *name, int value) {
     CCF_REQUIRE((value >= 0 && value <= 3) || (value >= 16 && value < 22), CCF_ERR_ARG,
                 "set_option: few_rows %d is neither 0..3 nor 16..21", value);
     g_few_rows = value;
+    return CCF_OK;
+  }
+  if (!strcmp(name, "few_rows_places")) {
+    CCF_REQUIRE(value >= -1 && value <= 1, CCF_ERR_ARG, "set_option: few_rows_places %d is neither -1, 0 nor 1", value);
+    g_few_places = value;
     return CCF_OK;
   }
   if (!strcmp(name, "gate_waves")) {

@@ -501,7 +501,8 @@ __device__ inline void build_plan(const PlanReq &rq, const int32_t *__restrict__
 // ffn.hip
 // Snapshot of the tuning knobs (ccf_set_option) that a grouped GEMM's plan and launches depend on.
 struct GemmOptions {
-  int variant, split_tail, split_tail_min_kt, split_max_parts, skinny_pct, fused_combine, skinny_tail, split_inside, few_rows;
+  int variant, split_tail, split_tail_min_kt, split_max_parts, skinny_pct, fused_combine, skinny_tail, split_inside, few_rows,
+      few_places;
 };
 GemmOptions forward_options();
 bool forward_plan_request(int which, int max_rows, int E, int d, int f, void *workspace, const GemmOptions &opt,
@@ -585,9 +586,11 @@ int thin_rows_gemm(const FewArgs &p, int epi, hipStream_t stream, const char *wh
 // mode: GemmOptions::few_rows (0: never, 1: by the rule, 2: always, 3: always, in the form of thin.hip where that can,
 // 16 + i: always and with tile shape i)
 bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_kn, int cus);
+// places: GemmOptions::few_places (-1: sums start at places of their own by the rule, 0: never, 1: wherever they can)
 // in_layer: before these weights are read again, as many bytes pass as they have (the layer's other product, or the weight
 // gradient)
-int few_rows_gemm(int mode, FewArgs p, int epi, bool b_kn, bool in_layer, int cus, hipStream_t stream, const char *what);
+int few_rows_gemm(int mode, int places, FewArgs p, int epi, bool b_kn, bool in_layer, int cus, hipStream_t stream,
+                  const char *what);
 
 // most entries of a table of per-run expert counts that the routing stage takes from the gate kernel
 long long route_rows_max_ints();

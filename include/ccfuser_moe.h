@@ -85,9 +85,11 @@ const char *ccf_last_error(void);
  *                     with that tile shape, 3 = cut over the wavefronts wherever that can be (at most 32 rows, [E, N, K]
  *                     weights), else as 2.  By the rule (1), column tiles of [E, N, K] weights of 160 MB and more over all
  *                     experts, K a multiple of 2048, at most 128 rows per expert on average, start their sums at K places of
- *                     their own, which go by the column alone; otherwise the sums of tiles of 64 or 128 rows are those of
- *                     the 256-row tiles.  The knobs above apply to the 256-row tiles: with any of the first six away
+ *                     their own, which go by the column alone ("few_rows_places"); otherwise the sums of tiles of 64 or
+ *                     128 rows are those of the 256-row tiles.  The knobs above apply to the 256-row tiles: with any of the first six away
  *                     from its default, they are used
+ *   "few_rows_places" -1 (default): the rule above; 0 = never: the sums of tiles of 64 or 128 rows are always those of the
+ *                     256-row tiles; 1 = in every mode of "few_rows", for all [E, N, K] weights with K a multiple of 2048
  *   "fused_combine"   0/1 (default 0): ccf_moe_forward with top_k = 2 adds the gate-weighted expert outputs
  *                     into the output in the second GEMM's epilogue (packed fp16 atomic adds onto zeros)
  *                     instead of running the combine pass; measured slower, kept for comparison

@@ -1372,6 +1372,86 @@ def test_places_of_a_sum_for_fewer_rows_than_experts():
         assert torch.equal(product(x[i:i + 1].contiguous(), *counts), out[i:i + 1]), i
 
 
+@pytest.mark.parametrize("K", [2048, 4096])
+def test_places_of_a_sum_in_every_tile_shape(K):
+    """Sums that start inside K, in tiles of all shapes with several tiles per workgroup, one and more M tiles an expert and
+    a last column tile that is not full, with and without non-temporal loads: the same bits from every shape, other
+    ones than in ascending order, and as near to the product in 64 bits as those (2-norms within 5 %: fp16 rounding dominates
+    both)."""
+    from ccfuser_amd import ops
+    counts, N = [1, 64, 65, 130, 0, 128, 33, 5, 127, 16, 260, 48, 2, 70, 64, 20, 17, 100, 3], 4136
+    E, R = len(counts), sum(counts)
+    _say(f"places in every shape K={K}")
+    g = torch.Generator(device="cuda").manual_seed(K)
+    rnd = lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, std, generator=g)
+    off = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    x, w, b, scale = rnd(R + 9, K), rnd(E, N, K, std=0.02), rnd(E, N), rnd(R)
+    perm = lambda n: torch.randperm(n, generator=g, device="cuda")[:R].int()
+    src, dst = perm(R + 9), perm(R)
+    kn = w.transpose(1, 2).contiguous()
+
+    def outputs(in_layer):
+        y = torch.empty(R, N, dtype=torch.float16, device="cuda")
+        plain = ops.ffn2(x, dst, off, R, w, b, y, row_scale=scale, src_row=src, in_layer=in_layer)
+        act, pre = ops.ffn1_keep(x, src, off, R, w, b)
+        return plain, ops.ffn1(x, src, off, R, w, b, in_layer=in_layer), act, pre
+
+    out = {}
+    try:
+        for shape in range(6):
+            ops.set_option("few_rows", 16 + shape)
+            for places in (1, 0):
+                ops.set_option("few_rows_places", places)
+                out[shape, places] = outputs(False)
+                for a, c in zip(outputs(True), out[shape, places]):
+                    assert torch.equal(a, c), (shape, places)
+                for a, c in zip(out[shape, places], out[0, places]):
+                    assert torch.equal(a, c), (shape, places)
+        ops.set_option("few_rows_places", 1)                      # [E, K, N] weights keep the ascending order
+        assert torch.equal(ops.ffn1(x, src, off, R, kn, b, w_kn=True), out[0, 0][1])
+    finally:
+        ops.set_option("few_rows", 1)
+        ops.set_option("few_rows_places", -1)
+    for a, c in zip(out[0, 1], out[0, 0]):
+        assert not torch.equal(a, c)
+    xs = x[src.long()].double()
+    pre = torch.cat([xs[off[e]:off[e + 1]] @ w[e].double().t() + b[e].double() for e in range(E)])
+    err = [float((out[0, p][3].double() - pre).norm()) for p in (1, 0)]
+    assert err[0] <= 1.05 * err[1], err
+    assert torch.equal(out[0, 1][1], out[0, 1][2])
+
+
+def test_places_of_a_sum_over_two_rounds_of_tiles():
+    """A decoding batch's first product by the rule: each workgroup has a second column tile, whose places are other ones.
+    No further from the product in 64 bits than the ascending sums (squares within 10 %: fp16 rounding dominates both), and
+    their bits with the places switched off."""
+    from ccfuser_amd import ops
+    E, rows, N, K = 8, 32, 14336, 4096
+    R = E * rows
+    _say("places over two rounds")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, std, generator=g)
+    off = (torch.arange(E + 1) * rows).int().cuda()
+    x, w, b = rnd(R, K), rnd(E, N, K, std=0.02), rnd(E, N)
+    out = {}
+    try:
+        for mode, places in ((1, -1), (2, -1), (1, 0)):
+            ops.set_option("few_rows", mode)
+            ops.set_option("few_rows_places", places)
+            out[mode, places] = ops.ffn2(x, None, off, R, w, b, torch.empty(R, N, dtype=torch.float16, device="cuda"))
+    finally:
+        ops.set_option("few_rows", 1)
+        ops.set_option("few_rows_places", -1)
+    assert torch.equal(out[1, 0], out[2, -1]) and not torch.equal(out[1, -1], out[1, 0])
+    sq = {key: 0.0 for key in out}
+    for e in range(E):
+        at = slice(e * rows, (e + 1) * rows)
+        ref = x[at].double() @ w[e].double().t() + b[e].double()
+        for key, y in out.items():
+            sq[key] += float((y[at].double() - ref).square().sum())
+    assert sq[1, -1] <= 1.1 * sq[1, 0], sq
+
+
 @pytest.mark.parametrize("counts,N,K", [
     ([513, 512, 511, 500, 257, 1, 0, 700], 3072, 768),       # remainders of one row, of none and of nearly a tile
     ([300] * 8, 4096, 256),                                  # the shortest K, two tiles an expert: just a round
