@@ -1317,11 +1317,22 @@ bool few_tiles_cut(int max_rows, int E, int n_tiles_n, int k_tiles, int epi_cost
 
 // Whether the 256-row tiles of evenly popular experts fill one round of workgroups or less, most probably (two standard
 // deviations of their number): a remainder's tile then runs beside the others, and skinny tiles in its place take nothing
-// off but add a reduction launch, and their pricing to the plan's.  A training step of 1999 tokens of 768 / 3072, 8
-// experts, whose first product and its input gradient have about 220 tiles: 20 kernels of 318 us -> 18 of 307, the step on
-// a slow host 349 -> 340 us.
-bool fits_one_round(int max_rows, int E, int n_tiles_n, int cus) {
+// off but add a reduction launch, and their pricing to the plan's.  The 20 kernels of a training step of 1999 tokens of 768 /
+// 3072, 8 experts, whose first product and its input gradient have about 220 tiles, take 318 us -> 18 of 307.
+// Uneven loads, which only the device knows, may make more tiles than a round, and a second one costs a whole tile: where K
+// is long the plan is left a choice unless such loads fit too, with remainders spread evenly over 0 to 256 rows (a standard
+// deviation more).  Microseconds with skinny tiles planned and without, Zipf loads of exponent 1.2 or 1.5: 12762 rows of 32
+// experts, K of 3136 101 and 131 (284 tiles); 1144 of 8, 2048: 88 and 98 (288); 3302 of 16, 2432: 101 and 115 (345).  Of 160 GEMMs
+// whose even loads fit, half of them with such loads, it takes the slower way by over 2 % in 7 (13 % at most), without this
+// condition in 11 (18 %); the mean gain is 7.5 %.
+constexpr int kOneRoundKT = 16;
+bool fits_one_round(int max_rows, int E, int n_tiles_n, int k_tiles, int cus) {
   if (static_cast<long long>(max_rows / Cfg5::BM) * n_tiles_n > cus) return false;
+  if (k_tiles > kOneRoundKT) {
+    const int used = E < max_rows ? E : max_rows;
+    const double uneven = static_cast<double>(max_rows) / Cfg5::BM + 0.5 * used + std::sqrt(used / 12.0);
+    if (uneven * n_tiles_n > cus) return false;
+  }
   const TileCount t = m_tiles(max_rows, E, Cfg5::BM);
   return (t.mean + 2 * std::sqrt(t.var)) * n_tiles_n <= cus;
 }
@@ -1365,7 +1376,7 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   g.split = opt.split_tail && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 8 && cut_pays &&
             g.grid <= kTailMaxParts && v.bm == Cfg5::BM && v.bn == Cfg5::BN && K / 64 >= opt.split_tail_min_kt;
   // remainder rows as skinny tiles: forward epilogues of the persistent 256 x 256 kernel (either weight layout)
-  const bool one_round = !g.split && opt.skinny_pct > 0 && fits_one_round(max_rows, E, n_tiles_n, g.grid);
+  const bool one_round = !g.split && opt.skinny_pct > 0 && fits_one_round(max_rows, E, n_tiles_n, kt_all, g.grid);
   g.skinny = opt.skinny_pct != 0 && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 64 &&
              cut_pays && !one_round &&
              v.bm == Cfg5::BM && v.bn == Cfg5::BN && v.persistent_plain && (!wide || g.split);

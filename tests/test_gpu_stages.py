@@ -1454,7 +1454,7 @@ def test_places_of_a_sum_over_two_rounds_of_tiles():
 
 @pytest.mark.parametrize("counts,N,K", [
     ([513, 512, 511, 500, 257, 1, 0, 700], 3072, 768),       # remainders of one row, of none and of nearly a tile
-    ([300] * 8, 4096, 256),                                  # the shortest K, two tiles an expert: just a round
+    ([300] * 8, 3840, 256),                                  # the shortest K, two tiles an expert: just inside a round
     ([2040], 7168, 1024),
 ])
 def test_one_round_of_tiles_has_no_skinny_tiles(counts, N, K):
@@ -1484,3 +1484,64 @@ def test_one_round_of_tiles_has_no_skinny_tiles(counts, N, K):
     for a, c in zip(res[1], res[0]):
         assert torch.equal(a, c)
         assert float((a.float() - ref).abs().max()) <= (2.0 ** -11 + K * 2.0 ** -24) * float(ref.abs().max()) + 1e-4
+
+
+def _launches(fn):
+    """Kernel launches of a call: the nodes of a graph that captures it."""
+    import ctypes as C
+    from ccfuser_amd import _lib
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        fn()
+    n = C.c_size_t(0)
+    get = _lib.lib().hipGraphGetNodes                         # of the HIP runtime that the library is linked to
+    assert get(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
+def _zipf_counts(E, R, skew):
+    w = torch.arange(1, E + 1).double() ** -skew
+    counts = (w / w.sum() * R).floor().long()
+    counts[0] += R - counts.sum()
+    return counts[torch.randperm(E, generator=torch.Generator().manual_seed(E))].tolist()
+
+
+@pytest.mark.parametrize("E,R,skew,N,K,one_round", [
+    (8, 3998, 0.0, 3072, 768, True),           # a training step's first product
+    (8, 3998, 0.0, 3328, 768, False),          # another column tile: two standard deviations beyond a round
+    (8, 2400, 0.0, 3840, 256, True),           # the shortest K, just inside a round
+    (8, 2400, 0.0, 4096, 256, False),
+    (16, 3644, 1.5, 3072, 768, True),          # uneven loads of more than a round (300 tiles), K too short to cut
+    (8, 3236, 0.0, 4096, 1024, True),          # where uneven loads might not fit: the last K that may, and the first that may not
+    (8, 3236, 0.0, 4096, 1088, False),
+    (16, 7000, 1.5, 1536, 3584, True),         # a long K whose uneven loads fit
+    (32, 12762, 1.5, 896, 3136, False),        # and one whose uneven loads do not (284 tiles): 130 us in tiles only, 100 with skinny ones
+])
+def test_one_round_of_tiles_by_sizes(E, R, skew, N, K, one_round):
+    """Which sizes of 256-row tiles plan neither skinny tiles nor a reduction launch, in both weight layouts; results
+    against fp32 (sums of K terms, half an fp16 step)."""
+    from ccfuser_amd import ops
+    _say(f"one round E={E} R={R} skew={skew} N={N} K={K}")
+    counts = _zipf_counts(E, R, skew)
+    g = torch.Generator(device="cuda").manual_seed(N + K + R)
+    rnd = lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda").normal_(0.0, std, generator=g)
+    off = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    x, w, b = rnd(R, K), rnd(E, N, K, std=K ** -0.5), rnd(E, N)
+    ws = ops.ffn_workspace(R, E, K, N, x)
+    tiles = sum(-(-c // 256) for c in counts) * -(-N // 256)
+    ref = torch.cat([x[off[e]:off[e + 1]].float() @ w[e].float().t() + b[e].float() for e in range(E)])
+    ops.set_option("few_rows", 0)
+    try:
+        for weight, kn in ((w, False), (w.transpose(1, 2).contiguous(), True)):
+            out = torch.empty(R, N, dtype=torch.float16, device="cuda")
+            call = lambda: ops.ffn1(x, None, off, R, weight, b, gelu=False, out=out, workspace=ws, w_kn=kn)
+            assert _launches(call) == (2 if one_round else 3), kn      # plan and product; with the reduction
+            call()
+            if skew and not one_round:                                 # the plan can still help loads of more than a round
+                assert tiles > 256 and ops.ffn_plan_info(ws, R, E, K, N, 1)["skinny_tiles"] > 0
+            tol = K * 2.0 ** -24 * K ** 0.5 + 2.0 ** -11 * ref.abs()
+            assert ((out.float() - ref).abs() <= tol + 1e-6).all()
+    finally:
+        ops.set_option("few_rows", 1)
