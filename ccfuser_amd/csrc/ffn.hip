@@ -1376,10 +1376,10 @@ GemmSetup setup_gemm(int max_rows, int E, int N, int K, int epi, bool b_kn, void
   g.split = opt.split_tail && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 8 && cut_pays &&
             g.grid <= kTailMaxParts && v.bm == Cfg5::BM && v.bn == Cfg5::BN && K / 64 >= opt.split_tail_min_kt;
   // remainder rows as skinny tiles: forward epilogues of the persistent 256 x 256 kernel (either weight layout)
-  const bool one_round = !g.split && opt.skinny_pct > 0 && fits_one_round(max_rows, E, n_tiles_n, kt_all, g.grid);
+  // (fits_one_round() last: 0.08 us on the host path, only for calls that it decides something for)
   g.skinny = opt.skinny_pct != 0 && epi <= (b_kn ? kEpiGelu : kEpiGeluKeep) && g.grid >= 64 &&
-             cut_pays && !one_round &&
-             v.bm == Cfg5::BM && v.bn == Cfg5::BN && v.persistent_plain && (!wide || g.split);
+             cut_pays && v.bm == Cfg5::BM && v.bn == Cfg5::BN && v.persistent_plain && (!wide || g.split) &&
+             !(!g.split && opt.skinny_pct > 0 && fits_one_round(max_rows, E, n_tiles_n, kt_all, g.grid));
   // skinny tiles may be cut along K (partial tiles in the split scratch, summed by the reduction launch) at any K,
   // also where the last round of 256-row tiles is not split
   g.cut = g.skinny && !wide && g.grid <= kTailMaxParts;
