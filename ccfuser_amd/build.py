@@ -45,6 +45,12 @@ ACC_CHECKED = {
     "ffn.hip": r"_ZN3ccf\S*grouped_gemm\S*",
     "probe.hip": r"_ZN3ccf\S*mfma_probe_kernel\S*",
 }
+# Sources whose kernels leave LDS reads written in inline asm in flight behind the statement that issues them, and the
+# kernels that do.  The compiler takes such a register as written at once: a copy of it, or another value put into it,
+# ahead of the wait would be silently wrong.  They are scanned for that, along all branches, and for spills.
+READS_CHECKED = {
+    "few.hip": r"_ZN3ccf\S*few_rows_kernel\S*",
+}
 _NOISE = "is not a recognized feature for this target"
 
 
@@ -90,6 +96,116 @@ def acc_register_violations(asm_text: str, name_regex: str):
     return bad
 
 
+_REGISTER = re.compile(r"(?<![\w.])([va])(?:(\d+)|\[(\w+)(?::(\w+))?\])")
+
+
+def _registers(operands: str) -> int:
+    """The vector and accumulation registers that an operand list names, as a bit mask."""
+    mask = 0
+    for kind, one, lo, hi in _REGISTER.findall(operands):
+        first = int(one or lo, 0)
+        last = int(hi, 0) if hi else first
+        mask |= ((1 << (last - first + 1)) - 1) << (first + (512 if kind == "a" else 0))
+    return mask
+
+
+def _instructions(body: str):
+    """(operation, operands) of every instruction of a kernel, and the index that each label stands for."""
+    code, labels = [], {}
+    for line in body.splitlines():
+        text = line.split(";")[0].split("//")[0].strip()
+        label = re.match(r"([.\w$]+):$", text)
+        if label:
+            labels[label.group(1)] = len(code)
+        elif text and not text.startswith("."):
+            op, _, operands = text.replace("\t", " ").partition(" ")
+            code.append((op, operands.strip()))
+    return code, labels
+
+
+def pending_read_violations(body: str):
+    """Instructions of a kernel that name the destination of an LDS or memory load ahead of the wait that covers it.
+
+    Loads of either kind return in order, so a wait for at most n of them leaves the n newest.  Per block of code the
+    state is, for either kind, the destinations by age, newest last; where branches meet, a destination has every age
+    that it may have, which can only find too much.  A load may overwrite the destination of an earlier one of its kind."""
+    code, labels = _instructions(body)
+    steps = []
+    for op, operands in code:
+        first, _, rest = operands.partition(",")
+        if op.startswith("ds_"):
+            loads = re.search(r"read|permute|swizzle|rtn", op) is not None
+            steps.append(("lds", _registers(rest if loads else operands), _registers(first) if loads else 0))
+        elif re.match(r"(global|buffer|scratch)_", op):
+            loads = "load" in op and "_lds_" not in op or "atomic" in op and "sc0" in operands
+            steps.append(("mem", _registers(rest if loads else operands), _registers(first) if loads else 0))
+        elif op == "s_waitcnt":
+            left = {kind: re.search(name + r"\((\d+)\)", operands) for kind, name in (("lds", "lgkmcnt"), ("mem", "vmcnt"))}
+            if "cnt(" not in operands:
+                raise ValueError(f"{op} {operands}")
+            steps.append(("wait", {kind: int(m.group(1)) for kind, m in left.items() if m}, 0))
+        elif op == "s_branch" or op.startswith("s_cbranch"):
+            steps.append(("jump" if op == "s_branch" else "branch", labels[operands], 0))
+        elif op == "s_endpgm":
+            steps.append(("end", 0, 0))
+        elif re.match(r"flat_|s_(setpc|swappc|call)", op):
+            raise ValueError(f"{op} {operands}")
+        else:
+            steps.append(("other", _registers(operands), 0))
+    heads = sorted({0, *labels.values(), *(i + 1 for i, s in enumerate(steps) if s[0] in ("jump", "branch", "end"))})
+    block_end = dict(zip(heads, heads[1:] + [len(steps)]))
+    entry, todo, bad = {0: {"lds": [], "mem": []}}, [0], set()
+
+    def meet(at, state):
+        known = entry.setdefault(at, {"lds": None, "mem": None})
+        grown = False
+        for kind, ages in state.items():
+            ages = ages[-64:]
+            old = known[kind]
+            if old is None:
+                known[kind], grown = list(ages), True
+                continue
+            old[:0] = [0] * (len(ages) - len(old))
+            for q in range(1, len(ages) + 1):
+                grown = grown or bool(ages[-q] & ~old[-q])
+                old[-q] |= ages[-q]
+        if grown:
+            todo.append(at)
+
+    while todo:
+        at = todo.pop()
+        state = {kind: list(ages) for kind, ages in entry[at].items()}
+        end = block_end.get(at, len(steps))
+        while at < end:
+            kind, named, dest = steps[at]
+            at += 1
+            if kind == "wait":
+                for which, left in named.items():
+                    del state[which][:max(len(state[which]) - left, 0)]
+            elif kind in ("jump", "branch"):
+                meet(named, state)
+                if kind == "jump":
+                    break
+            elif kind == "end":
+                break
+            else:
+                for which, ages in state.items():
+                    if any(p & (named if which == kind else named | dest) for p in ages):
+                        bad.add((at - 1, " ".join(code[at - 1])))
+                if kind != "other":
+                    state[kind].append(dest)
+        else:
+            if at < len(steps):
+                meet(at, state)
+    return [text for _, text in sorted(bad)]
+
+
+def spilled_bytes(asm_text: str, name_regex: str):
+    """{kernel: bytes of scratch memory a thread needs} from the kernels' metadata."""
+    records = re.findall(r"\.name:\s+(\S+)((?:(?!\.name:).)*?)\.private_segment_fixed_size:\s+(\d+)", asm_text, flags=re.S)
+    return {name: int(size) for name, _, size in records if re.fullmatch(name_regex, name)}
+
+
 def device_assembly(src: str, out: Path) -> str:
     rc, err = _run([HIPCC, *COMMON, *PER_FILE.get(src, []), "-S", "--cuda-device-only", str(CSRC / src), "-o", str(out)])
     if rc != 0:
@@ -101,10 +217,19 @@ def _check(src: str) -> None:
     obj_dir = CSRC / "_obj"
     obj_dir.mkdir(exist_ok=True)
     text = device_assembly(src, obj_dir / (src + ".s"))
-    bad = acc_register_violations(text, ACC_CHECKED[src])
-    if bad:
-        raise RuntimeError(f"{src}: the compiler uses accumulation registers that the kernels name themselves, "
-                           f"or spills; such a binary faults the GPU and is not linked: {bad[:3]}")
+    if src in ACC_CHECKED:
+        bad = acc_register_violations(text, ACC_CHECKED[src])
+        if bad:
+            raise RuntimeError(f"{src}: the compiler uses accumulation registers that the kernels name themselves, "
+                               f"or spills; such a binary faults the GPU and is not linked: {bad[:3]}")
+    if src in READS_CHECKED:
+        for name, body in kernel_bodies(text, READS_CHECKED[src]):
+            bad = pending_read_violations(body)
+            if bad:
+                raise RuntimeError(f"{src}: {name} touches the destination of a read in flight; not linked: {bad[:3]}")
+        bad = {k: n for k, n in spilled_bytes(text, READS_CHECKED[src]).items() if n}
+        if bad:
+            raise RuntimeError(f"{src}: spills next to reads in flight; not linked: {bad}")
 
 
 def _link(objs, lib: Path) -> None:
@@ -115,11 +240,11 @@ def _link(objs, lib: Path) -> None:
 
 
 def build(verbose: bool = True) -> Path:
-    """Compile every HIP source, scan the kernels that own their accumulation registers, and
+    """Compile every HIP source, scan the kernels that own their accumulation registers or leave reads in flight, and
     link both shared libraries.  Always recompiles."""
     srcs = SOURCES + PROBE_SOURCES
     with ThreadPoolExecutor(max_workers=8) as pool:
-        checks = [pool.submit(_check, s) for s in ACC_CHECKED]
+        checks = [pool.submit(_check, s) for s in {**ACC_CHECKED, **READS_CHECKED}]
         objs = dict(zip(srcs, pool.map(_compile, srcs)))
         for c in checks:
             c.result()

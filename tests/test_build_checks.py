@@ -85,3 +85,62 @@ def test_gate_kernels_keep_their_values_in_registers(tmp_path):
         forms["stream" if "stream" in name else "mfma"] += 1
     # tile widths 16 and 32, 1/2/4 slots, three list lengths of the selection
     assert forms["mfma"] >= 15 and forms["stream"] >= 15, forms
+
+
+def _few_rows_kernels(text):
+    from ccfuser_amd import build as B
+    return B.kernel_bodies(text, B.READS_CHECKED["few.hip"])
+
+
+@needs_hipcc
+def test_few_row_kernels_touch_no_read_in_flight(tmp_path):
+    """The few-row tiles read a half K step's fragments ahead of their use, in inline asm, across the loop's back edge: no
+    instruction may name such a register before its wait, and nothing may spill.  With the waits for the older half left
+    out, or one of its registers copied behind the reads, the scan finds it."""
+    import re
+    from ccfuser_amd import build as B
+    text = B.device_assembly("few.hip", tmp_path / "few.s")
+    kernels = _few_rows_kernels(text)
+    assert len(kernels) == 10, [name for name, _ in kernels]
+    spilled = B.spilled_bytes(text, B.READS_CHECKED["few.hip"])
+    assert len(spilled) == 10 and not any(spilled.values()), spilled
+    for name, body in kernels:
+        assert body.count("ds_read_b128") >= 24, name
+        assert B.pending_read_violations(body) == [], name
+    body = kernels[-1][1]
+    asm_waits = re.compile(r"(s_waitcnt lgkmcnt\()([1-9]\d*)(\))")
+    assert len(asm_waits.findall(body)) >= 6                                # one per tile shape
+    assert B.pending_read_violations(asm_waits.sub(lambda m: f"{m[1]}{int(m[2]) + 1}{m[3]}", body)) != []
+    for read in list(re.finditer(r"\n\tds_read_b128 v\[(\d+):\d+\][^\n]*", body))[::40]:
+        copy = f"\n\tv_mov_b32_e32 v255, v{read.group(1)}"
+        assert B.pending_read_violations(body[:read.end()] + copy + body[read.end():]) != [], read.group(0)
+
+
+@pytest.mark.parametrize("body,found", [
+    # waited for, also where an older read is the one that is used
+    ("ds_read_b128 v[0:3], v8\nds_read_b128 v[4:7], v8\ns_waitcnt lgkmcnt(1)\nv_mov_b32 v9, v0\ns_endpgm", []),
+    ("ds_read_b128 v[0:3], v8\nds_read_b128 v[4:7], v8\ns_waitcnt lgkmcnt(1)\nv_mov_b32 v9, v4\ns_endpgm", ["v_mov_b32 v9, v4"]),
+    # overwritten, and used as an address, while in flight
+    ("ds_read_b32 v0, v8\nv_mov_b32 v0, 0\ns_waitcnt lgkmcnt(0)\ns_endpgm", ["v_mov_b32 v0, 0"]),
+    ("ds_read_b32 v0, v8\nds_read_b32 v1, v0\ns_endpgm", ["ds_read_b32 v1, v0"]),
+    # across a back edge: the second turn copies what the first one left in flight
+    (".L1:\nv_mov_b32 v9, v1\nds_read_b32 v1, v8\ns_cbranch_scc1 .L1\ns_endpgm", ["v_mov_b32 v9, v1"]),
+    (".L1:\nv_mov_b32 v9, v1\nds_read_b32 v1, v8\ns_waitcnt lgkmcnt(0)\ns_cbranch_scc1 .L1\ns_endpgm", []),
+    # one of two ways to a place waits
+    ("ds_read_b32 v1, v8\ns_cbranch_scc1 .L1\ns_waitcnt lgkmcnt(0)\n.L1:\nv_mov_b32 v9, v1\ns_endpgm", ["v_mov_b32 v9, v1"]),
+    # memory loads have a count of their own; loads to LDS leave no register
+    ("global_load_dword v1, v[8:9], off\ns_waitcnt lgkmcnt(0)\nv_mov_b32 v2, v1\ns_endpgm", ["v_mov_b32 v2, v1"]),
+    ("global_load_dword v1, v[8:9], off\nglobal_load_lds_dwordx4 v[8:9], off\ns_waitcnt vmcnt(1)\nv_mov_b32 v2, v1\ns_endpgm", []),
+    # a load behind another one to the same register comes back behind it
+    ("ds_read_b32 v1, v8\nds_read_b32 v1, v7\ns_waitcnt lgkmcnt(0)\nv_mov_b32 v2, v1\ns_endpgm", []),
+])
+def test_the_scan_for_reads_in_flight(body, found):
+    from ccfuser_amd import build as B
+    assert B.pending_read_violations(body) == found
+
+
+def test_the_scan_refuses_what_it_cannot_follow():
+    from ccfuser_amd import build as B
+    for line in ("s_swappc_b64 s[30:31], s[0:1]", "flat_load_dword v0, v[2:3]", "s_waitcnt 0x0"):
+        with pytest.raises(ValueError):
+            B.pending_read_violations(line + "\ns_endpgm")
