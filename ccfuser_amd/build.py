@@ -51,6 +51,11 @@ ACC_CHECKED = {
 READS_CHECKED = {
     "few.hip": r"_ZN3ccf\S*few_rows_kernel\S*",
 }
+# Kernels with such reads whose branches depend on each other in ways that the scan cannot see, so that it finds uses on
+# ways that no wavefront takes: scanned for copies of pending registers, which the compiler makes where loops meet.
+COPIES_CHECKED = {
+    "ffn.hip": r"_ZN3ccf\S*grouped_gemm\S*",
+}
 _NOISE = "is not a recognized feature for this target"
 
 
@@ -123,8 +128,9 @@ def _instructions(body: str):
     return code, labels
 
 
-def pending_read_violations(body: str):
-    """Instructions of a kernel that name the destination of an LDS or memory load ahead of the wait that covers it.
+def pending_read_violations(body: str, copies_only: bool = False):
+    """Instructions of a kernel that name the destination of an LDS or memory load ahead of the wait that covers it;
+    copies_only: register moves that name an LDS read's.
 
     Loads of either kind return in order, so a wait for at most n of them leaves the n newest.  Per block of code the
     state is, for either kind, the destinations by age, newest last; where branches meet, a destination has every age
@@ -190,6 +196,8 @@ def pending_read_violations(body: str):
                 break
             else:
                 for which, ages in state.items():
+                    if copies_only and not (which == "lds" and re.match(r"v_(mov|accvgpr)", code[at - 1][0])):
+                        continue
                     if any(p & (named if which == kind else named | dest) for p in ages):
                         bad.add((at - 1, " ".join(code[at - 1])))
                 if kind != "other":
@@ -227,6 +235,11 @@ def _check(src: str) -> None:
             bad = pending_read_violations(body)
             if bad:
                 raise RuntimeError(f"{src}: {name} touches the destination of a read in flight; not linked: {bad[:3]}")
+    for name, body in kernel_bodies(text, COPIES_CHECKED[src]) if src in COPIES_CHECKED else []:
+        bad = pending_read_violations(body, copies_only=True)
+        if bad:
+            raise RuntimeError(f"{src}: {name} copies the destination of a read in flight; not linked: {bad[:3]}")
+    if src in READS_CHECKED:
         bad = {k: n for k, n in spilled_bytes(text, READS_CHECKED[src]).items() if n}
         if bad:
             raise RuntimeError(f"{src}: spills next to reads in flight; not linked: {bad}")
@@ -244,7 +257,7 @@ def build(verbose: bool = True) -> Path:
     link both shared libraries.  Always recompiles."""
     srcs = SOURCES + PROBE_SOURCES
     with ThreadPoolExecutor(max_workers=8) as pool:
-        checks = [pool.submit(_check, s) for s in {**ACC_CHECKED, **READS_CHECKED}]
+        checks = [pool.submit(_check, s) for s in {**ACC_CHECKED, **READS_CHECKED, **COPIES_CHECKED}]
         objs = dict(zip(srcs, pool.map(_compile, srcs)))
         for c in checks:
             c.result()

@@ -498,6 +498,7 @@ struct Ring16Mainloop {
       k2 += Cfg::BK;
       ph = ph == NSLOT - 1 ? 0 : ph + 1;
     }
+    frags_ready(a[0], b[0]);                         // the next step's, or tile's: the compiler may copy them from here on
     phase = ph;
   }
 
@@ -595,6 +596,7 @@ struct Ring16Mainloop {
     int phase = 0;
     reserve();
     zero_acc();
+    frags_ready(a[0], b[0]);                         // before the compiler copies them for the two loops below
     acc_settle();
     // past the end of K the last K tile is fetched again into slots nobody reads
     if (live_m == TM) {

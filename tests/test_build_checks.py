@@ -116,6 +116,19 @@ def test_few_row_kernels_touch_no_read_in_flight(tmp_path):
         assert B.pending_read_violations(body[:read.end()] + copy + body[read.end():]) != [], read.group(0)
 
 
+@needs_hipcc
+def test_256_row_kernels_copy_no_fragment_in_flight(tmp_path):
+    """The 256-row tiles' main loop ends with the next tile's fragments being read.  The compiler copies them between the
+    loops that it has for full and partly filled tiles, which must be behind their wait: a tile of few rows is through the
+    rest of its last step before the reads are."""
+    from ccfuser_amd import build as B
+    text = B.device_assembly("ffn.hip", tmp_path / "ffn.s")
+    kernels = [k for k in B.kernel_bodies(text, B.COPIES_CHECKED["ffn.hip"]) if "ds_read" in k[1]]
+    assert len(kernels) >= 20, [name for name, _ in kernels]
+    for name, body in kernels:
+        assert B.pending_read_violations(body, copies_only=True) == [], name
+
+
 @pytest.mark.parametrize("body,found", [
     # waited for, also where an older read is the one that is used
     ("ds_read_b128 v[0:3], v8\nds_read_b128 v[4:7], v8\ns_waitcnt lgkmcnt(1)\nv_mov_b32 v9, v0\ns_endpgm", []),
@@ -137,6 +150,13 @@ def test_few_row_kernels_touch_no_read_in_flight(tmp_path):
 def test_the_scan_for_reads_in_flight(body, found):
     from ccfuser_amd import build as B
     assert B.pending_read_violations(body) == found
+
+
+def test_the_scan_for_copies_only():
+    from ccfuser_amd import build as B
+    body = "ds_read_b32 v1, v8\nv_add_u32 v2, v1, v1\n{}\ns_waitcnt lgkmcnt(0)\nv_mov_b32 v3, v1\ns_endpgm"
+    assert B.pending_read_violations(body.format("v_mov_b64 v[4:5], v[0:1]"), copies_only=True) == ["v_mov_b64 v[4:5], v[0:1]"]
+    assert B.pending_read_violations(body.format("v_mov_b64 v[4:5], v[6:7]"), copies_only=True) == []
 
 
 def test_the_scan_refuses_what_it_cannot_follow():
