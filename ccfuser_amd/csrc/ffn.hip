@@ -873,7 +873,7 @@ grouped_gemm_persistent_kernel(GroupedArgs p, int slots_per_xcd) {
     const int k_end = KT * Cfg::BK;
 
     R::zero_acc();
-    R::frags_ready(fa[0], fb[0]);                     // the first tile's, behind the zeros
+    if constexpr (!kRows) R::frags_ready(fa[0], fb[0]);      // the first tile's, behind the zeros
 
     int next_row[kRows ? 1 : Cfg::A_DMA];             // A row of the next tile per tile load
     if constexpr (!kSeg) {

@@ -498,7 +498,9 @@ struct Ring16Mainloop {
       k2 += Cfg::BK;
       ph = ph == NSLOT - 1 ? 0 : ph + 1;
     }
-    frags_ready(a[0], b[0]);                         // the next step's, or tile's: the compiler may copy them from here on
+    // The next step's, or tile's, fragments: the compiler copies them from here on where its loops are for full and for
+    // partly filled tiles.  The form with both operands [K][.] has full ones only and no copies (the build scans for them).
+    if constexpr (!A_KM) frags_ready(a[0], b[0]);
     phase = ph;
   }
 
