@@ -14,14 +14,15 @@
 //     this one).  One workgroup of eight wavefronts per CU: two workgroups of four with half of the LDS each
 //     measured the same at many tiles and up to a quarter slower at one tile per CU, whose weights then stream
 //     through a pipeline of half the depth;
-//   * accumulation runs over K in 32-wide steps in ascending order, as in the 256-row tiles: same bits (large weights by
-//     the rule start inside K and go around: starts_apart()).
+//   * accumulation runs over K in 32-wide steps in ascending order, as in the 256-row tiles: same bits.  By the rule, tiles
+//     of large weights start inside K, at a place that the column gives, and go around: other bits than the 256-row tiles'
+//     and than those of a call of more rows, the same for every tile shape and slot of an expert (starts_apart()).
 //
-// Bound by streaming the weights from HBM at 5.3 - 5.7 TB/s where they are large, by the latency of a few dependent
+// Bound by streaming the weights from HBM at 6.2 - 6.7 TB/s where they are large, by the latency of a few dependent
 // steps where they are small.  FFN1 / FFN2 including their plan and reduction launches, 256-row tiles -> here:
-// 8 experts of 4096 / 14336, 32 rows each: 205 -> 165 and 176 -> 172 us, 83 rows each: 213 -> 191 and 201 -> 177;
-// 4 experts of 256 / 1024, 128 rows each: 20 -> 10 and 28 -> 10; FFN2 of 8 experts of 768 / 3072, 500 rows
-// each: 70 -> 38; 16 experts of 1024 / 4096, 64 rows each: 37 -> 28 and 53 -> 31.
+// 8 experts of 4096 / 14336, 32 rows each: 202 -> 150 and 192 -> 140 us, 83 rows each: 199 -> 171 and 203 -> 163;
+// 4 experts of 256 / 1024, 128 rows each: 21 -> 8 and 28 -> 10; FFN2 of 8 experts of 768 / 3072, 500 rows
+// each: 62 -> 37; 16 experts of 1024 / 4096, 64 rows each: 31 -> 28 and 44 -> 26.
 #include "ccf_common.h"
 #include "gelu.h"
 #include "gemm_tile.h"
@@ -37,7 +38,8 @@ constexpr int kFewLds = 163840;
 constexpr int kFewMaxRounds = 64;      // most tiles of a workgroup: one per lane of the tile table
 constexpr int kBK = 64;
 // A K step of 64 and an epilogue (GELU, plain) by tile shape, in microseconds: fitted to 2520 timed launches of all
-// shapes where the weights' bytes do not bound them, 4 to 9 % off each
+// shapes where the weights' bytes do not bound them, 4 to 9 % off each (before fragments were read ahead of their use, which
+// took up to 16 % off a step: see few_rows_fits)
 constexpr double kFewStepUs[6] = {0.274, 0.415, 0.705, 0.408, 0.600, 0.900};
 constexpr double kFewEpiUs[2][6] = {{1.3, 2.2, 3.2, 2.7, 5.5, 8.7}, {0.8, 0.6, 0.5, 1.7, 3.3, 5.7}};
 
@@ -519,7 +521,10 @@ bool few_rows_fits(int mode, int max_rows, int E, int N, int K, int epi, bool b_
   // experts.  Their loads scatter, so a launch whose tiles fill a round, or two, just so may take one more: rounds are
   // an expectation over the tile counts.  Of 840 GEMMs timed in both forms (28 widths and numbers of experts, 32 to 700
   // rows each, means over three loads) the rule takes one that is over 4 % slower in 45, most of them by staying with the
-  // 256-row tiles; rounding an expected count up did so in 57 and was up to 27 % slower than the 256-row tiles.
+  // 256-row tiles; rounding an expected count up did so in 57 and was up to 27 % slower than the 256-row tiles.  With
+  // fragments read ahead and sums that start apart, both only here, the prices stayed: of 347 GEMMs (10 widths, 60 to 600
+  // rows each, both weight layouts) 13 are over 4 % slower, 8 of them by staying with the 256-row tiles (20 % at most) and 5
+  // [E, K, N] or short ones by leaving them (30 % at most: 61 rows of 4 of 3072 / 11008, FFN2, 73 cut along K and 95 here).
   // The weights, once, from HBM at 5.5 TB/s overlap with the steps, but not fully.
   const double used = E < max_rows ? E : max_rows, kt = K / kBK, weights = 2.0 * used * N * K / 5.5e6;
   const TileCount mt[2] = {m_tiles(max_rows, E, 64), m_tiles(max_rows, E, 128)};

@@ -24,9 +24,13 @@ __device__ __forceinline__ float erf_of_twice(float h) {
 
 // erf-form GELU of v = 2 h: h + |h| erf(|v| / sqrt2).  The caller has h for the price of v: half of a sum is one fused
 // multiply-add with half of the other addend.  Measured in fp32 against the exact function over all fp16 values: within
-// 3.4e-6 and within 4e-6 |v| (v * Phi(v) by the polynomial of degree 17: 5.5e-5 and 1.3e-5; below |v| = 0.1 that one
-// had 4e-6 |v| too).  NaN for -inf, as the exact form's -inf * 0.  Nine full-rate instructions, twelve before; the FFN1
-// epilogue applies it to 256 values per lane and tile and is bound by this arithmetic.
+// 3.4e-6 and within 4e-6 |v|.  v * Phi(v) by the polynomial of degree 17 had 5.9e-5 up to |v| of 8, 6.9e-6 |v| beyond its
+// clamp and 1.1e-5 |v| at most; the largest error over |v| of either, that one and this, by |v|:
+//   to 1e-3 0.9e-7 and 2.4e-7, to 0.01 4e-7 and 1.0e-6, to 0.03 1.2e-6 and 2.3e-6, to 0.1 3.8e-6 and 3.9e-6, to 1 8.4e-6
+//   and 3.9e-6, to 2 8.4e-6 and 2.1e-6, to 4 9.5e-6 and 1.3e-6, beyond 1.1e-5 and 2e-7
+// So it is the worse one below 0.03, by 2e-4 of the rounding to fp16 that follows, and five times better for pre-activations of
+// variance 1 (root mean square 1.2e-6 for 5.9e-6).  NaN for -inf, as the exact form's -inf * 0.  Nine full-rate
+// instructions, twelve before; the FFN1 epilogue applies it to 256 values per lane and tile and is bound by this arithmetic.
 __device__ __forceinline__ float gelu_erf_of_twice(float h) {
   float g = fmaf(fabsf(h), erf_of_twice(h), h);
   // rounded to fp32 in every kernel: fused with a conversion to fp16 behind it, as the compiler would have it in some of
